@@ -38,6 +38,7 @@ SOURCES = {
     "gemm_i8.hip": [],
     "gemm_h16.hip": [],
     "kv_attention.hip": [],
+    "kv_chunk.hip": [],
     "decode_ops.hip": ["-ffp-contract=off"],
     "quantized.cpp": [],
     "static_workspace.cpp": [],

@@ -239,7 +239,21 @@ struct KvAttention {
     // reduce_group_rotary_kernel - before it attends (kv_attention returns hipErrorInvalidValue for other shapes).
     KvProjected projected = {};
 };
+// Calls of several tokens per slot attend on the matrix cores (kv_chunk.hip) once the streaming kernel would read this
+// many cached rows, counting one per workgroup and position of the caller's context bound. Measured (us, streaming /
+// chunk kernel with its append and merge launches; 32/8 heads x 128, f16 unless named, slots x tokens at context):
+// 1x8 at 2000 (128 Ki rows) 17.6 / 18, 4x16 at 256 (128 Ki) 18.2 / 17; 1x16 at 2000 (256 Ki) 25.8 / 23.3, bf16 24.1 / 24.5,
+// u8 26.5 / 27; 1x64 at 2000 (1 Mi) 72 / 30; 2x500 at 2000 (16 Mi) 1034 / 77, bf16 1097 / 99, u8 1322 / 112.
+constexpr uint64_t kKvChunkMinRows = 192 * 1024;
+bool kv_chunk_supported(const KvAttention& p);
+struct KvChunkGrid {
+    int row_waves;   // 32 query rows each: 4, or 2 where a slot has no more
+    uint64_t units;  // (slot, kv head, 32 * row_waves query rows)
+    uint32_t round;  // positions a workgroup takes per round
+};
+KvChunkGrid kv_chunk_grid(const KvAttention& p);
 struct KvLaunchShape {
+    bool chunk;
     bool streaming;
     int waves;  // per workgroup of the streaming kernel: 4 or 8
     uint32_t splits;

@@ -12,6 +12,7 @@
 //                          writes the output, or (m, l, acc) partials when the context is split
 //      kv_attend_any_kernel  the same for widths / groups the streaming kernel does not cover
 //   2. kv_merge_kernel     combines the partials of the splits
+// Calls of many tokens per slot run on kv_chunk.hip instead (see kv_attention_shape).
 //      (Letting the last split to finish combine them inside the attend kernel was measured: the
 //      device-wide fences it needs cost far more than this second launch.)
 //
@@ -23,194 +24,23 @@
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <type_traits>
 
 #include "decode_math.h"
 #include "et_hip.h"
 #include "kernels.h"
+#include "kv_device.h"
 #include "quantize_halves.h"
 
 namespace et {
 namespace {
 
-constexpr uint32_t kNoBlock = 0xffffffffu;
-constexpr float kLowest = -1.0e30f;  // "no score yet": finite, so that exp2(kLowest - m) = 0 without NaN
-
-// Element types of a slab besides float and __half.
-struct Bf16 {
-    uint16_t bits;
-};
-struct U8 {  // the int8-quantized tier: byte = round(x / scale) + 128, one f32 scale per row and head
-    uint8_t byte;
-};
-
-struct KvArgs {
-    void* k_slab;
-    void* v_slab;
-    float* k_scales;  // [max_tokens, kv_heads], the U8 tier only
-    float* v_scales;
-    const uint32_t* table;
-    const uint32_t* cursors;
-    const uint32_t* advances;
-    const float* q;
-    const float* k;
-    const float* v;
-    float* out;
-    float* partial;
-    unsigned long long* status;
-    uint32_t max_tokens, kv_heads, width, block_size;
-    int32_t block_shift;  // log2(block_size), or -1 when it is not a power of two
-    uint32_t table_stride, active_batch, query_heads, tokens, context_window, window;
-    uint32_t splits, max_context;
-    float scale_log2;  // scale * log2(e)
-    uint8_t* prepared;       // see KvAttention::prepared; null = none, or a quantiser launch follows
-    uint32_t vector_tiles;   // of the prepared activations: ceil(batch / 32)
-    KvProjected projected;   // see KvAttention::projected; shares == null: q, k, v above
-};
-
-struct Span {
-    uint32_t cursor, advance, needed, start;
-    uint32_t code;   // the first check of kv_prepare that fails, 0 = none
-    uint64_t value;  // what that check reports; cursor + advance needs 33 bits
-    bool ok;
-};
-
-// kv_prepare (napi/mod.rs:3588-3609) on device-resident cursors.
-__device__ Span slot_span(const KvArgs& a, uint32_t slot) {
-    Span s;
-    s.cursor = a.cursors[slot];
-    s.advance = a.advances[slot];
-    // The reference adds in usize and cannot wrap; a cursor near 2^32 (an idle slot's -1) must fail
-    // a check here, before any table access, instead of wrapping to a small context.
-    const uint64_t needed = static_cast<uint64_t>(s.cursor) + s.advance;
-    const uint64_t start = a.context_window != 0 && needed > a.context_window ? needed - a.context_window : 0;
-    s.code = 0;
-    s.value = 0;
-    if (s.advance == 0 || s.advance > a.tokens) {
-        s.code = kKvBadAdvance;
-        s.value = s.advance;
-    } else if (needed - start > a.max_tokens) {
-        s.code = kKvOverCapacity;
-        s.value = needed - start;
-    } else if ((needed + a.block_size - 1) / a.block_size > a.table_stride) {
-        s.code = kKvShortTable;
-        s.value = needed;
-    } else if (needed > a.max_context) {  // max_context is 32 bits wide: passing means no wrap below
-        s.code = kKvOverDeclared;
-        s.value = needed;
-    }
-    s.ok = s.code == 0;
-    s.needed = s.ok ? static_cast<uint32_t>(needed) : 0;
-    s.start = s.ok ? static_cast<uint32_t>(start) : 0;
-    return s;
-}
-
-__device__ __forceinline__ uint32_t block_of(const KvArgs& a, uint32_t position) {
-    return a.block_shift >= 0 ? position >> a.block_shift : position / a.block_size;
-}
-__device__ __forceinline__ uint32_t within_block(const KvArgs& a, uint32_t position) {
-    return a.block_shift >= 0 ? position & (a.block_size - 1) : position % a.block_size;
-}
-
-__device__ __forceinline__ void slab_store(float* slab, uint64_t at, float value) { slab[at] = value; }
-__device__ __forceinline__ void slab_store(__half* slab, uint64_t at, float value) {
-    slab[at] = __float2half_rn(value);
-}
-// the value a slab of this type holds after storing `value`
-__device__ __forceinline__ float slab_round(const float*, float value) { return value; }
-__device__ __forceinline__ float slab_round(const __half*, float value) {
-    return __half2float(__float2half_rn(value));
-}
-__device__ __forceinline__ float slab_load(const float* slab, uint64_t at) { return slab[at]; }
-__device__ __forceinline__ float slab_load(const __half* slab, uint64_t at) { return __half2float(slab[at]); }
-// bf16::from_f32 (half 2.7.1): NaN keeps its top bits and gets a quiet bit, else round to nearest even.
-__device__ __forceinline__ uint32_t bf16_bits(float value) {
-    const uint32_t x = __float_as_uint(value);
-    if ((x & 0x7fffffffu) > 0x7f800000u) return (x >> 16) | 0x0040u;
-    return (x + 0x7fffu + ((x >> 16) & 1u)) >> 16;
-}
-__device__ __forceinline__ void slab_store(Bf16* slab, uint64_t at, float value) {
-    slab[at].bits = static_cast<uint16_t>(bf16_bits(value));
-}
-__device__ __forceinline__ float slab_round(const Bf16*, float value) { return __uint_as_float(bf16_bits(value) << 16); }
-__device__ __forceinline__ float slab_load(const Bf16* slab, uint64_t at) {
-    return __uint_as_float(static_cast<uint32_t>(slab[at].bits) << 16);
-}
-// The U8 tier (napi/mod.rs:3397-3437, :3467-3478): scale = max|x| / 127 + 1e-12 over the row of a
-// head, byte = clamp(round(x / scale), +-127) + 128 (halves away from zero), value = (byte - 128) * scale.
-__device__ __forceinline__ float u8_scale(float row_maximum) { return row_maximum / 127.0f + 1e-12f; }
-__device__ __forceinline__ uint32_t u8_byte(float value, float scale) {
-    return static_cast<uint32_t>(fminf(fmaxf(roundf(value / scale), -127.0f), 127.0f) + 128.0f);
-}
-__device__ __forceinline__ float u8_value(uint32_t byte, float scale) {
-    return (static_cast<float>(byte) - 128.0f) * scale;
-}
-
 __global__ void kv_zero_kernel(float* out, uint64_t count, unsigned long long* status, uint32_t slots) {
     const uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i < count) out[i] = 0.f;
     if (i < slots) status[i] = 0;
-}
-
-// The status word of a slot: 0, or code << 56 | value. Written by one wave per slot, which also
-// checks that the rows of the new positions lie inside the pool.
-__device__ void write_slot_status(const KvArgs& a, uint32_t slot, const Span& s, int lane) {
-    uint32_t code = s.code;
-    uint64_t value = s.value;
-    if (s.ok) {
-        uint32_t worst = 0;
-        for (uint32_t token = lane; token < s.advance; token += 64) {
-            const uint32_t position = s.cursor + token;
-            const uint64_t row = static_cast<uint64_t>(a.table[static_cast<uint64_t>(slot) * a.table_stride +
-                                                               block_of(a, position)]) * a.block_size +
-                                 within_block(a, position);
-            if (row >= a.max_tokens) worst = max(worst, static_cast<uint32_t>(min(row, uint64_t{0xffffffffu})));
-        }
-        for (int offset = 32; offset > 0; offset >>= 1) worst = max(worst, __shfl_xor(worst, offset));
-        if (worst != 0) {
-            code = kKvBlockOutside;
-            value = worst;
-        }
-    }
-    if (lane == 0) a.status[slot] = (static_cast<unsigned long long>(code) << 56) | value;
-}
-
-// Positions a query attends to (napi/mod.rs:3481-3483).
-__device__ __forceinline__ void query_range(const KvArgs& a, const Span& s, uint32_t token,
-                                            uint32_t& begin, uint32_t& end) {
-    end = min(s.cursor + token + 1, s.needed);
-    begin = s.start;
-    if (a.window != 0) begin = max(end > a.window ? end - a.window : 0u, s.start);
-    begin = min(begin, end);
-}
-
-template <int CTRL>
-__device__ __forceinline__ float dpp_f32(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
-}
-
-// Sum over the LANES lanes of an aligned group; every lane gets the total.
-template <int LANES>
-__device__ __forceinline__ float group_sum(float v) {
-    if constexpr (LANES >= 2) v += dpp_f32<0xB1>(v);    // quad_perm [1,0,3,2]
-    if constexpr (LANES >= 4) v += dpp_f32<0x4E>(v);    // quad_perm [2,3,0,1]
-    if constexpr (LANES >= 8) v += dpp_f32<0x141>(v);   // row_half_mirror
-    if constexpr (LANES >= 16) v += dpp_f32<0x140>(v);  // row_mirror
-    if constexpr (LANES >= 32) v += __shfl_xor(v, 16);
-    if constexpr (LANES >= 64) v += __shfl_xor(v, 32);
-    return v;
-}
-
-template <int LANES>
-__device__ __forceinline__ float group_max(float v) {
-    if constexpr (LANES >= 2) v = fmaxf(v, dpp_f32<0xB1>(v));
-    if constexpr (LANES >= 4) v = fmaxf(v, dpp_f32<0x4E>(v));
-    if constexpr (LANES >= 8) v = fmaxf(v, dpp_f32<0x141>(v));
-    if constexpr (LANES >= 16) v = fmaxf(v, dpp_f32<0x140>(v));
-    if constexpr (LANES >= 32) v = fmaxf(v, __shfl_xor(v, 16));
-    if constexpr (LANES >= 64) v = fmaxf(v, __shfl_xor(v, 32));
-    return v;
 }
 
 // Sixteen bytes of a slab row as floats.
@@ -951,6 +781,26 @@ uint32_t positions_per_step(const KvAttention& p, int g, int waves) {
 KvLaunchShape kv_attention_shape(const KvAttention& p) {
     KvLaunchShape shape{};
     const int g = streaming_group(p);
+    const uint64_t queries = static_cast<uint64_t>(p.active_batch) * p.query_heads * p.tokens;
+    const uint64_t streamed = static_cast<uint64_t>(p.active_batch) * p.tokens * p.kv_heads *
+                              (g != 0 ? p.query_heads / p.kv_heads / g : 0);
+    if (kv_chunk_supported(p) && streamed * p.max_context >= kKvChunkMinRows) {
+        // One workgroup per compute unit; a split of at least four rounds, or its start and end cost more than
+        // the compute units it brings in.
+        const KvChunkGrid grid = kv_chunk_grid(p);
+        const uint64_t context = p.max_context;
+        uint64_t splits = grid.units == 0 || grid.units >= 256 ? 1 : 256 / grid.units;
+        splits = std::min(splits, (context + 4 * grid.round - 1) / (4 * grid.round));
+        const uint64_t room = static_cast<uint64_t>(kKvTableEntries - 2) * p.block_size;
+        const uint64_t reach = room > 2 * grid.round ? room - grid.round : grid.round;
+        splits = std::max(splits, (context + reach - 1) / reach);
+        shape.chunk = true;
+        shape.waves = 8;
+        shape.splits = static_cast<uint32_t>(splits);
+        shape.workgroups = grid.units * splits;
+        shape.workspace_bytes = splits > 1 ? queries * splits * (p.width + 2) * sizeof(float) : 0;
+        return shape;
+    }
     shape.streaming = g != 0;
     const uint64_t rows = static_cast<uint64_t>(p.active_batch) * p.tokens *
                           (shape.streaming ? p.kv_heads * ((p.query_heads / p.kv_heads) / g) : p.query_heads);
@@ -980,7 +830,6 @@ KvLaunchShape kv_attention_shape(const KvAttention& p) {
     if (splits == 0) splits = 1;
     shape.splits = static_cast<uint32_t>(splits);
     shape.workgroups = rows * splits;
-    const uint64_t queries = static_cast<uint64_t>(p.active_batch) * p.query_heads * p.tokens;
     shape.workspace_bytes = splits > 1 ? queries * splits * (p.width + 2) * sizeof(float) : 0;
     return shape;
 }
@@ -1043,7 +892,9 @@ hipError_t kv_attention(const KvAttention& p, void* workspace, hipStream_t strea
     if (p.active_batch == 0) return finish(hipGetLastError());
 
     hipError_t error;
-    if (shape.streaming) {
+    if (shape.chunk) {
+        error = kv_chunk(p.slab_dtype, a, kv_chunk_grid(p).row_waves, static_cast<uint32_t>(shape.workgroups), stream);
+    } else if (shape.streaming) {
         const int g = streaming_group(p);
         const uint32_t workgroups = static_cast<uint32_t>(shape.workgroups);
         switch (p.slab_dtype) {

@@ -85,6 +85,7 @@ const char* kernel_name(const et_kv_layer& layer, uint64_t query_heads, uint64_t
     if (layer_geometry(layer, &p, &error) != ET_OK || query_geometry(query_heads, tokens, &p, &error) != ET_OK)
         return "";
     const KvLaunchShape shape = kv_attention_shape(p);
+    if (shape.chunk) return shape.splits > 1 ? "kv_append+kv_chunk+kv_merge" : "kv_append+kv_chunk";
     if (shape.streaming) return shape.splits > 1 ? "kv_attend+kv_merge" : "kv_attend";
     return shape.splits > 1 ? "kv_attend_any+kv_merge" : "kv_attend_any";
 }
@@ -210,8 +211,8 @@ int attention_into(const et_kv_layer& layer, const quantized::TensorView& q, con
     const KvLaunchShape shape = kv_attention_shape(p);
     if (projected != nullptr && !shape.streaming)
         return fail(error, ET_ERR_UNSUPPORTED, "kv attention: this geometry's kernel takes q, k and v as tensors");
-    if (shape.streaming) {
-        // the streaming kernel moves 16 bytes per lane
+    if (shape.streaming || shape.chunk) {
+        // these kernels move 16 bytes per lane
         const auto misaligned = [](const void* pointer) { return reinterpret_cast<uintptr_t>(pointer) % 16 != 0; };
         if (misaligned(p.k_slab) || misaligned(p.v_slab))
             return fail(error, ET_ERR_INVALID, "kv attention: slabs must be 16-byte aligned");

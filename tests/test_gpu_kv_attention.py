@@ -193,6 +193,38 @@ def test_long_context_is_split(et, device, dtype):
     compare(again, run_oracle(case, scale))
 
 
+# `bound`: the caller's bound of the context, by which the kernel is chosen and the context split
+@pytest.mark.parametrize("dtype", [np.float16, "bf16", "u8"])
+@pytest.mark.parametrize("width,query_heads,kv_heads,tokens,contexts,advances,windows,bound,split", [
+    (128, 4, 1, 2, [0, 62, 127], [2, 2, 1], (0, 0), 40000, True),     # the fewest tokens; most splits are empty
+    (128, 3, 1, 43, [85, 21, 1], [43, 43, 40], (0, 0), 4000, True),   # 129 query rows: one past a workgroup's
+    (128, 24, 8, 43, [0, 20, 85, 96] * 5, [43, 43, 43, 1] * 5, (0, 0), 200, False),  # the same without splits
+    (128, 8, 8, 32, [96, 300] * 16, [32] * 32, (0, 0), 332, False),   # one query head per kv head, 32 rows
+    (64, 8, 1, 33, [223, 0, 95], [33, 33, 33], (0, 0), 4000, True),   # width 64: a round is 256 positions
+    (64, 16, 8, 9, [223, 247, 40, 3] * 8, [9] * 32, (0, 0), 256, False),
+    (128, 8, 2, 20, [3000, 2500], [20, 7], (0, 0), 3020, True),       # full splits
+    (128, 8, 2, 70, [400, 333], [70, 70], (0, 37), 3000, True),       # rows of a wave that see disjoint positions
+    (64, 4, 2, 65, [500, 120], [65, 64], (210, 0), 3000, True),
+])
+def test_chunks_on_the_matrix_cores(et, device, dtype, width, query_heads, kv_heads, tokens, contexts, advances, windows,
+                                    bound, split):
+    rng = np.random.default_rng(width + tokens)
+    case = make_case(rng, slots=len(contexts), query_heads=query_heads, kv_heads=kv_heads, width=width, block_size=16,
+                     contexts=contexts, tokens=tokens, advances=advances, dtype=dtype)
+    # rows of q far apart in size: the kernel scales each by a power of two of its own
+    case["q"] *= np.exp2(rng.integers(-8, 3, case["q"].shape[:3])).astype(np.float32)[..., None]
+    scale, options = 1.0 / np.sqrt(width), dict(context_window=windows[0], window=windows[1])
+    got = run_gpu(et, device, case, scale, max_context=bound, **options)
+    assert et.kv_attention_kernel(got[3], query_heads, tokens) == "kv_append+kv_chunk" + ("+kv_merge" if split else "")
+    want = run_oracle(case, scale, **options)
+    compare(got, want)
+    # q and the weights enter the matrix cores with 22 bits or more and every sum is f32: an output is a mean of values
+    # of size 1, off by a few 2^-22 of the largest plus what its exponents, |score| * log2(e) <= 64, lose in f32 (2^-19)
+    assert np.abs(got[0] - want[0]).max() <= 1e-5
+    again = run_gpu(et, device, case, scale, max_context=bound, **options)
+    assert np.array_equal(got[0].view(np.uint32), again[0].view(np.uint32))
+
+
 def test_one_workspace_serves_calls_of_any_geometry(et, device):
     workspace = torch.full((64 << 20,), 255, dtype=torch.uint8, device=device)
     rng = np.random.default_rng(11)
