@@ -31,7 +31,6 @@
 #include <algorithm>
 #include <atomic>
 #include <cstdint>
-#include <cstdlib>
 
 #include "et_codecs.h"
 #include "gemv_common.h"
@@ -44,6 +43,7 @@ namespace {
 constexpr int kConsumers = 8;
 constexpr uint32_t kLdsBytes = 160u * 1024u;
 constexpr uint32_t kGroupRows = 16u;    // rows of W per matrix instruction
+constexpr uint32_t kNarrowColumns = 4096u;  // wider rows: gemv_mma_wide_kernel
 // Activations as fixed point: X = rint(x * kLimbRange / max|x|), |X| < 2^22. Adding kLimbMagic to the
 // scaled value makes the float's mantissa the integer X + 0x408080 (the sum lies in [2^23, 2^24), where
 // floats are the integers): one fused multiply-add quantises, rounds to nearest even and offsets.
@@ -52,11 +52,11 @@ constexpr float kLimbMagic = 12582912.0f + 32896.0f;    // 1.5 * 2^23 + 0x8080
 
 constexpr uint32_t kMostGroups = 4u;    // groups of a range: its rows' partial sums wait in LDS for the end
 
-// Per consumer wave: [limb planes of one vector, 544 bytes apart][sums per vector and 32 columns]
-// [units per vector and 256 columns]. Once the A operands are in registers the first part holds the
+// Per consumer wave: [limb planes of one vector, 544 bytes apart][sums and unit per vector and 256 columns]. Once the A operands are in registers the first part holds the
 // wave's partial sums: [group][vector group][lane].
+constexpr uint32_t kSumsFloats = 12u;  // of one (vector, unit): eight sums, the unit, padding to whole float4s
 constexpr uint32_t kLimbPitch = 544u;  // 512 bytes of a limb plane + 32: the three planes start in different banks
-constexpr uint32_t kSumsAt = 2048u, kUnitsAt = 2560u, kWaveScratch = 2624u;
+constexpr uint32_t kSumsAt = 2048u, kWaveScratch = 2048u + 8u * 2u * kSumsFloats * 4u;
 static_assert(3u * kLimbPitch <= kSumsAt && kMostGroups * 2u * 256u <= kSumsAt, "planes and partial sums share the first part");
 struct Control {
     uint32_t landed[8];  // copies of loader w that have landed
@@ -77,18 +77,6 @@ __device__ __forceinline__ float dpp(float v) {
 }
 
 typedef int v4i __attribute__((ext_vector_type(4)));
-
-#ifdef ET_MMA_PROBES
-// timing experiments only: [workgroup][wave][slot] wall-clock stamps (100 MHz)
-__device__ uint64_t mma_stamps[1024 * 16 * 16];
-#define ET_STAMP(slot)                                                                                          \
-    do {                                                                                                        \
-        if (PROBE == 4 && lane_id == 0 && blockIdx.x < 1024)                                                    \
-            mma_stamps[(blockIdx.x * 16 + wave) * 16 + (slot)] = wall_clock64();                                \
-    } while (0)
-#else
-#define ET_STAMP(slot) do {} while (0)
-#endif
 
 __device__ __forceinline__ long pack(uint32_t low, uint32_t high) {
     return static_cast<long>((static_cast<uint64_t>(high) << 32) | low);
@@ -113,15 +101,15 @@ __device__ __forceinline__ void split_quad(int x0, int x1, int x2, int x3, uint3
 //   rp     the unit in the lane's row of the LDS image
 //   q      the lane's K index: which 8 of a block's 32 columns its operand registers hold
 //   a      A operands of the wave's sixteen 32-column blocks, per group of four vectors
-//   sums   f32 sums of the lane's vector over the unit's eight blocks (next vector group: + 64 floats)
-//   units  value of one unit of limb 0 of the lane's vector in this unit (next vector group: + 8 floats)
+//   sums   f32 sums of the lane's vector over the unit's eight blocks, then the value of one unit of limb 0
+//          (next vector group: + sums_step floats)
 // ---------------------------------------------------------------------------
 struct Q4KMma {
     static constexpr uint32_t kUnitBytes = 144u;  // one super-block
     static __device__ __forceinline__ uint32_t chunk(uint32_t q) { return q; }
-    template <int VG, int UNIT>
-    static __device__ __forceinline__ void contract(const uint8_t* rp, uint32_t q, const long (&a)[VG][16],
-                                                    const float* sums, const float* units, float (&total)[VG]) {
+    template <int VG, int UNIT, int BLOCKS>
+    static __device__ __forceinline__ void contract(const uint8_t* rp, uint32_t q, const long (&a)[VG][BLOCKS],
+                                                    const float* sums, uint32_t sums_step, float (&total)[VG]) {
         const uint4 h = *reinterpret_cast<const uint4*>(rp);
         const float d = half_bits_to_float(h.x & 0xffffu), dmin = half_bits_to_float(h.x >> 16);
         // (scale, min) of the eight sub-blocks, a byte each: crates/runtime-cpu/src/quantized.rs:77-86
@@ -157,8 +145,8 @@ struct Q4KMma {
         const float m6 = static_cast<float>((mn[1] >> 16) & 0xffu), m7 = static_cast<float>(mn[1] >> 24);
 #pragma unroll
         for (int g = 0; g < VG; g++) {
-            const float4 s0 = *reinterpret_cast<const float4*>(sums + 64 * g);
-            const float4 s1 = *reinterpret_cast<const float4*>(sums + 64 * g + 4);
+            const float4 s0 = *reinterpret_cast<const float4*>(sums + sums_step * g);
+            const float4 s1 = *reinterpret_cast<const float4*>(sums + sums_step * g + 4);
             float neg = m0 * s0.x;
             neg = fmaf(m1, s0.y, neg);
             neg = fmaf(m2, s0.z, neg);
@@ -170,7 +158,7 @@ struct Q4KMma {
             float f = static_cast<float>(acc[g][0]);
             f = fmaf(256.0f, static_cast<float>(acc[g][1]), f);
             f = fmaf(65536.0f, static_cast<float>(acc[g][2]), f);
-            total[g] += d * (units[8 * g] * f) - dmin * neg;
+            total[g] += d * (sums[sums_step * g + 8] * f) - dmin * neg;
         }
     }
 };
@@ -183,16 +171,16 @@ struct Q4KMma {
 struct Q40Mma {
     static constexpr uint32_t kUnitBytes = 144u;  // eight blocks of 18 bytes
     static __device__ __forceinline__ uint32_t chunk(uint32_t q) { return ((q & 1u) << 1) | (q >> 1); }
-    template <int VG, int UNIT>
-    static __device__ __forceinline__ void contract(const uint8_t* rp, uint32_t q, const long (&a)[VG][16],
-                                                    const float* sums, const float* units, float (&total)[VG]) {
+    template <int VG, int UNIT, int BLOCKS>
+    static __device__ __forceinline__ void contract(const uint8_t* rp, uint32_t q, const long (&a)[VG][BLOCKS],
+                                                    const float* sums, uint32_t sums_step, float (&total)[VG]) {
         const uint32_t half = q >> 1, shift = (q & 1u) * 4u;
         float pos[VG], corr[VG], s[VG][8];
 #pragma unroll
         for (int g = 0; g < VG; g++) {
             pos[g] = corr[g] = 0.f;
-            const float4 s0 = *reinterpret_cast<const float4*>(sums + 64 * g);
-            const float4 s1 = *reinterpret_cast<const float4*>(sums + 64 * g + 4);
+            const float4 s0 = *reinterpret_cast<const float4*>(sums + sums_step * g);
+            const float4 s1 = *reinterpret_cast<const float4*>(sums + sums_step * g + 4);
             s[g][0] = s0.x, s[g][1] = s0.y, s[g][2] = s0.z, s[g][3] = s0.w;
             s[g][4] = s1.x, s[g][5] = s1.y, s[g][6] = s1.z, s[g][7] = s1.w;
         }
@@ -222,7 +210,7 @@ struct Q40Mma {
             }
         }
 #pragma unroll
-        for (int g = 0; g < VG; g++) total[g] += units[8 * g] * pos[g] - 8.0f * corr[g];
+        for (int g = 0; g < VG; g++) total[g] += sums[sums_step * g + 8] * pos[g] - 8.0f * corr[g];
     }
 };
 
@@ -231,9 +219,9 @@ struct Q40Mma {
 struct Q5KMma {
     static constexpr uint32_t kUnitBytes = 176u;
     static __device__ __forceinline__ uint32_t chunk(uint32_t q) { return q; }
-    template <int VG, int UNIT>
-    static __device__ __forceinline__ void contract(const uint8_t* rp, uint32_t q, const long (&a)[VG][16],
-                                                    const float* sums, const float* units, float (&total)[VG]) {
+    template <int VG, int UNIT, int BLOCKS>
+    static __device__ __forceinline__ void contract(const uint8_t* rp, uint32_t q, const long (&a)[VG][BLOCKS],
+                                                    const float* sums, uint32_t sums_step, float (&total)[VG]) {
         const uint4 h = *reinterpret_cast<const uint4*>(rp);
         const float d = half_bits_to_float(h.x & 0xffffu), dmin = half_bits_to_float(h.x >> 16);
         const uint32_t sc[2] = {h.y & 0x3f3f3f3fu, (h.w & 0x0f0f0f0fu) | ((h.y >> 2) & 0x30303030u)};
@@ -268,8 +256,8 @@ struct Q5KMma {
         const float m6 = static_cast<float>((mn[1] >> 16) & 0xffu), m7 = static_cast<float>(mn[1] >> 24);
 #pragma unroll
         for (int g = 0; g < VG; g++) {
-            const float4 s0 = *reinterpret_cast<const float4*>(sums + 64 * g);
-            const float4 s1 = *reinterpret_cast<const float4*>(sums + 64 * g + 4);
+            const float4 s0 = *reinterpret_cast<const float4*>(sums + sums_step * g);
+            const float4 s1 = *reinterpret_cast<const float4*>(sums + sums_step * g + 4);
             float neg = m0 * s0.x;
             neg = fmaf(m1, s0.y, neg);
             neg = fmaf(m2, s0.z, neg);
@@ -281,7 +269,7 @@ struct Q5KMma {
             float f = static_cast<float>(acc[g][0]);
             f = fmaf(256.0f, static_cast<float>(acc[g][1]), f);
             f = fmaf(65536.0f, static_cast<float>(acc[g][2]), f);
-            total[g] += d * (units[8 * g] * f) - dmin * neg;
+            total[g] += d * (sums[sums_step * g + 8] * f) - dmin * neg;
         }
     }
 };
@@ -291,9 +279,9 @@ struct Q5KMma {
 struct Q80Mma {
     static constexpr uint32_t kUnitBytes = 272u;
     static __device__ __forceinline__ uint32_t chunk(uint32_t q) { return q; }
-    template <int VG, int UNIT>
-    static __device__ __forceinline__ void contract(const uint8_t* rp, uint32_t q, const long (&a)[VG][16],
-                                                    const float*, const float* units, float (&total)[VG]) {
+    template <int VG, int UNIT, int BLOCKS>
+    static __device__ __forceinline__ void contract(const uint8_t* rp, uint32_t q, const long (&a)[VG][BLOCKS],
+                                                    const float* sums, uint32_t sums_step, float (&total)[VG]) {
         float pos[VG];
 #pragma unroll
         for (int g = 0; g < VG; g++) pos[g] = 0.f;
@@ -321,11 +309,11 @@ struct Q80Mma {
             }
         }
 #pragma unroll
-        for (int g = 0; g < VG; g++) total[g] += units[8 * g] * pos[g];
+        for (int g = 0; g < VG; g++) total[g] += sums[sums_step * g + 8] * pos[g];
     }
 };
 
-template <class T, int VG, int LOADERS, int DEPTH, int PROBE = 0>
+template <class T, int VG, int LOADERS, int DEPTH>
 __global__ __launch_bounds__(64 * (kConsumers + LOADERS)) void gemv_mma_kernel(
     const uint8_t* __restrict__ weight, const float* __restrict__ x, uint64_t x_row_stride,
     const float* __restrict__ bias, float* __restrict__ y, uint32_t rows, uint32_t columns, uint32_t rows_per_wg,
@@ -339,7 +327,6 @@ __global__ __launch_bounds__(64 * (kConsumers + LOADERS)) void gemv_mma_kernel(
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t wg_row0 = blockIdx.x * rows_per_wg;
     if (wg_row0 >= rows) return;
-    ET_STAMP(0);
     const uint32_t wg_rows = min(rows_per_wg, rows - wg_row0);
     const uint32_t row_units = columns >> 8;
     const uint32_t row_bytes = row_units * T::kUnitBytes;
@@ -364,7 +351,7 @@ __global__ __launch_bounds__(64 * (kConsumers + LOADERS)) void gemv_mma_kernel(
         uint32_t next = loader;  // number of the wave's next copy
         const auto copy = [&]() {
             // never a copy without a lane: the image ends with bytes of W and padding is shorter than a copy
-            if (PROBE != 2 && PROBE != 3 && column < row_bytes && from < end)
+            if (column < row_bytes && from < end)
                 // streamed once: non-temporal (aux bit 1), the caches keep nothing of it
                 __builtin_amdgcn_global_load_lds(reinterpret_cast<const uint4*>(source + from),
                                                  reinterpret_cast<uint4*>(lds + next * 1024u), 16, 0, 2);
@@ -380,24 +367,19 @@ __global__ __launch_bounds__(64 * (kConsumers + LOADERS)) void gemv_mma_kernel(
         // loads: issued ahead of it they delay those loads, and with them everything else.
         // (measured: issued ahead of the barrier, 0.9 to 1.5 us per launch slower)
         __syncthreads();
-        ET_STAMP(1);
         const uint32_t head = min(mine, static_cast<uint32_t>(DEPTH));
         for (uint32_t i = 0; i < head; i++) copy();
-        ET_STAMP(2);
         uint32_t landed = 0;
         for (uint32_t i = head; i < mine; i++) {  // only with DEPTH copies in flight
             // the oldest copy in flight has landed: say so, then take its place in the queue
             __builtin_amdgcn_s_waitcnt(vmcnt_only(DEPTH - 1));
             lds_store_unseen(landed_address, ++landed);
-            if (landed == 1u) ET_STAMP(3);
             copy();
         }
-        ET_STAMP(4);
         for (uint32_t left = head; left > 0u; left--) {
             wait_copies_in_flight(left - 1u);
             lds_store_unseen(landed_address, ++landed);
         }
-        ET_STAMP(5);
         return;
     }
 
@@ -406,8 +388,7 @@ __global__ __launch_bounds__(64 * (kConsumers + LOADERS)) void gemv_mma_kernel(
     const uint32_t first_unit = 2u * wave;  // the wave's columns: units first_unit, first_unit + 1
     const uint32_t my_units = row_units > first_unit ? min(2u, row_units - first_unit) : 0u;
     uint8_t* scratch = lds + kScratchAt + wave * kWaveScratch;
-    float* sums = reinterpret_cast<float*>(scratch + kSumsAt);    // [vector][block of the slice]
-    float* units = reinterpret_cast<float*>(scratch + kUnitsAt);  // [vector][unit of the slice]
+    float* sums = reinterpret_cast<float*>(scratch + kSumsAt);    // [vector][unit of the slice][kSumsFloats]
 
     // Activation loads first: nothing of the consumers' may queue behind a copy. Lane j holds columns
     // 8j .. 8j+7 of the slice: chunk j % 4 of block j / 4.
@@ -426,7 +407,6 @@ __global__ __launch_bounds__(64 * (kConsumers + LOADERS)) void gemv_mma_kernel(
     }
     if (threadIdx.x < 16) reinterpret_cast<uint32_t*>(control)[threadIdx.x] = 0u;
     __syncthreads();  // the only barrier: the counters are zero before anybody counts
-    ET_STAMP(1);
 
     // 23-bit fixed point per vector and 256-column unit, X = rint(x * kLimbRange / max|x|), in three
     // balanced signed-byte limbs; the limbs go through the wave's scratch into the lanes that hold
@@ -465,8 +445,9 @@ __global__ __launch_bounds__(64 * (kConsumers + LOADERS)) void gemv_mma_kernel(
 #pragma unroll
         for (int k = 0; k < 3; k++)
             *reinterpret_cast<uint2*>(scratch + k * kLimbPitch + lane_id * 8u) = make_uint2(low[k], high[k]);
-        if ((lane_id & 3u) == 0u) sums[v * 16 + (lane_id >> 2)] = total;
-        if ((lane_id & 31u) == 0u) units[v * 2 + (lane_id >> 5)] = unit;
+        float* of_unit = sums + (2u * v + (lane_id >> 5)) * kSumsFloats;
+        if ((lane_id & 3u) == 0u) of_unit[(lane_id & 31u) >> 2] = total;
+        if ((lane_id & 31u) == 0u) of_unit[8] = unit;
         asm volatile("" ::: "memory");  // LDS serves a wave in order: written above, read below
         if (((lane_id & 15u) >> 2) == static_cast<uint32_t>(v & 3) && (lane_id & 3u) != 3u) {
             const uint8_t* plane = scratch + (lane_id & 3u) * kLimbPitch + T::chunk(lane_id >> 4) * 8u;
@@ -478,7 +459,6 @@ __global__ __launch_bounds__(64 * (kConsumers + LOADERS)) void gemv_mma_kernel(
         }
     }
     asm volatile("" ::: "memory");
-    ET_STAMP(2);
 
     const uint32_t n = lane_id & 15u, q = lane_id >> 4;
     const uint32_t groups = (wg_rows + kGroupRows - 1u) / kGroupRows;
@@ -486,21 +466,18 @@ __global__ __launch_bounds__(64 * (kConsumers + LOADERS)) void gemv_mma_kernel(
     for (uint32_t group = 0; group < groups; group++) {
         const uint32_t last_row = min(group * kGroupRows + kGroupRows, wg_rows) - 1u;
         const bool landed = await_copies_in_turn<LOADERS>(control->landed, lane_id, (last_row * pitch + row_bytes + 1023u) >> 10, patience);
-        ET_STAMP(3 + 3 * group);
         float total[VG];
 #pragma unroll
         for (int g = 0; g < VG; g++) total[g] = 0.f;
-        if (PROBE != 1 && PROBE != 3 && landed && my_units != 0u) {
+        if (landed && my_units != 0u) {
             // rows past the end of the range read its last row again and are not stored
             const uint8_t* rp = lds + min(group * kGroupRows + n, wg_rows - 1u) * pitch + first_unit * T::kUnitBytes;
-            if (my_units > 1u) {  // both in one block: the second unit's LDS reads overtake the first's arithmetic
-                T::template contract<VG, 0>(rp, q, a, sums + q * 16u, units + q * 2u, total);
-                T::template contract<VG, 1>(rp + T::kUnitBytes, q, a, sums + q * 16u + 8u, units + q * 2u + 1u, total);
-            } else {
-                T::template contract<VG, 0>(rp, q, a, sums + q * 16u, units + q * 2u, total);
-            }
+            const float* of_vector = sums + 2u * q * kSumsFloats;
+            constexpr uint32_t kStep = 4u * 2u * kSumsFloats;  // to the next vector group
+            T::template contract<VG, 0>(rp, q, a, of_vector, kStep, total);
+            // in one block with the first: the second unit's LDS reads overtake the first's arithmetic
+            if (my_units > 1u) T::template contract<VG, 1>(rp + T::kUnitBytes, q, a, of_vector + kSumsFloats, kStep, total);
         }
-        ET_STAMP(4 + 3 * group);
 #pragma unroll
         for (int g = 0; g < VG; g++) partial[(group * VG + g) * 64u + lane_id] = total[g];
     }
@@ -508,7 +485,6 @@ __global__ __launch_bounds__(64 * (kConsumers + LOADERS)) void gemv_mma_kernel(
     // pair in wave order (the same bits on every run) and stores sixteen rows of four vectors.
     const uint32_t summed_address = lds_address(&control->summed);
     lds_arrive(summed_address, lane_id == 0);
-    ET_STAMP(15);
     if (!lds_await(summed_address, kConsumers, patience)) return;
     for (uint32_t pair = wave; pair < groups * VG; pair += kConsumers) {
         const uint32_t group = pair / VG, g = pair - group * VG;
@@ -522,92 +498,375 @@ __global__ __launch_bounds__(64 * (kConsumers + LOADERS)) void gemv_mma_kernel(
             y[static_cast<uint64_t>(vector) * rows + wg_row0 + row] = value;
         }
     }
-    ET_STAMP(14);
 }
 
-// Rows of a workgroup's range: a two-hundred-fifty-sixth of the matrix when its image fits LDS (and
-// its groups the partial sums' slots); else the matrix is cut into the fewest rounds of 256 ranges that do.
-uint32_t range_rows(uint32_t rows, uint32_t row_bytes) {
-    const uint32_t pitch = image_pitch(row_bytes);
-    const uint32_t most = std::min((kScratchAt - row_bytes) / pitch + 1u, kMostGroups * kGroupRows);
+// ---------------------------------------------------------------------------
+// Rows wider than 4096 columns. The A operands of a whole row no longer fit the consumers' registers, and a workgroup
+// holds few rows (sixteen of 14336 columns fill LDS), so that quantising the activations once per workgroup would cost
+// more than everything else: gemv_mma_prepare_kernel does it once per call and leaves A operands in the order of the
+// lanes that take them. The row is then walked in SLICES of eight 256-column units, one per consumer wave, whose operands
+// arrive from L2 a slice ahead; one or two groups of sixteen rows are contracted and their sums stay in registers. The
+// image of W lies slice after slice - [slice][row][slice bytes, padded to an odd number of 16-byte pieces so that
+// sixteen rows at one column offset spread over the banks] - and lands in that order, so the first slices are
+// contracted while the last ones are still in flight.
+// Activations are 24-bit fixed point per vector and unit (the launches of gemv_limb.hip that this replaces hold 24 bits
+// too): X = rint(x * 127 * 2^16 / max|x|), limbs in [-128, 127].
+// ---------------------------------------------------------------------------
+constexpr uint32_t kSliceUnits = kConsumers;
+constexpr int kWideGroups = 2;
+// Per consumer wave: the sums of its units, [slice][vector][kSumsFloats], and at the end its partial sums,
+// [group][vector group][lane]. The image ends below the waves' scratch.
+constexpr uint32_t kWidePartials = kWideGroups * 2u * 256u;
+__host__ __device__ constexpr uint32_t wide_scratch(uint32_t row_units, uint32_t vectors) {
+    const uint32_t sums = (row_units + kSliceUnits - 1u) / kSliceUnits * vectors * kSumsFloats * 4u;
+    return sums > kWidePartials ? sums : kWidePartials;
+}
+constexpr float kWideRange = 8323072.0f;  // 127 * 2^16
+
+// One (unit, vector) of the prepared activations: the three rows of the A operand that are the vector's,
+// [block pair][limb][K index][16 bytes], then the f32 sums of the unit's eight blocks and the unit of limb 0. Nothing is
+// kept for the zero rows and absent vectors: every workgroup reads all of this from L2.
+constexpr uint32_t kWideRecordSumsAt = 768u, kWideRecord = 768u + kSumsFloats * 4u;
+
+__host__ __device__ constexpr uint32_t slice_pitch(uint32_t slice_bytes) { return slice_bytes + (slice_bytes / 16u % 2u == 0 ? 16u : 0u); }
+
+// Limb k of four 24-bit values X + 0x808080 into one dword each, as split_quad.
+__device__ __forceinline__ void split_quad_24(int x0, int x1, int x2, int x3, uint32_t (&limb)[3]) {
+    const uint32_t a = __builtin_amdgcn_perm(x1, x0, 0x05010400u), b = __builtin_amdgcn_perm(x3, x2, 0x05010400u);
+    const uint32_t c = __builtin_amdgcn_perm(x1, x0, 0x0c0c0602u), d = __builtin_amdgcn_perm(x3, x2, 0x0c0c0602u);
+    limb[0] = __builtin_amdgcn_perm(b, a, 0x05040100u) ^ 0x80808080u;
+    limb[1] = __builtin_amdgcn_perm(b, a, 0x07060302u) ^ 0x80808080u;
+    limb[2] = __builtin_amdgcn_perm(d, c, 0x05040100u) ^ 0x80808080u;
+}
+
+// A wave per (unit, vector).
+template <class T>
+__global__ __launch_bounds__(64) void gemv_mma_prepare_kernel(const float* __restrict__ x, uint64_t x_row_stride,
+                                                              uint8_t* __restrict__ prepared) {
+    __shared__ uint32_t planes[3][64];
+    const uint32_t unit = blockIdx.x, v = blockIdx.y, lane_id = threadIdx.x;
+    uint8_t* out = prepared + (static_cast<uint64_t>(unit) * gridDim.y + v) * kWideRecord;
+    const float4 f = *reinterpret_cast<const float4*>(x + v * x_row_stride + unit * 256u + lane_id * 4u);
+    float amax = fmaxf(fmaxf(fmaxf(fabsf(f.x), fabsf(f.y)), fabsf(f.z)), fabsf(f.w));
+    float sum = (f.x + f.y) + (f.z + f.w);
+    sum += dpp<0xB1>(sum);
+    sum += dpp<0x4E>(sum);
+    sum += dpp<0x141>(sum);  // eight lanes: the block's 32 columns
+    amax = fmaxf(amax, dpp<0xB1>(amax));
+    amax = fmaxf(amax, dpp<0x4E>(amax));
+    amax = fmaxf(amax, dpp<0x141>(amax));
+    amax = fmaxf(amax, dpp<0x140>(amax));
+    amax = fmaxf(amax, __shfl_xor(amax, 16));
+    amax = fmaxf(amax, __shfl_xor(amax, 32));
+    const bool nonzero = amax >= 1e-30f;
+    const float inv = nonzero ? kWideRange / amax : 0.f;
+    // to nearest even: a rounding with a bias would meet the mean of W's quants, which is not zero
+    const auto fixed = [&](float value) { return static_cast<int>(rintf(value * inv)) + 0x808080; };
+    uint32_t limb[3];
+    split_quad_24(fixed(f.x), fixed(f.y), fixed(f.z), fixed(f.w), limb);
+#pragma unroll
+    for (int k = 0; k < 3; k++) planes[k][lane_id] = limb[k];
+    float* sums = reinterpret_cast<float*>(out + kWideRecordSumsAt);
+    if ((lane_id & 7u) == 0u) sums[lane_id >> 3] = sum;
+    if (lane_id == 0u) sums[8] = nonzero ? amax * (1.0f / kWideRange) : 0.f;
+    __syncthreads();
+    if (lane_id < 48u) {  // lane: block pair, limb k, K index q
+        const uint32_t pair = lane_id / 12u, k = lane_id % 12u >> 2, q = lane_id & 3u;
+        const uint32_t* plane = planes[k] + pair * 16u + T::chunk(q) * 2u;  // block 2 pair; the next one 8 words on
+        *reinterpret_cast<uint4*>(out + lane_id * 16u) = make_uint4(plane[0], plane[1], plane[8], plane[9]);
+    }
+}
+
+template <class T, int VG, int LOADERS, int DEPTH, int AHEAD>
+__global__ __launch_bounds__(64 * (kConsumers + LOADERS)) void gemv_mma_wide_kernel(
+    const uint8_t* __restrict__ weight, const uint8_t* __restrict__ prepared, const float* __restrict__ bias,
+    float* __restrict__ y, uint32_t rows, uint32_t columns, uint32_t rows_per_wg, uint32_t vectors, uint32_t spin_limit,
+    uint32_t* timeouts) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    static_assert(DEPTH >= 1 && DEPTH <= 8 && LOADERS >= 1 && LOADERS <= 8, "wait_copies_in_flight counts to seven");
+    Control* control = reinterpret_cast<Control*>(lds + kControlAt);
+
+    const uint32_t lane_id = threadIdx.x & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t wg_row0 = blockIdx.x * rows_per_wg;
+    if (wg_row0 >= rows) return;
+    const uint32_t wg_rows = min(rows_per_wg, rows - wg_row0);
+    const uint32_t row_units = columns >> 8, row_bytes = row_units * T::kUnitBytes;
+    // whole slices, then one of the remaining units (its rows closer together)
+    constexpr uint32_t kSliceBytes = kSliceUnits * T::kUnitBytes, kPitch = slice_pitch(kSliceBytes);
+    const uint32_t whole = row_units / kSliceUnits, rest_units = row_units % kSliceUnits;
+    const uint32_t rest_bytes = rest_units * T::kUnitBytes, rest_pitch = slice_pitch(rest_bytes);
+    const uint32_t slices = whole + (rest_units != 0u ? 1u : 0u);
+    const uint32_t rest_at = whole * wg_rows * kPitch;
+
+    if (wave >= static_cast<uint32_t>(kConsumers)) {
+        // ---- loaders: 1 KiB copies in turn, front to back over the image ------------------------
+        const uint32_t loader = wave - kConsumers;
+        // the image ends with the last byte of the last row of the last slice
+        const uint32_t image_bytes = rest_units != 0u ? rest_at + (wg_rows - 1u) * rest_pitch + rest_bytes
+                                                      : rest_at - kPitch + kSliceBytes;
+        const uint32_t copies = (image_bytes + 1023u) >> 10;
+        const uint32_t mine = copies > loader ? (copies - loader + LOADERS - 1u) / LOADERS : 0u;
+        const uint8_t* source = weight + static_cast<uint64_t>(wg_row0) * row_bytes;
+        const uint32_t landed_address = lds_address(&control->landed[loader]);
+        // where this lane's 16 bytes of the wave's next copy lie: image byte `at`, in a whole slice byte `column` of
+        // its row (a step at a time: two divisions per copy kept the loaders from filling their queues)
+        constexpr uint32_t kStep = LOADERS * 1024u, kStepRows = kStep / kPitch, kStepColumns = kStep % kPitch;
+        uint32_t next = loader, at = loader * 1024u + lane_id * 16u;
+        uint32_t row = at / kPitch, column = at % kPitch, slice = row / wg_rows;
+        row -= slice * wg_rows;
+        const auto copy = [&]() {
+            const uint8_t* from = source + row * row_bytes + slice * kSliceBytes + column;
+            bool live = column < kSliceBytes && at < image_bytes;
+            if (at >= rest_at) {
+                const uint32_t line = (at - rest_at) / rest_pitch, byte = (at - rest_at) - line * rest_pitch;
+                from = source + line * row_bytes + whole * kSliceBytes + byte;
+                live = byte < rest_bytes && at < image_bytes;
+            }
+            // padding is shorter than a copy and the image ends with bytes of W: never a copy without a lane
+            if (live)
+                // streamed once: non-temporal (aux bit 1), the caches keep nothing of it
+                __builtin_amdgcn_global_load_lds(reinterpret_cast<const uint4*>(from), reinterpret_cast<uint4*>(lds + next * 1024u),
+                                                 16, 0, 2);
+            next += LOADERS;
+            at += kStep;
+            column += kStepColumns;
+            row += kStepRows;
+            if (column >= kPitch) {
+                column -= kPitch;
+                row++;
+            }
+            while (row >= wg_rows) {
+                row -= wg_rows;
+                slice++;
+            }
+        };
+        __syncthreads();  // the consumers' first operand loads go ahead of the copies
+        const uint32_t head = min(mine, static_cast<uint32_t>(DEPTH));
+        for (uint32_t i = 0; i < head; i++) copy();
+        uint32_t landed = 0;
+        for (uint32_t i = head; i < mine; i++) {  // only with DEPTH copies in flight
+            __builtin_amdgcn_s_waitcnt(vmcnt_only(DEPTH - 1));
+            lds_store_unseen(landed_address, ++landed);
+            copy();
+        }
+        for (uint32_t left = head; left > 0u; left--) {
+            wait_copies_in_flight(left - 1u);
+            lds_store_unseen(landed_address, ++landed);
+        }
+        return;
+    }
+
+    // ---- consumers --------------------------------------------------------------------------------
+    Patience patience{spin_limit, timeouts};
+    const uint32_t n = lane_id & 15u, q = lane_id >> 4;
+    const uint32_t scratch_bytes = wide_scratch(row_units, vectors);
+    uint8_t* scratch = lds + kControlAt - (kConsumers - wave) * scratch_bytes;
+    const uint8_t* my_units = prepared + static_cast<uint64_t>(wave) * vectors * kWideRecord;
+    const uint64_t slice_stride = static_cast<uint64_t>(kSliceUnits) * vectors * kWideRecord;
+    // the wave's own slices: the row's last slice may have no unit for it
+    const uint32_t my_slices = (row_units + kSliceUnits - 1u - wave) / kSliceUnits;
+    union Operands {
+        uint4 raw[VG][4];
+        long a[VG][8];
+    };
+    const auto load = [&](Operands& operands, uint32_t slice) {  // as A operand: row n = 4 * vector + limb
+#pragma unroll
+        for (int g = 0; g < VG; g++) {
+            const uint32_t vector = 4u * g + (n >> 2);
+            const uint8_t* from = my_units + slice * slice_stride + vector * kWideRecord + ((n & 3u) * 4u + q) * 16u;
+#pragma unroll
+            for (int p = 0; p < 4; p++) {
+                operands.raw[g][p] = make_uint4(0u, 0u, 0u, 0u);
+                if (vector < vectors && (n & 3u) != 3u) operands.raw[g][p] = *reinterpret_cast<const uint4*>(from + p * 192);
+            }
+        }
+    };
+    // AHEAD slices of operands are in flight while one is contracted: an L2 read takes longer than a slice
+    Operands operands[AHEAD + 1];
+#pragma unroll
+    for (int i = 0; i < AHEAD; i++)
+        if (static_cast<uint32_t>(i) < my_slices) load(operands[i], i);
+    float* sums = reinterpret_cast<float*>(scratch);
+    for (uint32_t i = lane_id; i < my_slices * vectors * 3u; i += 64u) {
+        const uint32_t record = i / 3u, slice = record / vectors, vector = record - slice * vectors;
+        *reinterpret_cast<float4*>(sums + 4u * i) = *reinterpret_cast<const float4*>(
+            my_units + slice * slice_stride + vector * kWideRecord + kWideRecordSumsAt + (i - 3u * record) * 16u);
+    }
+    if (threadIdx.x < 16) reinterpret_cast<uint32_t*>(control)[threadIdx.x] = 0u;
+    __syncthreads();  // the only barrier: the counters are zero before anybody counts
+
+    const uint32_t groups = (wg_rows + kGroupRows - 1u) / kGroupRows;
+    const float* of_result = sums + min(q, vectors - 1u) * kSumsFloats;  // result rows past `vectors` are not stored
+    const uint32_t sums_step = (min(q + 4u, vectors - 1u) - min(q, vectors - 1u)) * kSumsFloats;
+    float total[kWideGroups][VG];
+#pragma unroll
+    for (int i = 0; i < kWideGroups; i++)
+#pragma unroll
+        for (int g = 0; g < VG; g++) total[i][g] = 0.f;
+    for (uint32_t first = 0; first < my_slices; first += AHEAD + 1) {
+#pragma unroll
+        for (int i = 0; i <= AHEAD; i++) {  // unrolled: operand sets change their roles, not their registers
+            const uint32_t slice = first + i;
+            if (slice >= my_slices) break;
+            if (slice + AHEAD < my_slices) load(operands[(i + AHEAD) % (AHEAD + 1)], slice + AHEAD);
+            const bool in_rest = slice == whole;
+            const uint32_t pitch = in_rest ? rest_pitch : kPitch, bytes = in_rest ? rest_bytes : kSliceBytes;
+            const uint32_t slice_at = slice * wg_rows * kPitch;
+#pragma unroll
+            for (int group = 0; group < kWideGroups; group++) {
+                if (static_cast<uint32_t>(group) >= groups) break;
+                const uint32_t last_row = min(group * kGroupRows + kGroupRows, wg_rows) - 1u;
+                if (!await_copies_in_turn<LOADERS>(control->landed, lane_id, (slice_at + last_row * pitch + bytes + 1023u) >> 10, patience))
+                    continue;
+                // rows past the end of the range read its last row again and are not stored
+                const uint8_t* rp = lds + slice_at + min(group * kGroupRows + n, wg_rows - 1u) * pitch + wave * T::kUnitBytes;
+                T::template contract<VG, 0>(rp, q, operands[i].a, of_result + slice * vectors * kSumsFloats, sums_step, total[group]);
+            }
+        }
+    }
+    asm volatile("" ::: "memory");  // the sums are read no more
+    float* partial = reinterpret_cast<float*>(scratch);
+#pragma unroll
+    for (int group = 0; group < kWideGroups; group++)
+#pragma unroll
+        for (int g = 0; g < VG; g++) partial[(group * VG + g) * 64u + lane_id] = total[group][g];
+    // as in gemv_mma_kernel: the eight partial sums of a pair are added in wave order
+    const uint32_t summed_address = lds_address(&control->summed);
+    lds_arrive(summed_address, lane_id == 0);
+    if (!lds_await(summed_address, kConsumers, patience)) return;
+    for (uint32_t pair = wave; pair < groups * VG; pair += kConsumers) {
+        const uint32_t group = pair / VG, g = pair - group * VG;
+        float value = 0.f;
+#pragma unroll
+        for (int w = 0; w < kConsumers; w++)
+            value += reinterpret_cast<const float*>(lds + kControlAt - (kConsumers - w) * scratch_bytes)[pair * 64u + lane_id];
+        const uint32_t vector = 4u * g + q, row = group * kGroupRows + n;
+        if (vector < vectors && row < wg_rows) {
+            if (bias != nullptr) value += bias[wg_row0 + row];
+            y[static_cast<uint64_t>(vector) * rows + wg_row0 + row] = value;
+        }
+    }
+}
+
+// Rows of W whose slices fit a workgroup's LDS.
+uint32_t wide_rows_that_fit(uint64_t columns, uint32_t vectors, uint32_t unit_bytes) {
+    const uint32_t units = static_cast<uint32_t>(columns >> 8), whole = units / kSliceUnits, rest = units % kSliceUnits;
+    const uint32_t scratch = kConsumers * wide_scratch(units, vectors);
+    if (scratch >= kControlAt) return 0;
+    const uint32_t per_row = whole * slice_pitch(kSliceUnits * unit_bytes) + (rest != 0 ? slice_pitch(rest * unit_bytes) : 0u);
+    return std::min((kControlAt - scratch) / per_row, kWideGroups * kGroupRows);
+}
+
+// Rows of a workgroup's range: a two-hundred-fifty-sixth of the matrix when `most` rows (what fits LDS and the
+// partial sums' slots) hold it; else the matrix is cut into the fewest rounds of 256 ranges that do.
+uint32_t range_rows(uint32_t rows, uint32_t most) {
     const uint32_t share = (rows + 255u) / 256u;
     if (share <= most) return share;
     const uint32_t rounds = (share + most - 1u) / most;
     return (rows + 256u * rounds - 1u) / (256u * rounds);
 }
+uint32_t rows_that_fit(uint32_t row_bytes) {
+    return std::min((kScratchAt - row_bytes) / image_pitch(row_bytes) + 1u, kMostGroups * kGroupRows);
+}
 
-template <class T, int VG, int LOADERS, int DEPTH, int PROBE = 0>
-hipError_t launch(const uint8_t* weight, const float* x, uint64_t x_row_stride, const float* bias, float* y,
-                  uint32_t rows, uint32_t columns, uint32_t vectors, hipStream_t stream) {
-    static std::atomic<bool> allowed[64];
+// The whole LDS of a compute unit has to be allowed once per kernel and device.
+template <typename Kernel>
+hipError_t allow_lds(Kernel kernel, std::atomic<bool> (&allowed)[64]) {
     int device = 0;
     if (hipError_t status = hipGetDevice(&device)) return status;
     if (device < 0 || device >= 64) return hipErrorInvalidDevice;
-    const auto kernel = gemv_mma_kernel<T, VG, LOADERS, DEPTH, PROBE>;
     if (!allowed[device].load(std::memory_order_acquire)) {
         if (hipError_t status = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                                     hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes))
             return status;
         allowed[device].store(true, std::memory_order_release);
     }
+    return hipSuccess;
+}
+
+template <class T, int VG, int LOADERS, int DEPTH>
+hipError_t launch(const uint8_t* weight, const float* x, uint64_t x_row_stride, const float* bias, float* y,
+                  uint32_t rows, uint32_t columns, uint32_t vectors, hipStream_t stream) {
+    static std::atomic<bool> allowed[64];
+    const auto kernel = gemv_mma_kernel<T, VG, LOADERS, DEPTH>;
+    if (hipError_t status = allow_lds(kernel, allowed)) return status;
     HandoverState handover;
     if (hipError_t status = handover_state(&handover)) return status;
-    const uint32_t rows_per_wg = range_rows(rows, (columns >> 8) * T::kUnitBytes);
+    const uint32_t rows_per_wg = range_rows(rows, rows_that_fit((columns >> 8) * T::kUnitBytes));
     const uint32_t grid = (rows + rows_per_wg - 1u) / rows_per_wg;
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * (kConsumers + LOADERS)), kLdsBytes, stream, weight, x, x_row_stride,
                        bias, y, rows, columns, rows_per_wg, vectors, handover.limit, handover.timeouts);
     return hipGetLastError();
 }
 
+template <class T, int VG, int LOADERS, int DEPTH, int AHEAD>
+hipError_t launch_wide(const uint8_t* weight, const float* x, uint64_t x_row_stride, const float* bias, float* y,
+                       uint32_t rows, uint32_t columns, uint32_t vectors, uint8_t* prepared, hipStream_t stream) {
+    static std::atomic<bool> allowed[64];
+    const auto kernel = gemv_mma_wide_kernel<T, VG, LOADERS, DEPTH, AHEAD>;
+    if (hipError_t status = allow_lds(kernel, allowed)) return status;
+    HandoverState handover;
+    if (hipError_t status = handover_state(&handover)) return status;
+    hipLaunchKernelGGL(gemv_mma_prepare_kernel<T>, dim3(columns >> 8, vectors), dim3(64), 0, stream, x, x_row_stride, prepared);
+    if (hipError_t status = hipGetLastError()) return status;
+    const uint32_t rows_per_wg = range_rows(rows, wide_rows_that_fit(columns, vectors, T::kUnitBytes));
+    const uint32_t grid = (rows + rows_per_wg - 1u) / rows_per_wg;
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * (kConsumers + LOADERS)), kLdsBytes, stream, weight, prepared, bias, y,
+                       rows, columns, rows_per_wg, vectors, handover.limit, handover.timeouts);
+    return hipGetLastError();
+}
+
 template <class T>
 hipError_t launch_vectors(const uint8_t* weight, const float* x, uint64_t x_row_stride, const float* bias, float* y,
-                          uint32_t rows, uint32_t columns, uint32_t vectors, hipStream_t stream) {
-#ifdef ET_MMA_PROBES
-    // timing experiments only (never in the product build): ET_HIP_MMA_VARIANT picks a launch shape or a probe
-    static const int variant = [] { const char* v = std::getenv("ET_HIP_MMA_VARIANT"); return v ? std::atoi(v) : 0; }();
-#define ET_V(N, ...) case N: return launch<T, __VA_ARGS__>(weight, x, x_row_stride, bias, y, rows, columns, vectors, stream)
-    if (vectors <= 4) switch (variant) {
-        ET_V(1, 1, 8, 4, 1); ET_V(2, 1, 8, 4, 2); ET_V(3, 1, 8, 5); ET_V(4, 1, 8, 6); ET_V(5, 1, 4, 8); ET_V(6, 1, 8, 8);
-        ET_V(7, 1, 8, 3); ET_V(8, 1, 4, 6); ET_V(9, 1, 8, 4, 3); ET_V(10, 1, 8, 4, 4);
-        default: break;
-    } else switch (variant) {
-        ET_V(1, 2, 4, 8, 1); ET_V(2, 2, 4, 8, 2); ET_V(3, 2, 8, 4); ET_V(4, 2, 8, 5); ET_V(5, 2, 4, 6); ET_V(6, 2, 2, 8);
-        ET_V(9, 2, 4, 8, 3); ET_V(10, 2, 4, 8, 4);
-        default: break;
-    }
-#undef ET_V
-#endif
-    if (vectors <= 4) return launch<T, 1, 8, 4>(weight, x, x_row_stride, bias, y, rows, columns, vectors, stream);
+                          uint32_t rows, uint32_t columns, uint32_t vectors, uint8_t* prepared, hipStream_t stream) {
     // two vector groups keep 64 registers of A operands: twelve waves leave each 168
+    if (columns > kNarrowColumns) {
+        if (prepared == nullptr) return hipErrorInvalidValue;
+        if (vectors <= 4) return launch_wide<T, 1, 8, 4, 2>(weight, x, x_row_stride, bias, y, rows, columns, vectors, prepared, stream);
+        return launch_wide<T, 2, 4, 8, 1>(weight, x, x_row_stride, bias, y, rows, columns, vectors, prepared, stream);
+    }
+    if (vectors <= 4) return launch<T, 1, 8, 4>(weight, x, x_row_stride, bias, y, rows, columns, vectors, stream);
     return launch<T, 2, 4, 8>(weight, x, x_row_stride, bias, y, rows, columns, vectors, stream);
 }
 
 }  // namespace
 
-#ifdef ET_MMA_PROBES
-extern "C" int et_hip_mma_stamps(uint64_t* out, uint64_t count) {
-    return hipMemcpyFromSymbol(out, HIP_SYMBOL(mma_stamps), count * 8);
-}
-#endif
-
 bool gemv_mma_supported(int32_t codec, uint64_t rows, uint64_t columns, uint32_t vectors) {
     if (codec != kQ4_K && codec != kQ4_0 && codec != kQ5_K && codec != kQ8_0) return false;
     if (vectors < 2 || vectors > kGemvMmaMaxVectors) return false;
-    // one image row is at most 16 units; the copies are 16 bytes wide (a unit is a multiple of 16 bytes)
-    if (columns == 0 || columns % 256 != 0 || columns > 4096) return false;
+    // the copies are 16 bytes wide (a unit is a multiple of 16 bytes)
+    if (columns == 0 || columns % 256 != 0) return false;
     // with less than a group of rows to a compute unit most of every matrix instruction is padding
-    return rows >= 256u * 8u && rows <= 0xffffffffull;
+    if (rows < 256u * 8u || rows > 0xffffffffull) return false;
+    if (columns <= kNarrowColumns) return true;
+    // Wider rows, against the launches of gemv_limb.hip (two or three vectors each): Q4_K 4096 x 14336, 2 / 3 / 4 / 5 / 6
+    // vectors 13.8 / 14.6 / 15.6 / 18.6 / 18.9 us (20.4 / 26.0 / 37.1 / 44.6 / 50.2); 3000 x 8192, 4 vectors 10.9 (18.1); Q8_0
+    // 4096 x 14336, whose ranges of eight rows take two rounds of workgroups, 2 / 3 / 6 vectors 23 / 24 / 31 (23 / 30 / 57).
+    // A second round of ranges is worth it from three vectors on where LDS holds less than a group of sixteen rows.
+    // From seven vectors on the batch kernels' plans hold prepared inputs, which callers may share between plans;
+    // taller matrices keep the launches that their plans name (one call of more rounds would still be faster: 14336 x 5120,
+    // 4 vectors 18.2 against 41.4 us).
+    if (vectors > 6u || columns > (1u << 20)) return false;
+    const uint32_t unit_bytes = static_cast<uint32_t>(256 / block_values(codec) * block_bytes(codec));
+    const uint32_t fit = wide_rows_that_fit(columns, vectors, unit_bytes);
+    return rows <= 256u * fit || (vectors > 2u && fit >= 8u && fit < kGroupRows && rows <= 512u * fit);
+}
+
+uint64_t gemv_mma_prepared_bytes(uint64_t columns, uint32_t vectors) {
+    if (columns <= kNarrowColumns) return 0;
+    return (columns >> 8) * vectors * kWideRecord;
 }
 
 hipError_t gemv_mma(int32_t codec, const uint8_t* weight, const float* x, uint64_t x_row_stride, const float* bias,
-                    float* y, uint64_t rows, uint64_t columns, uint32_t vectors, hipStream_t stream) {
+                    float* y, uint64_t rows, uint64_t columns, uint32_t vectors, uint8_t* prepared, hipStream_t stream) {
     const uint32_t n = static_cast<uint32_t>(rows), k = static_cast<uint32_t>(columns);
     if (!gemv_mma_supported(codec, rows, columns, vectors)) return hipErrorInvalidValue;
     switch (codec) {
-        case kQ4_K: return launch_vectors<Q4KMma>(weight, x, x_row_stride, bias, y, n, k, vectors, stream);
-        case kQ5_K: return launch_vectors<Q5KMma>(weight, x, x_row_stride, bias, y, n, k, vectors, stream);
-        case kQ4_0: return launch_vectors<Q40Mma>(weight, x, x_row_stride, bias, y, n, k, vectors, stream);
-        case kQ8_0: return launch_vectors<Q80Mma>(weight, x, x_row_stride, bias, y, n, k, vectors, stream);
+        case kQ4_K: return launch_vectors<Q4KMma>(weight, x, x_row_stride, bias, y, n, k, vectors, prepared, stream);
+        case kQ5_K: return launch_vectors<Q5KMma>(weight, x, x_row_stride, bias, y, n, k, vectors, prepared, stream);
+        case kQ4_0: return launch_vectors<Q40Mma>(weight, x, x_row_stride, bias, y, n, k, vectors, prepared, stream);
+        case kQ8_0: return launch_vectors<Q80Mma>(weight, x, x_row_stride, bias, y, n, k, vectors, prepared, stream);
         default: return hipErrorInvalidValue;
     }
 }

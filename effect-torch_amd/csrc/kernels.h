@@ -50,9 +50,12 @@ hipError_t gemv_limb(int32_t codec, const uint8_t* weight, const float* x, uint6
 // x rows must be 16-byte aligned (x pointer and x_row_stride * 4).
 constexpr uint32_t kGemvMmaMaxVectors = 8;
 bool gemv_mma_supported(int32_t codec, uint64_t rows, uint64_t columns, uint32_t vectors);
+// Rows wider than 4096 columns take quantised activations that a first launch leaves in `prepared`
+// (gemv_mma_prepared_bytes(...) bytes, 16-byte aligned; 0 = not used).
+uint64_t gemv_mma_prepared_bytes(uint64_t columns, uint32_t vectors);
 hipError_t gemv_mma(int32_t codec, const uint8_t* weight, const float* x, uint64_t x_row_stride,
                     const float* bias, float* y, uint64_t rows, uint64_t columns, uint32_t vectors,
-                    hipStream_t stream);
+                    uint8_t* prepared, hipStream_t stream);
 
 // ---- gemv_generic.hip: every codec, any whole number of blocks, vectors <= 4 ----
 constexpr uint32_t kGemvGenericMaxVectors = 4;

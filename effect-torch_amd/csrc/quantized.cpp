@@ -156,6 +156,7 @@ int select_kernel(et_linear_plan* plan, std::string* error) {
             // one pass over W for all the vectors
             plan->kernel = LinearKernel::kGemvMma;
             plan->vectors_per_launch = kGemvMmaMaxVectors;
+            plan->q_offset = take({gemv_mma_prepared_bytes(plan->columns, static_cast<uint32_t>(plan->vectors))});
         } else if (plan->vectors >= kGemmMinVectors && gemm_h16_supported(plan->codec, plan->columns)) {
             plan_matrix_core(LinearKernel::kGemmHalf, 2);
         } else if (plan->vectors >= kGemmMinVectors && gemm_i8_supported(plan->codec, plan->columns)) {
@@ -279,7 +280,9 @@ const char* kernel_name(const et_linear_plan& plan) {
         case LinearKernel::kNone: return "none";
         case LinearKernel::kGemvLimb: return plan.kernel_label.c_str();
         case LinearKernel::kGemvGeneric: return "gemv_generic";
-        case LinearKernel::kGemvMma: return "gemv_mma";
+        case LinearKernel::kGemvMma:
+            return gemv_mma_prepared_bytes(plan.columns, static_cast<uint32_t>(plan.vectors)) != 0 ? "gemv_mma_prepare+gemv_mma_wide"
+                                                                                                  : "gemv_mma";
         case LinearKernel::kGemmI8:
             return plan.k_splits > 1 ? "quantize_act+gemm_i8+reduce" : "quantize_act+gemm_i8";
         case LinearKernel::kGemmLimb:
@@ -740,16 +743,26 @@ int linear_enqueue(const et_linear_plan& plan, const float* x, uint64_t x_row_st
         return ET_OK;
     }
 
-    for (uint64_t v0 = 0; v0 < plan.vectors; v0 += plan.vectors_per_launch) {
+    LinearKernel kernel = plan.kernel;
+    uint32_t per_launch = plan.vectors_per_launch;
+    uint8_t* mma_prepared = nullptr;
+    if (kernel == LinearKernel::kGemvMma) {
+        const uint64_t bytes = gemv_mma_prepared_bytes(plan.columns, static_cast<uint32_t>(plan.vectors));
+        if (bytes != 0 && scratch != nullptr && workspace_bytes >= plan.q_offset + bytes) mma_prepared = scratch + plan.q_offset;
+        if (bytes != 0 && mma_prepared == nullptr) {  // aligned activations need no workspace elsewhere in this family
+            kernel = LinearKernel::kGemvLimb;
+            per_launch = gemv_limb_max_vectors(plan.codec);
+        }
+    }
+    for (uint64_t v0 = 0; v0 < plan.vectors; v0 += per_launch) {
         if (v0 != 0 && cancelled(cancel)) return fail(error, ET_ERR_CANCELLED, "operation aborted");
-        const uint32_t count = static_cast<uint32_t>(
-            plan.vectors - v0 < plan.vectors_per_launch ? plan.vectors - v0 : plan.vectors_per_launch);
+        const uint32_t count = static_cast<uint32_t>(plan.vectors - v0 < per_launch ? plan.vectors - v0 : per_launch);
         const float* xv = x + v0 * x_row_stride;
         float* yv = y + v0 * plan.rows;
         hipError_t status;
-        if (plan.kernel == LinearKernel::kGemvMma)
-            status = gemv_mma(plan.codec, weight, xv, x_row_stride, bias, yv, plan.rows, plan.columns, count, s);
-        else if (plan.kernel == LinearKernel::kGemvLimb && gemv_limb_supported(plan.codec, plan.columns, count))
+        if (kernel == LinearKernel::kGemvMma)
+            status = gemv_mma(plan.codec, weight, xv, x_row_stride, bias, yv, plan.rows, plan.columns, count, mma_prepared, s);
+        else if (kernel == LinearKernel::kGemvLimb && gemv_limb_supported(plan.codec, plan.columns, count))
             status = gemv_limb(plan.codec, weight, xv, x_row_stride, bias, yv, plan.rows, plan.columns,
                                count, s);
         else

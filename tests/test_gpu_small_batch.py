@@ -21,10 +21,10 @@ def planned_kernel(et, codec, rows, columns, vectors, bias=False):
     return et.RawLinear(et.GgmlQuant(codec), rows, columns, vectors, bias).requirements.kernel
 
 
-def check(et, device, codec, rows, columns, vectors, rng, bias=None, x_scale=1.0):
+def check(et, device, codec, rows, columns, vectors, rng, bias=None, x_scale=1.0, kernel="gemv_mma"):
     weight = synth.random_weight(codec, rows, columns, rng)
     x = synth.random_activations(vectors, columns, rng, x_scale)
-    assert planned_kernel(et, codec, rows, columns, vectors, bias is not None) == "gemv_mma"
+    assert planned_kernel(et, codec, rows, columns, vectors, bias is not None) == kernel
     print(f"gemv_mma codec={codec} rows={rows} columns={columns} vectors={vectors}", flush=True)
     abandoned = et.handover_timeouts()
     got = run_linear(et, device, codec, rows, columns, x, weight, bias)
@@ -63,6 +63,32 @@ def test_shapes(et, device, codec, vectors, rows, columns):
     rng = np.random.default_rng(7 * codec + vectors + rows + columns)
     bias = rng.standard_normal(rows).astype(np.float32) if rows % 2 else None
     check(et, device, codec, rows, columns, vectors, rng, bias)
+
+
+@pytest.mark.parametrize("codec", CODECS)
+@pytest.mark.parametrize("vectors,rows,columns", [
+    (2, 2048, 4352),     # seventeen units: a last slice of one
+    (4, 2100, 8192),     # whole slices only; ranges of nine rows, the last of three
+    (5, 4096, 6400),     # sixteen rows per range, a last slice of one unit
+    (6, 4100, 5120),     # ranges of seventeen rows: a group of one; a half slice at the end
+    (3, 4096, 14336),    # the widest configuration: seven slices (Q8_0: two rounds of ranges of eight rows)
+])
+def test_rows_wider_than_4096_columns(et, device, codec, vectors, rows, columns):
+    rng = np.random.default_rng(17 * codec + vectors + rows + columns)
+    bias = rng.standard_normal(rows).astype(np.float32) if rows % 8 else None
+    check(et, device, codec, rows, columns, vectors, rng, bias, kernel="gemv_mma_prepare+gemv_mma_wide")
+
+
+def test_wide_rows_without_a_workspace(et, device):
+    # aligned activations need no workspace in the vector kernels: the call then runs the launches that quantise themselves
+    rows, columns, vectors = 2048, 8192, 5
+    rng = np.random.default_rng(3)
+    weight = synth.random_weight(oracle.Q4_K, rows, columns, rng)
+    x = synth.random_activations(vectors, columns, rng)
+    plan = et.RawLinear(et.GgmlQuant.Q4_K, rows, columns, vectors)
+    y = torch.empty(vectors, rows, device=device)
+    plan.enqueue(to_dev(x, device), to_dev(weight, device), None, y)
+    close(y.cpu().numpy(), oracle.linear_into(oracle.Q4_K, rows, columns, x, weight))
 
 
 @pytest.mark.parametrize("name", ["q4_0_gemv_11008x4096", "q4_k_gemv_14336x4096", "q8_0_gemv_4096x4096"])
