@@ -174,6 +174,28 @@ def test_linear_kats(et, device):
     assert y.tolist() == [[2048.0, 2048.0, 2048.0]]
 
 
+@pytest.mark.parametrize("count", [1, 255, 256, 257, 4096, 4097, 9001])
+@pytest.mark.parametrize("dtype", [torch.int64, torch.uint32])
+def test_embedding_reports_the_lowest_bad_position(et, device, count, dtype):
+    # one workgroup checks 256 positions at a time, sixteen rounds in flight: bad ones at the edges of both
+    rng = np.random.default_rng(count)
+    rows = 40
+    table = synth.random_weight(oracle.Q8_0, rows, 64, rng)
+    ids = rng.integers(0, rows, count)
+    w = to_dev(table, device)
+    out = torch.zeros((count, 64), device=device)
+    plan = et.embedding_requirements(torch.from_numpy(ids).to(device).to(dtype), w, et.GgmlQuant.Q8_0, (rows, 64))
+    et.embedding_into(torch.from_numpy(ids).to(device).to(dtype), w, et.GgmlQuant.Q8_0, out, plan)
+    assert np.array_equal(out.cpu().numpy(), oracle.embedding_into(oracle.Q8_0, rows, 64, ids, table))
+    for position in sorted({0, count // 2, min(255, count - 1), min(4096, count - 1), count - 1}):
+        bad = ids.copy()
+        bad[position:] = rows + 1  # every later one is bad too
+        bad[position] = rows + 2
+        with pytest.raises(et.QuantizedError) as info:
+            et.embedding_into(torch.from_numpy(bad).to(device).to(dtype), w, et.GgmlQuant.Q8_0, out, plan)
+        assert str(info.value) == f"quantized_embedding: index {rows + 2} is outside 0..{rows}"
+
+
 @pytest.mark.parametrize("codec", K_QUANTS)
 @pytest.mark.parametrize("vectors", [1, 3, 4, 5, 16, 17])
 def test_linear_cross_backend_protocol(et, device, codec, vectors):
