@@ -7,11 +7,13 @@ fallback: if the shared object is missing this module raises on import of
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "lib", "libet_hip.so")
 CALIBRATE_LIB_PATH = os.path.join(HERE, "lib", "libet_hip_calibrate.so")
+HOST_CALLS_PATH = os.path.join(HERE, "lib", "et_host_calls.so")
 
 # et_status
 OK, ERR_UNSUPPORTED, ERR_EXECUTION, ERR_CANCELLED, ERR_UNAVAILABLE, ERR_INVALID = range(6)
@@ -239,6 +241,7 @@ CALIBRATE_SIGNATURES = {
 
 _lib = None
 _calibrate_lib = None
+_host_calls = None
 
 
 class NativeLibraryMissing(ImportError):
@@ -260,6 +263,21 @@ def lib() -> ctypes.CDLL:
             fn.argtypes = argtypes
         _lib = handle
     return _lib
+
+
+def host_calls():
+    """The CPython module of ``csrc/host_calls.cpp``: the execute calls from torch tensors without ctypes. Its functions
+    return a negative status, before anything has happened, for arguments that they leave to the ctypes path."""
+    global _host_calls
+    if _host_calls is None:
+        lib()
+        if not os.path.exists(HOST_CALLS_PATH):
+            raise NativeLibraryMissing(f"{HOST_CALLS_PATH} is missing: build it with `python effect-torch_amd/build.py`")
+        spec = importlib.util.spec_from_file_location("et_host_calls", HOST_CALLS_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        _host_calls = module
+    return _host_calls
 
 
 def calibrate_lib() -> ctypes.CDLL:

@@ -1,5 +1,6 @@
 """Builds libet_hip.so (the C-ABI library of include/et_hip.h) and libet_hip_calibrate.so (the
-measurement aids of include/et_hip_calibrate.h) for gfx950 with hipcc.
+measurement aids of include/et_hip_calibrate.h) for gfx950 with hipcc, and et_host_calls.so (the CPython
+module that hands torch tensors to the C ABI) with g++.
 
 Usage: ``python build.py`` from anywhere. The libraries land next to this file
 under ``lib/``; the first is what the tests, the smoke check and the benchmark
@@ -8,9 +9,11 @@ those aids. hipcc cross-compiles, so no GPU is needed to build.
 """
 from __future__ import annotations
 
+import importlib.util
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -20,6 +23,7 @@ LIB_DIR = os.path.join(HERE, "lib")
 OBJ_DIR = os.path.join(HERE, "build")
 LIB_PATH = os.path.join(LIB_DIR, "libet_hip.so")
 CALIBRATE_LIB_PATH = os.path.join(LIB_DIR, "libet_hip_calibrate.so")
+HOST_CALLS_PATH = os.path.join(LIB_DIR, "et_host_calls.so")
 
 # Packed-FP32 instructions are switched off for all device code.
 COMMON = [
@@ -74,12 +78,30 @@ def _compile(item):
     return name, obj, log
 
 
+def _torch_dir() -> str:
+    return importlib.util.find_spec("torch").submodule_search_locations[0]
+
+
+def _compile_host_calls():
+    obj = os.path.join(OBJ_DIR, "host_calls.o")
+    torch_dir = _torch_dir()
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM", "-I", sysconfig.get_paths()["include"],
+           "-I", os.path.join(torch_dir, "include"), "-I", os.path.join(torch_dir, "include", "torch", "csrc", "api", "include"),
+           "-I", "/opt/rocm/include", "-I", INCLUDE, "-c", os.path.join(CSRC, "host_calls.cpp"), "-o", obj]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"g++ failed for host_calls.cpp:\n{proc.stderr}")
+    return obj
+
+
 def build(verbose: bool = False) -> str:
     os.makedirs(LIB_DIR, exist_ok=True)
     os.makedirs(OBJ_DIR, exist_ok=True)
     items = list(SOURCES.items()) + list(CALIBRATE_SOURCES.items())
     with ThreadPoolExecutor(max_workers=8) as pool:
+        host_calls = pool.submit(_compile_host_calls)
         results = list(pool.map(_compile, items))
+        host_obj = host_calls.result()
     for name, _, log in results:
         if verbose and log.strip():
             print(f"[{name}]\n{log}", file=sys.stderr)
@@ -93,6 +115,12 @@ def build(verbose: bool = False) -> str:
         proc = subprocess.run(link, capture_output=True, text=True)
         if proc.returncode != 0:
             raise RuntimeError(f"link failed:\n{proc.stderr}")
+    # torch's libraries are in the process by the time the module is imported; the operators' library lies next to it
+    link = ["g++", "-shared", "-o", HOST_CALLS_PATH, host_obj, "-L", os.path.join(_torch_dir(), "lib"), "-ltorch_python",
+            "-ltorch_cpu", "-lc10", "-lc10_hip", "-L", LIB_DIR, "-let_hip", "-Wl,-rpath,$ORIGIN"]
+    proc = subprocess.run(link, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"link failed:\n{proc.stderr}")
     return LIB_PATH
 
 

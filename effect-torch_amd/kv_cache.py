@@ -14,7 +14,7 @@ from typing import Optional, Sequence
 import torch
 
 from . import _native as N
-from .quantized import CancellationFlag, QuantizedError, _check, _desc, _ref, _stream_handle
+from .quantized import CancellationFlag, QuantizedError, _cancel_address, _check, _desc, _ref, _stream_handle
 
 _SLAB_DTYPES = {torch.float32: N.DTYPE_F32, torch.float16: N.DTYPE_F16, torch.bfloat16: N.DTYPE_BF16,
                 torch.uint8: N.DTYPE_U8}
@@ -106,6 +106,18 @@ def kv_attention_into(layer: KvLayer, q: torch.Tensor, k: torch.Tensor, v: torch
 
     ``prepared_for`` (a :class:`RawLinear` whose activations are the result, one token per slot) and
     ``prepared``: also leaves that plan's prepared input behind (``et_hip_kv_attention_prepared_into``)."""
+    if prepared_for is None and workspace is not None:
+        taken = N.host_calls().kv_attention_into(
+            layer.k_slab, layer.v_slab, layer.k_scales, layer.v_scales, layer.block_table, layer.cursors, layer.advances,
+            layer.block_size, layer.max_context, layer.active_batch, layer.context_window, q, k, v, scale, window or 0,
+            destination, workspace, None if stream is None else _stream_handle(stream), _cancel_address(cancelled))
+        if taken != -1:
+            code, status = taken
+            _check(code)
+            if synchronize:
+                kv_attention_status_check(layer, q.shape[-2], status)
+                return None
+            return status
     struct = layer.struct()
     tokens = q.shape[-2] if q.dim() >= 2 else 0
     heads = q.shape[-3] if q.dim() >= 3 else 0

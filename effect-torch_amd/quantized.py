@@ -149,6 +149,10 @@ class CancellationFlag:
         return ctypes.cast(ctypes.byref(self._value), ctypes.c_void_p)
 
 
+def _cancel_address(cancelled: Optional[CancellationFlag]) -> Optional[int]:
+    return None if cancelled is None else ctypes.addressof(cancelled._value)
+
+
 class QuantizedRequirements:
     """Frozen plan of one quantized linear (crates/runtime-cpu/src/quantized.rs:35-42)."""
 
@@ -218,8 +222,12 @@ def linear_into(input: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.
                 cancelled: Optional[CancellationFlag] = None, *,
                 workspace: Optional[torch.Tensor] = None, stream=None) -> None:
     """Execute step (crates/runtime-cpu/src/quantized.rs:419-499): enqueues on ``stream``."""
-    if int(codec) != int(requirements.codec):
+    if codec is not requirements.codec and int(codec) != int(requirements.codec):
         raise QuantizedError(N.ERR_EXECUTION, "quantized_linear: codec does not match the immutable plan")
+    status = N.host_calls().linear_into(requirements._handle.value, input, weight, bias, destination, workspace,
+                                        None if stream is None else _stream_handle(stream), _cancel_address(cancelled))
+    if status >= 0:
+        return _check(status)
     descs = (_desc(input), _desc(weight), _desc(bias), _desc(destination))
     ws_ptr = workspace.data_ptr() if workspace is not None else None
     ws_bytes = workspace.numel() * workspace.element_size() if workspace is not None else 0
@@ -264,13 +272,19 @@ def embedding_into(indexes: torch.Tensor, weight: torch.Tensor, codec: GgmlQuant
     reference's error is raised here; otherwise the status tensor is returned
     for :func:`embedding_status_check` after the caller's own fence.
     """
-    if int(codec) != int(requirements.codec):
+    if codec is not requirements.codec and int(codec) != int(requirements.codec):
         raise QuantizedError(N.ERR_EXECUTION, "quantized_embedding: codec does not match the immutable plan")
-    status = torch.empty(N.STATUS_BYTES, dtype=torch.uint8, device=destination.device)
-    descs = (_desc(indexes), _desc(weight), _desc(destination))
-    _check(N.lib().et_hip_embedding_into(requirements._handle, _ref(descs[0]), _ref(descs[1]),
-                                         _ref(descs[2]), status.data_ptr(), _stream_handle(stream),
-                                         cancelled.ptr if cancelled is not None else None))
+    taken = N.host_calls().embedding_into(requirements._handle.value, indexes, weight, destination,
+                                          None if stream is None else _stream_handle(stream), _cancel_address(cancelled))
+    if taken != -1:
+        code, status = taken
+        _check(code)
+    else:
+        status = torch.empty(N.STATUS_BYTES, dtype=torch.uint8, device=destination.device)
+        descs = (_desc(indexes), _desc(weight), _desc(destination))
+        _check(N.lib().et_hip_embedding_into(requirements._handle, _ref(descs[0]), _ref(descs[1]),
+                                             _ref(descs[2]), status.data_ptr(), _stream_handle(stream),
+                                             cancelled.ptr if cancelled is not None else None))
     if not synchronize:
         return status
     embedding_status_check(requirements, status)

@@ -382,3 +382,26 @@ def test_projections_left_as_k_shares_layout_and_validation(et):
     narrow.shares = prepared.data_ptr()
     fails("this geometry's kernel takes q, k and v as tensors", layer=odd, shares=narrow,
           destination=torch.zeros(32, 32, 1, 12))
+
+
+def test_host_calls_leave_other_arguments_to_the_ctypes_path(et):
+    # the CPython module takes plain device tensors only; anything else comes back as -1 before anything has happened,
+    # and the ctypes path words the error
+    import torch
+    from effect_torch_amd import _native
+    calls = _native.host_calls()
+    x, w, y = torch.zeros(2, 256), torch.zeros((4, 144), dtype=torch.uint8), torch.zeros(2, 4)
+    plan = et.linear_requirements(x, w, None, et.GgmlQuant.Q4_K, (4, 256))
+    handle = plan._handle.value
+    for arguments in ((), (handle, x, w, None, y, None, 0, None), (handle, None, w, None, y, None, 0, None),
+                      (handle, "x", w, None, y, None, 0, None), (handle, x.to_sparse(), w, None, y, None, 0, None),
+                      ("plan", x, w, None, y, None, 0, None), (handle, x, w, None, y, None, -1, None)):
+        assert calls.linear_into(*arguments) == -1
+    assert calls.embedding_into(handle, x, w, y, 0, None) == -1
+    assert calls.kv_attention_into() == -1 and calls.kv_attention_into(*[None] * 20) == -1
+    with pytest.raises(et.QuantizedError, match="unsupported dtype torch.int8"):
+        et.linear_into(x.to(torch.int8), w, None, et.GgmlQuant.Q4_K, y, plan, stream=0)
+    flag = et.CancellationFlag()
+    flag.cancel()
+    with pytest.raises(et.Cancelled, match="operation aborted"):
+        et.linear_into(x, w, None, et.GgmlQuant.Q4_K, y, plan, flag, stream=0)
