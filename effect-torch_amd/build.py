@@ -41,6 +41,7 @@ SOURCES = {
     "quantize_act.hip": ["-ffp-contract=off"],
     "gemm_i8.hip": [],
     "gemm_h16.hip": [],
+    "gemm_h16_wide.hip": [],
     "kv_attention.hip": [],
     "kv_chunk.hip": [],
     "decode_ops.hip": ["-ffp-contract=off"],

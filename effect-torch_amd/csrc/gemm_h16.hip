@@ -5,9 +5,9 @@
 //           - sum_s  dmin[n, s] * sum_g m_g[n] * xsum[m, g]
 // s = 256-column stage (one Q4_K super-block), g = its eight 32-column sub-blocks.
 //
-// Activations are 24-bit fixed point per vector and stage, X = rint(x * (2^23 - 1) / max|x|), split
-// into two balanced 12-bit halves X = 4096 * hi + lo with |lo|, |hi| <= 2048: integers a half float
-// holds exactly. The tiles hold hi and lo / 4096 (exact as well: a power of two), so that both halves
+// Activations are scaled per vector and stage, X = x * (2^23 - 1) / max|x|, and split into X = 4096 * hi + lo with
+// |lo|, |hi| <= 2048: hi an integer a half float holds exactly, lo rounded to the eleven bits of a half float
+// (quantize_halves.h). The tiles hold hi and lo / 4096, so that both halves
 // of a sub-block add up in ONE accumulator, hi * w + (lo / 4096) * w = X * w / 4096, and the factor
 // 4096 rides on the row scale: one multiply-add per element and stage in the epilogue. On the weight side the 6-bit sub-block scale is folded into the operand:
 // sc_g * nib <= 63 * 15 = 945 (Q5_K: 63 * 31 = 1953), exact in a half float as well. Every product (< 2^21) is exact in
@@ -29,19 +29,11 @@
 #include <cstdint>
 #include <type_traits>
 
-#include "decode_math.h"
-#include "et_codecs.h"
-#include "gemv_common.h"
-#include "kernels.h"
+#include "gemm_h16_device.h"
 
 namespace et {
 namespace {
 
-typedef _Float16 v8h __attribute__((ext_vector_type(8)));
-typedef _Float16 v2h __attribute__((ext_vector_type(2)));
-typedef float v16f __attribute__((ext_vector_type(16)));
-
-constexpr int kStageBlocks = 8;
 constexpr int kConsumers = 8;
 constexpr int kWeightLoaders = 2;
 constexpr int kActivationLoaders = 2;
@@ -52,57 +44,12 @@ constexpr int kThreads = 64 * (kConsumers + kLoaders);
 // workgroup copies per weight row; two groups (64 rows) make twice as many workgroups.
 // NARROW = at most sixteen vectors: see Operands.
 
-constexpr float kPlaneRatio = 4096.0f;          // what the accumulators lack: the tiles hold hi and lo / 4096
-constexpr uint32_t kBlob = tile_blob_bytes(2);  // in memory and in LDS
-constexpr uint32_t kUnitAt = 32768u;            // unit[m]
-constexpr uint32_t kSumsAt = 32768u + 128u;     // xsum[g][m]
 constexpr int kActivationJobs = kBlob / 1024;
 static_assert(kBlob % 1024 == 0, "whole copy instructions");
 
-// (scale, min) of Q4_K sub-block g (crates/runtime-cpu/src/quantized.rs:77-86).
-__device__ __forceinline__ void q4k_scale_min(const uint4& header, uint32_t g, uint32_t& sc, uint32_t& mn) {
-    const uint32_t shift = 8u * (g & 3u);
-    const uint32_t s0 = (header.y >> shift) & 0xffu;
-    const uint32_t s1 = (header.z >> shift) & 0xffu;
-    const uint32_t s2 = (header.w >> shift) & 0xffu;
-    sc = g < 4 ? (s0 & 63u) : ((s2 & 0x0fu) | ((s0 >> 6) << 4));
-    mn = g < 4 ? (s1 & 63u) : ((s2 >> 4) | ((s1 >> 6) << 4));
-}
-
-// s_waitcnt immediate that waits for vmcnt <= n only (gfx9 encoding: vmcnt in bits 3:0 and 15:14).
-constexpr int vmcnt_only(int n) {
-    return (n & 0xf) | ((n >> 4) << 14) | (0x7 << 4) | (0xf << 8);
-}
-
-// A row's share of a stage, as it lies in memory: a Q4_K super-block is d, dmin, scales[12], qs[128];
-// a Q5_K one d, dmin, scales[12], qh[32] (the fifth bits: bit g of qh[c] belongs to column c of
-// sub-block g), qs[128] (crates/runtime-cpu/src/quantized.rs:180-234).
-// Super-blocks whose size is not a multiple of sixteen (Q6_K: 210 bytes = ql[128], qh[64], sixteen int8
-// scales, d; Q3_K: 110 = hmask[32], qs[64], scales[12], d; Q2_K: 84 = scales[16], qs[64], d, dmin;
-// crates/runtime-cpu/src/quantized.rs:117-176, 238-261) get an LDS row of the next multiple: every
-// 16-byte chunk holds the stage's bytes at the same offset except the last one, which is taken from the
-// stage's last sixteen bytes - so no copy reads past the stage (or the weight buffer). Q3_K and Q6_K
-// stages start on 2-byte boundaries; global_load_lds takes such sources, more slowly.
-template <int CODEC>
-struct Codec {
-    static_assert(CODEC == kQ2_K || CODEC == kQ3_K || CODEC == kQ4_K || CODEC == kQ5_K || CODEC == kQ6_K,
-                  "the K-quants");
-    static constexpr uint32_t kStageBytes = block_bytes(CODEC);            // in memory
-    static constexpr uint32_t kRowBytes = (kStageBytes + 15u) / 16u * 16u;  // in LDS
-    static constexpr uint32_t kQuantsAt = CODEC == kQ5_K ? 48u : 16u;       // Q4_K / Q5_K
-    // where the stage's last sixteen bytes lie in the LDS row: d (and dmin) are read from there
-    static constexpr uint32_t kTailAt = kRowBytes - 16u, kTailFrom = kStageBytes - 16u;
-    // byte of the stage that LDS byte `within` (a multiple of 16) of the row holds
-    static __device__ __forceinline__ uint32_t source_of(uint32_t within) {
-        return kRowBytes != kStageBytes && within == kTailAt ? kTailFrom : within;
-    }
-    // LDS offset of stage byte `at` of the tail
-    static constexpr uint32_t in_tail(uint32_t at) { return kTailAt + (at - kTailFrom); }
-};
-
 template <int CODEC, int RG, int AX, int AW>
 struct Shape {
-    static constexpr uint32_t kRowBytes = Codec<CODEC>::kRowBytes;
+    static constexpr uint32_t kRowBytes = HalfStage<CODEC>::kRowBytes;
     static constexpr int kRowGroups = RG, kSplit = kConsumers / RG, kBlocksPerWave = kStageBlocks / kSplit;
     static constexpr uint32_t kRows = 32 * RG;
     static constexpr uint32_t kWeightBytes = kRows * kRowBytes;
@@ -118,66 +65,6 @@ struct Shape {
     static constexpr uint32_t kExchangeBytes = (kSplit - 1) * kRowGroups * 16 * 64 * 4;
     static constexpr uint32_t kLdsBytes = kRingBytes > kExchangeBytes ? kRingBytes : kExchangeBytes;
 };
-
-// Eight nibbles (two dwords of four, one per byte) as eight half floats times `scale`:
-// 0x6400 | n is the half float 1024 + n, and (1024 + n) * scale - 1024 * scale, one fused
-// multiply-add per pair, is n * scale exactly (1024 * scale <= 64512 is a half float).
-template <int OFFSET = 0>
-__device__ __forceinline__ v8h nibbles_times(uint32_t first, uint32_t second, v2h scale) {
-    // OFFSET is subtracted from every byte first: (1024 + n) * scale - (1024 + OFFSET) * scale
-    const v2h offset = {static_cast<_Float16>(1024.0f + OFFSET), static_cast<_Float16>(1024.0f + OFFSET)};
-    union {
-        uint32_t word[4];
-        v2h pair[4];
-        v8h all;
-    } u;
-    u.word[0] = __builtin_amdgcn_perm(0x64646464u, first, 0x04010400u);   // bytes 0, 1
-    u.word[1] = __builtin_amdgcn_perm(0x64646464u, first, 0x04030402u);   // bytes 2, 3
-    u.word[2] = __builtin_amdgcn_perm(0x64646464u, second, 0x04010400u);
-    u.word[3] = __builtin_amdgcn_perm(0x64646464u, second, 0x04030402u);
-#pragma unroll
-    for (int i = 0; i < 4; i++) u.pair[i] = __builtin_elementwise_fma(u.pair[i], scale, -(offset * scale));
-    return u.all;
-}
-
-// The matrices of one launch: contractions that share their activations (the q / k / v projections
-// of a decode step) run as one grid over the row tiles of all of them.
-struct Member {
-    const uint8_t* weight;
-    const float* bias;
-    const float* residual;
-    float* y;
-    uint32_t rows;
-    uint32_t first_tile;  // of the launch's row tiles
-};
-struct Group {
-    Member member[kGemmGroupMost];
-    uint32_t count;
-    uint32_t row_tiles;  // of all members together
-};
-
-// Eight bytes as eight half floats, (n - OFFSET) * scale in two exact steps (for offsets whose product
-// with the scale a half float does not hold: 1028 * 31).
-template <int OFFSET>
-__device__ __forceinline__ v8h bytes_minus_times(uint32_t first, uint32_t second, v2h scale) {
-#pragma clang fp contract(off)
-    const v2h offset = {static_cast<_Float16>(1024.0f + OFFSET), static_cast<_Float16>(1024.0f + OFFSET)};
-    union {
-        uint32_t word[4];
-        v2h pair[4];
-        v8h all;
-    } u;
-    u.word[0] = __builtin_amdgcn_perm(0x64646464u, first, 0x04010400u);
-    u.word[1] = __builtin_amdgcn_perm(0x64646464u, first, 0x04030402u);
-    u.word[2] = __builtin_amdgcn_perm(0x64646464u, second, 0x04010400u);
-    u.word[3] = __builtin_amdgcn_perm(0x64646464u, second, 0x04030402u);
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const v2h centred = u.pair[i] - offset;
-        u.pair[i] = centred * scale;
-    }
-    return u.all;
-}
 
 // The activation operands of sub-block b for one lane (matrix row i = in_half, K group = half), two per
 // 16-column chunk in the order they are contracted: low and high plane of vector i - or, NARROW (at most
@@ -229,7 +116,7 @@ __global__ __launch_bounds__(kThreads) void gemm_h16_kernel(
     const Group group, const uint8_t* __restrict__ tiles, uint32_t vector_tiles, uint32_t columns,
     uint32_t vectors, uint32_t k_splits, float* __restrict__ partials) {
     using S = Shape<CODEC, RG, AX, AW>;
-    constexpr uint32_t kRowBytes = S::kRowBytes, kQuantsAt = Codec<CODEC>::kQuantsAt, kStageBytes = Codec<CODEC>::kStageBytes;
+    constexpr uint32_t kRowBytes = S::kRowBytes, kQuantsAt = HalfStage<CODEC>::kQuantsAt, kStageBytes = HalfStage<CODEC>::kStageBytes;
     constexpr int NB = S::kBlocksPerWave;
     constexpr int kSplit = S::kSplit, kRowGroups = S::kRowGroups, kWeightJobs = S::kWeightJobs;
     constexpr uint32_t kRows = S::kRows, kWeightBytes = S::kWeightBytes;
@@ -306,7 +193,7 @@ __global__ __launch_bounds__(kThreads) void gemm_h16_kernel(
                 const uint32_t at = job * 1024u + lane * 16u;
                 const uint32_t row = min(row0 + at / kRowBytes, rows - 1u);
                 const uint8_t* src = weight + row * row_bytes + static_cast<uint64_t>(first_stage + s) * kStageBytes +
-                                     Codec<CODEC>::source_of(at % kRowBytes);
+                                     HalfStage<CODEC>::source_of(at % kRowBytes);
                 if constexpr (PROBE == kProbeNoCopies || PROBE == kProbeNoWeightCopies || PROBE == kProbeActivationCopiesOnly) continue;
                 __builtin_amdgcn_global_load_lds(reinterpret_cast<const uint4*>(src),
                                                  reinterpret_cast<uint4*>(region + job * 1024u), 16, 0, 0);
@@ -352,7 +239,7 @@ __global__ __launch_bounds__(kThreads) void gemm_h16_kernel(
         if constexpr (CODEC == kQ3_K) {
             // value = d * (sc - 32) * (v - 4), v = two bits of qs | the hmask bit << 2, a 6-bit scale per 16
             // columns; |(sc - 32) * (v - 4)| <= 128 is exact in a half float. No minimum term.
-            const float d_block = half_bits_to_float(*reinterpret_cast<const uint16_t*>(row_in_slot + Codec<CODEC>::in_tail(108u)));
+            const float d_block = half_bits_to_float(*reinterpret_cast<const uint16_t*>(row_in_slot + HalfStage<CODEC>::in_tail(108u)));
             const float unit = *reinterpret_cast<const float*>(slot + kUnitAt + in_half * 4u);
             const uint4 hm = *reinterpret_cast<const uint4*>(row_in_slot + 16u * half);  // hmask of these columns
             v16f p = zero;
@@ -361,8 +248,8 @@ __global__ __launch_bounds__(kThreads) void gemm_h16_kernel(
                 const uint32_t b = b_base + bb, n = b >> 2, t = b & 3u;
                 const uint4 qs = *reinterpret_cast<const uint4*>(row_in_slot + 32u + 32u * n + 16u * half);
                 // scale of group 8 n + 2 t + half: nibble n of packed[2 t + half], top bits from packed[8 + ..]
-                const uint32_t low_byte = row_in_slot[Codec<CODEC>::in_tail(96u) + 2u * t + half];
-                const uint32_t high_byte = row_in_slot[Codec<CODEC>::in_tail(104u) + 2u * (t & 1u) + half];
+                const uint32_t low_byte = row_in_slot[HalfStage<CODEC>::in_tail(96u) + 2u * t + half];
+                const uint32_t high_byte = row_in_slot[HalfStage<CODEC>::in_tail(104u) + 2u * (t & 1u) + half];
                 const int sc = static_cast<int>(((low_byte >> (4u * n)) & 15u) |
                                                 (((high_byte >> (2u * (2u * n + (t >> 1)))) & 3u) << 4)) - 32;
                 const uint32_t bit = 4u * n + t;
@@ -387,7 +274,7 @@ __global__ __launch_bounds__(kThreads) void gemm_h16_kernel(
             // value = d * sc * v - dmin * mn with a 4-bit scale and minimum per 16 columns. The minima ride
             // on the matrix cores too: a weight operand that is mn in all sixteen columns sums the
             // activations of the run times mn (acc_min is then the second pair of accumulators).
-            const uint32_t dd = *reinterpret_cast<const uint32_t*>(row_in_slot + Codec<CODEC>::in_tail(80u));
+            const uint32_t dd = *reinterpret_cast<const uint32_t*>(row_in_slot + HalfStage<CODEC>::in_tail(80u));
             const float d_block = half_bits_to_float(dd & 0xffffu), dmin_block = half_bits_to_float(dd >> 16);
             const float unit = *reinterpret_cast<const float*>(slot + kUnitAt + in_half * 4u);
             v16f p = zero, m = zero;  // products, and the sums of the activations times the minima
@@ -424,7 +311,7 @@ __global__ __launch_bounds__(kThreads) void gemm_h16_kernel(
             // of a 32-column block are one such run. sc * (q - 32) reaches 4096, too wide for a half
             // float, so sc = 16 * s_hi + s_lo (s_lo 0..15, s_hi -8..7) and both parts are contracted:
             // four accumulators, (X_lo, X_hi) x (s_lo, s_hi), joined once per stage.
-            const float d_block = half_bits_to_float(*reinterpret_cast<const uint16_t*>(row_in_slot + Codec<CODEC>::in_tail(208u)));
+            const float d_block = half_bits_to_float(*reinterpret_cast<const uint16_t*>(row_in_slot + HalfStage<CODEC>::in_tail(208u)));
             const float unit = *reinterpret_cast<const float*>(slot + kUnitAt + in_half * 4u);
             v16f p_l = zero, p_h = zero;  // by scale part; both activation halves go into one sum
 #pragma unroll
@@ -661,6 +548,11 @@ __global__ __launch_bounds__(256) void reduce_group_rotary_kernel(const Group gr
 
 }  // namespace
 
+// Up to here two of the wide kernel's four activation tiles would be padding.
+constexpr uint64_t kGemmWideFrom = 64;
+// Its weight copies add 32-bit byte offsets to a tile's first row: 256 rows of less than 2^23 bytes each.
+constexpr uint64_t kGemmWideColumns = 1u << 23;
+
 bool gemm_h16_supported(int32_t codec, uint64_t columns) {
     return (codec == kQ2_K || codec == kQ3_K || codec == kQ4_K || codec == kQ5_K || codec == kQ6_K) &&
            columns % 256 == 0 && columns > 0;
@@ -679,17 +571,58 @@ GemmGroupGeometry gemm_h16_group_geometry(int32_t codec, const uint64_t* rows, u
         const uint64_t share = (stages + splits - 1) / splits;
         return static_cast<uint32_t>((stages + share - 1) / share);
     };
-    uint64_t small = 0, large = 0;
+    uint64_t small = 0, large = 0, wide = 0;
+    const uint32_t wide_rows = gemm_h16_wide_rows(codec);
     for (uint32_t i = 0; i < count; i++) {
         small += (rows[i] + 63) / 64;
         large += (rows[i] + 127) / 128;
+        wide += (rows[i] + wide_rows - 1) / wide_rows;
     }
     // 128-row workgroups (half the activation copies per weight row) once they fill the device without
     // sharing K. (With K shares they measured slower than 64-row workgroups: 14336 x 4096 with 32 vectors
     // 25.1 against 23.7 us, 4096 x 4096 16.3 against 13.8 us.)
     // (Q6_K: 128 rows of 224 bytes per stage leave no room for a weight ring.)
-    if (codec != kQ6_K && large * vector_tiles >= 192) return GemmGroupGeometry{128, large, 1};
-    return GemmGroupGeometry{64, small, shares(small * vector_tiles)};
+    const GemmGroupGeometry narrow = codec != kQ6_K && large * vector_tiles >= 192
+                                         ? GemmGroupGeometry{128, large, 1}
+                                         : GemmGroupGeometry{64, small, shares(small * vector_tiles)};
+    if (vectors <= kGemmWideFrom || columns >= kGemmWideColumns || vectors > 0xffffffffull) return narrow;
+    // Prompts: the wide kernel where it takes less time. A compute unit runs one workgroup at a time, so a launch takes
+    // as many turns of a share's stages as its busiest XCD has workgroups per compute unit; a stage of 256 columns takes,
+    // from launches of 1000 vectors on 14336 x 4096, the microseconds of StageTimes. K shares cost what their sums move,
+    // written and read at 4 TB/s, and a launch; the wide kernel also its first copies and its stores, which no other
+    // workgroup covers. (Whole calls, narrow / wide in us: Q4_K 14336 x 4096 with 1000, 256 and 70 vectors 419 / 288,
+    // 115 / 85, 55 / 47; 4096 x 4096 with 1000, 512 and 200 vectors 129 / 95, 65 / 59 and 33 / 38, the last one stays
+    // narrow; 11008 x 2048 with 300 vectors 66 / 71, narrow as well; Q6_K 14336 x 4096 with 1000 and 70 724 / 460, 71 / 63.)
+    struct StageTimes {
+        double rows64, rows128, wide;
+    };
+    const StageTimes us = codec == kQ2_K   ? StageTimes{1.3, 2.2, 6.1}
+                          : codec == kQ3_K ? StageTimes{1.1, 1.8, 7.6}
+                          : codec == kQ5_K ? StageTimes{1.15, 1.95, 8.5}
+                          : codec == kQ6_K ? StageTimes{1.6, 0.0, 6.9}
+                                           : StageTimes{1.05, 1.8, 8.4};
+    uint64_t launch_rows = 0;
+    for (uint32_t i = 0; i < count; i++) launch_rows += rows[i];
+    const auto cost = [&](uint64_t on_an_xcd, uint64_t splits, double stage_us) {
+        const double turns = static_cast<double>((on_an_xcd + 31) / 32);
+        const double sums = splits > 1 ? 3.0 + 8.0e-6 / 4 * static_cast<double>(splits) * static_cast<double>(vectors) * static_cast<double>(launch_rows) : 0.0;
+        return turns * static_cast<double>((stages + splits - 1) / splits) * stage_us + sums;
+    };
+    const double narrow_us = cost((narrow.row_tiles + 7) / 8 * vector_tiles * narrow.k_splits, narrow.k_splits,
+                                  narrow.tile_rows == 128 ? us.rows128 : us.rows64);
+    GemmGroupGeometry best = narrow;
+    double best_us = narrow_us - 6.0;
+    const uint64_t wide_groups = (vectors + kGemmWideVectors - 1) / kGemmWideVectors;
+    for (uint64_t splits = 1; splits <= stages && splits <= 16; splits++) {
+        const uint64_t share = (stages + splits - 1) / splits;
+        if ((stages + share - 1) / share != splits) continue;  // an empty share
+        const double wide_us = cost((wide * splits + 7) / 8 * wide_groups, splits, us.wide);
+        if (wide_us < best_us) {
+            best_us = wide_us;
+            best = GemmGroupGeometry{wide_rows, wide, static_cast<uint32_t>(splits), true};
+        }
+    }
+    return best;
 }
 
 uint64_t gemm_h16_group_partial_bytes(int32_t codec, const uint64_t* rows, uint32_t count, uint64_t columns,
@@ -715,6 +648,18 @@ hipError_t sum_shares(const Group& group, const float* partials, uint32_t vector
     return hipGetLastError();
 }
 
+// Members of at most 2^32 - 1 rows each: their tiles of 64 rows or more fit 32 bits.
+Group group_of(const GemmMember* members, uint32_t count, uint32_t tile_rows) {
+    Group group = {};
+    group.count = count;
+    for (uint32_t i = 0; i < count; i++) {
+        group.member[i] = Member{members[i].weight, members[i].bias, members[i].residual, members[i].y,
+                                 static_cast<uint32_t>(members[i].rows), group.row_tiles};
+        group.row_tiles += static_cast<uint32_t>((members[i].rows + tile_rows - 1) / tile_rows);
+    }
+    return group;
+}
+
 template <int CODEC, int RG, int AX, int AW, bool NARROW, int PROBE = kProbeNone>
 hipError_t launch_tiles(const GemmMember* members, uint32_t count, const uint8_t* tiles, float* partials,
                         uint32_t columns, uint32_t vectors, uint32_t k_splits, hipStream_t stream, bool leave_shares,
@@ -722,16 +667,9 @@ hipError_t launch_tiles(const GemmMember* members, uint32_t count, const uint8_t
     using S = Shape<CODEC, RG, AX, AW>;
     static_assert(S::kLdsBytes <= 160 * 1024, "LDS of a gfx950 CU: 160 KiB, all of it dynamic here");
     const auto kernel = gemm_h16_kernel<CODEC, RG, AX, AW, NARROW, PROBE>;
-    Group group = {};
-    group.count = count;
-    uint64_t row_tiles = 0;
-    for (uint32_t i = 0; i < count; i++) {
-        group.member[i] = Member{members[i].weight, members[i].bias, members[i].residual, members[i].y,
-                                 static_cast<uint32_t>(members[i].rows), static_cast<uint32_t>(row_tiles)};
-        row_tiles += (members[i].rows + S::kRows - 1) / S::kRows;
-    }
-    if (row_tiles > 0x00ffffffull) return hipErrorInvalidValue;
-    group.row_tiles = static_cast<uint32_t>(row_tiles);
+    const Group group = group_of(members, count, S::kRows);
+    if (group.row_tiles > 0x00ffffffu) return hipErrorInvalidValue;
+    const uint64_t row_tiles = group.row_tiles;
     // More than 64 KiB of dynamic LDS has to be allowed once per kernel and device.
     static std::atomic<bool> allowed[64] = {};  // callers may enqueue from several threads; setting twice is harmless
     int device = 0;
@@ -786,6 +724,11 @@ hipError_t gemm_h16_group(int32_t codec, const GemmMember* members, uint32_t cou
     if (rotary != nullptr && (g.k_splits == 1 || partials == nullptr)) return hipErrorInvalidValue;
     if (partials == nullptr && g.k_splits > 1) {  // nowhere to keep shares: 64-row workgroups, whole K each
         g = GemmGroupGeometry{64, 0, 1};
+    }
+    if (g.wide) {
+        const Group group = group_of(members, count, g.tile_rows);
+        if (hipError_t status = gemm_h16_wide(codec, group, tiles, columns, vectors, g.k_splits, partials, stream)) return status;
+        return sum_shares(group, partials, vectors, g.k_splits, g.tile_rows, stream, leave_shares, rotary);
     }
     // weight lead: what the activation ring (three slots of 34 KiB) leaves of LDS
     if (codec == kQ6_K)  // 64-row tiles only (gemm_h16_group_geometry): 128 rows of 224 bytes leave no room for a ring

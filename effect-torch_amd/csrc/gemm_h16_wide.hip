@@ -1,0 +1,421 @@
+// gemm_h16.hip's contraction (the same operands: exact integers in half floats) for prompts. A workgroup contracts 128
+// vectors with 256 weight rows (Q2_K, Q6_K: 128), so that weights are unpacked once for 128 (64) vectors instead of for
+// every 32, and an activation tile is copied for 256 rows instead of 64 or 128.
+//
+// Bound: instruction issue. Eight waves, two per SIMD, each 128 vectors x 32 rows (Q2_K, Q6_K, which contract two operands
+// per weight: 64 x 32). Matrix and vector instructions of a SIMD take their time one after the other on this device, also
+// from two waves: a Q4_K wave's stage of 256 columns is 128 half-float matrix instructions (32 cycles each), 16 f32 ones for
+// the minima (64) and about 510 vector instructions (4): 7160 cycles by that sum, 7860 measured at the 2.1 GHz the
+// device holds. What helped was therefore fewer vector instructions (waves of 64 x 64 unpack every weight twice: 282 ->
+// 296 us) and not the latencies: operands fetched only behind each barrier measured the same. LDS is 14 % busy.
+// Every wave unpacks its own weight rows from the packed bytes in LDS. There are no loader waves (a third wave per SIMD
+// would leave 168 registers each): the waves ask for the next sub-blocks' activations and the next stage's weights
+// themselves, through inline assembly, because any LDS read next to a copy that the compiler can see waits for it.
+//
+// Whole calls (us, gemm_h16_kernel / this): 14336 x 4096 with 1000 vectors Q4_K 420 / 288 (407 TFLOP/s), Q5_K 453 / 285,
+// Q6_K 724 / 460, Q3_K 415 / 255, Q2_K 512 / 405; Q4_K 4096 x 14336 with 1000 396 / 278, 14336 x 4096 with 256 115 / 85.
+// Relative error against 64 bits there (2-norm, 1e-7): Q4_K 1.75 / 1.71, Q6_K 1.66 / 1.63, Q2_K 1.84 / 1.76: one chain of
+// sums over the stage's eight sub-blocks instead of two or four, from activations that are rounded less (quantize_halves.h).
+#include <hip/hip_runtime.h>
+
+#include <atomic>
+#include <cstdint>
+
+#include "gemm_h16_device.h"
+
+namespace et {
+namespace {
+
+constexpr int kWaves = 8;
+constexpr int kTiles = kGemmWideVectors / 32;        // activation tiles per workgroup
+constexpr int kSlots = 4;                            // sub-blocks of activations in LDS: two landed, two on their way
+constexpr uint32_t kSlotBytes = kTiles * 2 * 2048u;  // per tile and plane four 8-column parts of 512 bytes
+constexpr int kActivationCopies = 2;                 // per wave and sub-block: one plane of one tile
+static_assert(kTiles * 2 == kWaves && kStageBlocks % kSlots == 0, "a wave copies one plane of one tile; slots start anew per stage");
+
+template <int CODEC>
+struct Wide {
+    static constexpr bool kMinima = CODEC == kQ4_K || CODEC == kQ5_K;  // a minimum per sub-block, against xsum
+    // weight operands per sixteen columns: Q6_K splits its scale, Q2_K contracts its minima
+    static constexpr int kParts = CODEC == kQ6_K || CODEC == kQ2_K ? 2 : 1;
+    static constexpr int kMT = kParts == 2 ? 2 : 4;  // 32-vector tiles per wave, against 32 rows
+    static constexpr int kWavesM = kTiles / kMT, kWavesN = kWaves / kWavesM;
+    static constexpr uint32_t kRows = 32u * kWavesN;
+    static constexpr uint32_t kRowBytes = HalfStage<CODEC>::kRowBytes;
+    static constexpr uint32_t kWeightBytes = kRows * kRowBytes;
+    static constexpr int kWeightJobs = kWeightBytes / 1024;
+    static_assert(kWeightBytes % 1024 == 0, "whole copy instructions");
+    static constexpr int kRounds = (kWeightJobs + kWaves - 1) / kWaves;  // weight copies per wave and stage, one per sub-block
+    static_assert(kRounds <= kStageBlocks - 2, "landed before the last sub-block");
+    // the activation slots; one stage of unit[m] (512 bytes, copied twice) and of xsum; two stages of weights
+    static constexpr uint32_t kUnitsAt = kSlots * kSlotBytes, kSumsAt = kUnitsAt + 1024u,
+                              kWeightsAt = kSumsAt + (kMinima ? 4096u : 0u), kLdsBytes = kWeightsAt + 2 * kWeightBytes;
+    static_assert(kLdsBytes <= 160 * 1024, "LDS of a gfx950 CU: 160 KiB, all of it dynamic here");
+    // copies that a wave asks for in front of the activations during sub-block b: the stage's tables, next weights
+    static constexpr int ahead(int b, bool last) { return (b == 0 ? 1 : 0) + (!last && b < kRounds ? 1 : 0); }
+};
+
+// 1 KiB from `base` + a byte offset per lane to LDS address `to` + 16 bytes per lane.
+__device__ __forceinline__ void copy_to_lds(const uint8_t* base, uint32_t lane_offset, uint32_t to) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                 :
+                 : "s"(to), "v"(lane_offset), "s"(base)
+                 : "memory");  // m0 is a reserved register: nothing else in this file sets it
+}
+
+// The packed bytes of one lane's columns 32 b + 16 half .. + 16 of a row, as they come out of LDS.
+struct Raw {
+    uint4 low, high;
+    uint32_t scale, scale_top;
+};
+// What all of a row's sub-blocks share: d, dmin and the scales (Q4_K, Q5_K); the fifth (Q5_K) or top (Q3_K) bits.
+struct Shared {
+    uint4 header, bits;
+};
+template <int CODEC>
+__device__ __forceinline__ Shared fetch_shared(const uint8_t* row, uint32_t half) {
+    Shared s = {};
+    if constexpr (CODEC == kQ4_K || CODEC == kQ5_K) s.header = *reinterpret_cast<const uint4*>(row);
+    if constexpr (CODEC == kQ5_K) s.bits = *reinterpret_cast<const uint4*>(row + 16u + 16u * half);
+    if constexpr (CODEC == kQ3_K) s.bits = *reinterpret_cast<const uint4*>(row + 16u * half);
+    return s;
+}
+template <int CODEC>
+__device__ __forceinline__ Raw fetch(const uint8_t* row, int b, uint32_t half) {
+    const uint32_t n = b >> 2, t = b & 3;
+    Raw r = {};
+    if constexpr (CODEC == kQ4_K || CODEC == kQ5_K) {
+        r.low = *reinterpret_cast<const uint4*>(row + HalfStage<CODEC>::kQuantsAt + 32u * (b >> 1) + 16u * half);
+    } else if constexpr (CODEC == kQ6_K) {
+        r.low = *reinterpret_cast<const uint4*>(row + 64u * n + 32u * (t & 1u) + 16u * half);
+        r.high = *reinterpret_cast<const uint4*>(row + 128u + 32u * n + 16u * half);
+        r.scale = row[192u + 8u * n + 2u * t + half];
+    } else if constexpr (CODEC == kQ3_K) {
+        r.low = *reinterpret_cast<const uint4*>(row + 32u + 32u * n + 16u * half);
+        r.scale = row[HalfStage<CODEC>::in_tail(96u) + 2u * t + half];
+        r.scale_top = row[HalfStage<CODEC>::in_tail(104u) + 2u * (t & 1u) + half];
+    } else {
+        r.low = *reinterpret_cast<const uint4*>(row + 16u + 32u * n + 16u * half);
+        r.scale = row[2u * b + half];
+    }
+    return r;
+}
+__device__ __forceinline__ v2h twice(int value) {
+    const _Float16 h = static_cast<_Float16>(static_cast<float>(value));
+    return v2h{h, h};
+}
+// The weight operands of those columns, eight by eight: gemm_h16_kernel's values.
+template <int CODEC>
+__device__ __forceinline__ void operands(const Raw& raw, const Shared& shared, int b, v8h out[2][Wide<CODEC>::kParts]) {
+    const uint32_t n = b >> 2, t = b & 3;
+    const uint32_t low[4] = {raw.low.x, raw.low.y, raw.low.z, raw.low.w}, high[4] = {raw.high.x, raw.high.y, raw.high.z, raw.high.w};
+    const uint32_t bits[4] = {shared.bits.x, shared.bits.y, shared.bits.z, shared.bits.w};
+    uint32_t w[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        if constexpr (CODEC == kQ4_K || CODEC == kQ5_K) {
+            w[i] = (low[i] >> ((b & 1) * 4)) & 0x0f0f0f0fu;
+            if constexpr (CODEC == kQ5_K) w[i] |= ((bits[i] >> b) & 0x01010101u) << 4;
+        } else if constexpr (CODEC == kQ6_K) {
+            w[i] = ((low[i] >> ((t >> 1) * 4u)) & 0x0f0f0f0fu) | (((high[i] >> (2u * t)) & 0x03030303u) << 4);
+        } else {
+            w[i] = (low[i] >> (2u * t)) & 0x03030303u;
+            if constexpr (CODEC == kQ3_K) w[i] |= ((bits[i] >> (4u * n + t)) & 0x01010101u) << 2;
+        }
+    }
+    if constexpr (CODEC == kQ4_K || CODEC == kQ5_K) {
+        uint32_t sc, mn;
+        q4k_scale_min(shared.header, b, sc, mn);
+        const v2h scale = twice(sc);
+        out[0][0] = nibbles_times(w[0], w[1], scale);
+        out[1][0] = nibbles_times(w[2], w[3], scale);
+    } else if constexpr (CODEC == kQ6_K) {
+        const int sc = static_cast<int8_t>(raw.scale);
+        const v2h scale_low = twice(sc & 15), scale_high = twice(sc >> 4);
+        out[0][0] = nibbles_times<32>(w[0], w[1], scale_low);
+        out[1][0] = nibbles_times<32>(w[2], w[3], scale_low);
+        out[0][1] = nibbles_times<32>(w[0], w[1], scale_high);
+        out[1][1] = nibbles_times<32>(w[2], w[3], scale_high);
+    } else if constexpr (CODEC == kQ3_K) {
+        const int sc = static_cast<int>(((raw.scale >> (4u * n)) & 15u) |
+                                        (((raw.scale_top >> (2u * (2u * n + (t >> 1)))) & 3u) << 4)) - 32;
+        const v2h scale = twice(sc);
+        out[0][0] = bytes_minus_times<4>(w[0], w[1], scale);
+        out[1][0] = bytes_minus_times<4>(w[2], w[3], scale);
+    } else {
+        const v2h scale = twice(raw.scale & 15u), m = twice(raw.scale >> 4);
+        out[0][0] = nibbles_times(w[0], w[1], scale);
+        out[1][0] = nibbles_times(w[2], w[3], scale);
+        out[0][1] = out[1][1] = v8h{m.x, m.x, m.x, m.x, m.x, m.x, m.x, m.x};
+    }
+}
+
+template <int CODEC>
+__global__ __launch_bounds__(64 * kWaves, 2) void gemm_h16_wide_kernel(const Group group, const uint8_t* __restrict__ tiles,
+                                                                       uint32_t vector_tiles, uint32_t columns,
+                                                                       uint32_t vectors, uint32_t k_splits,
+                                                                       float* __restrict__ partials) {
+    using W = Wide<CODEC>;
+    constexpr uint32_t kRowBytes = W::kRowBytes, kStageBytes = HalfStage<CODEC>::kStageBytes;
+    constexpr int MT = W::kMT, P = W::kParts;
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+
+    // Workgroups go to the eight XCDs round-robin: the vector groups of one (row tile, K share) run on the same XCD, next
+    // to each other in time, so the later ones find the weights in its L2. (Row tiles whole to an XCD each, as in
+    // gemm_h16.hip, leave some XCDs a second turn: 5000 x 3072 with 333 vectors 72 us.)
+    const uint32_t xcd = blockIdx.x & 7u, turn = blockIdx.x >> 3;
+    const uint32_t vector_groups = (vector_tiles + kTiles - 1u) / kTiles;
+    const uint32_t vector_group = turn % vector_groups, pair = (turn / vector_groups) * 8u + xcd;
+    const uint32_t row_tile = pair / k_splits, k_share = pair % k_splits;
+    if (row_tile >= group.row_tiles) return;
+    uint32_t which = 0;
+    for (uint32_t i = 1; i < group.count; i++)
+        if (row_tile >= group.member[i].first_tile) which = i;
+    const Member& member = group.member[which];
+    const uint32_t rows = member.rows;
+
+    const uint32_t lane = threadIdx.x & 63u, half = lane >> 5, in_half = lane & 31u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t wave_n = wave % W::kWavesN, wave_m = wave / W::kWavesN;
+    const uint32_t all_stages = columns / 256u, share = (all_stages + k_splits - 1u) / k_splits;
+    const uint32_t first_stage = k_share * share;  // < all_stages: the launcher leaves no share empty
+    const uint32_t stages = min(share, all_stages - first_stage);
+    const uint32_t row_bytes = all_stages * kStageBytes;
+    const uint32_t row0 = (row_tile - member.first_tile) * W::kRows;  // in the member's own rows
+    const uint32_t first_vector_tile = vector_group * kTiles + wave_m * MT;
+    const bool working = first_vector_tile < vector_tiles;  // else every vector of this wave is padding
+
+    // ---- copies ----
+    const uint32_t lds0 = lds_address(lds);
+    // activations: wave w copies plane w & 1 of tile w / 2 (of the last tile where there are no more)
+    const uint32_t copied_tile = min(vector_group * kTiles + (wave >> 1), vector_tiles - 1u);
+    const uint8_t* const blobs = tiles + (static_cast<uint64_t>(first_stage) * vector_tiles + copied_tile) * kBlob + (wave & 1u) * 16384u;
+    const uint64_t blob_stride = static_cast<uint64_t>(vector_tiles) * kBlob;
+    const auto copy_activations = [&](uint32_t stage, int b) {
+        const uint8_t* from = blobs + stage * blob_stride + b * 2048u;
+        const uint32_t to = lds0 + (b % kSlots) * kSlotBytes + wave * 2048u;
+#pragma unroll
+        for (uint32_t i = 0; i < kActivationCopies; i++) copy_to_lds(from + i * 1024u, lane * 16u, to + i * 1024u);
+    };
+    // weights: the stage's bytes of the rows, row after row, as HalfStage lays them out
+    uint32_t weight_from[W::kRounds];
+#pragma unroll
+    for (int i = 0; i < W::kRounds; i++) {
+        const uint32_t at = (i * kWaves + wave) % W::kWeightJobs * 1024u + lane * 16u;
+        weight_from[i] = min(at / kRowBytes, rows - 1u - row0) * row_bytes + HalfStage<CODEC>::source_of(at % kRowBytes);
+    }
+    const uint8_t* const weights = member.weight + static_cast<uint64_t>(row0) * row_bytes + static_cast<uint64_t>(first_stage) * kStageBytes;
+    const auto copy_weights = [&](uint32_t stage, int round) {
+        copy_to_lds(weights + static_cast<uint64_t>(stage) * kStageBytes, weight_from[round],
+                    lds0 + W::kWeightsAt + (stage & 1u) * W::kWeightBytes + (round * kWaves + wave) % W::kWeightJobs * 1024u);
+    };
+    // xsum[g][m], 1 KiB per tile (waves 0 to 3), and the units of all tiles (the others, each the same bytes: every wave
+    // asks for one copy, so that all of them count alike)
+    const auto copy_tables = [&](uint32_t stage) {
+        const uint8_t* base = tiles + static_cast<uint64_t>(first_stage + stage) * blob_stride + static_cast<uint64_t>(vector_group) * kTiles * kBlob;
+        const uint32_t tiles_left = vector_tiles - 1u - vector_group * kTiles;
+        if (W::kMinima && wave < kTiles)
+            copy_to_lds(base + min(wave, tiles_left) * kBlob + ::et::kSumsAt, lane * 16u, lds0 + W::kSumsAt + wave * 1024u);
+        else
+            copy_to_lds(base + kUnitAt, min((lane >> 3) & 3u, tiles_left) * kBlob + (lane & 7u) * 16u, lds0 + W::kUnitsAt);
+    };
+
+    v16f acc[MT], zero;
+#pragma unroll
+    for (int r = 0; r < 16; r++) zero[r] = 0.f;
+#pragma unroll
+    for (int m = 0; m < MT; m++) acc[m] = zero;
+
+    const auto row_of = [&](uint32_t stage) {  // this lane's row in LDS
+        return lds + W::kWeightsAt + (stage & 1u) * W::kWeightBytes + (wave_n * 32u + in_half) * kRowBytes;
+    };
+    const uint8_t* const activations = lds + wave_m * MT * 4096u + half * 1024u + in_half * 16u;
+    const auto load = [&](int b, int plane, int chunk, v8h x[MT]) {
+#pragma unroll
+        for (int m = 0; m < MT; m++)
+            x[m] = *reinterpret_cast<const v8h*>(activations + (b % kSlots) * kSlotBytes + m * 4096u + plane * 2048u + chunk * 512u);
+    };
+
+    // Sub-block b of a stage begins. Landed behind its barrier: the activations of sub-block b + 1, and whatever was
+    // asked for before them two sub-blocks ago. Free: the slot of sub-block b - 1, in a stage's first sub-block also the
+    // other stage's weights and the tables of the stage before.
+    const auto begin = [&](uint32_t stage, bool last, int b) {
+        if (!last) wait_copies_in_flight(kActivationCopies + (b > 0 ? W::ahead(b - 1, false) : 0));
+        else wait_copies_in_flight(b < 6 ? kActivationCopies + (b > 0 ? W::ahead(b - 1, true) : 0) : 0);
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (b == 0) copy_tables(stage);
+        if (!last && b < W::kRounds) copy_weights(stage + 1u, b);
+        if (b + kSlots - 1 < kStageBlocks) copy_activations(stage, b + kSlots - 1);
+        else if (!last) copy_activations(stage + 1u, b + kSlots - 1 - kStageBlocks);
+    };
+#pragma unroll
+    for (int i = 0; i < W::kRounds; i++) copy_weights(0, i);
+#pragma unroll
+    for (int b = 0; b < kSlots - 1; b++) copy_activations(0, b);
+    wait_copies_in_flight(kActivationCopies);  // all but the last sub-block's
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (!working) {
+        for (uint32_t stage = 0; stage < stages; stage++) {
+#pragma unroll
+            for (int b = 0; b < kStageBlocks; b++) begin(stage, stage + 1u == stages, b);
+        }
+        return;
+    }
+    Shared shared = fetch_shared<CODEC>(row_of(0), half);
+    v8h w[2][P], x[2][MT];
+    operands<CODEC>(fetch<CODEC>(row_of(0), 0, half), shared, 0, w);
+    load(0, 0, 0, x[0]);
+
+    for (uint32_t stage = 0; stage < stages; stage++) {
+        const bool last = stage + 1u == stages;
+        v16f p[P][MT];
+        Shared shared_next;
+#pragma unroll
+        for (int b = 0; b < kStageBlocks; b++) {
+            begin(stage, last, b);
+            // Four turns of matrix instructions, low and high plane of both sixteen-column chunks. Behind each the next
+            // turn's activations are read; behind the first also the next sub-block's packed bytes, which become weight
+            // operands behind the third.
+            const int bn = (b + 1) % kStageBlocks;
+            const uint8_t* const row_n = row_of(b + 1 < kStageBlocks ? stage : stage + 1u);
+            Raw raw;
+            v8h next[2][P];
+#pragma unroll
+            for (int turn = 0; turn < 4; turn++) {
+                const int chunk = turn >> 1, plane = turn & 1;
+                if (turn < 3) load(b, (turn + 1) & 1, (turn + 1) >> 1, x[(turn + 1) & 1]);
+                else load(bn, 0, 0, x[0]);
+                if (turn == 0) {
+                    if (bn == 0) shared_next = fetch_shared<CODEC>(row_n, half);
+                    raw = fetch<CODEC>(row_n, bn, half);
+                }
+                if (turn == 2) operands<CODEC>(raw, bn == 0 ? shared_next : shared, bn, next);
+#pragma unroll
+                for (int m = 0; m < MT; m++)
+#pragma unroll
+                    for (int k = 0; k < P; k++)
+                        p[k][m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[plane][m], w[chunk][k], b + turn == 0 ? zero : p[k][m], 0, 0, 0);
+                // reads first, then the matrix instructions with the operands' arithmetic between them
+                __builtin_amdgcn_sched_group_barrier(0x100, MT + 1, 0);
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, 10, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int chunk = 0; chunk < 2; chunk++)
+#pragma unroll
+                for (int k = 0; k < P; k++) w[chunk][k] = next[chunk][k];
+        }
+        // acc += p * unit[m] * d[n] - sum_g (dmin * m_g)[n] * xsum[m, g]; vectors of a lane: 8 (r / 4) + 4 half + r % 4
+        const uint8_t* row = row_of(stage);
+        uint32_t dd = 0;
+        if constexpr (W::kMinima) dd = shared.header.x;
+        else if constexpr (CODEC == kQ3_K) dd = *reinterpret_cast<const uint16_t*>(row + HalfStage<CODEC>::in_tail(108u));
+        else if constexpr (CODEC == kQ6_K) dd = *reinterpret_cast<const uint16_t*>(row + HalfStage<CODEC>::in_tail(208u));
+        else dd = *reinterpret_cast<const uint32_t*>(row + HalfStage<CODEC>::in_tail(80u));
+        const float d = kPlaneRatio * half_bits_to_float(dd & 0xffffu), dmin = half_bits_to_float(dd >> 16);
+        float minimum[kStageBlocks / 2];  // of sub-blocks 2 j + half
+        if constexpr (W::kMinima) {
+#pragma unroll
+            for (int j = 0; j < kStageBlocks / 2; j++) {
+                uint32_t sc, mn;
+                q4k_scale_min(shared.header, 2u * j + half, sc, mn);
+                minimum[j] = dmin * static_cast<float>(mn);
+            }
+        }
+#pragma unroll
+        for (int m = 0; m < MT; m++) {
+            v16f below = zero;  // K = 2 per instruction, lane half h supplies sub-block 2 j + h
+            if constexpr (W::kMinima) {
+#pragma unroll
+                for (int j = 0; j < kStageBlocks / 2; j++)
+                    below = __builtin_amdgcn_mfma_f32_32x32x2f32(
+                        *reinterpret_cast<const float*>(lds + W::kSumsAt + (wave_m * MT + m) * 1024u + (2u * j + half) * 128u + in_half * 4u),
+                        minimum[j], below, 0, 0, 0);
+            }
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const float4 units = *reinterpret_cast<const float4*>(lds + W::kUnitsAt + (wave_m * MT + m) * 128u + (8u * j + 4u * half) * 4u);
+                const float unit[4] = {units.x, units.y, units.z, units.w};
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const int r = 4 * j + i;
+                    if constexpr (W::kMinima) acc[m][r] += fmaf(p[0][m][r], unit[i] * d, -below[r]);
+                    else if constexpr (CODEC == kQ6_K) acc[m][r] = fmaf(fmaf(16.0f, p[P - 1][m][r], p[0][m][r]), unit[i] * d, acc[m][r]);
+                    else if constexpr (CODEC == kQ2_K)
+                        acc[m][r] = fmaf(fmaf(p[0][m][r], d, -p[P - 1][m][r] * (kPlaneRatio * dmin)), unit[i], acc[m][r]);
+                    else acc[m][r] = fmaf(p[0][m][r], unit[i] * d, acc[m][r]);
+                }
+            }
+        }
+        shared = shared_next;
+    }
+
+    // ---- add bias, store ----
+    const uint64_t launch_rows = static_cast<uint64_t>(group.row_tiles) * W::kRows;
+    const uint32_t in_tile = wave_n * 32u + in_half, n_out = row0 + in_tile;
+    if (n_out >= rows) return;
+    const float bias = member.bias != nullptr ? member.bias[n_out] : 0.f;
+    const uint32_t launch_row = row_tile * W::kRows + in_tile;  // among the rows of all members
+#pragma unroll
+    for (int m = 0; m < MT; m++) {
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            const uint32_t v = (first_vector_tile + m) * 32u + 8u * (r >> 2) + 4u * half + (r & 3u);
+            if (v >= vectors) continue;
+            if (k_splits == 1) {
+                // residual may be y itself: every output is read, then written, by this lane only
+                const uint64_t at = static_cast<uint64_t>(v) * rows + n_out;
+                const float value = acc[m][r] + bias;
+                member.y[at] = member.residual != nullptr ? value + member.residual[at] : value;
+            } else {
+                partials[(static_cast<uint64_t>(k_share) * vectors + v) * launch_rows + launch_row] = acc[m][r];
+            }
+        }
+    }
+}
+
+template <int CODEC>
+hipError_t launch(const Group& group, const uint8_t* tiles, uint32_t columns, uint32_t vectors, uint32_t k_splits,
+                  float* partials, hipStream_t stream) {
+    using W = Wide<CODEC>;
+    static_assert(W::kRows == gemm_h16_wide_rows(CODEC), "the planner's tile height");
+    const auto kernel = gemm_h16_wide_kernel<CODEC>;
+    // More than 64 KiB of dynamic LDS has to be allowed once per kernel and device.
+    static std::atomic<bool> allowed[64] = {};  // callers may enqueue from several threads; setting twice is harmless
+    int device = 0;
+    if (hipError_t status = hipGetDevice(&device)) return status;
+    if (device < 0 || device >= 64) return hipErrorInvalidDevice;
+    if (!allowed[device].load(std::memory_order_acquire)) {
+        if (hipError_t status = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                                    hipFuncAttributeMaxDynamicSharedMemorySize, W::kLdsBytes))
+            return status;
+        allowed[device].store(true, std::memory_order_release);
+    }
+    const uint32_t vector_tiles = (vectors + 31u) / 32u, vector_groups = (vector_tiles + kTiles - 1u) / kTiles;
+    const uint64_t grid = (static_cast<uint64_t>(group.row_tiles) * k_splits + 7u) / 8u * 8u * vector_groups;
+    if (grid > 0x7fffffffull) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(grid)), dim3(64 * kWaves), W::kLdsBytes, stream, group, tiles,
+                       vector_tiles, columns, vectors, k_splits, partials);
+    return hipGetLastError();
+}
+}  // namespace
+
+hipError_t gemm_h16_wide(int32_t codec, const Group& group, const uint8_t* tiles, uint32_t columns, uint32_t vectors,
+                         uint32_t k_splits, float* partials, hipStream_t stream) {
+    switch (codec) {
+        case kQ2_K: return launch<kQ2_K>(group, tiles, columns, vectors, k_splits, partials, stream);
+        case kQ3_K: return launch<kQ3_K>(group, tiles, columns, vectors, k_splits, partials, stream);
+        case kQ4_K: return launch<kQ4_K>(group, tiles, columns, vectors, k_splits, partials, stream);
+        case kQ5_K: return launch<kQ5_K>(group, tiles, columns, vectors, k_splits, partials, stream);
+        case kQ6_K: return launch<kQ6_K>(group, tiles, columns, vectors, k_splits, partials, stream);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+}  // namespace et

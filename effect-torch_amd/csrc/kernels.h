@@ -6,6 +6,8 @@
 
 #include <cstdint>
 
+#include "et_codecs.h"
+
 namespace et {
 
 constexpr int kMaxRank = 8;
@@ -80,8 +82,8 @@ hipError_t quantize_activations(const float* x, uint64_t x_row_stride, uint64_t 
 // in all a multiple of 4096 bytes.
 // limbs = 1: int8 activations, scale = max|x| / 127.
 // limbs = 3: 24-bit fixed point in three balanced signed bytes, scale = max|x| / (127 * 65536).
-// limbs = 2 is the layout of gemm_h16: 24-bit fixed point per vector and 256-column stage in two
-// balanced 12-bit halves, each a half float:
+// limbs = 2 is the layout of gemm_h16: x in units of max|x| / (2^23 - 1) per vector and 256-column stage, as a whole
+// multiple of 4096 and a rest, each a half float (quantize_halves.h):
 //   half l (0: low / 4096, 1: high), 8-column part c (0..31), vector m: 8 half floats at  l*16384 + c*512 + m*16
 //   unit[m] f32 (max|x| / (2^23 - 1)) at  32768 + m*4
 //   xsum[sub-block g (0..7)][m] f32 at  32768 + 128 + g*128 + m*4
@@ -149,12 +151,16 @@ struct GemmMember {
     float* y;               // [vectors, rows]
     uint64_t rows;
 };
-// Rows per workgroup (64 or 128), row tiles of that height over all members, K shares.
+// Rows per workgroup, row tiles of that height over all members, K shares; wide: gemm_h16_wide.hip's kernel, with 128
+// vectors per workgroup instead of 32.
 struct GemmGroupGeometry {
     uint32_t tile_rows;
     uint64_t row_tiles;
     uint32_t k_splits;
+    bool wide = false;
 };
+constexpr uint32_t kGemmWideVectors = 128;
+constexpr uint32_t gemm_h16_wide_rows(int32_t codec) { return codec == kQ2_K || codec == kQ6_K ? 128u : 256u; }
 GemmGroupGeometry gemm_h16_group_geometry(int32_t codec, const uint64_t* rows, uint32_t count, uint64_t columns,
                                           uint64_t vectors);
 uint64_t gemm_h16_group_partial_bytes(int32_t codec, const uint64_t* rows, uint32_t count, uint64_t columns,

@@ -288,6 +288,8 @@ const char* kernel_name(const et_linear_plan& plan) {
         case LinearKernel::kGemmLimb:
             return plan.k_splits > 1 ? "quantize_limbs+gemm_i8+reduce" : "quantize_limbs+gemm_i8";
         case LinearKernel::kGemmHalf:
+            if (gemm_h16_group_geometry(plan.codec, &plan.rows, 1, plan.columns, plan.vectors).wide)
+                return plan.k_splits > 1 ? "quantize_halves+gemm_h16_wide+reduce" : "quantize_halves+gemm_h16_wide";
             return plan.k_splits > 1 ? "quantize_halves+gemm_h16+reduce" : "quantize_halves+gemm_h16";
     }
     return "?";

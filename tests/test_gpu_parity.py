@@ -265,6 +265,39 @@ def test_linear_many_vectors_f32_matrix_core_tiles(et, device, codec, vectors, r
     close(got, exact, oracle_noise=0)
 
 
+@pytest.mark.parametrize("codec,vectors,rows,columns", [
+    (oracle.Q4_K, 65, 14001, 4096),   # the last tile of 32 vectors holds one; a ragged last row tile; K shares
+    (oracle.Q4_K, 1000, 14300, 256),  # one stage: nothing to prefetch; 104 vectors in the last group
+    (oracle.Q4_K, 385, 8001, 4352),   # one vector in the last group; seventeen stages in uneven shares
+    (oracle.Q4_K, 129, 14336, 8448),
+    (oracle.Q5_K, 128, 14336, 4096),  # whole tiles
+    (oracle.Q5_K, 385, 4001, 4096),
+    (oracle.Q3_K, 70, 14100, 5120),
+    (oracle.Q6_K, 1000, 8000, 256),   # two operands per weight: 128-row tiles, half of the waves' vectors may be padding
+    (oracle.Q6_K, 225, 4097, 2304),
+    (oracle.Q2_K, 161, 14336, 4096),
+    (oracle.Q2_K, 480, 4096, 4352),
+])
+def test_prompts_on_the_wide_kernel(et, device, codec, vectors, rows, columns):
+    rng = np.random.default_rng(rows + columns + vectors)
+    weight = synth.random_weight(codec, rows, columns, rng)
+    x = synth.random_activations(vectors, columns, rng)
+    x[vectors // 2, :300] = 0.0  # a whole stage and part of the next: unit 0
+    bias = rng.standard_normal(rows).astype(np.float32)
+    assert "gemm_h16_wide" in et.RawLinear(et.GgmlQuant(codec), rows, columns, vectors, True).requirements.kernel
+    print(f"wide codec={codec} vectors={vectors} rows={rows} columns={columns}", flush=True)
+    got = run_linear(et, device, codec, rows, columns, x, weight, bias)
+    again = run_linear(et, device, codec, rows, columns, x, weight, bias)
+    assert np.array_equal(got, again)
+    decoded = et.dequantize_rows(to_dev(weight, device), et.GgmlQuant(codec), (rows, columns)).double()
+    exact = (to_dev(x, device).double() @ decoded.T + to_dev(bias, device).double()).cpu().numpy()
+    close(got, exact, oracle_noise=0)
+    # Rounding errors of random sign, each at most half an ulp (rms 2^-24 / sqrt(3) of the running sum, whose square grows
+    # evenly): 32 matrix instructions per stage chain, 33 stages at most, a handful per element: sqrt(32/2 + 33/2 + 4) of them
+    # are 2.1e-7, the activations' own rounding 1e-7
+    assert np.linalg.norm(got - exact) <= 2.5e-7 * np.linalg.norm(exact)
+
+
 @pytest.mark.parametrize("mode", ["F32", "INT8"])
 @pytest.mark.parametrize("codec,vectors,rows,columns", [(oracle.Q4_K, 32, 1024, 4096), (oracle.Q4_K, 32, 4096, 4096),
                                                         (oracle.Q4_K, 32, 4096, 14336), (oracle.Q5_K, 32, 4096, 4096),
