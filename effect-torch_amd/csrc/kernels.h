@@ -249,11 +249,13 @@ struct KvAttention {
     KvProjected projected = {};
 };
 // Calls of several tokens per slot attend on the matrix cores (kv_chunk.hip) once the streaming kernel would read this
-// many cached rows, counting one per workgroup and position of the caller's context bound. Measured (us, streaming /
-// chunk kernel with its append and merge launches; 32/8 heads x 128, f16 unless named, slots x tokens at context):
-// 1x8 at 2000 (128 Ki rows) 17.6 / 18, 4x16 at 256 (128 Ki) 18.2 / 17; 1x16 at 2000 (256 Ki) 25.8 / 23.3, bf16 24.1 / 24.5,
-// u8 26.5 / 27; 1x64 at 2000 (1 Mi) 72 / 30; 2x500 at 2000 (16 Mi) 1034 / 77, bf16 1097 / 99, u8 1322 / 112.
-constexpr uint64_t kKvChunkMinRows = 192 * 1024;
+// many cached rows, counting one per workgroup and position of the caller's context bound, and where that many
+// workgroups share them. Measured (us, streaming / chunk kernel with its append and merge launches; 32/8 heads x 128,
+// slots x tokens at context): 1x16 at 2000 (256 Ki rows, 32 workgroups) u8 25.3 / 30.0; 1x32 at 2000 (512 Ki, 32)
+// u8 37.1 / 41.0, bf16 34.0 / 39.7; 6x16 at 600 (450 Ki, 96) f16 45.0 / 25.5; 8x16 at 512 (512 Ki, 64) u8 56.2 / 29.2;
+// 1x64 at 2000 (1 Mi, 64) f16 71 / 34; 2x500 at 2000 (16 Mi, 256) f16 1036 / 83, bf16 1097 / 107, u8 1322 / 110.
+constexpr uint64_t kKvChunkMinRows = 384 * 1024;
+constexpr uint64_t kKvChunkMinWorkgroups = 64;
 bool kv_chunk_supported(const KvAttention& p);
 struct KvChunkGrid {
     int row_waves;   // 32 query rows each: 4, or 2 where a slot has no more

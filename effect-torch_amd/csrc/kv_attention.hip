@@ -794,12 +794,14 @@ KvLaunchShape kv_attention_shape(const KvAttention& p) {
         const uint64_t room = static_cast<uint64_t>(kKvTableEntries - 2) * p.block_size;
         const uint64_t reach = room > 2 * grid.round ? room - grid.round : grid.round;
         splits = std::max(splits, (context + reach - 1) / reach);
-        shape.chunk = true;
-        shape.waves = 8;
-        shape.splits = static_cast<uint32_t>(splits);
-        shape.workgroups = grid.units * splits;
-        shape.workspace_bytes = splits > 1 ? queries * splits * (p.width + 2) * sizeof(float) : 0;
-        return shape;
+        if (grid.units * splits >= kKvChunkMinWorkgroups) {
+            shape.chunk = true;
+            shape.waves = 8;
+            shape.splits = static_cast<uint32_t>(splits);
+            shape.workgroups = grid.units * splits;
+            shape.workspace_bytes = splits > 1 ? queries * splits * (p.width + 2) * sizeof(float) : 0;
+            return shape;
+        }
     }
     shape.streaming = g != 0;
     const uint64_t rows = static_cast<uint64_t>(p.active_batch) * p.tokens *

@@ -16,7 +16,11 @@
 //
 // Precision: K and V enter the matrix cores as the slab holds them (f16, bf16, or the u8 tier's integers, all exact);
 // q and the weights are f32 and enter in pieces whose sum they are to 22 bits (two half floats; q scaled by a power
-// of two per row and the weights by 2^12, so that the pieces stay normal) or 24 bits (three bfloat16). Sums are f32.
+// of two per row and the weights by 2^12, so that the pieces stay normal) or 24 bits (three bfloat16). Sums are f32, in
+// short chains: four column chunks of a score, or a step's positions of an output, from zero and the small pieces first,
+// then added to the total. One chain over everything was the larger part of the error (against 64 bits, 1e-7, two slots
+// of 500 tokens at context 2000, streaming kernel / one chain / this: f16 2.4 / 4.3 / 2.6, u8 with 5 x 12 tokens
+// 3.0 / 4.9 / 2.9) and the chains cost 6 us there.
 //
 // Eight waves in kGroups groups of kRowWaves: the waves of a group share 32 query rows each, the groups take tiles of
 // positions in turn and meet in LDS at the end, so that each SIMD has two waves to issue from. Tiles lie in LDS as in
@@ -24,9 +28,9 @@
 // is copied (global_load_lds; the u8 tier passes through registers, where it becomes half floats and bfloat16) while
 // this one is contracted.
 //
-// Bound: the matrix pipe. A round of 128 positions of a compute unit is 128 matrix instructions per SIMD, 4096 clocks of
-// the 5300 it takes (two slots of 500 tokens at context 2000, 32/8 heads x 128, f16: 77 us, the kernel alone 70, where
-// the streaming kernel took 1034).
+// Bound: the matrix pipe. A round of 128 positions of a compute unit is 128 matrix instructions per SIMD, 4096 clocks
+// (two slots of 500 tokens at context 2000, 32/8 heads x 128, f16: 83 us with the other launches, where the streaming
+// kernel took 1036; bf16 107 / 1097, u8 110 / 1322).
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 
@@ -199,6 +203,50 @@ __device__ __forceinline__ uint2 read_transposed(const uint8_t* from) {
     return u.raw;
 }
 
+__device__ __forceinline__ float slab_value(const __half* slab, const float*, uint64_t row, int width, int column) {
+    return slab_load(slab, row * width + column);
+}
+__device__ __forceinline__ float slab_value(const Bf16* slab, const float*, uint64_t row, int width, int column) {
+    return slab_load(slab, row * width + column);
+}
+__device__ __forceinline__ float slab_value(const U8* slab, const float* scales, uint64_t row, int width, int column) {
+    return u8_value(slab[row * width + column].byte, scales[row]);
+}
+
+// One query row over positions [begin, end) by one wave in plain f32, position by position: the row's maximum, the sum of
+// its weights and its weighted values.
+template <typename T, int W>
+__device__ void attend_row(const KvArgs& a, uint32_t slot, uint32_t kv_head, uint64_t query, uint32_t begin, uint32_t end,
+                           int lane, float& m, float& l, float (&o)[W / 64]) {
+    const T *k_slab = static_cast<const T*>(a.k_slab), *v_slab = static_cast<const T*>(a.v_slab);
+    m = kLowest;
+    l = 0.f;
+#pragma unroll
+    for (int i = 0; i < W / 64; i++) o[i] = 0.f;
+    for (uint32_t first = begin; first < end; first += 64) {
+        const uint32_t position = min(first + lane, end - 1), count = min(end - first, 64u);
+        const uint64_t block = static_cast<uint64_t>(a.table[static_cast<uint64_t>(slot) * a.table_stride + block_of(a, position)]) *
+                               a.block_size;
+        const uint32_t at = block >= a.max_tokens ? 0u : min(static_cast<uint32_t>(block) + within_block(a, position), a.max_tokens - 1);
+        const uint64_t key = static_cast<uint64_t>(at) * a.kv_heads + kv_head;
+        float dot = 0.f;
+        for (int column = 0; column < W; column++) dot = fmaf(a.q[query * W + column], slab_value(k_slab, a.k_scales, key, W, column), dot);
+        const float score = static_cast<uint32_t>(lane) < count ? dot * a.scale_log2 : -INFINITY;
+        const float next = fmaxf(m, group_max<64>(score)), keep = __builtin_amdgcn_exp2f(m - next);
+        m = next;
+        const float weight = static_cast<uint32_t>(lane) < count ? __builtin_amdgcn_exp2f(score - m) : 0.f;
+        l = fmaf(l, keep, group_sum<64>(weight));
+#pragma unroll
+        for (int i = 0; i < W / 64; i++) o[i] *= keep;
+        for (uint32_t p = 0; p < count; p++) {
+            const float w = __shfl(weight, static_cast<int>(p));
+            const uint64_t value = static_cast<uint64_t>(__shfl(at, static_cast<int>(p))) * a.kv_heads + kv_head;
+#pragma unroll
+            for (int i = 0; i < W / 64; i++) o[i] = fmaf(w, slab_value(v_slab, a.v_scales, value, W, lane + 64 * i), o[i]);
+        }
+    }
+}
+
 template <typename T, int W, int RW>
 __global__ __launch_bounds__(kChunkThreads, 2) void kv_chunk_kernel(const KvArgs a) {
     using S = Slab<T>;
@@ -358,11 +406,11 @@ __global__ __launch_bounds__(kChunkThreads, 2) void kv_chunk_kernel(const KvArgs
     }
 
     float m = kLowest, l = 0.f;
-    v16f o[kDimTiles];
+    v16f o[kDimTiles], zero;
 #pragma unroll
-    for (int t = 0; t < kDimTiles; t++)
+    for (int r = 0; r < 16; r++) zero[r] = 0.f;
 #pragma unroll
-        for (int r = 0; r < 16; r++) o[t][r] = 0.f;
+    for (int t = 0; t < kDimTiles; t++) o[t] = zero;
 
     // K operand of a 32-position block: position in_half, pieces 2c + half. V operand: positions
     // 16c + 8a + 4 half + (0..3), of which this lane's address names row (lane & 15) / 4 and four of sixteen columns.
@@ -379,17 +427,19 @@ __global__ __launch_bounds__(kChunkThreads, 2) void kv_chunk_kernel(const KvArgs
 #pragma unroll
             for (int u = 0; u < U; u++)
 #pragma unroll
-                for (int r = 0; r < 16; r++) score[u][r] = 0.f;
+                for (int first = 0; first < kKeyChunks; first += 4) {
+                    typename KE::v8 key[4];
 #pragma unroll
-            for (int c = 0; c < kKeyChunks; c++) {
+                    for (int c = 0; c < 4; c++)
+                        key[c] = *reinterpret_cast<const typename KE::v8*>(buffer + 32 * (b + u) * Shape::kRowBytes + key_row +
+                                                                           (((2 * (first + c) + half) ^ key_swizzle) << 4));
+                    v16f sum = zero;
 #pragma unroll
-                for (int u = 0; u < U; u++) {
-                    const typename KE::v8 key = *reinterpret_cast<const typename KE::v8*>(
-                        buffer + 32 * (b + u) * Shape::kRowBytes + key_row + (((2 * c + half) ^ key_swizzle) << 4));
+                    for (int p = KE::kPieces - 1; p >= 0; p--)
 #pragma unroll
-                    for (int p = 0; p < KE::kPieces; p++) score[u] = KE::mfma(key, q[p][c], score[u]);
+                        for (int c = 0; c < 4; c++) sum = KE::mfma(key[c], q[p][first + c], sum);
+                    score[u] = first == 0 ? sum : score[u] + sum;
                 }
-            }
             if constexpr (S::kScaled) {
 #pragma unroll
                 for (int u = 0; u < U; u++)
@@ -427,6 +477,9 @@ __global__ __launch_bounds__(kChunkThreads, 2) void kv_chunk_kernel(const KvArgs
 #pragma unroll
                     for (int r = 0; r < 16; r++) o[t][r] *= keep;
             }
+            // The weights of the whole step, then the values 32 columns at a time.
+            typename VE::v8 pieces[2 * U][VE::kPieces];
+            float step_sum = 0.f;
 #pragma unroll
             for (int u = 0; u < U; u++) {
 #pragma unroll
@@ -435,7 +488,7 @@ __global__ __launch_bounds__(kChunkThreads, 2) void kv_chunk_kernel(const KvArgs
 #pragma unroll
                     for (int i = 0; i < 8; i++) {
                         weight[i] = __builtin_amdgcn_exp2f(fmaf(score[u][8 * c + i], unit, -m));
-                        l += weight[i];
+                        step_sum += weight[i];
                     }
                     if constexpr (S::kScaled) {
 #pragma unroll
@@ -448,25 +501,30 @@ __global__ __launch_bounds__(kChunkThreads, 2) void kv_chunk_kernel(const KvArgs
                             weight[4 * j + 3] *= v4.w;
                         }
                     }
-                    typename VE::v8 pieces[VE::kPieces];
-                    split<VE>(weight, pieces);
-                    union {
-                        uint2 raw[2];
-                        typename VE::v8 all;
-                    } value[kDimTiles];
-#pragma unroll
-                    for (int t = 0; t < kDimTiles; t++)
-#pragma unroll
-                        for (int h = 0; h < 2; h++) {
-                            const uint32_t r = 32 * (b + u) + 16 * c + 8 * h + value_row;
-                            value[t].raw[h] = read_transposed(values + r * Shape::kRowBytes +
-                                                              (((4 * t + value_piece) ^ Shape::swizzle(r)) << 4) + (lane & 1) * 8);
-                        }
-#pragma unroll
-                    for (int p = 0; p < VE::kPieces; p++)
-#pragma unroll
-                        for (int t = 0; t < kDimTiles; t++) o[t] = VE::mfma(value[t].all, pieces[p], o[t]);
+                    split<VE>(weight, pieces[2 * u + c]);
                 }
+            }
+            l += step_sum;
+#pragma unroll
+            for (int t = 0; t < kDimTiles; t++) {
+                union {
+                    uint2 raw[2];
+                    typename VE::v8 all;
+                } value[2 * U];
+#pragma unroll
+                for (int c = 0; c < 2 * U; c++)
+#pragma unroll
+                    for (int h = 0; h < 2; h++) {
+                        const uint32_t r = 32 * b + 16 * c + 8 * h + value_row;
+                        value[c].raw[h] = read_transposed(values + r * Shape::kRowBytes +
+                                                          (((4 * t + value_piece) ^ Shape::swizzle(r)) << 4) + (lane & 1) * 8);
+                    }
+                v16f sum = zero;
+#pragma unroll
+                for (int p = VE::kPieces - 1; p >= 0; p--)
+#pragma unroll
+                    for (int c = 0; c < 2 * U; c++) sum = VE::mfma(value[c].all, pieces[c][p], sum);
+                o[t] += sum;
             }
         }
     };
@@ -483,6 +541,11 @@ __global__ __launch_bounds__(kChunkThreads, 2) void kv_chunk_kernel(const KvArgs
             __syncthreads();
         }
     }
+    // NaN where a sum is not finite
+#pragma unroll
+    for (int t = 0; t < kDimTiles; t++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) l = fmaf(o[t][r], 0.f, l);
     l += other_half(l, lane);
 
     // All groups leave their sums in LDS (the tiles and the table are read no more); each group's wave then joins a
@@ -498,7 +561,6 @@ __global__ __launch_bounds__(kChunkThreads, 2) void kv_chunk_kernel(const KvArgs
 #pragma unroll
         for (int r = 0; r < 16; r++) sums_of(group, t)[64 * r] = o[t][r];
     __syncthreads();
-    if (row >= rows || !s.ok) return;
     float share_of[kGroups], top = kLowest, total = 0.f;
 #pragma unroll
     for (int g = 0; g < kGroups; g++) top = fmaxf(top, weights_of(g)[0]);
@@ -507,25 +569,52 @@ __global__ __launch_bounds__(kChunkThreads, 2) void kv_chunk_kernel(const KvArgs
         share_of[g] = __builtin_amdgcn_exp2f(weights_of(g)[0] - top);
         total = fmaf(share_of[g], weights_of(g)[64], total);
     }
-    float* record = a.partial + (query * a.splits + split_index) * (W + 2);
-    if (a.splits != 1 && group == 0 && half == 0) {
-        record[0] = top;
-        record[1] = total;
-    }
-    float* to = (a.splits == 1 ? a.out + query * W : record + 2) + 4 * half;
-    const float divisor = a.splits == 1 ? total : 1.0f;
-    for (int t = group; t < kDimTiles; t += kGroups) {
+    const bool live = row < rows && s.ok, again = live && !(fabsf(total) < INFINITY);
+    if (live && !again) {
+        float* record = a.partial + (query * a.splits + split_index) * (W + 2);
+        if (a.splits != 1 && group == 0 && half == 0) {
+            record[0] = top;
+            record[1] = total;
+        }
+        float* to = (a.splits == 1 ? a.out + query * W : record + 2) + 4 * half;
+        const float divisor = a.splits == 1 ? total : 1.0f;
+        for (int t = group; t < kDimTiles; t += kGroups) {
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            v4f joined;
+            for (int j = 0; j < 4; j++) {
+                v4f joined;
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                float value = 0.f;
+                for (int i = 0; i < 4; i++) {
+                    float value = 0.f;
 #pragma unroll
-                for (int g = 0; g < kGroups; g++) value = fmaf(share_of[g], sums_of(g, t)[64 * (4 * j + i)], value);
-                joined[i] = value / divisor;
+                    for (int g = 0; g < kGroups; g++) value = fmaf(share_of[g], sums_of(g, t)[64 * (4 * j + i)], value);
+                    joined[i] = value / divisor;
+                }
+                *reinterpret_cast<v4f*>(to + 32 * t + 8 * j) = joined;
             }
-            *reinterpret_cast<v4f*>(to + 32 * t + 8 * j) = joined;
+        }
+    }
+    // An infinity or NaN in a K or V row spoils the matrix products of every query row it shares a tile with, also of those
+    // that do not see its position, and a product of pieces overflows or meets inf - inf before the product itself does.
+    // Such rows are attended to once more, without pieces and over their own positions alone.
+    uint64_t left = __builtin_amdgcn_ballot_w64(again) & 0xffffffffull;
+    for (int turn = 0; left != 0; left &= left - 1, turn++) {
+        if (turn % kGroups != group) continue;
+        const int which = __builtin_ctzll(left);
+        const uint32_t begin_of = __shfl(max(row_begin, my_begin), which), end_of = __shfl(min(row_end, my_end), which);
+        const uint32_t at = first_row + 32 * row_wave + which;
+        const uint64_t query_of = (static_cast<uint64_t>(slot) * a.query_heads + kv_head * group_size + at % group_size) * a.tokens +
+                                  at / group_size;
+        float m_of, l_of, o_of[W / 64];
+        attend_row<T, W>(a, slot, kv_head, query_of, begin_of, end_of, lane, m_of, l_of, o_of);
+        float* record = a.partial + (query_of * a.splits + split_index) * (W + 2);
+        if (a.splits != 1 && lane == 0) {
+            record[0] = m_of;
+            record[1] = l_of;
+        }
+#pragma unroll
+        for (int i = 0; i < W / 64; i++) {
+            if (a.splits == 1) a.out[query_of * W + lane + 64 * i] = o_of[i] / l_of;
+            else record[2 + lane + 64 * i] = o_of[i];
         }
     }
 }

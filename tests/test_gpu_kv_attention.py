@@ -196,15 +196,15 @@ def test_long_context_is_split(et, device, dtype):
 # `bound`: the caller's bound of the context, by which the kernel is chosen and the context split
 @pytest.mark.parametrize("dtype", [np.float16, "bf16", "u8"])
 @pytest.mark.parametrize("width,query_heads,kv_heads,tokens,contexts,advances,windows,bound,split", [
-    (128, 4, 1, 2, [0, 62, 127], [2, 2, 1], (0, 0), 40000, True),     # the fewest tokens; most splits are empty
-    (128, 3, 1, 43, [85, 21, 1], [43, 43, 40], (0, 0), 4000, True),   # 129 query rows: one past a workgroup's
+    (128, 4, 1, 2, [0, 62, 127], [2, 2, 1], (0, 0), 70000, True),     # the fewest tokens; most splits are empty
+    (128, 3, 1, 43, [85, 21, 1], [43, 43, 40], (0, 0), 8000, True),   # 129 query rows: one past a workgroup's
     (128, 24, 8, 43, [0, 20, 85, 96] * 5, [43, 43, 43, 1] * 5, (0, 0), 200, False),  # the same without splits
     (128, 8, 8, 32, [96, 300] * 16, [32] * 32, (0, 0), 332, False),   # one query head per kv head, 32 rows
-    (64, 8, 1, 33, [223, 0, 95], [33, 33, 33], (0, 0), 4000, True),   # width 64: a round is 256 positions
+    (64, 8, 1, 33, [223, 0, 95], [33, 33, 33], (0, 0), 8000, True),   # width 64: a round is 256 positions
     (64, 16, 8, 9, [223, 247, 40, 3] * 8, [9] * 32, (0, 0), 256, False),
-    (128, 8, 2, 20, [3000, 2500], [20, 7], (0, 0), 3020, True),       # full splits
+    (128, 8, 2, 20, [3000, 2500], [20, 7], (0, 0), 10000, True),       # full splits
     (128, 8, 2, 70, [400, 333], [70, 70], (0, 37), 3000, True),       # rows of a wave that see disjoint positions
-    (64, 4, 2, 65, [500, 120], [65, 64], (210, 0), 3000, True),
+    (64, 4, 2, 65, [500, 120], [65, 64], (210, 0), 8000, True),
 ])
 def test_chunks_on_the_matrix_cores(et, device, dtype, width, query_heads, kv_heads, tokens, contexts, advances, windows,
                                     bound, split):
@@ -223,6 +223,26 @@ def test_chunks_on_the_matrix_cores(et, device, dtype, width, query_heads, kv_he
     assert np.abs(got[0] - want[0]).max() <= 1e-5
     again = run_gpu(et, device, case, scale, max_context=bound, **options)
     assert np.array_equal(got[0].view(np.uint32), again[0].view(np.uint32))
+
+
+@pytest.mark.parametrize("dtype", [np.float16, "bf16"])
+@pytest.mark.parametrize("width,bound", [(128, 300), (128, 9000), (64, 300)])  # one split, several, the narrow kernel
+def test_values_that_are_not_finite_stay_with_the_rows_that_see_them(et, device, dtype, width, bound):
+    rng = np.random.default_rng(width + bound)
+    tokens, slots = 40, 20
+    case = make_case(rng, slots=slots, query_heads=8, kv_heads=2, width=width, block_size=16, contexts=[70, 257] * 10, tokens=tokens,
+                     advances=[tokens] * slots, dtype=dtype)
+    case["v"][0, 0, 33, 5] = np.inf       # seen by the tokens from 33 on
+    case["v"][1, 1, 39, 7] = np.nan
+    case["k"][2, 0, 30, 3] = np.inf       # a score of +inf or -inf, by the sign of q
+    case["k"][3, 1, 39, 2] = -np.inf
+    case["q"][4, 3, 11, 1] = np.nan
+    scale = 1.0 / np.sqrt(width)
+    got = run_gpu(et, device, case, scale, max_context=bound)
+    assert et.kv_attention_kernel(got[3], 8, tokens).startswith("kv_append+kv_chunk")
+    want = run_oracle(case, scale)
+    assert np.isinf(want[0]).any() and np.isnan(want[0]).any() and np.isfinite(want[0]).mean() > 0.9
+    np.testing.assert_allclose(got[0], want[0], rtol=0, atol=1e-4)  # this file's bar; the same infinities and NaN
 
 
 def test_one_workspace_serves_calls_of_any_geometry(et, device):
