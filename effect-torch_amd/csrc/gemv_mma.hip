@@ -54,7 +54,7 @@ constexpr uint32_t kMostGroups = 4u;    // groups of a range: its rows' partial 
 
 // Per consumer wave: [limb planes of one vector, 544 bytes apart][sums and unit per vector and 256 columns]. Once the A operands are in registers the first part holds the
 // wave's partial sums: [group][vector group][lane].
-constexpr uint32_t kSumsFloats = 12u;  // of one (vector, unit): eight sums, the unit, padding to whole float4s
+constexpr uint32_t kSumsFloats = 12u;  // of one (vector, unit): eight sums, one or four units of limb 0, whole float4s
 constexpr uint32_t kLimbPitch = 544u;  // 512 bytes of a limb plane + 32: the three planes start in different banks
 constexpr uint32_t kSumsAt = 2048u, kWaveScratch = 2048u + 8u * 2u * kSumsFloats * 4u;
 static_assert(3u * kLimbPitch <= kSumsAt && kMostGroups * 2u * 256u <= kSumsAt, "planes and partial sums share the first part");
@@ -96,18 +96,28 @@ __device__ __forceinline__ void split_quad(int x0, int x1, int x2, int x3, uint3
     limb[2] = (__builtin_amdgcn_perm(d, c, 0x05040100u) + 0x40404040u) ^ 0x80808080u;
 }
 
+// sum += unit * (the value of three limb sums), which start anew.
+__device__ __forceinline__ void scaled_limbs(int (&acc)[3], float unit, float& sum) {
+    float f = static_cast<float>(acc[0]);
+    f = fmaf(256.0f, static_cast<float>(acc[1]), f);
+    f = fmaf(65536.0f, static_cast<float>(acc[2]), f);
+    sum = fmaf(unit, f, sum);
+    acc[0] = acc[1] = acc[2] = 0;
+}
+
 // ---------------------------------------------------------------------------
 // Codec traits: one 256-column unit (kUnitBytes) of sixteen rows against the A operands.
 //   rp     the unit in the lane's row of the LDS image
 //   q      the lane's K index: which 8 of a block's 32 columns its operand registers hold
 //   a      A operands of the wave's sixteen 32-column blocks, per group of four vectors
-//   sums   f32 sums of the lane's vector over the unit's eight blocks, then the value of one unit of limb 0
+//   sums   f32 sums of the lane's vector over the unit's eight blocks, then the value of one unit of limb 0:
+//          SCALES = 1 for all of the unit's columns, SCALES = 4 for every 64 of them
 //          (next vector group: + sums_step floats)
 // ---------------------------------------------------------------------------
 struct Q4KMma {
     static constexpr uint32_t kUnitBytes = 144u;  // one super-block
     static __device__ __forceinline__ uint32_t chunk(uint32_t q) { return q; }
-    template <int VG, int UNIT, int BLOCKS>
+    template <int VG, int UNIT, int SCALES, int BLOCKS>
     static __device__ __forceinline__ void contract(const uint8_t* rp, uint32_t q, const long (&a)[VG][BLOCKS],
                                                     const float* sums, uint32_t sums_step, float (&total)[VG]) {
         const uint4 h = *reinterpret_cast<const uint4*>(rp);
@@ -118,8 +128,9 @@ struct Q4KMma {
         // keeps the minima packed, a byte-to-float conversion each, instead of a mask per byte
         asm volatile("" : "+v"(mn[0]), "+v"(mn[1]));
         int acc[VG][3];
+        float pos[VG];
 #pragma unroll
-        for (int g = 0; g < VG; g++) acc[g][0] = acc[g][1] = acc[g][2] = 0;
+        for (int g = 0; g < VG; g++) acc[g][0] = acc[g][1] = acc[g][2] = 0, pos[g] = 0.f;
         const v4i zero = {0, 0, 0, 0};
 #pragma unroll
         for (int p = 0; p < 4; p++) {
@@ -136,6 +147,7 @@ struct Q4KMma {
                 // block dots are below 2^17, scales below 2^6: 24-bit multiplies, exact int32 sums
 #pragma unroll
                 for (int k = 0; k < 3; k++) acc[g][k] += __mul24(c0[k], s_lo) + __mul24(c1[k], s_hi);
+                if constexpr (SCALES == 4) scaled_limbs(acc[g], sums[sums_step * g + 8 + p], pos[g]);
             }
         }
         // (the compiler turns these into v_cvt_f32_ubyte0..3)
@@ -155,10 +167,8 @@ struct Q4KMma {
             neg = fmaf(m5, s1.y, neg);
             neg = fmaf(m6, s1.z, neg);
             neg = fmaf(m7, s1.w, neg);
-            float f = static_cast<float>(acc[g][0]);
-            f = fmaf(256.0f, static_cast<float>(acc[g][1]), f);
-            f = fmaf(65536.0f, static_cast<float>(acc[g][2]), f);
-            total[g] += d * (sums[sums_step * g + 8] * f) - dmin * neg;
+            if constexpr (SCALES == 1) scaled_limbs(acc[g], sums[sums_step * g + 8], pos[g]);
+            total[g] += d * pos[g] - dmin * neg;
         }
     }
 };
@@ -171,7 +181,7 @@ struct Q4KMma {
 struct Q40Mma {
     static constexpr uint32_t kUnitBytes = 144u;  // eight blocks of 18 bytes
     static __device__ __forceinline__ uint32_t chunk(uint32_t q) { return ((q & 1u) << 1) | (q >> 1); }
-    template <int VG, int UNIT, int BLOCKS>
+    template <int VG, int UNIT, int SCALES, int BLOCKS>
     static __device__ __forceinline__ void contract(const uint8_t* rp, uint32_t q, const long (&a)[VG][BLOCKS],
                                                     const float* sums, uint32_t sums_step, float (&total)[VG]) {
         const uint32_t half = q >> 1, shift = (q & 1u) * 4u;
@@ -205,12 +215,13 @@ struct Q40Mma {
                 float f1 = static_cast<float>(c1[0]);
                 f1 = fmaf(256.0f, static_cast<float>(c1[1]), f1);
                 f1 = fmaf(65536.0f, static_cast<float>(c1[2]), f1);
-                pos[g] = fmaf(db, f1, fmaf(da, f0, pos[g]));
+                if constexpr (SCALES == 4) pos[g] = fmaf(sums[sums_step * g + 8 + c], fmaf(db, f1, da * f0), pos[g]);
+                else pos[g] = fmaf(db, f1, fmaf(da, f0, pos[g]));
                 corr[g] = fmaf(db, s[g][2 * c + 1], fmaf(da, s[g][2 * c], corr[g]));
             }
         }
 #pragma unroll
-        for (int g = 0; g < VG; g++) total[g] += sums[sums_step * g + 8] * pos[g] - 8.0f * corr[g];
+        for (int g = 0; g < VG; g++) total[g] += (SCALES == 4 ? pos[g] : sums[sums_step * g + 8] * pos[g]) - 8.0f * corr[g];
     }
 };
 
@@ -219,7 +230,7 @@ struct Q40Mma {
 struct Q5KMma {
     static constexpr uint32_t kUnitBytes = 176u;
     static __device__ __forceinline__ uint32_t chunk(uint32_t q) { return q; }
-    template <int VG, int UNIT, int BLOCKS>
+    template <int VG, int UNIT, int SCALES, int BLOCKS>
     static __device__ __forceinline__ void contract(const uint8_t* rp, uint32_t q, const long (&a)[VG][BLOCKS],
                                                     const float* sums, uint32_t sums_step, float (&total)[VG]) {
         const uint4 h = *reinterpret_cast<const uint4*>(rp);
@@ -229,8 +240,9 @@ struct Q5KMma {
         asm volatile("" : "+v"(mn[0]), "+v"(mn[1]));
         const uint2 fifth = *reinterpret_cast<const uint2*>(rp + 16 + 8 * q);  // columns 8q..8q+7, all sub-blocks
         int acc[VG][3];
+        float pos[VG];
 #pragma unroll
-        for (int g = 0; g < VG; g++) acc[g][0] = acc[g][1] = acc[g][2] = 0;
+        for (int g = 0; g < VG; g++) acc[g][0] = acc[g][1] = acc[g][2] = 0, pos[g] = 0.f;
         const v4i zero = {0, 0, 0, 0};
 #pragma unroll
         for (int p = 0; p < 4; p++) {
@@ -248,6 +260,7 @@ struct Q5KMma {
                 // block dots are below 2^18, scales below 2^6
 #pragma unroll
                 for (int k = 0; k < 3; k++) acc[g][k] += __mul24(c0[k], s_lo) + __mul24(c1[k], s_hi);
+                if constexpr (SCALES == 4) scaled_limbs(acc[g], sums[sums_step * g + 8 + p], pos[g]);
             }
         }
         const float m0 = static_cast<float>(mn[0] & 0xffu), m1 = static_cast<float>((mn[0] >> 8) & 0xffu);
@@ -266,10 +279,8 @@ struct Q5KMma {
             neg = fmaf(m5, s1.y, neg);
             neg = fmaf(m6, s1.z, neg);
             neg = fmaf(m7, s1.w, neg);
-            float f = static_cast<float>(acc[g][0]);
-            f = fmaf(256.0f, static_cast<float>(acc[g][1]), f);
-            f = fmaf(65536.0f, static_cast<float>(acc[g][2]), f);
-            total[g] += d * (sums[sums_step * g + 8] * f) - dmin * neg;
+            if constexpr (SCALES == 1) scaled_limbs(acc[g], sums[sums_step * g + 8], pos[g]);
+            total[g] += d * pos[g] - dmin * neg;
         }
     }
 };
@@ -279,7 +290,7 @@ struct Q5KMma {
 struct Q80Mma {
     static constexpr uint32_t kUnitBytes = 272u;
     static __device__ __forceinline__ uint32_t chunk(uint32_t q) { return q; }
-    template <int VG, int UNIT, int BLOCKS>
+    template <int VG, int UNIT, int SCALES, int BLOCKS>
     static __device__ __forceinline__ void contract(const uint8_t* rp, uint32_t q, const long (&a)[VG][BLOCKS],
                                                     const float* sums, uint32_t sums_step, float (&total)[VG]) {
         float pos[VG];
@@ -305,11 +316,12 @@ struct Q80Mma {
                 float f1 = static_cast<float>(c1[0]);
                 f1 = fmaf(256.0f, static_cast<float>(c1[1]), f1);
                 f1 = fmaf(65536.0f, static_cast<float>(c1[2]), f1);
-                pos[g] = fmaf(db, f1, fmaf(da, f0, pos[g]));
+                if constexpr (SCALES == 4) pos[g] = fmaf(sums[sums_step * g + 8 + c], fmaf(db, f1, da * f0), pos[g]);
+                else pos[g] = fmaf(db, f1, fmaf(da, f0, pos[g]));
             }
         }
 #pragma unroll
-        for (int g = 0; g < VG; g++) total[g] += sums[sums_step * g + 8] * pos[g];
+        for (int g = 0; g < VG; g++) total[g] += SCALES == 4 ? pos[g] : sums[sums_step * g + 8] * pos[g];
     }
 };
 
@@ -474,9 +486,9 @@ __global__ __launch_bounds__(64 * (kConsumers + LOADERS)) void gemv_mma_kernel(
             const uint8_t* rp = lds + min(group * kGroupRows + n, wg_rows - 1u) * pitch + first_unit * T::kUnitBytes;
             const float* of_vector = sums + 2u * q * kSumsFloats;
             constexpr uint32_t kStep = 4u * 2u * kSumsFloats;  // to the next vector group
-            T::template contract<VG, 0>(rp, q, a, of_vector, kStep, total);
+            T::template contract<VG, 0, 1>(rp, q, a, of_vector, kStep, total);
             // in one block with the first: the second unit's LDS reads overtake the first's arithmetic
-            if (my_units > 1u) T::template contract<VG, 1>(rp + T::kUnitBytes, q, a, of_vector + kSumsFloats, kStep, total);
+            if (my_units > 1u) T::template contract<VG, 1, 1>(rp + T::kUnitBytes, q, a, of_vector + kSumsFloats, kStep, total);
         }
 #pragma unroll
         for (int g = 0; g < VG; g++) partial[(group * VG + g) * 64u + lane_id] = total[g];
@@ -509,8 +521,9 @@ __global__ __launch_bounds__(64 * (kConsumers + LOADERS)) void gemv_mma_kernel(
 // image of W lies slice after slice - [slice][row][slice bytes, padded to an odd number of 16-byte pieces so that
 // sixteen rows at one column offset spread over the banks] - and lands in that order, so the first slices are
 // contracted while the last ones are still in flight.
-// Activations are 24-bit fixed point per vector and unit (the launches of gemv_limb.hip that this replaces hold 24 bits
-// too): X = rint(x * 127 * 2^16 / max|x|), limbs in [-128, 127].
+// Activations are 24-bit fixed point per vector and 64 columns, as in gemv_limb.hip, whose launches this replaces:
+// X = rint(x * 127 * 2^16 / max|x|), limbs in [-128, 127]. One unit per 256 columns would let a single large activation
+// coarsen 255 others instead of 63.
 // ---------------------------------------------------------------------------
 constexpr uint32_t kSliceUnits = kConsumers;
 constexpr int kWideGroups = 2;
@@ -524,7 +537,7 @@ __host__ __device__ constexpr uint32_t wide_scratch(uint32_t row_units, uint32_t
 constexpr float kWideRange = 8323072.0f;  // 127 * 2^16
 
 // One (unit, vector) of the prepared activations: the three rows of the A operand that are the vector's,
-// [block pair][limb][K index][16 bytes], then the f32 sums of the unit's eight blocks and the unit of limb 0. Nothing is
+// [block pair][limb][K index][16 bytes], then the f32 sums of the unit's eight blocks and the four units of limb 0. Nothing is
 // kept for the zero rows and absent vectors: every workgroup reads all of this from L2.
 constexpr uint32_t kWideRecordSumsAt = 768u, kWideRecord = 768u + kSumsFloats * 4u;
 
@@ -555,9 +568,7 @@ __global__ __launch_bounds__(64) void gemv_mma_prepare_kernel(const float* __res
     amax = fmaxf(amax, dpp<0xB1>(amax));
     amax = fmaxf(amax, dpp<0x4E>(amax));
     amax = fmaxf(amax, dpp<0x141>(amax));
-    amax = fmaxf(amax, dpp<0x140>(amax));
-    amax = fmaxf(amax, __shfl_xor(amax, 16));
-    amax = fmaxf(amax, __shfl_xor(amax, 32));
+    amax = fmaxf(amax, dpp<0x140>(amax));  // sixteen lanes: 64 columns
     const bool nonzero = amax >= 1e-30f;
     const float inv = nonzero ? kWideRange / amax : 0.f;
     // to nearest even: a rounding with a bias would meet the mean of W's quants, which is not zero
@@ -568,7 +579,7 @@ __global__ __launch_bounds__(64) void gemv_mma_prepare_kernel(const float* __res
     for (int k = 0; k < 3; k++) planes[k][lane_id] = limb[k];
     float* sums = reinterpret_cast<float*>(out + kWideRecordSumsAt);
     if ((lane_id & 7u) == 0u) sums[lane_id >> 3] = sum;
-    if (lane_id == 0u) sums[8] = nonzero ? amax * (1.0f / kWideRange) : 0.f;
+    if ((lane_id & 15u) == 0u) sums[8u + (lane_id >> 4)] = nonzero ? amax * (1.0f / kWideRange) : 0.f;
     __syncthreads();
     if (lane_id < 48u) {  // lane: block pair, limb k, K index q
         const uint32_t pair = lane_id / 12u, k = lane_id % 12u >> 2, q = lane_id & 3u;
@@ -721,7 +732,7 @@ __global__ __launch_bounds__(64 * (kConsumers + LOADERS)) void gemv_mma_wide_ker
                     continue;
                 // rows past the end of the range read its last row again and are not stored
                 const uint8_t* rp = lds + slice_at + min(group * kGroupRows + n, wg_rows - 1u) * pitch + wave * T::kUnitBytes;
-                T::template contract<VG, 0>(rp, q, operands[i].a, of_result + slice * vectors * kSumsFloats, sums_step, total[group]);
+                T::template contract<VG, 0, 4>(rp, q, operands[i].a, of_result + slice * vectors * kSumsFloats, sums_step, total[group]);
             }
         }
     }

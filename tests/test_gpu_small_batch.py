@@ -79,6 +79,42 @@ def test_rows_wider_than_4096_columns(et, device, codec, vectors, rows, columns)
     check(et, device, codec, rows, columns, vectors, rng, bias, kernel="gemv_mma_prepare+gemv_mma_wide")
 
 
+# Bytes of a 256-column unit that make its first 64 columns' weights zero: {offset: bytes}.
+ZERO_FIRST_64 = {
+    oracle.Q4_K: {2: [0] * 2, 16: [0] * 32},            # no minimum; nibbles of sub-blocks 0 and 1
+    oracle.Q5_K: {2: [0] * 2, 16: None, 48: [0] * 32},  # None: their fifth bits
+    oracle.Q4_0: {0: [0] * 2, 18: [0] * 2},             # the block scales: a quant of 8 is only zero after a subtraction
+    oracle.Q8_0: {2: [0] * 32, 36: [0] * 32},
+}
+
+
+@pytest.mark.parametrize("codec", CODECS)
+@pytest.mark.parametrize("vectors", [3, 6])
+def test_wide_rows_beside_a_large_activation(et, device, codec, vectors):
+    # One activation of 2^20 among each 256, its 64 columns' weights zero: the other columns keep 24 bits of their own
+    # size. Fixed point with 127 * 2^16 units to the largest of 64 columns is off by at most 1.5 units (half a unit
+    # of rounding, one of the scaled value's two roundings); the rest is f32 sums of at most 64 terms per chain.
+    rows, columns = 2080, 8448
+    rng = np.random.default_rng(400 + 10 * codec + vectors)
+    weight = synth.random_weight(codec, rows, columns, rng)
+    units = weight.reshape(rows, columns // 256, -1)
+    for offset, values in ZERO_FIRST_64[codec].items():
+        if values is None:
+            units[:, :, offset:offset + 32] &= 0xFC
+        else:
+            units[:, :, offset:offset + len(values)] = values
+    weight = units.reshape(rows, -1)
+    x = synth.random_activations(vectors, columns, rng)
+    x[:, 5::256] = 2.0 ** 20
+    assert planned_kernel(et, codec, rows, columns, vectors) == "gemv_mma_prepare+gemv_mma_wide"
+    got = run_linear(et, device, codec, rows, columns, x, weight)
+    w = oracle.decode_rows(codec, weight, columns).astype(np.float64)
+    assert not w.reshape(rows, -1, 256)[:, :, :64].any()
+    unit = np.abs(x.astype(np.float64)).reshape(vectors, -1, 64).max(-1) / (127 * 65536)
+    bound = 1.5 * unit @ np.abs(w).reshape(rows, -1, 64).sum(-1).T + 64 * 2.0 ** -24 * np.abs(x.astype(np.float64)) @ np.abs(w).T
+    assert (np.abs(got - x.astype(np.float64) @ w.T) <= bound).all()
+
+
 def test_wide_rows_without_a_workspace(et, device):
     # aligned activations need no workspace in the vector kernels: the call then runs the launches that quantise themselves
     rows, columns, vectors = 2048, 8192, 5
