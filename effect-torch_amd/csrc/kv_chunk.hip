@@ -15,12 +15,18 @@
 // and the weights never move between lanes.
 //
 // Precision: K and V enter the matrix cores as the slab holds them (f16, bf16, or the u8 tier's integers, all exact);
-// q and the weights are f32 and enter in pieces whose sum they are to 22 bits (two half floats; q scaled by a power
-// of two per row and the weights by 2^12, so that the pieces stay normal) or 24 bits (three bfloat16). Sums are f32, in
-// short chains: four column chunks of a score, or a step's positions of an output, from zero and the small pieces first,
-// then added to the total. One chain over everything was the larger part of the error (against 64 bits, 1e-7, two slots
-// of 500 tokens at context 2000, streaming kernel / one chain / this: f16 2.4 / 4.3 / 2.6, u8 with 5 x 12 tokens
-// 3.0 / 4.9 / 2.9) and the chains cost 6 us there.
+// q and the weights are f32 and enter in pieces whose sum they are: three bfloat16 (24 bits, all of an f32), or two half
+// floats where K or V are half floats (23 bits: every fourth value is off by its last bit; q scaled by a power of two per
+// row and the weights by 2^12, so that the pieces stay normal). Sums are f32, in short chains: four column chunks of a
+// score, or a step's positions of an output, from zero and the small pieces first, then added to the total. Exponents are
+// taken against the row's own maximum, so that those of the large weights are small numbers: with the 2^12 inside the
+// exponent (weights up to exp2(12)) its rounding was the larger part of the error. Against 64 bits (2-norm, 1e-7;
+// streaming kernel / 2^12 in the exponent / this), 32/8 heads x 128, ragged contexts, two slots of 500 tokens at context
+// 2000: f16 2.1 / 2.4 / 1.7, bf16 2.1 / 2.3 / 1.5, u8 2.7 / 2.7 / 2.5; eight of 64 at 512: f16 1.9 / 2.4 / 1.6, bf16 1.9 /
+// 2.2 / 1.4, u8 2.5 / 2.5 / 2.2; four of 100 at 800, 16/8 heads x 64: f16 2.3 / 2.3 / 1.6. With scores sixteen times as large
+// the scores' own error rules: f16 5.4 / 5.3 / 5.3 and bf16 5.3 / 4.6 / 4.6 at 8 x 64, u8 6.6 / 7.4 / 7.3 at 5 x 12 tokens and
+// context 2000. (A third half float of q takes 0.1 off the u8 tier's error at ordinary scores and costs 35 % of its time,
+// f16 20 %; one chain over everything would add 1.7.)
 //
 // Eight waves in kGroups groups of kRowWaves: the waves of a group share 32 query rows each, the groups take tiles of
 // positions in turn and meet in LDS at the end, so that each SIMD has two waves to issue from. Tiles lie in LDS as in
@@ -49,11 +55,10 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 typedef float v2f __attribute__((ext_vector_type(2)));
 typedef float v4f __attribute__((ext_vector_type(4), aligned(4)));  // of rows that are only whole floats aligned
 
-// An element type of the matrix cores, and how many pieces of it make an f32.
+// An element type of the matrix cores.
 struct Half {
     typedef _Float16 v8 __attribute__((ext_vector_type(8)));
     typedef _Float16 v2 __attribute__((ext_vector_type(2)));
-    static constexpr int kPieces = 2;
     static __device__ __forceinline__ v16f mfma(v8 a, v8 b, v16f c) {
         return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
     }
@@ -61,33 +66,32 @@ struct Half {
 struct BFloat {
     typedef __bf16 v8 __attribute__((ext_vector_type(8)));
     typedef __bf16 v2 __attribute__((ext_vector_type(2)));
-    static constexpr int kPieces = 3;
     static __device__ __forceinline__ v16f mfma(v8 a, v8 b, v16f c) {
         return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
     }
 };
 
-// Eight f32 as kPieces vectors of E, each the rounded rest of the ones before.
-template <typename E>
-__device__ __forceinline__ void split(const float (&x)[8], typename E::v8 (&out)[E::kPieces]) {
+// Eight f32 as N vectors of E, each the rounded rest of the ones before.
+template <typename E, int N>
+__device__ __forceinline__ void split(const float (&x)[8], typename E::v8 (&out)[N]) {
     union Piece {
         typename E::v8 all;
         typename E::v2 pair[4];
-    } u[E::kPieces];
+    } u[N];
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         v2f rest = {x[2 * i], x[2 * i + 1]};
 #pragma unroll
-        for (int p = 0; p < E::kPieces; p++) {
+        for (int p = 0; p < N; p++) {
             u[p].pair[i] = __builtin_convertvector(rest, typename E::v2);
-            if (p + 1 < E::kPieces) {
+            if (p + 1 < N) {
                 rest.x -= static_cast<float>(u[p].pair[i].x);
                 rest.y -= static_cast<float>(u[p].pair[i].y);
             }
         }
     }
 #pragma unroll
-    for (int p = 0; p < E::kPieces; p++) out[p] = u[p].all;
+    for (int p = 0; p < N; p++) out[p] = u[p].all;
 }
 
 // Slab types: the elements K and V are contracted in, and eight values of a slab row as those.
@@ -100,6 +104,8 @@ struct Slab<__half> {
     using Raw = uint4;
     static constexpr bool kScaled = false;
     static constexpr int kBytes = 2;
+    static constexpr int kQueryPieces = 2, kWeightPieces = 2;
+    static constexpr float kWeightScale = 4096.0f;  // the half-float pieces of small weights stay normal
     static constexpr int kBlocksPerStep = 2;  // 32-position blocks per softmax step
     static __device__ __forceinline__ uint4 key(Raw raw) { return raw; }
     static __device__ __forceinline__ uint4 value(Raw raw) { return raw; }
@@ -111,6 +117,8 @@ struct Slab<Bf16> {
     using Raw = uint4;
     static constexpr bool kScaled = false;
     static constexpr int kBytes = 2;
+    static constexpr int kQueryPieces = 3, kWeightPieces = 3;
+    static constexpr float kWeightScale = 1.0f;
     static constexpr int kBlocksPerStep = 1;  // three pieces of q leave no registers for two
     static __device__ __forceinline__ uint4 key(Raw raw) { return raw; }
     static __device__ __forceinline__ uint4 value(Raw raw) { return raw; }
@@ -123,6 +131,8 @@ struct Slab<U8> {
     using Raw = uint2;
     static constexpr bool kScaled = true;
     static constexpr int kBytes = 1;
+    static constexpr int kQueryPieces = 2, kWeightPieces = 3;
+    static constexpr float kWeightScale = 1.0f;
     static constexpr int kBlocksPerStep = 1;
     static __device__ __forceinline__ uint4 key(Raw raw) {
         union {
@@ -156,7 +166,6 @@ struct Slab<U8> {
 };
 
 constexpr int kChunkWaves = 8, kChunkThreads = 64 * kChunkWaves;
-constexpr float kWeightBias = 12.0f;  // log2 of what the weights are scaled by
 
 // RW row waves share a tile (32 * RW query rows per workgroup), 8 / RW groups of them take tiles in turn.
 template <typename T, int W, int RW>
@@ -255,7 +264,7 @@ __global__ __launch_bounds__(kChunkThreads, 2) void kv_chunk_kernel(const KvArgs
     using Raw = typename S::Raw;
     using Shape = ChunkShape<T, W, RW>;
     constexpr int kGroups = Shape::kGroups, kRows = Shape::kRows, kTile = Shape::kTile, kCopies = Shape::kCopies;
-    constexpr int kKeyChunks = W / 16, kDimTiles = W / 32;
+    constexpr int kKeyChunks = W / 16, kDimTiles = W / 32, kQueryPieces = S::kQueryPieces, kWeightPieces = S::kWeightPieces;
     constexpr int U = S::kBlocksPerStep < kTile / 32 ? S::kBlocksPerStep : kTile / 32;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     uint32_t* rows_of_block = reinterpret_cast<uint32_t*>(lds + Shape::kTableAt);
@@ -368,7 +377,7 @@ __global__ __launch_bounds__(kChunkThreads, 2) void kv_chunk_kernel(const KvArgs
     if (rounds != 0) fetch(tile_begin, 0);
 
     // q in pieces, scaled so that the row's largest component lies in [2^9, 2^10); the score's unit undoes it.
-    typename KE::v8 q[KE::kPieces][kKeyChunks];
+    typename KE::v8 q[kQueryPieces][kKeyChunks];
     float unit;
     {
         const auto load = [&](int c, float (&x)[8]) {
@@ -398,10 +407,10 @@ __global__ __launch_bounds__(kChunkThreads, 2) void kv_chunk_kernel(const KvArgs
             load(c, x);
 #pragma unroll
             for (int i = 0; i < 8; i++) x[i] *= up;
-            typename KE::v8 pieces[KE::kPieces];
-            split<KE>(x, pieces);
+            typename KE::v8 pieces[kQueryPieces];
+            split<KE, kQueryPieces>(x, pieces);
 #pragma unroll
-            for (int p = 0; p < KE::kPieces; p++) q[p][c] = pieces[p];
+            for (int p = 0; p < kQueryPieces; p++) q[p][c] = pieces[p];
         }
     }
 
@@ -435,7 +444,7 @@ __global__ __launch_bounds__(kChunkThreads, 2) void kv_chunk_kernel(const KvArgs
                                                                            (((2 * (first + c) + half) ^ key_swizzle) << 4));
                     v16f sum = zero;
 #pragma unroll
-                    for (int p = KE::kPieces - 1; p >= 0; p--)
+                    for (int p = kQueryPieces - 1; p >= 0; p--)
 #pragma unroll
                         for (int c = 0; c < 4; c++) sum = KE::mfma(key[c], q[p][first + c], sum);
                     score[u] = first == 0 ? sum : score[u] + sum;
@@ -467,7 +476,7 @@ __global__ __launch_bounds__(kChunkThreads, 2) void kv_chunk_kernel(const KvArgs
 #pragma unroll
                 for (int r = 0; r < 16; r++) top = fmaxf(top, score[u][r]);
             top = fmaxf(top, other_half(top, lane));
-            const float next = fmaxf(m, fmaf(top, unit, -kWeightBias));  // the weights are 2^12 times exp(score - max)
+            const float next = fmaxf(m, top * unit);
             if (__builtin_amdgcn_ballot_w64(next != m) != 0) {
                 const float keep = __builtin_amdgcn_exp2f(m - next);
                 m = next;
@@ -478,7 +487,7 @@ __global__ __launch_bounds__(kChunkThreads, 2) void kv_chunk_kernel(const KvArgs
                     for (int r = 0; r < 16; r++) o[t][r] *= keep;
             }
             // The weights of the whole step, then the values 32 columns at a time.
-            typename VE::v8 pieces[2 * U][VE::kPieces];
+            typename VE::v8 pieces[2 * U][kWeightPieces];
             float step_sum = 0.f;
 #pragma unroll
             for (int u = 0; u < U; u++) {
@@ -488,6 +497,7 @@ __global__ __launch_bounds__(kChunkThreads, 2) void kv_chunk_kernel(const KvArgs
 #pragma unroll
                     for (int i = 0; i < 8; i++) {
                         weight[i] = __builtin_amdgcn_exp2f(fmaf(score[u][8 * c + i], unit, -m));
+                        if constexpr (S::kWeightScale != 1.0f) weight[i] *= S::kWeightScale;
                         step_sum += weight[i];
                     }
                     if constexpr (S::kScaled) {
@@ -501,7 +511,7 @@ __global__ __launch_bounds__(kChunkThreads, 2) void kv_chunk_kernel(const KvArgs
                             weight[4 * j + 3] *= v4.w;
                         }
                     }
-                    split<VE>(weight, pieces[2 * u + c]);
+                    split<VE, kWeightPieces>(weight, pieces[2 * u + c]);
                 }
             }
             l += step_sum;
@@ -521,7 +531,7 @@ __global__ __launch_bounds__(kChunkThreads, 2) void kv_chunk_kernel(const KvArgs
                     }
                 v16f sum = zero;
 #pragma unroll
-                for (int p = VE::kPieces - 1; p >= 0; p--)
+                for (int p = kWeightPieces - 1; p >= 0; p--)
 #pragma unroll
                     for (int c = 0; c < 2 * U; c++) sum = VE::mfma(value[c].all, pieces[c][p], sum);
                 o[t] += sum;
@@ -566,7 +576,7 @@ __global__ __launch_bounds__(kChunkThreads, 2) void kv_chunk_kernel(const KvArgs
     for (int g = 0; g < kGroups; g++) top = fmaxf(top, weights_of(g)[0]);
 #pragma unroll
     for (int g = 0; g < kGroups; g++) {
-        share_of[g] = __builtin_amdgcn_exp2f(weights_of(g)[0] - top);
+        share_of[g] = __builtin_amdgcn_exp2f(weights_of(g)[0] - top) * (1.0f / S::kWeightScale);
         total = fmaf(share_of[g], weights_of(g)[64], total);
     }
     const bool live = row < rows && s.ok, again = live && !(fabsf(total) < INFINITY);

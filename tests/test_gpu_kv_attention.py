@@ -218,11 +218,30 @@ def test_chunks_on_the_matrix_cores(et, device, dtype, width, query_heads, kv_he
     assert et.kv_attention_kernel(got[3], query_heads, tokens) == "kv_append+kv_chunk" + ("+kv_merge" if split else "")
     want = run_oracle(case, scale, **options)
     compare(got, want)
-    # q and the weights enter the matrix cores with 22 bits or more and every sum is f32: an output is a mean of values
+    # q and the weights enter the matrix cores with 23 bits or more and every sum is f32: an output is a mean of values
     # of size 1, off by a few 2^-22 of the largest plus what its exponents, |score| * log2(e) <= 64, lose in f32 (2^-19)
     assert np.abs(got[0] - want[0]).max() <= 1e-5
     again = run_gpu(et, device, case, scale, max_context=bound, **options)
     assert np.array_equal(got[0].view(np.uint32), again[0].view(np.uint32))
+
+
+@pytest.mark.parametrize("dtype", [np.float16, "bf16"])
+@pytest.mark.parametrize("width", [128, 64])
+def test_chunks_are_as_close_to_64_bits_as_the_streaming_kernel(et, device, dtype, width):
+    # Scores of size 1 to 5 (log2 units) carry an f32 rounding each, and so does the exponent that they become: 2^-24 of a
+    # number below 4 twice, times ln 2, about 1e-7 of a weight; the sums add as much again. 2e-7 is what the streaming
+    # kernel shows (1.9e-7 to 2.4e-7); exponents near 12 instead of 0 would alone add 1.6e-7.
+    rng = np.random.default_rng(width)
+    tokens, slots = 64, 8
+    case = make_case(rng, slots=slots, query_heads=16, kv_heads=8, width=width, block_size=16, contexts=[448] * slots, tokens=tokens,
+                     advances=[tokens] * slots, dtype=dtype)
+    scale = 1.0 / np.sqrt(width)
+    got = run_gpu(et, device, case, scale)
+    assert et.kv_attention_kernel(got[3], 16, tokens).startswith("kv_append+kv_chunk")
+    want = run_oracle(case, scale)[0].astype(np.float64)
+    error = np.linalg.norm(got[0] - want) / np.linalg.norm(want)
+    print(f"chunk error {error:.3g}", flush=True)
+    assert error <= 2.0e-7
 
 
 @pytest.mark.parametrize("dtype", [np.float16, "bf16"])
