@@ -55,24 +55,35 @@ __device__ __forceinline__ uint64_t index_value(const void* indexes, int index_i
     return value;
 }
 
-// The status block by one workgroup: the lowest position of a bad index and its VALUE, so the host can word the error like
-// crates/runtime-cpu/src/quantized.rs:570-583; or kNoBadIndex and 0.
-__device__ void report_bad_index(const void* indexes, int index_is_i64, const IndexLayout& layout, uint64_t count,
-                                 uint64_t table_rows, unsigned long long* status) {
-    constexpr int kAtOnce = 16;  // loads in flight per thread
+// The status block is the lowest position of a bad index and its VALUE, so the host can word the error like
+// crates/runtime-cpu/src/quantized.rs:570-583; or kNoBadIndex and 0. Two ways to write it:
+//
+// Few indexes (lookup_checks_itself): an extra workgroup of the lookup's own launch checks all of them and writes the
+// block while the others decode.
+// Many, or strided: the block is cleared first, the workgroups that decode check their own index, and a third launch
+// adds the value.
+constexpr uint32_t kChecksInFlight = 16;                        // loads in flight per thread of the checking workgroup
+constexpr uint64_t kMostSelfChecked = 256u * kChecksInFlight;  // indexes it takes in one round
+
+// Two launches less (contiguous ids in a captured graph, three launches / one in us: one id of 4096 Q4_K columns 6.9 / 4.8,
+// 1000 ids 10.6 / 7.7, 4096 ids 22.1 / 20.1; 4096 ids of 32 Q8_0 columns 8.2 / 5.7). One workgroup takes more than 4096 ids
+// in rounds, each a memory latency that narrow rows do not hide (100 000 ids of 256 columns 73 / 97), and strided
+// ids cost each of its threads sixteen times a division per dimension (1000 ids 7.1 / 11.4).
+bool lookup_checks_itself(const IndexLayout& layout, uint64_t count) { return layout.contiguous && count <= kMostSelfChecked; }
+
+__device__ void report_bad_index(const void* indexes, int index_is_i64, uint64_t offset, uint32_t count, uint64_t table_rows,
+                                 unsigned long long* status) {
     __shared__ unsigned long long lowest[256];
     unsigned long long position = kNoBadIndex;
-    for (uint64_t first = threadIdx.x; first < count && position == kNoBadIndex; first += 256 * kAtOnce) {
-        bool bad[kAtOnce];
+    bool bad[kChecksInFlight];
 #pragma unroll
-        for (int i = 0; i < kAtOnce; i++) {
-            const uint64_t p = first + 256u * i;
-            index_value(indexes, index_is_i64, source_index(layout, p < count ? p : first), table_rows, bad[i]);
-        }
-#pragma unroll
-        for (int i = kAtOnce - 1; i >= 0; i--)
-            if (bad[i] && first + 256u * i < count) position = first + 256u * i;
+    for (uint32_t i = 0; i < kChecksInFlight; i++) {
+        const uint32_t p = threadIdx.x + 256u * i;
+        index_value(indexes, index_is_i64, offset + (p < count ? p : 0u), table_rows, bad[i]);
     }
+#pragma unroll
+    for (int i = kChecksInFlight - 1; i >= 0; i--)
+        if (bad[i] && threadIdx.x + 256u * i < count) position = threadIdx.x + 256u * i;
     lowest[threadIdx.x] = position;
     __syncthreads();
     for (uint32_t step = 128; step > 0; step >>= 1) {
@@ -80,40 +91,51 @@ __device__ void report_bad_index(const void* indexes, int index_is_i64, const In
         __syncthreads();
     }
     if (threadIdx.x == 0) {
-        bool bad;
+        bool ignored;
         status[0] = lowest[0];
-        status[1] = lowest[0] == kNoBadIndex
-                        ? 0ull
-                        : index_value(indexes, index_is_i64, source_index(layout, lowest[0]), table_rows, bad);
+        status[1] = lowest[0] == kNoBadIndex ? 0ull : index_value(indexes, index_is_i64, offset + lowest[0], table_rows, ignored);
     }
 }
 
-// With indexes, workgroup (0, 0) checks all of them and writes the status block while the others decode: two launches less
-// than clearing it first and completing it afterwards (one id 6.4 -> 4.3 us, 100 ids 6.8 -> 4.5, 5000 ids 25.1 -> 23.5;
-// called one by one from the host 20 -> 14 us for up to 2000 ids). Stores that bypass the caches would take 3 us off 5000
-// ids and put 9 us onto the launch that reads them.
+__global__ void status_init_kernel(unsigned long long* status) {
+    if (threadIdx.x == 0) {
+        status[0] = kNoBadIndex;
+        status[1] = 0;
+    }
+}
+
+__global__ void status_finalize_kernel(const void* indexes, int index_is_i64, IndexLayout layout, uint64_t table_rows,
+                                       unsigned long long* status) {
+    if (threadIdx.x != 0 || status[0] == kNoBadIndex) return;
+    bool ignored;
+    status[1] = index_value(indexes, index_is_i64, source_index(layout, status[0]), table_rows, ignored);
+}
+
 // One workgroup per (output row, four 1024-column chunks): the row's index is read once per workgroup
 // and everything per lane is 32-bit arithmetic (a 64-bit division per item, as a flat grid-stride
-// loop over all outputs needs, costs more than the decode itself).
-template <int CODEC>
+// loop over all outputs needs, costs more than the decode itself). CHECKER: workgroup (0, 0) checks all the indexes.
+template <int CODEC, bool CHECKER>
 __global__ __launch_bounds__(256) void dequant_rows_kernel(
     const uint8_t* __restrict__ weight, const void* __restrict__ indexes, int index_is_i64,
     IndexLayout layout, uint64_t out_rows, uint64_t table_rows, uint32_t columns,
     uint64_t row_bytes, float* __restrict__ out, unsigned long long* status) {
     constexpr uint32_t kValues = block_values(CODEC);
     constexpr uint32_t kBytes = block_bytes(CODEC);
+    constexpr uint32_t kCheckers = CHECKER ? 1u : 0u;
     const uint32_t chunks = (columns + 1023u) >> 10;
-    const uint32_t checkers = indexes != nullptr ? 1u : 0u;
-    if (blockIdx.x < checkers) {
-        if (blockIdx.y == 0) report_bad_index(indexes, index_is_i64, layout, out_rows, table_rows, status);
+    if (blockIdx.x < kCheckers) {
+        if (blockIdx.y == 0) report_bad_index(indexes, index_is_i64, layout.offset, static_cast<uint32_t>(out_rows), table_rows, status);
         return;
     }
-    for (uint64_t p = blockIdx.x - checkers; p < out_rows; p += gridDim.x - checkers) {
+    for (uint64_t p = blockIdx.x - kCheckers; p < out_rows; p += gridDim.x - kCheckers) {
         uint64_t row = p;
         if (indexes != nullptr) {
             bool bad;
             row = index_value(indexes, index_is_i64, source_index(layout, p), table_rows, bad);
-            if (bad) continue;  // skipped, like the reference's Metal kernel
+            if (bad) {  // skipped, like the reference's Metal kernel
+                if (!CHECKER && blockIdx.y == 0 && threadIdx.x == 0) atomicMin(status, static_cast<unsigned long long>(p));
+                continue;
+            }
         }
         const uint8_t* packed_row = weight + row * row_bytes;
         float* out_row = out + p * columns;
@@ -147,11 +169,25 @@ hipError_t launch_dequant(const uint8_t* weight, const void* indexes, int index_
     if (out_rows == 0 || columns == 0) return hipSuccess;
     // The loops in the kernel take what the grid limits leave over.
     const uint64_t chunks = (((columns + 1023) >> 10) + kChunksPerPass - 1) / kChunksPerPass;
-    const uint32_t grid_x = static_cast<uint32_t>(out_rows < (1u << 24) ? out_rows : (1u << 24)) + (indexes != nullptr ? 1u : 0u);
+    const uint32_t grid_x = static_cast<uint32_t>(out_rows < (1u << 24) ? out_rows : (1u << 24));
     const uint32_t grid_y = static_cast<uint32_t>(chunks < 1024 ? chunks : 1024);
-    hipLaunchKernelGGL(dequant_rows_kernel<CODEC>, dim3(grid_x, grid_y), dim3(256), 0,
+    auto* status_words = static_cast<unsigned long long*>(status);
+    if (indexes != nullptr && lookup_checks_itself(layout, out_rows)) {
+        hipLaunchKernelGGL((dequant_rows_kernel<CODEC, true>), dim3(grid_x + 1, grid_y), dim3(256), 0,
+                           stream, weight, indexes, index_is_i64, layout, out_rows, table_rows,
+                           static_cast<uint32_t>(columns), row_bytes, out, status_words);
+        return hipGetLastError();
+    }
+    if (indexes != nullptr) {
+        hipLaunchKernelGGL(status_init_kernel, dim3(1), dim3(64), 0, stream, status_words);
+    }
+    hipLaunchKernelGGL((dequant_rows_kernel<CODEC, false>), dim3(grid_x, grid_y), dim3(256), 0,
                        stream, weight, indexes, index_is_i64, layout, out_rows, table_rows,
-                       static_cast<uint32_t>(columns), row_bytes, out, static_cast<unsigned long long*>(status));
+                       static_cast<uint32_t>(columns), row_bytes, out, status_words);
+    if (indexes != nullptr) {
+        hipLaunchKernelGGL(status_finalize_kernel, dim3(1), dim3(64), 0, stream, indexes,
+                           index_is_i64, layout, table_rows, status_words);
+    }
     return hipGetLastError();
 }
 
