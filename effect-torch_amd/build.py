@@ -11,6 +11,7 @@ from __future__ import annotations
 
 import importlib.util
 import os
+import shutil
 import subprocess
 import sys
 import sysconfig
@@ -79,20 +80,33 @@ def _compile(item):
     return name, obj, log
 
 
-def _torch_dir() -> str:
-    return importlib.util.find_spec("torch").submodule_search_locations[0]
+def _host_calls_needs() -> str:
+    """What this machine lacks to build et_host_calls.so ('' = nothing): callers of the C ABI alone do without."""
+    torch = importlib.util.find_spec("torch")
+    if torch is None:
+        return "torch"
+    if shutil.which("g++") is None:
+        return "g++"
+    for header in (os.path.join(sysconfig.get_paths()["include"], "Python.h"),
+                   os.path.join(torch.submodule_search_locations[0], "include", "ATen", "ATen.h")):
+        if not os.path.exists(header):
+            return header
+    return ""
 
 
-def _compile_host_calls():
+def _build_host_calls():
     obj = os.path.join(OBJ_DIR, "host_calls.o")
-    torch_dir = _torch_dir()
-    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM", "-I", sysconfig.get_paths()["include"],
-           "-I", os.path.join(torch_dir, "include"), "-I", os.path.join(torch_dir, "include", "torch", "csrc", "api", "include"),
-           "-I", "/opt/rocm/include", "-I", INCLUDE, "-c", os.path.join(CSRC, "host_calls.cpp"), "-o", obj]
-    proc = subprocess.run(cmd, capture_output=True, text=True)
-    if proc.returncode != 0:
-        raise RuntimeError(f"g++ failed for host_calls.cpp:\n{proc.stderr}")
-    return obj
+    torch_dir = importlib.util.find_spec("torch").submodule_search_locations[0]
+    compile_ = ["g++", "-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM", "-I", sysconfig.get_paths()["include"],
+                "-I", os.path.join(torch_dir, "include"), "-I", os.path.join(torch_dir, "include", "torch", "csrc", "api", "include"),
+                "-I", "/opt/rocm/include", "-I", INCLUDE, "-c", os.path.join(CSRC, "host_calls.cpp"), "-o", obj]
+    # torch's libraries are in the process by the time the module is imported; the operators' library lies next to it
+    link = ["g++", "-shared", "-o", HOST_CALLS_PATH, obj, "-L", os.path.join(torch_dir, "lib"), "-ltorch_python",
+            "-ltorch_cpu", "-lc10", "-lc10_hip", "-L", LIB_DIR, "-let_hip", "-Wl,-rpath,$ORIGIN"]
+    for command in (compile_, link):
+        proc = subprocess.run(command, capture_output=True, text=True)
+        if proc.returncode != 0:
+            raise RuntimeError(f"g++ failed for host_calls.cpp:\n{proc.stderr}")
 
 
 def build(verbose: bool = False) -> str:
@@ -100,9 +114,7 @@ def build(verbose: bool = False) -> str:
     os.makedirs(OBJ_DIR, exist_ok=True)
     items = list(SOURCES.items()) + list(CALIBRATE_SOURCES.items())
     with ThreadPoolExecutor(max_workers=8) as pool:
-        host_calls = pool.submit(_compile_host_calls)
         results = list(pool.map(_compile, items))
-        host_obj = host_calls.result()
     for name, _, log in results:
         if verbose and log.strip():
             print(f"[{name}]\n{log}", file=sys.stderr)
@@ -116,12 +128,14 @@ def build(verbose: bool = False) -> str:
         proc = subprocess.run(link, capture_output=True, text=True)
         if proc.returncode != 0:
             raise RuntimeError(f"link failed:\n{proc.stderr}")
-    # torch's libraries are in the process by the time the module is imported; the operators' library lies next to it
-    link = ["g++", "-shared", "-o", HOST_CALLS_PATH, host_obj, "-L", os.path.join(_torch_dir(), "lib"), "-ltorch_python",
-            "-ltorch_cpu", "-lc10", "-lc10_hip", "-L", LIB_DIR, "-let_hip", "-Wl,-rpath,$ORIGIN"]
-    proc = subprocess.run(link, capture_output=True, text=True)
-    if proc.returncode != 0:
-        raise RuntimeError(f"link failed:\n{proc.stderr}")
+    # after the libraries: they are there for callers of the C ABI whatever becomes of the Python module
+    lacking = _host_calls_needs()
+    if lacking:
+        if os.path.exists(HOST_CALLS_PATH):
+            os.remove(HOST_CALLS_PATH)  # of other sources, maybe
+        print(f"{HOST_CALLS_PATH} is not built: there is no {lacking} (only the Python package needs it)", file=sys.stderr)
+    else:
+        _build_host_calls()
     return LIB_PATH
 
 

@@ -33,6 +33,31 @@ def test_library_exports_every_declared_symbol(et):
         assert not hasattr(_native.lib(), symbol), f"{symbol} belongs in the measurement library"
 
 
+def test_the_libraries_are_built_where_the_python_module_cannot_be(monkeypatch, tmp_path, capsys):
+    # a caller of the C ABI alone has neither torch nor Python's headers: the build links both libraries all the same
+    import importlib.util
+    spec = importlib.util.spec_from_file_location("_et_build", os.path.join(ROOT, "effect-torch_amd", "build.py"))
+    builder = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(builder)
+    commands = []
+
+    class Done:
+        returncode, stdout, stderr = 0, "", ""
+
+    monkeypatch.setattr(builder.subprocess, "run", lambda command, **_: commands.append(command) or Done())
+    for name in ("LIB_DIR", "OBJ_DIR"):
+        monkeypatch.setattr(builder, name, str(tmp_path))
+    for name in ("LIB_PATH", "CALIBRATE_LIB_PATH", "HOST_CALLS_PATH"):
+        monkeypatch.setattr(builder, name, str(tmp_path / os.path.basename(getattr(builder, name))))
+    (tmp_path / "et_host_calls.so").write_text("of other sources")
+    find_spec = importlib.util.find_spec
+    monkeypatch.setattr(builder.importlib.util, "find_spec", lambda name, *rest: None if name == "torch" else find_spec(name, *rest))
+    assert builder.build() == builder.LIB_PATH
+    linked = [command[command.index("-o") + 1] for command in commands if "-shared" in command]
+    assert linked == [builder.LIB_PATH, builder.CALIBRATE_LIB_PATH]
+    assert not (tmp_path / "et_host_calls.so").exists() and "there is no torch" in capsys.readouterr().err
+
+
 def test_codec_tables(et):
     Q = et.GgmlQuant
     assert [(q.ggml_name, q.block_bytes) for q in (Q.Q2_K, Q.Q3_K, Q.Q4_K, Q.Q5_K, Q.Q6_K)] == [
