@@ -212,46 +212,172 @@ __device__ __forceinline__ uint2 read_transposed(const uint8_t* from) {
     return u.raw;
 }
 
-__device__ __forceinline__ float slab_value(const __half* slab, const float*, uint64_t row, int width, int column) {
-    return slab_load(slab, row * width + column);
+// Eight values of a slab row as f32: what the slab holds.
+__device__ __forceinline__ void slab_values(const __half*, const uint4& raw, float, float (&out)[8]) {
+    union {
+        uint4 all;
+        Half::v8 half;
+    } u;
+    u.all = raw;
+#pragma unroll
+    for (int i = 0; i < 8; i++) out[i] = static_cast<float>(u.half[i]);
 }
-__device__ __forceinline__ float slab_value(const Bf16* slab, const float*, uint64_t row, int width, int column) {
-    return slab_load(slab, row * width + column);
+__device__ __forceinline__ void slab_values(const Bf16*, const uint4& raw, float, float (&out)[8]) {
+    const uint32_t word[4] = {raw.x, raw.y, raw.z, raw.w};
+#pragma unroll
+    for (int i = 0; i < 8; i++) out[i] = __uint_as_float(i & 1 ? word[i / 2] & 0xffff0000u : word[i / 2] << 16);
 }
-__device__ __forceinline__ float slab_value(const U8* slab, const float* scales, uint64_t row, int width, int column) {
-    return u8_value(slab[row * width + column].byte, scales[row]);
+__device__ __forceinline__ void slab_values(const U8*, const uint2& raw, float scale, float (&out)[8]) {
+#pragma unroll
+    for (int i = 0; i < 8; i++) out[i] = u8_value(((i < 4 ? raw.x : raw.y) >> (8 * (i & 3))) & 0xffu, scale);
 }
 
-// One query row over positions [begin, end) by one wave in plain f32, position by position: the row's maximum, the sum of
-// its weights and its weighted values.
+// Up to kRowsAtOnce query rows of one (slot, kv head) by one wave in plain f32, each over its own positions
+// [begin, end): the streaming kernel's scheme. W / 8 lanes share a position and hold sixteen bytes of its rows each
+// (eight of the u8 tier), so that a K / V row is read once for all of them; 2 * 64 / (W / 8) positions are contracted
+// while the next ones are on their way. The running maximum, sum and weighted values are a lane group's own until the end.
+// Bound: its vector instructions, about forty per query row and position of a lane group.
+constexpr int kRowsAtOnce = 8;
 template <typename T, int W>
-__device__ void attend_row(const KvArgs& a, uint32_t slot, uint32_t kv_head, uint64_t query, uint32_t begin, uint32_t end,
-                           int lane, float& m, float& l, float (&o)[W / 64]) {
-    const T *k_slab = static_cast<const T*>(a.k_slab), *v_slab = static_cast<const T*>(a.v_slab);
-    m = kLowest;
-    l = 0.f;
+__device__ void attend_rows(const KvArgs& a, uint32_t slot, uint32_t kv_head, uint32_t split_index, uint32_t count,
+                            const uint32_t (&query)[kRowsAtOnce], const uint32_t (&begin)[kRowsAtOnce],
+                            const uint32_t (&end)[kRowsAtOnce], int lane) {
+    using S = Slab<T>;
+    using Raw = typename S::Raw;
+    constexpr int R = kRowsAtOnce, U = 2;
+    constexpr uint32_t kLanes = W / 8, kAt = 64 / kLanes;
+    const uint32_t column = lane % kLanes * 8, offset = lane / kLanes;
+    // any position of the rows, and those that all of them see
+    uint32_t lo = 0xffffffffu, hi = 0, all_lo = 0, all_hi = 0xffffffffu;
 #pragma unroll
-    for (int i = 0; i < W / 64; i++) o[i] = 0.f;
-    for (uint32_t first = begin; first < end; first += 64) {
-        const uint32_t position = min(first + lane, end - 1), count = min(end - first, 64u);
-        const uint64_t block = static_cast<uint64_t>(a.table[static_cast<uint64_t>(slot) * a.table_stride + block_of(a, position)]) *
-                               a.block_size;
-        const uint32_t at = block >= a.max_tokens ? 0u : min(static_cast<uint32_t>(block) + within_block(a, position), a.max_tokens - 1);
-        const uint64_t key = static_cast<uint64_t>(at) * a.kv_heads + kv_head;
-        float dot = 0.f;
-        for (int column = 0; column < W; column++) dot = fmaf(a.q[query * W + column], slab_value(k_slab, a.k_scales, key, W, column), dot);
-        const float score = static_cast<uint32_t>(lane) < count ? dot * a.scale_log2 : -INFINITY;
-        const float next = fmaxf(m, group_max<64>(score)), keep = __builtin_amdgcn_exp2f(m - next);
-        m = next;
-        const float weight = static_cast<uint32_t>(lane) < count ? __builtin_amdgcn_exp2f(score - m) : 0.f;
-        l = fmaf(l, keep, group_sum<64>(weight));
+    for (int r = 0; r < R; r++) {
+        if (r >= static_cast<int>(count)) continue;
+        if (begin[r] < end[r]) {
+            lo = min(lo, begin[r]);
+            hi = max(hi, end[r]);
+        }
+        all_lo = max(all_lo, begin[r]);
+        all_hi = min(all_hi, end[r]);
+    }
+    float q[R][8], o[R][8], m[R], l[R];
 #pragma unroll
-        for (int i = 0; i < W / 64; i++) o[i] *= keep;
-        for (uint32_t p = 0; p < count; p++) {
-            const float w = __shfl(weight, static_cast<int>(p));
-            const uint64_t value = static_cast<uint64_t>(__shfl(at, static_cast<int>(p))) * a.kv_heads + kv_head;
+    for (int r = 0; r < R; r++) {
+        m[r] = kLowest;
+        l[r] = 0.f;
+        const v4f* source = reinterpret_cast<const v4f*>(a.q + static_cast<uint64_t>(query[r]) * W + column);
+        const v4f low = source[0], high = source[1];
 #pragma unroll
-            for (int i = 0; i < W / 64; i++) o[i] = fmaf(w, slab_value(v_slab, a.v_scales, value, W, lane + 64 * i), o[i]);
+        for (int i = 0; i < 8; i++) {
+            q[r][i] = (i < 4 ? low[i & 3] : high[i & 3]) * a.scale_log2;
+            o[r][i] = 0.f;
+        }
+    }
+    // slab row of a position: first its block's row, which has to arrive before the row itself can be asked for
+    const uint32_t* table = a.table + static_cast<uint64_t>(slot) * a.table_stride;
+    const auto position_of = [&](uint32_t first, int u) { return min(first + u * kAt + offset, hi - 1); };
+    const auto load = [&](const uint32_t (&block)[U], uint32_t first, Raw (&k)[U], Raw (&v)[U], float (&k_scale)[U], float (&v_scale)[U]) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const uint64_t base = static_cast<uint64_t>(block[u]) * a.block_size;
+            const uint32_t at = base >= a.max_tokens ? 0u
+                                                     : min(static_cast<uint32_t>(base) + within_block(a, position_of(first, u)), a.max_tokens - 1);
+            const uint64_t row = static_cast<uint64_t>(at) * a.kv_heads + kv_head;
+            k[u] = *reinterpret_cast<const Raw*>(static_cast<const char*>(a.k_slab) + (row * W + column) * S::kBytes);
+            v[u] = *reinterpret_cast<const Raw*>(static_cast<const char*>(a.v_slab) + (row * W + column) * S::kBytes);
+            if constexpr (S::kScaled) {
+                k_scale[u] = a.k_scales[row];
+                v_scale[u] = a.v_scales[row];
+            }
+        }
+    };
+    const auto blocks = [&](uint32_t first, uint32_t (&block)[U]) {
+#pragma unroll
+        for (int u = 0; u < U; u++) block[u] = table[block_of(a, position_of(first, u))];
+    };
+    uint32_t block[U];
+    Raw k_next[U], v_next[U];
+    float k_scale[U] = {}, v_scale[U] = {};
+    if (lo < hi) {
+        blocks(lo, block);
+        load(block, lo, k_next, v_next, k_scale, v_scale);
+        blocks(lo + U * kAt, block);
+    }
+    for (uint32_t first = lo; first < hi; first += U * kAt) {
+        float key[U][8], value[U][8];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            slab_values(static_cast<const T*>(nullptr), k_next[u], k_scale[u], key[u]);
+            slab_values(static_cast<const T*>(nullptr), v_next[u], v_scale[u], value[u]);
+        }
+        if (first + U * kAt < hi) {
+            load(block, first + U * kAt, k_next, v_next, k_scale, v_scale);
+            blocks(first + 2 * U * kAt, block);
+        }
+        const bool whole = first >= all_lo && first + U * kAt <= all_hi;  // every row sees all of these
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            if (r >= static_cast<int>(count)) continue;
+            float score[U], top = m[r], total = 0.f;
+            bool seen[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const uint32_t position = first + u * kAt + offset;
+                seen[u] = whole || (position >= begin[r] && position < end[r]);
+                float part = 0.f;
+#pragma unroll
+                for (int i = 0; i < 8; i++) part = fmaf(q[r][i], key[u][i], part);
+                part = group_sum<kLanes>(part);
+                score[u] = seen[u] ? part : -INFINITY;
+                top = fmaxf(top, score[u]);
+            }
+            const float keep = __builtin_amdgcn_exp2f(m[r] - top);
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                score[u] = __builtin_amdgcn_exp2f(score[u] - top);
+                total += score[u];
+            }
+            m[r] = top;
+            l[r] = fmaf(l[r], keep, total);
+#pragma unroll
+            for (int i = 0; i < 8; i++) o[r][i] *= keep;
+#pragma unroll
+            for (int u = 0; u < U; u++)
+#pragma unroll
+                // a weight of zero does not hide an infinite value: positions that are not seen add nothing
+                for (int i = 0; i < 8; i++) o[r][i] = fmaf(score[u], seen[u] ? value[u][i] : 0.f, o[r][i]);
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        if (r >= static_cast<int>(count)) continue;
+        float top = m[r];
+#pragma unroll
+        for (uint32_t step = kLanes; step < 64; step *= 2) top = fmaxf(top, __shfl_xor(top, step));
+        const float share = __builtin_amdgcn_exp2f(m[r] - top);
+        float total = l[r] * share;
+#pragma unroll
+        for (int i = 0; i < 8; i++) o[r][i] *= share;
+#pragma unroll
+        for (uint32_t step = kLanes; step < 64; step *= 2) {
+            total += __shfl_xor(total, step);
+#pragma unroll
+            for (int i = 0; i < 8; i++) o[r][i] += __shfl_xor(o[r][i], step);
+        }
+        float* record = a.partial + (static_cast<uint64_t>(query[r]) * a.splits + split_index) * (W + 2);
+        if (a.splits != 1 && lane == 0) {
+            record[0] = top;
+            record[1] = total;
+        }
+        if (offset == 0) {
+            float* to = (a.splits == 1 ? a.out + static_cast<uint64_t>(query[r]) * W : record + 2) + column;
+            const float divisor = a.splits == 1 ? total : 1.0f;
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                v4f joined;
+#pragma unroll
+                for (int i = 0; i < 4; i++) joined[i] = o[r][4 * j + i] / divisor;
+                *reinterpret_cast<v4f*>(to + 4 * j) = joined;
+            }
         }
     }
 }
@@ -605,27 +731,24 @@ __global__ __launch_bounds__(kChunkThreads, 2) void kv_chunk_kernel(const KvArgs
     }
     // An infinity or NaN in a K or V row spoils the matrix products of every query row it shares a tile with, also of those
     // that do not see its position, and a product of pieces overflows or meets inf - inf before the product itself does.
-    // Such rows are attended to once more, without pieces and over their own positions alone.
-    uint64_t left = __builtin_amdgcn_ballot_w64(again) & 0xffffffffull;
-    for (int turn = 0; left != 0; left &= left - 1, turn++) {
-        if (turn % kGroups != group) continue;
-        const int which = __builtin_ctzll(left);
-        const uint32_t begin_of = __shfl(max(row_begin, my_begin), which), end_of = __shfl(min(row_end, my_end), which);
-        const uint32_t at = first_row + 32 * row_wave + which;
-        const uint64_t query_of = (static_cast<uint64_t>(slot) * a.query_heads + kv_head * group_size + at % group_size) * a.tokens +
-                                  at / group_size;
-        float m_of, l_of, o_of[W / 64];
-        attend_row<T, W>(a, slot, kv_head, query_of, begin_of, end_of, lane, m_of, l_of, o_of);
-        float* record = a.partial + (query_of * a.splits + split_index) * (W + 2);
-        if (a.splits != 1 && lane == 0) {
-            record[0] = m_of;
-            record[1] = l_of;
-        }
+    // Such rows are attended to once more, without pieces and over their own positions alone. Two slots of 500 tokens at
+    // context 2000 with a NaN at position 0 of one, which all its rows see: f16 1337 us, u8 1494 (all finite 89 and 122; row
+    // after row, a lane to a position, 6617 and 7408; the streaming kernel 1036 and 1322 whatever the values); eight slots
+    // of 64 tokens at context 512, f16, 363 (1691); a NaN in one row of q of the former 178 (332).
+    uint32_t left = static_cast<uint32_t>(__builtin_amdgcn_ballot_w64(again));
+    const uint32_t begin_here = max(row_begin, my_begin), end_here = min(row_end, my_end);
+    for (int turn = 0; left != 0; turn++) {
+        uint32_t query_of[kRowsAtOnce], begin_of[kRowsAtOnce], end_of[kRowsAtOnce], count = 0;
 #pragma unroll
-        for (int i = 0; i < W / 64; i++) {
-            if (a.splits == 1) a.out[query_of * W + lane + 64 * i] = o_of[i] / l_of;
-            else record[2 + lane + 64 * i] = o_of[i];
+        for (int r = 0; r < kRowsAtOnce; r++) {
+            const int which = left != 0 ? __builtin_ctz(left) : 0;
+            count += left != 0 ? 1 : 0;
+            left &= left - 1;
+            query_of[r] = __builtin_amdgcn_readlane(static_cast<uint32_t>(query), which);
+            begin_of[r] = __builtin_amdgcn_readlane(begin_here, which);
+            end_of[r] = __builtin_amdgcn_readlane(end_here, which);
         }
+        if (turn % kGroups == group) attend_rows<T, W>(a, slot, kv_head, split_index, count, query_of, begin_of, end_of, lane);
     }
 }
 

@@ -264,6 +264,49 @@ def test_values_that_are_not_finite_stay_with_the_rows_that_see_them(et, device,
     np.testing.assert_allclose(got[0], want[0], rtol=0, atol=1e-4)  # this file's bar; the same infinities and NaN
 
 
+def time_of_calls(call, calls=3, takes=5):
+    """The least time of a call, in us, over takes of a few in a row."""
+    call()
+    times = []
+    for _ in range(takes):
+        begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        begin.record()
+        for _ in range(calls):
+            call()
+        end.record()
+        torch.cuda.synchronize()
+        times.append(begin.elapsed_time(end) * 1000 / calls)
+    return min(times)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.uint8])
+def test_a_value_that_is_not_finite_costs_no_more_than_a_pass_per_token(et, device, dtype):
+    # one NaN at position 0 is seen by every query row of its slot, so that all of them are attended to once more, in f32:
+    # about the work of the streaming kernel, which takes eleven to twelve times the chunk kernel's time at this size.
+    # (measured: 11 to 15 times; one query row after the other, 60 to 80 times)
+    torch.manual_seed(5)
+    slots, tokens, context, kv_heads, width = 2, 500, 2000, 8, 128
+    blocks = context // 16
+    slab = lambda: (torch.randint(1, 256, (slots * context, kv_heads, width), device=device, dtype=dtype)  # noqa: E731
+                    if dtype == torch.uint8 else torch.randn(slots * context, kv_heads, width, device=device).to(dtype))
+    scales = {name: torch.full((slots * context, kv_heads), 0.02, device=device) for name in ("k_scales", "v_scales")}
+    layer = et.KvLayer(slab(), slab(), 16, torch.arange(slots * blocks, device=device, dtype=torch.int32).reshape(slots, blocks),
+                       torch.full((slots,), context - tokens, device=device, dtype=torch.int32),
+                       torch.full((slots,), tokens, device=device, dtype=torch.int32), context,
+                       **(scales if dtype == torch.uint8 else {}))
+    q, k, v = (torch.randn(slots, heads, tokens, width, device=device) for heads in (32, kv_heads, kv_heads))
+    out, workspace = torch.empty_like(q), et.kv_attention_workspace(layer, 32, tokens)
+    call = lambda: et.kv_attention_into(layer, q, k, v, 0.09, None, out, workspace=workspace, synchronize=False)  # noqa: E731
+    assert et.kv_attention_kernel(layer, 32, tokens).startswith("kv_append+kv_chunk")
+    finite = time_of_calls(call)
+    for slot in range(slots):
+        (scales["v_scales"] if dtype == torch.uint8 else layer.v_slab)[slot * context] = float("nan")
+    spoilt = time_of_calls(call)
+    assert out.isnan().all()
+    print(f"{dtype}: {finite:.0f} us, with a NaN at position 0 {spoilt:.0f} us", flush=True)
+    assert spoilt <= 30 * finite
+
+
 def test_one_workspace_serves_calls_of_any_geometry(et, device):
     workspace = torch.full((64 << 20,), 255, dtype=torch.uint8, device=device)
     rng = np.random.default_rng(11)
