@@ -488,7 +488,9 @@ __global__ __launch_bounds__(kChunkThreads, 2) void kv_chunk_kernel(const KvArgs
                 *reinterpret_cast<uint4*>(to) = S::key(k_raw[i]);
                 *reinterpret_cast<uint4*>(to + Shape::kTileBytes) = S::value(v_raw[i]);
                 if (lane % Shape::kPieces == 0) {
-                    scales[tile_row(i)] = k_scale[i];
+                    // Of a K row with an infinite scale every value is infinite or, byte 128, NaN, and so are its products with q:
+                    // NaN, not the infinity that the scale makes of the whole sum (-inf would pass for a weight of zero).
+                    scales[tile_row(i)] = fabsf(k_scale[i]) < INFINITY ? k_scale[i] : NAN;
                     scales[kTile + tile_row(i)] = v_scale[i];
                 }
             }

@@ -264,6 +264,28 @@ def test_values_that_are_not_finite_stay_with_the_rows_that_see_them(et, device,
     np.testing.assert_allclose(got[0], want[0], rtol=0, atol=1e-4)  # this file's bar; the same infinities and NaN
 
 
+@pytest.mark.parametrize("width,bound", [(128, 320), (128, 9000), (64, 320)])
+def test_scales_that_are_not_finite_stay_with_the_rows_that_see_them(et, device, width, bound):
+    # the u8 tier: its bytes are always finite, a scale (of a row written from an infinity or NaN) or q need not be
+    rng = np.random.default_rng(width + bound)
+    tokens, slots, window = 40, 20, 60
+    contexts = [70, 257] * 10
+    case = make_case(rng, slots=slots, query_heads=8, kv_heads=2, width=width, block_size=16, contexts=contexts, tokens=tokens,
+                     advances=[tokens] * slots, dtype="u8")
+    row_of = lambda slot, position: case["table"][slot, position // 16] * 16 + position % 16  # noqa: E731
+    case["v_scales"][row_of(0, contexts[0] - 30), 0] = np.inf   # the window's last tokens see it no more
+    case["v_scales"][row_of(1, contexts[1] - 25), 1] = np.nan
+    case["k_scales"][row_of(2, contexts[2] - 30), 0] = np.nan
+    case["k_scales"][row_of(3, contexts[3] - 50), 1] = np.inf
+    case["q"][4, 3, 11, 1] = np.nan
+    scale = 1.0 / np.sqrt(width)
+    got = run_gpu(et, device, case, scale, max_context=bound, window=window)
+    assert et.kv_attention_kernel(got[3], 8, tokens).startswith("kv_append+kv_chunk")
+    want = run_oracle(case, scale, window=window)
+    assert np.isinf(want[0]).any() and np.isnan(want[0]).any() and np.isfinite(want[0]).mean() > 0.9
+    np.testing.assert_allclose(got[0], want[0], rtol=0, atol=1e-4)  # this file's bar; the same infinities and NaN
+
+
 def time_of_calls(call, calls=3, takes=5):
     """The least time of a call, in us, over takes of a few in a row."""
     call()
