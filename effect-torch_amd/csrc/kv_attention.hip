@@ -776,33 +776,9 @@ uint32_t positions_per_step(const KvAttention& p, int g, int waves) {
     return waves * (64 / lanes) * (g >= 8 ? 2 : 4);
 }
 
-}  // namespace
-
-KvLaunchShape kv_attention_shape(const KvAttention& p) {
+KvLaunchShape shape_without_chunks(const KvAttention& p, int g) {
     KvLaunchShape shape{};
-    const int g = streaming_group(p);
     const uint64_t queries = static_cast<uint64_t>(p.active_batch) * p.query_heads * p.tokens;
-    const uint64_t streamed = static_cast<uint64_t>(p.active_batch) * p.tokens * p.kv_heads *
-                              (g != 0 ? p.query_heads / p.kv_heads / g : 0);
-    if (kv_chunk_supported(p) && streamed * p.max_context >= kKvChunkMinRows) {
-        // One workgroup per compute unit; a split of at least four rounds, or its start and end cost more than
-        // the compute units it brings in.
-        const KvChunkGrid grid = kv_chunk_grid(p);
-        const uint64_t context = p.max_context;
-        uint64_t splits = grid.units == 0 || grid.units >= 256 ? 1 : 256 / grid.units;
-        splits = std::min(splits, (context + 4 * grid.round - 1) / (4 * grid.round));
-        const uint64_t room = static_cast<uint64_t>(kKvTableEntries - 2) * p.block_size;
-        const uint64_t reach = room > 2 * grid.round ? room - grid.round : grid.round;
-        splits = std::max(splits, (context + reach - 1) / reach);
-        if (grid.units * splits >= kKvChunkMinWorkgroups) {
-            shape.chunk = true;
-            shape.waves = 8;
-            shape.splits = static_cast<uint32_t>(splits);
-            shape.workgroups = grid.units * splits;
-            shape.workspace_bytes = splits > 1 ? queries * splits * (p.width + 2) * sizeof(float) : 0;
-            return shape;
-        }
-    }
     shape.streaming = g != 0;
     const uint64_t rows = static_cast<uint64_t>(p.active_batch) * p.tokens *
                           (shape.streaming ? p.kv_heads * ((p.query_heads / p.kv_heads) / g) : p.query_heads);
@@ -833,6 +809,67 @@ KvLaunchShape kv_attention_shape(const KvAttention& p) {
     shape.splits = static_cast<uint32_t>(splits);
     shape.workgroups = rows * splits;
     shape.workspace_bytes = splits > 1 ? queries * splits * (p.width + 2) * sizeof(float) : 0;
+    return shape;
+}
+
+// Two to four tokens per slot and one query head per kv head: a chunk workgroup's 64 rows hold two to four live ones, and
+// the streaming kernel reads the context that few times. Both kernels' times from their workgroups, in turns of the
+// compute units, and the positions each takes, in us; the constants fit 342 launches (2 to 4 tokens, 8 to 32 heads,
+// context 128 to 6000) to 6 % in the mean and 25 % at most. With 2 tokens, streaming / chunk, 32 slots of 32 heads x 128 at
+// 512: f16 64 / 69, bf16 69 / 89, u8 69 / 83; 61 slots at 267: 82 / 107, 88 / 133, 99 / 128; but 8 at 2000: 69 / 51, 71 / 65,
+// 62 / 61. From five tokens on, and with two or more query heads per kv head, the chunk kernel was ahead at every size that
+// the limits above let through (0.2 to 1.0 of the streaming kernel's time).
+constexpr uint32_t kKvFewTokens = 4;
+bool streaming_is_faster(const KvAttention& p, const KvLaunchShape& streaming, uint64_t chunk_units, uint64_t chunk_splits) {
+    struct Times {
+        double chunk_turn, chunk_position, chunk_bytes, merge;     // per turn; per 1000 positions of a turn; of all units
+        double launch, turn, position, bytes;                      // the streaming kernel's
+    };
+    static constexpr Times kTimes[2][3] = {
+        // f16, bf16, u8
+        {{7.7, 9.3, 1.6, 7.1, 6.0, 1.0, 5.4, 2.6}, {8.1, 11.5, 0.3, 7.9, 6.7, 1.5, 5.5, 2.4}, {9.1, 13.8, 0.0, 9.6, 7.6, 1.8, 6.7, 3.2}},
+        {{7.8, 11.7, 11.6, 6.2, 2.3, 1.0, 11.9, 1.8}, {9.0, 17.6, 11.6, 7.3, 3.0, 1.4, 12.0, 1.4}, {10.3, 23.3, 0.0, 9.1, 7.7, 2.2, 9.8, 0.8}},
+    };
+    const Times& us = kTimes[p.width == 128][p.slab_dtype == ET_DTYPE_F16 ? 0 : p.slab_dtype == ET_DTYPE_BF16 ? 1 : 2];
+    const double context = p.max_context / 1000.0;
+    const auto turns = [](uint64_t workgroups, uint64_t resident) { return static_cast<double>((workgroups + resident - 1) / resident); };
+    const uint64_t resident = streaming.waves == 8 ? 256 : 512;
+    const double chunk = turns(chunk_units * chunk_splits, 256) * (us.chunk_turn + us.chunk_position * context / chunk_splits) +
+                         us.chunk_bytes * context * chunk_units / 256 + (chunk_splits > 1 ? us.merge : 0.0);
+    const double rows = static_cast<double>(streaming.workgroups / streaming.splits);
+    const double streamed = us.launch + turns(streaming.workgroups, resident) * (us.turn + us.position * context / streaming.splits) +
+                            us.bytes * context * rows / 256;
+    return chunk > 0.95 * streamed;
+}
+
+}  // namespace
+
+KvLaunchShape kv_attention_shape(const KvAttention& p) {
+    const int g = streaming_group(p);
+    KvLaunchShape shape = shape_without_chunks(p, g);
+    const uint64_t queries = static_cast<uint64_t>(p.active_batch) * p.query_heads * p.tokens;
+    const uint64_t streamed = static_cast<uint64_t>(p.active_batch) * p.tokens * p.kv_heads *
+                              (g != 0 ? p.query_heads / p.kv_heads / g : 0);
+    if (kv_chunk_supported(p) && streamed * p.max_context >= kKvChunkMinRows) {
+        // One workgroup per compute unit; a split of at least four rounds, or its start and end cost more than
+        // the compute units it brings in.
+        const KvChunkGrid grid = kv_chunk_grid(p);
+        const uint64_t context = p.max_context;
+        uint64_t splits = grid.units == 0 || grid.units >= 256 ? 1 : 256 / grid.units;
+        splits = std::min(splits, (context + 4 * grid.round - 1) / (4 * grid.round));
+        const uint64_t room = static_cast<uint64_t>(kKvTableEntries - 2) * p.block_size;
+        const uint64_t reach = room > 2 * grid.round ? room - grid.round : grid.round;
+        splits = std::max(splits, (context + reach - 1) / reach);
+        const bool few = p.tokens <= kKvFewTokens && p.query_heads == p.kv_heads;
+        if (grid.units * splits >= kKvChunkMinWorkgroups && !(few && streaming_is_faster(p, shape, grid.units, splits))) {
+            shape.chunk = true;
+            shape.streaming = false;
+            shape.waves = 8;
+            shape.splits = static_cast<uint32_t>(splits);
+            shape.workgroups = grid.units * splits;
+            shape.workspace_bytes = splits > 1 ? queries * splits * (p.width + 2) * sizeof(float) : 0;
+        }
+    }
     return shape;
 }
 

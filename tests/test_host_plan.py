@@ -267,6 +267,27 @@ def test_kv_attention_validation_follows_the_reference(et):
         _kv_layer(et, torch, dtype=torch.uint8)
 
 
+@pytest.mark.parametrize("query_heads,kv_heads,width,dtype,slots,tokens,context,kernel", [
+    # us measured, streaming / chunk kernel
+    (32, 32, 128, "bfloat16", 32, 2, 512, "kv_attend"),                     # 69 / 89
+    (32, 32, 128, "float16", 61, 2, 267, "kv_attend"),                      # 82 / 107
+    (8, 8, 128, "uint8", 44, 2, 1710, "kv_attend"),                         # 67 / 97
+    (16, 16, 64, "bfloat16", 19, 2, 1137, "kv_attend"),                     # 35 / 43
+    (32, 32, 128, "bfloat16", 2, 4, 1759, "kv_attend"),                     # 26 / 31: two workgroups to a unit, with splits
+    (32, 32, 128, "uint8", 3, 3, 3503, "kv_append+kv_chunk+kv_merge"),      # 94 / 58: the streaming kernel takes two turns
+    (8, 8, 128, "bfloat16", 58, 4, 1973, "kv_append+kv_chunk"),             # 203 / 138
+    (32, 32, 128, "bfloat16", 43, 5, 602, "kv_append+kv_chunk"),            # 229 / 158
+    (64, 8, 128, "bfloat16", 35, 2, 827, "kv_append+kv_chunk"),             # 88 / 60: eight query heads share a kv head
+])
+def test_few_tokens_per_slot_attend_on_the_kernel_that_is_faster(et, query_heads, kv_heads, width, dtype, slots, tokens, context,
+                                                                 kernel):
+    import torch
+    scales = {name: torch.ones(4096, kv_heads) for name in ("k_scales", "v_scales")} if dtype == "uint8" else {}
+    layer = _kv_layer(et, torch, slots=slots, kv_heads=kv_heads, width=width, max_tokens=4096, block_size=16,
+                      dtype=getattr(torch, dtype), max_context=context, **scales)
+    assert et.kv_attention_kernel(layer, query_heads, tokens) == kernel
+
+
 def test_kv_attention_launch_shapes_and_status_wording(et):
     import ctypes
     import struct
