@@ -264,6 +264,20 @@ def test_values_that_are_not_finite_stay_with_the_rows_that_see_them(et, device,
     np.testing.assert_allclose(got[0], want[0], rtol=0, atol=1e-4)  # this file's bar; the same infinities and NaN
 
 
+@pytest.mark.parametrize("dtype", [np.float16, "bf16", "u8"])
+@pytest.mark.parametrize("block_size", [1, 5])  # 1: a split ends where its blocks fill the kernel's table in LDS
+def test_chunks_page_through_blocks_of_any_size(et, device, dtype, block_size):
+    rng = np.random.default_rng(block_size)
+    tokens, slots = 20, 16
+    case = make_case(rng, slots=slots, query_heads=8, kv_heads=4, width=128, block_size=block_size, contexts=[3980, 1500] + [60] * 14,
+                     tokens=tokens, advances=[tokens, 13] * 8, dtype=dtype)
+    got = run_gpu(et, device, case, 0.09)
+    assert et.kv_attention_kernel(got[3], 8, tokens) == "kv_append+kv_chunk+kv_merge"
+    want = run_oracle(case, 0.09)
+    compare(got, want)
+    assert np.abs(got[0] - want[0]).max() <= 1e-5  # as in test_chunks_on_the_matrix_cores
+
+
 @pytest.mark.parametrize("width,bound", [(128, 320), (128, 9000), (64, 320)])
 def test_scales_that_are_not_finite_stay_with_the_rows_that_see_them(et, device, width, bound):
     # the u8 tier: its bytes are always finite, a scale (of a row written from an infinity or NaN) or q need not be
@@ -284,6 +298,67 @@ def test_scales_that_are_not_finite_stay_with_the_rows_that_see_them(et, device,
     want = run_oracle(case, scale, window=window)
     assert np.isinf(want[0]).any() and np.isnan(want[0]).any() and np.isfinite(want[0]).mean() > 0.9
     np.testing.assert_allclose(got[0], want[0], rtol=0, atol=1e-4)  # this file's bar; the same infinities and NaN
+
+
+@pytest.mark.parametrize("dtype", [np.float16, "bf16", "u8"])
+@pytest.mark.parametrize("bound,split", [(300, False), (9000, True)])
+def test_chunk_slots_that_are_inactive_or_fail_a_check(et, device, dtype, bound, split):
+    # slot 3 advances by more than the chunk, slots 32 and 33 are not active: the other slots' results are what they are without
+    # them, the failing one's are not touched (its partial records neither written nor read: the workspace holds NaN)
+    rng = np.random.default_rng(bound)
+    tokens, slots, active = 40, 34, 32
+    case = make_case(rng, slots=slots, query_heads=8, kv_heads=2, width=128, block_size=16, contexts=[70, 133] * 17, tokens=tokens,
+                     advances=[tokens] * slots, dtype=dtype)
+    workspace = torch.full((32 << 20,), 255, dtype=torch.uint8, device=device)
+    want = run_gpu(et, device, case, 0.09, active_batch=active, max_context=bound, workspace=workspace)
+    assert et.kv_attention_kernel(want[3], 8, tokens) == "kv_append+kv_chunk" + ("+kv_merge" if split else "")
+    compare(want, run_oracle(case, 0.09, active_batch=active))
+    assert np.all(want[0][active:] == 0)
+    case["advances"][3] = tokens + 1
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(device)  # noqa: E731
+    slab = lambda a: dev(a.view(np.int16)).view(torch.bfloat16) if dtype == "bf16" else dev(a)  # noqa: E731
+    scales = {name: dev(case[name]) for name in ("k_scales", "v_scales") if case[name] is not None}
+    layer = et.KvLayer(slab(case["k_slab"]), slab(case["v_slab"]), 16, dev(case["table"].view(np.int32)),
+                       dev(case["cursors"].view(np.int32)), dev(case["advances"].view(np.int32)), bound, active_batch=active, **scales)
+    q = dev(case["q"])
+    out = torch.full_like(q, float("nan"))
+    workspace.fill_(255)
+    status = et.kv_attention_into(layer, q, dev(case["k"]), dev(case["v"]), 0.09, None, out, workspace=workspace, synchronize=False)
+    with pytest.raises(et.QuantizedError, match=f"kv attention: advance {tokens + 1} out of range for chunk length {tokens}"):
+        et.kv_attention_status_check(layer, tokens, status)
+    good = [slot for slot in range(slots) if slot != 3]
+    out = out.cpu().numpy()
+    assert np.array_equal(out[good].view(np.uint32), want[0][good].view(np.uint32))
+    assert np.isnan(out[3]).all()
+
+
+@pytest.mark.parametrize("dtype", [np.float16, "bf16", "u8"])
+@pytest.mark.parametrize("width", [128, 64])
+def test_chunks_with_a_negative_scale_and_rows_that_are_whole_floats_aligned(et, device, dtype, width):
+    rng = np.random.default_rng(width)
+    tokens, slots, scale = 33, 20, -0.11
+    case = make_case(rng, slots=slots, query_heads=16, kv_heads=4, width=width, block_size=16, contexts=[223, 90] * 10, tokens=tokens,
+                     advances=[tokens] * slots, dtype=dtype)
+    want = run_oracle(case, scale)
+    got = run_gpu(et, device, case, scale)
+    assert et.kv_attention_kernel(got[3], 16, tokens).startswith("kv_append+kv_chunk")
+    compare(got, want)
+    assert np.abs(got[0] - want[0]).max() <= 1e-5  # as in test_chunks_on_the_matrix_cores
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(device)  # noqa: E731
+    slab = lambda a: dev(a.view(np.int16)).view(torch.bfloat16) if dtype == "bf16" else dev(a)  # noqa: E731
+
+    def one_float_off(array):
+        buffer = torch.full((array.size + 1,), float("nan"), device=device)
+        buffer[1:] = dev(array).reshape(-1)
+        return buffer[1:].reshape(array.shape)
+
+    scales = {name: dev(case[name]) for name in ("k_scales", "v_scales") if case[name] is not None}
+    layer = et.KvLayer(slab(case["k_slab"]), slab(case["v_slab"]), 16, dev(case["table"].view(np.int32)),
+                       dev(case["cursors"].view(np.int32)), dev(case["advances"].view(np.int32)), case["max_context"], **scales)
+    q, k, v = (one_float_off(case[name]) for name in ("q", "k", "v"))
+    out = one_float_off(np.full(case["q"].shape, np.nan, np.float32))
+    et.kv_attention_into(layer, q, k, v, scale, None, out)
+    assert np.array_equal(out.cpu().numpy().view(np.uint32), got[0].view(np.uint32))
 
 
 def time_of_calls(call, calls=3, takes=5):
