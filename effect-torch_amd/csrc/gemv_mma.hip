@@ -851,13 +851,16 @@ bool gemv_mma_supported(int32_t codec, uint64_t rows, uint64_t columns, uint32_t
     // with less than a group of rows to a compute unit most of every matrix instruction is padding
     if (rows < 256u * 8u || rows > 0xffffffffull) return false;
     if (columns <= kNarrowColumns) return true;
-    // Wider rows, against the launches of gemv_limb.hip (two or three vectors each): Q4_K 4096 x 14336, 2 / 3 / 4 / 5 / 6
-    // vectors 13.8 / 14.6 / 15.6 / 18.6 / 18.9 us (20.4 / 26.0 / 37.1 / 44.6 / 50.2); 3000 x 8192, 4 vectors 10.9 (18.1); Q8_0
-    // 4096 x 14336, whose ranges of eight rows take two rounds of workgroups, 2 / 3 / 6 vectors 23 / 24 / 31 (23 / 30 / 57).
-    // A second round of ranges is worth it from three vectors on where LDS holds less than a group of sixteen rows.
-    // From seven vectors on the batch kernels' plans hold prepared inputs, which callers may share between plans;
-    // taller matrices keep the launches that their plans name (one call of more rounds would still be faster: 14336 x 5120,
-    // 4 vectors 18.2 against 41.4 us).
+    // Wider rows, against the launches of gemv_limb.hip (two or three vectors each), us, this / those: Q4_K 4096 x 14336 with
+    // 2 / 3 / 5 vectors 12.9 / 13.2 / 17.2 against 17.1 / 22.3 / 39.7; Q8_0 3072 x 12800, whose ranges take two rounds of
+    // workgroups, 3 vectors 19.9 (23.9), 2 vectors slower: a second round of ranges is worth it from three vectors on where
+    // LDS holds less than a group of sixteen rows.
+    // Two vectors on at most 8192 columns are one launch there, without the preparing one: 2048 x 7936 Q4_K 10.2 (8.0), Q8_0
+    // 10.0 (7.7), 4096 x 8192 Q8_0 11.3 (9.7); 5120 x 4608 Q4_K 10.6 (11.2) is the most that is given away. Wider ones take
+    // twice the launches' slices: 3072 x 8704 Q4_K 10.6 (14.3).
+    // Not taken up: from seven vectors on the batch kernels' plans hold prepared inputs, which callers may share between
+    // plans; more rounds of ranges, although they would be faster at least once (14336 x 5120, 4 vectors 18.2 against 41.4).
+    if (vectors == 2u && columns <= 8192u) return false;
     if (vectors > 6u || columns > (1u << 20)) return false;
     const uint32_t unit_bytes = static_cast<uint32_t>(256 / block_values(codec) * block_bytes(codec));
     const uint32_t fit = wide_rows_that_fit(columns, vectors, unit_bytes);

@@ -67,7 +67,8 @@ def test_shapes(et, device, codec, vectors, rows, columns):
 
 @pytest.mark.parametrize("codec", CODECS)
 @pytest.mark.parametrize("vectors,rows,columns", [
-    (2, 2048, 4352),     # seventeen units: a last slice of one
+    (3, 2048, 4352),     # seventeen units: a last slice of one
+    (2, 2048, 8448),     # two vectors: wider than 8192 columns
     (4, 2100, 8192),     # whole slices only; ranges of nine rows, the last of three
     (5, 4096, 6400),     # sixteen rows per range, a last slice of one unit
     (6, 4100, 5120),     # ranges of seventeen rows: a group of one; a half slice at the end

@@ -228,6 +228,17 @@ def test_embedding_status_wording(et):
         assert N.last_error() == f"quantized_embedding: index {value} is outside 0..1"
 
 
+@pytest.mark.parametrize("codec,row_bytes", [("Q4_K", 144), ("Q5_K", 176), ("Q4_0", 144), ("Q8_0", 272)])
+def test_two_vectors_on_rows_of_8192_columns_stay_one_launch(et, codec, row_bytes):
+    # us measured at 2048 x 7936, gemv_limb / prepare + wide: Q4_K 8.0 / 10.2, Q8_0 7.7 / 10.0; at 3072 x 8704 14.3 / 10.6
+    import torch
+    for vectors, columns, kernel in ((2, 4352, "gemv_limb"), (2, 8192, "gemv_limb"), (2, 8448, "gemv_mma_prepare+gemv_mma_wide"),
+                                     (3, 8192, "gemv_mma_prepare+gemv_mma_wide")):
+        plan = et.linear_requirements(torch.zeros(vectors, columns), torch.zeros(2048, columns // 256 * row_bytes, dtype=torch.uint8),
+                                      None, et.GgmlQuant[codec], (2048, columns))
+        assert plan.kernel == kernel
+
+
 def _kv_layer(et, torch, *, slots=2, kv_heads=2, width=8, max_tokens=32, block_size=4, dtype=None, **kw):
     dtype = dtype or torch.float32
     slab = torch.zeros(max_tokens, kv_heads, width, dtype=dtype)
