@@ -1,5 +1,5 @@
 // f32-accurate contraction of Q4_K or Q5_K weights with a batch of activation vectors on the gfx950
-// matrix cores, with every operand an exact small integer held in a half float.
+// matrix cores: weights times their sub-block scales are exact small integers in half floats, activations two half floats each.
 //
 //   y[m, n] = sum_s  unit[m, s] * d[n, s] * sum_g sum_i (sc_g[n] * nib[n, g, i]) * X[m, g, i]
 //           - sum_s  dmin[n, s] * sum_g m_g[n] * xsum[m, g]
@@ -10,8 +10,8 @@
 // (quantize_halves.h). The tiles hold hi and lo / 4096, so that both halves
 // of a sub-block add up in ONE accumulator, hi * w + (lo / 4096) * w = X * w / 4096, and the factor
 // 4096 rides on the row scale: one multiply-add per element and stage in the epilogue. On the weight side the 6-bit sub-block scale is folded into the operand:
-// sc_g * nib <= 63 * 15 = 945 (Q5_K: 63 * 31 = 1953), exact in a half float as well. Every product (< 2^21) is exact in
-// the f32 the matrix core accumulates in, so v_mfma_f32_32x32x16_f16 sums whole super-blocks with
+// sc_g * nib <= 63 * 15 = 945 (Q5_K: 63 * 31 = 1953), exact in a half float as well. Every product (of two
+// numbers of at most eleven bits) is exact in the f32 the matrix core accumulates in, so v_mfma_f32_32x32x16_f16 sums whole super-blocks with
 // f32 accumulation error only, and the f32 scales unit[m] * d[n] are applied once per stage instead
 // of once per 32-column block: the per-element VALU work, which bounds the int8 kernel with
 // three-byte activations (gemm_i8.hip: a convert and multiply-adds per element and block), shrinks

@@ -1,4 +1,4 @@
-// gemm_h16.hip's contraction (the same operands: exact integers in half floats) for prompts. A workgroup contracts 128
+// gemm_h16.hip's contraction (the same operands in half floats) for prompts. A workgroup contracts 128
 // vectors with 256 weight rows (Q2_K, Q6_K: 128), so that weights are unpacked once for 128 (64) vectors instead of for
 // every 32, and an activation tile is copied for 256 rows instead of 64 or 128.
 //
@@ -7,7 +7,9 @@
 // from two waves: a Q4_K wave's stage of 256 columns is 128 half-float matrix instructions (32 cycles each), 16 f32 ones for
 // the minima (64) and about 510 vector instructions (4): 7160 cycles by that sum, 7860 measured at the 2.1 GHz the
 // device holds. What helped was therefore fewer vector instructions (waves of 64 x 64 unpack every weight twice: 282 ->
-// 296 us) and not the latencies: operands fetched only behind each barrier measured the same. LDS is 14 % busy.
+// 296 us) and not the latencies: operands fetched only behind each barrier measured the same. Counted at
+// 14336 x 4096 with 1000 vectors: matrix 60 %, vector 22 % of the cycles of busy compute units, which are busy 81 % of the
+// launch (448 workgroups on 256 compute units), no LDS bank conflicts.
 // Every wave unpacks its own weight rows from the packed bytes in LDS. There are no loader waves (a third wave per SIMD
 // would leave 168 registers each): the waves ask for the next sub-blocks' activations and the next stage's weights
 // themselves, through inline assembly, because any LDS read next to a copy that the compiler can see waits for it.

@@ -607,7 +607,6 @@ __global__ __launch_bounds__(64 * (kConsumers + LOADERS)) void gemv_mma_wide_ker
     constexpr uint32_t kSliceBytes = kSliceUnits * T::kUnitBytes, kPitch = slice_pitch(kSliceBytes);
     const uint32_t whole = row_units / kSliceUnits, rest_units = row_units % kSliceUnits;
     const uint32_t rest_bytes = rest_units * T::kUnitBytes, rest_pitch = slice_pitch(rest_bytes);
-    const uint32_t slices = whole + (rest_units != 0u ? 1u : 0u);
     const uint32_t rest_at = whole * wg_rows * kPitch;
 
     if (wave >= static_cast<uint32_t>(kConsumers)) {

@@ -253,7 +253,10 @@ struct KvAttention {
 // workgroups share them. Measured (us, streaming / chunk kernel with its append and merge launches; 32/8 heads x 128,
 // slots x tokens at context): 1x16 at 2000 (256 Ki rows, 32 workgroups) u8 25.3 / 30.0; 1x32 at 2000 (512 Ki, 32)
 // u8 37.1 / 41.0, bf16 34.0 / 39.7; 6x16 at 600 (450 Ki, 96) f16 45.0 / 25.5; 8x16 at 512 (512 Ki, 64) u8 56.2 / 29.2;
-// 1x64 at 2000 (1 Mi, 64) f16 71 / 34; 2x500 at 2000 (16 Mi, 256) f16 1036 / 83, bf16 1097 / 107, u8 1322 / 110.
+// 1x64 at 2000 (1 Mi, 64) f16 71 / 34; 2x500 at 2000 (16 Mi, 256) f16 1036 / 93, bf16 1097 / 115, u8 1322 / 126.
+// Other head counts and width 64 at the lower limits: 23x4 at 748 (537 Ki, 184; 16/8 heads x 64) f16 23.3 / 18.6, u8 34.1 / 24.8;
+// 4x8 at 794 (595 Ki, 64; 24/8 x 128) bf16 33.0 / 24.8; 1x12 at 1219 (457 Ki, 96; 32/32 x 128) f16 21.8 / 21.9, u8 31.8 / 27.2.
+// One query head per kv head and two to four tokens: streaming_is_faster (kv_attention.hip).
 constexpr uint64_t kKvChunkMinRows = 384 * 1024;
 constexpr uint64_t kKvChunkMinWorkgroups = 64;
 bool kv_chunk_supported(const KvAttention& p);

@@ -34,9 +34,11 @@
 // is copied (global_load_lds; the u8 tier passes through registers, where it becomes half floats and bfloat16) while
 // this one is contracted.
 //
-// Bound: the matrix pipe. A round of 128 positions of a compute unit is 128 matrix instructions per SIMD, 4096 clocks
-// (two slots of 500 tokens at context 2000, 32/8 heads x 128, f16: 83 us with the other launches, where the streaming
-// kernel took 1036; bf16 107 / 1097, u8 110 / 1322).
+// Bound: instruction issue. Matrix and vector instructions of a SIMD take their time one after the other on this device;
+// two slots of 500 tokens at context 2000, 32/8 heads x 128: matrix 38 %, vector (softmax, the weights' pieces, the adds of
+// the short chains) 45 % of the cycles of busy compute units (u8: 33 and 51 %), no LDS bank conflicts, compute units busy 76 %
+// of the launch (their workgroups have 1500 to 2000 positions). 93 us with the append launch, where the streaming kernel
+// took 1036; bf16 115 / 1097, u8 126 / 1322.
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 
@@ -734,7 +736,7 @@ __global__ __launch_bounds__(kChunkThreads, 2) void kv_chunk_kernel(const KvArgs
     // An infinity or NaN in a K or V row spoils the matrix products of every query row it shares a tile with, also of those
     // that do not see its position, and a product of pieces overflows or meets inf - inf before the product itself does.
     // Such rows are attended to once more, without pieces and over their own positions alone. Two slots of 500 tokens at
-    // context 2000 with a NaN at position 0 of one, which all its rows see: f16 1337 us, u8 1494 (all finite 89 and 122; row
+    // context 2000 with a NaN at position 0 of one, which all its rows see: f16 1337 us, u8 1494 (all finite 93 and 126; row
     // after row, a lane to a position, 6617 and 7408; the streaming kernel 1036 and 1322 whatever the values); eight slots
     // of 64 tokens at context 512, f16, 363 (1691); a NaN in one row of q of the former 178 (332).
     uint32_t left = static_cast<uint32_t>(__builtin_amdgcn_ballot_w64(again));

@@ -22,8 +22,8 @@ __device__ __forceinline__ int dpp_i32(int v) {
 
 // Activations for gemm_h16: per vector and 256-column stage, x = unit * X with unit = amax / (2^23 - 1) and
 // X = 4096 * hi + lo: hi the nearest integer to X / 4096 (|hi| <= 2048: exact in a half float), lo the rest, written as the
-// half float nearest to lo / 4096 - eleven significant bits of |lo| <= 2048, so 2^-12 of X's range at worst and finer
-// wherever lo is small. X is x / unit to within one rounding: the quotient by a multiplication with 1 / unit, corrected
+// half float nearest to lo / 4096 - eleven significant bits of |lo| <= 2048, so off by half a unit of X at most (2^-24
+// of the stage's largest value) and by less wherever lo is small. X is x / unit to within one rounding: the quotient by a multiplication with 1 / unit, corrected
 // by its remainder. (A whole number lo from the product alone: relative error of a contraction with 20 vectors x 4096
 // columns, 1e-7, before / now Q5_K 1.46 / 1.20, Q6_K 1.58 / 1.37, Q2_K 1.64 / 1.43; no slower.) The two products of a weight with these operands add
 // up to X * w / 4096 in one accumulator. xsum[g] = unit * (sum of X over sub-block g).

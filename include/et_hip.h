@@ -146,7 +146,9 @@ uint64_t et_hip_linear_plan_output_bytes(const et_linear_plan* plan);
 /* Device scratch the execute step needs (int8 activations, gathered strided
  * input); the caller allocates at least this many bytes, 256-byte aligned. May be 0. */
 uint64_t et_hip_linear_plan_workspace_bytes(const et_linear_plan* plan);
-/* Name of the selected kernel variant, for profiles and diagnostics. */
+/* Name of the selected kernel variant, for profiles and diagnostics: of calls that bring the plan's
+ * workspace. (et_hip_linear_enqueue takes few aligned vectors without one too, and then runs a
+ * "gemv_mma_prepare+gemv_mma_wide" plan as gemv_limb launches.) */
 const char* et_hip_linear_plan_kernel(const et_linear_plan* plan);
 /* Algorithmic bytes of one execution: packed weight + f32 input + f32 output (+ bias). */
 uint64_t et_hip_linear_plan_algorithmic_bytes(const et_linear_plan* plan);
