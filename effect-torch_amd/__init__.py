@@ -13,6 +13,7 @@ from .quantized import (  # noqa: F401
     QuantizedError,
     QuantizedRequirements,
     LinearGroup,
+    LinearStep,
     RawLinear,
     STATIC_WORKSPACE_BYTES,
     MFMA_OPERATIONS,

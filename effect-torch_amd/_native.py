@@ -67,6 +67,18 @@ class EtRotaryAfter(ctypes.Structure):
     ]
 
 
+class EtStepInput(ctypes.Structure):
+    """``et_step_input`` of include/et_hip.h."""
+
+    _fields_ = [
+        ("x", ctypes.c_void_p),
+        ("normed", ctypes.c_int32),
+        ("norm_weight_dtype", ctypes.c_int32),
+        ("norm_weight", ctypes.c_void_p),
+        ("eps", ctypes.c_double),
+    ]
+
+
 class EtGroupShares(ctypes.Structure):
     """``et_group_shares`` of include/et_hip.h."""
 
@@ -177,6 +189,9 @@ SIGNATURES = {
                                                                    ctypes.POINTER(EtGroupShares), _vp, _vp]),
     "et_hip_linear_enqueue_prepared_then_norm": (ctypes.c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _u64, _vp, _vp, _i32,
                                                                 ctypes.c_double, _vp, _u64, _vp, _vp]),
+    "et_hip_linear_step_supported": (ctypes.c_int, [_vp, ctypes.c_uint32, _i32]),
+    "et_hip_linear_enqueue_step": (ctypes.c_int, [_vp, ctypes.c_uint32, ctypes.POINTER(EtStepInput), _vp, _vp, _vp, _i32,
+                                                  _vp, _vp]),
     "et_hip_embedding_requirements": (ctypes.c_int, [_T, _T, _i32, _u64, _u64, _PP]),
     "et_hip_embedding_plan_destroy": (None, [_vp]),
     "et_hip_embedding_plan_output_rank": (_i32, [_vp]),

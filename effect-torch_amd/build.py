@@ -36,6 +36,7 @@ COMMON = [
 SOURCES = {
     "dequant.hip": ["-ffp-contract=off"],
     "gemv_limb.hip": [],
+    "gemv_step.hip": [],
     "gemv_mma.hip": [],
     "lds_handover.cpp": [],
     "gemv_generic.hip": [],

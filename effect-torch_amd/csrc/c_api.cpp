@@ -299,6 +299,23 @@ int et_hip_linear_enqueue_prepared_group_shares(const et_linear_plan* const* pla
     });
 }
 
+int et_hip_linear_step_supported(const et_linear_plan* const* plans, uint32_t count, int32_t silu_mul) {
+    return et::quantized::linear_step_supported(plans, count, silu_mul != 0) ? 1 : 0;
+}
+
+int et_hip_linear_enqueue_step(const et_linear_plan* const* plans, uint32_t count, const et_step_input* input,
+                               const uint8_t* const* weights, const float* const* residuals, float* const* ys,
+                               int32_t silu_mul, void* stream, const volatile int32_t* cancel) {
+    return guarded([&](std::string* error) -> int {
+        if (input == nullptr) {
+            *error = "quantized_linear: NULL input";
+            return ET_ERR_INVALID;
+        }
+        return et::quantized::linear_enqueue_step(plans, count, *input, weights, residuals, ys, silu_mul != 0, stream,
+                                                  cancel, error);
+    });
+}
+
 int et_hip_linear_enqueue_prepared_then_norm(const et_linear_plan* plan, const void* prepared,
                                              const uint8_t* weight, const float* bias, const float* residual,
                                              float* y, void* workspace, uint64_t workspace_bytes,

@@ -97,6 +97,7 @@ __device__ __forceinline__ void rotate_pair(float a_in, float b_in, uint32_t off
 // Tensor.silu (packages/core/src/Tensor.ts:1537-1540) times the up projection. Tensor.sigmoid is
 // tanh(x / 2) / 2 + 1 / 2, every step rounded to f32 (Tensor.ts:1240-1245).
 __device__ __forceinline__ float silu_mul_one(float gate, float up) {
+#pragma clang fp contract(off)
     const float sigmoid = tanhf(gate * 0.5f) * 0.5f + 0.5f;
     return (gate * sigmoid) * up;
 }

@@ -47,6 +47,28 @@ hipError_t gemv_limb(int32_t codec, const uint8_t* weight, const float* x, uint6
                      const float* bias, float* y, uint64_t rows, uint64_t columns, uint32_t vectors,
                      hipStream_t stream);
 
+// ---- gemv_step.hip: one vector against up to four matrices of one codec and width in one launch ----
+// y_i = W_i f(x) (+ residual_i, which may be y_i), f(x) = x, or rms_norm(x) * norm_weight (null: ones; floats or halves)
+// when `normed`; silu_mul (two matrices of the same rows): y_0 = silu(W_0 f(x)) * (W_1 f(x)), residuals and y_1 unused.
+// x is 16-byte aligned.
+constexpr uint32_t kGemvStepMost = 4;
+struct GemvStep {
+    const float* x;
+    int normed;
+    const void* norm_weight;
+    int norm_weight_is_half;
+    double eps;
+    uint64_t columns, row_bytes;
+    bool silu_mul;
+    uint32_t count;
+    uint64_t rows[kGemvStepMost];
+    const uint8_t* weight[kGemvStepMost];
+    const float* residual[kGemvStepMost];
+    float* y[kGemvStepMost];
+};
+bool gemv_step_supported(int32_t codec, uint64_t columns, bool silu_mul);
+hipError_t gemv_step(int32_t codec, const GemvStep& step, hipStream_t stream);
+
 // ---- gemv_mma.hip: dequant-GEMV for 2..8 vectors on v_mfma_i32_16x16x32_i8 (Q4_K, Q5_K, Q4_0, Q8_0) ----
 // W is streamed once through LDS whatever the number of vectors; f32-accurate like gemv_limb.
 // x rows must be 16-byte aligned (x pointer and x_row_stride * 4).

@@ -689,6 +689,62 @@ int linear_enqueue_prepared_then_norm(const et_linear_plan& plan, const void* pr
     return ET_OK;
 }
 
+bool linear_step_supported(const et_linear_plan* const* plans, uint32_t count, bool silu_mul) {
+    static_assert(ET_HIP_LINEAR_GROUP_MOST == kGemvStepMost, "the header's bound is the kernel's");
+    if (plans == nullptr || count == 0 || count > kGemvStepMost) return false;
+    if (silu_mul && count != 2) return false;
+    for (uint32_t i = 0; i < count; i++) {
+        const et_linear_plan* plan = plans[i];
+        if (plan == nullptr || plan->kernel != LinearKernel::kGemvLimb || plan->vectors != 1 || plan->has_bias ||
+            plan->codec != plans[0]->codec || plan->columns != plans[0]->columns || plan->rows > 0x0fffffffull)
+            return false;
+    }
+    if (silu_mul && plans[0]->rows != plans[1]->rows) return false;
+    return gemv_step_supported(plans[0]->codec, plans[0]->columns, silu_mul);
+}
+
+int linear_enqueue_step(const et_linear_plan* const* plans, uint32_t count, const et_step_input& input,
+                        const uint8_t* const* weights, const float* const* residuals, float* const* ys, bool silu_mul,
+                        void* stream, const volatile int32_t* cancel, std::string* error) {
+    if (!linear_step_supported(plans, count, silu_mul))
+        return fail(error, ET_ERR_UNSUPPORTED, "quantized_linear: these plans have no launch with the operators around them");
+    if (weights == nullptr || ys == nullptr || input.x == nullptr)
+        return fail(error, ET_ERR_INVALID, "quantized_linear: NULL device pointer");
+    if (reinterpret_cast<uintptr_t>(input.x) % 16 != 0)
+        return fail(error, ET_ERR_INVALID, "quantized_linear: activations must be 16-byte aligned");
+    GemvStep step{};
+    step.x = input.x;
+    step.normed = input.normed != 0;
+    if (step.normed) {
+        if (input.norm_weight_dtype != ET_DTYPE_F32 && input.norm_weight_dtype != ET_DTYPE_F16)
+            return fail(error, ET_ERR_UNSUPPORTED, "rms_norm: the weight must be f32 or f16");
+        step.norm_weight = input.norm_weight;
+        step.norm_weight_is_half = input.norm_weight_dtype == ET_DTYPE_F16;
+        step.eps = input.eps;
+    }
+    step.columns = plans[0]->columns;
+    step.row_bytes = plans[0]->encoded_row_bytes;
+    step.silu_mul = silu_mul;
+    step.count = count;
+    const uintptr_t x_begin = reinterpret_cast<uintptr_t>(input.x), x_end = x_begin + 4 * step.columns;
+    for (uint32_t i = 0; i < count; i++) {
+        step.rows[i] = plans[i]->rows;
+        step.weight[i] = weights[i];
+        step.residual[i] = residuals != nullptr && !silu_mul ? residuals[i] : nullptr;
+        step.y[i] = ys[i];
+        if (weights[i] == nullptr || (ys[i] == nullptr && !(silu_mul && i == 1)))
+            return fail(error, ET_ERR_INVALID, "quantized_linear: NULL device pointer");
+        // every workgroup reads all of x while others already write
+        const uintptr_t y_begin = reinterpret_cast<uintptr_t>(ys[i]);
+        if (ys[i] != nullptr && y_begin < x_end && x_begin < y_begin + 4 * plans[i]->rows)
+            return fail(error, ET_ERR_INVALID, "quantized_linear: a result overlaps the activations of its launch");
+    }
+    if (cancelled(cancel)) return fail(error, ET_ERR_CANCELLED, "operation aborted");
+    if (hipError_t status = gemv_step(plans[0]->codec, step, as_stream(stream)))
+        return hip_failure(error, "quantized_linear", status);
+    return ET_OK;
+}
+
 int linear_enqueue(const et_linear_plan& plan, const float* x, uint64_t x_row_stride,
                    const uint8_t* weight, const float* bias, float* y, void* workspace,
                    uint64_t workspace_bytes, void* stream, const volatile int32_t* cancel,

@@ -144,6 +144,12 @@ int linear_enqueue_prepared_then_norm(const et_linear_plan& plan, const void* pr
                                       double eps, void* next_prepared, uint64_t next_prepared_bytes, void* stream,
                                       const volatile int32_t* cancel, std::string* error);
 
+// Contractions of one vector with the operators around them in one launch (et_hip_linear_enqueue_step in et_hip.h).
+bool linear_step_supported(const et_linear_plan* const* plans, uint32_t count, bool silu_mul);
+int linear_enqueue_step(const et_linear_plan* const* plans, uint32_t count, const et_step_input& input,
+                        const uint8_t* const* weights, const float* const* residuals, float* const* ys, bool silu_mul,
+                        void* stream, const volatile int32_t* cancel, std::string* error);
+
 int embedding_requirements(const TensorView& indexes, const TensorView& weight, int32_t codec,
                            uint64_t rows, uint64_t columns, et_embedding_plan* plan,
                            std::string* error);

@@ -21,11 +21,12 @@ from typing import Dict, List, Optional, Sequence
 
 import torch
 
+from ._native import EtGroupShares
 from .decode_ops import (RotaryLayout, add_into, gather_rows_into, greedy_tokens, greedy_workspace_bytes,
                          rms_norm_into, rotary_into, rotary_pair_into, silu_mul_into)
 from .kv_cache import (KvLayer, kv_attention_into, kv_attention_kernel, kv_attention_projected_into,
                        kv_attention_workspace, kv_commit)
-from .quantized import ActivationMode, GgmlQuant, LinearGroup, RawLinear
+from .quantized import ActivationMode, GgmlQuant, LinearGroup, LinearStep, RawLinear
 
 LINEARS = ("wq", "wk", "wv", "wo", "gate", "up", "down")
 
@@ -61,7 +62,8 @@ class LlamaDecoder:
     ``fused``: one quantisation per distinct input, residual sums in the contraction epilogues,
     norms / SiLU * up / rotary computed inside the launches next to them where the plans can
     (``on_the_fly``); otherwise one launch sequence per operator, as the reference's executor runs
-    them. The results agree within the f32 bars either way.
+    them, except that a single sequence whose plans can (``chained``) has norms, residual sums and
+    SiLU * up computed inside the contractions' launches. The results agree within the f32 bars either way.
     """
 
     def __init__(self, shape: LlamaShape, codec: GgmlQuant, slots: int, weights: Sequence[Dict[str, torch.Tensor]],
@@ -89,14 +91,26 @@ class LlamaDecoder:
             self.qkv_group = LinearGroup([plans["wq"], plans["wk"], plans["wv"]])
             self.ffn_group = LinearGroup([plans["gate"], plans["up"]])
             self.group_ws = u8(max(self.qkv_group.workspace_bytes, self.ffn_group.workspace_bytes))
+        # one sequence: contractions of one vector with the operators around them
+        self.chain = {"qkv": LinearStep([plans["wq"], plans["wk"], plans["wv"]]), "wo": LinearStep([plans["wo"]]),
+                      "ffn": LinearStep([plans["gate"], plans["up"]], silu_mul=True), "down": LinearStep([plans["down"]]),
+                      "head": LinearStep([plans["head"]])}
+        self.chained = not fused and all(step.supported for step in self.chain.values())
         self.kv_ws = kv_attention_workspace(kv[0], shape.heads, 1)
         # q / k / v can stay the K shares of their group launch when the attention kernel is the one that sums them
-        self.project_in_attention = (self.on_the_fly and self.qkv_group.shares_layout().count > 1 and
-                                     kv_attention_kernel(kv[0], shape.heads, 1).split("+")[0] == "kv_attend")
+        streaming = lambda layer: kv_attention_kernel(layer, shape.heads, 1).split("+")[0] == "kv_attend"  # noqa: E731
+        self.project_in_attention = (all(streaming(layer) for layer in kv) if self.chained else
+                                     self.on_the_fly and self.qkv_group.shares_layout().count > 1 and streaming(kv[0]))
         self.greedy_ws = u8(greedy_workspace_bytes(slots, shape.vocab))
         kv_width = shape.kv_heads * shape.head_dim
         self.x, self.h = f32(slots, shape.hidden), f32(slots, shape.hidden)
-        self.q, self.k, self.v = f32(slots, shape.hidden), f32(slots, kv_width), f32(slots, kv_width)
+        if self.chained:  # side by side, as the one share of a launch over the rows of all three
+            qkv = f32(slots, shape.hidden + 2 * kv_width)
+            self.q, self.k, self.v = qkv.split([shape.hidden, kv_width, kv_width], dim=1)
+            self.qkv_rows = EtGroupShares(qkv.data_ptr(), 1, slots, qkv.shape[1],
+                                          (0, shape.hidden, shape.hidden + kv_width, 0))
+        else:
+            self.q, self.k, self.v = f32(slots, shape.hidden), f32(slots, kv_width), f32(slots, kv_width)
         self.attended, self.projected = f32(slots, shape.hidden), f32(slots, shape.hidden)
         self.gate, self.up, self.down = f32(slots, shape.ffn), f32(slots, shape.ffn), f32(slots, shape.hidden)
         self.logits = f32(slots, shape.vocab)
@@ -154,6 +168,21 @@ class LlamaDecoder:
             plans["down"].enqueue_prepared_then_norm(self.shared_ffn, w["down"], None, x, self.linear_ws, following,
                                                      norm_weight, eps, self.shared_hidden, residual=x)
             return
+        if self.chained:
+            chain = self.chain
+            chain["qkv"].enqueue(x, [w["wq"], w["wk"], w["wv"]], [q, k, v], norm=(self.norms[index][0], eps))
+            if self.project_in_attention:  # the attention kernel rotates q and k at the slot's cursor
+                self.status.append(kv_attention_projected_into(
+                    kvl, self.qkv_rows, (0, 1, 2), (None, None, None), self.cursors, theta, 1.0, half_split, self.scale, None,
+                    attended4, workspace=self.kv_ws, synchronize=False))
+            else:
+                rotary_pair_into(q4, k4, self.cursors, theta, 1.0, half_split, q4, k4)
+                self.status.append(kv_attention_into(kvl, q4, k4, v4, self.scale, None, attended4, workspace=self.kv_ws,
+                                                     synchronize=False))
+            chain["wo"].enqueue(self.attended, [w["wo"]], [x], residuals=[x])
+            chain["ffn"].enqueue(x, [w["gate"], w["up"]], [self.gate], norm=(self.norms[index][1], eps))
+            chain["down"].enqueue(self.gate, [w["down"]], [x], residuals=[x])
+            return
         rms_norm_into(x, self.norms[index][0], eps, h)
         if self.fused:
             plans["wq"].prepare_input(h, self.shared_hidden)
@@ -193,6 +222,8 @@ class LlamaDecoder:
         """logits = head(final_norm(x))."""
         if self.on_the_fly:  # the last layer has left the normed, prepared x behind
             self.plans["head"].enqueue_prepared(self.shared_hidden, self.head, None, self.logits, self.linear_ws)
+        elif self.chained:
+            self.chain["head"].enqueue(self.x, [self.head], [self.logits], norm=(self.final_norm, self.shape.eps))
         else:
             rms_norm_into(self.x, self.final_norm, self.shape.eps, self.h)
             self.plans["head"].enqueue(self.h, self.head, None, self.logits, self.linear_ws)

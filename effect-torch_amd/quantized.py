@@ -558,6 +558,45 @@ class LinearGroup:
                            biases, residuals, stream, cancelled)
 
 
+class LinearStep:
+    """Up to four :class:`RawLinear` plans of one vector, one codec and one width that run in one launch together with the
+    operators around them (``et_hip_linear_enqueue_step``); ``silu_mul``: two plans, the gate and the up projection."""
+
+    def __init__(self, plans: Sequence["RawLinear"], silu_mul: bool = False):
+        self.plans, self.silu_mul = list(plans), silu_mul
+        self._handles = (ctypes.c_void_p * len(self.plans))(*[p.requirements._handle for p in self.plans])
+
+    @property
+    def supported(self) -> bool:
+        return bool(N.lib().et_hip_linear_step_supported(self._handles, len(self.plans), int(self.silu_mul)))
+
+    def enqueue(self, x: torch.Tensor, weights: Sequence[torch.Tensor], ys: Sequence[torch.Tensor], *,
+                norm: Optional[tuple] = None, residuals: Optional[Sequence[Optional[torch.Tensor]]] = None, stream=None,
+                cancelled: Optional[CancellationFlag] = None) -> None:
+        """``ys[i] = W_i f(x) (+ residuals[i])``, ``f(x) = rms_norm(x) * weight`` for ``norm = (weight, eps)``; ``silu_mul``:
+        ``ys[0] = silu(W_0 f(x)) * (W_1 f(x))``."""
+        count = len(self.plans)
+        if len(weights) != count or len(ys) != (1 if self.silu_mul else count):
+            raise QuantizedError(N.ERR_INVALID, f"quantized_linear: a launch of {count} plans got {len(weights)} weights and "
+                                                f"{len(ys)} results")
+        for index, plan in enumerate(self.plans):
+            plan._check_input(x)
+            plan._check_weight(weights[index])
+            if index < len(ys):
+                plan._check_output(ys[index], residuals[index] if residuals is not None else None)
+        weight, eps = norm if norm is not None else (None, 0.0)
+        if weight is not None:
+            self.plans[0]._holds("norm weight", weight, weight.element_size() * self.plans[0].columns)
+        pointers = lambda tensors: (ctypes.c_void_p * count)(  # noqa: E731
+            *[t.data_ptr() if t is not None else None for t in tensors])
+        source = N.EtStepInput(x.data_ptr(), int(norm is not None), _weight_dtype(weight),
+                               weight.data_ptr() if weight is not None else None, float(eps))
+        _check(N.lib().et_hip_linear_enqueue_step(
+            self._handles, count, ctypes.byref(source), pointers(weights),
+            pointers(residuals) if residuals is not None else None, pointers(ys), int(self.silu_mul),
+            _stream_handle(stream), cancelled.ptr if cancelled is not None else None))
+
+
 def _group_then_rotary(group: "LinearGroup", prepared, weights, ys, workspace, rotate, offsets, theta, sign, layout,
                        head_dim, biases, residuals, stream, cancelled) -> None:
     count = len(group.plans)

@@ -282,6 +282,25 @@ int et_hip_linear_enqueue_prepared_then_norm(const et_linear_plan* plan, const v
                                              uint64_t next_prepared_bytes, void* stream,
                                              const volatile int32_t* cancel);
 
+/* Up to ET_HIP_LINEAR_GROUP_MOST contractions of ONE vector in one launch together with the operators around them, for a
+ * decode step of a single sequence: y_i = W_i f(x) (+ residual_i, which may be y_i), f(x) = x or, `normed`,
+ * rms_norm(x) * norm_weight (rms_norm_forward_into_impl; [columns] f32 or f16, or NULL); with `silu_mul`, two plans of
+ * the same rows: y_0 = silu(W_0 f(x)) * (W_1 f(x)), residuals and ys[1] unused. Plans of one vector, one codec and one
+ * width, without bias, whose kernel is the dequant-GEMV of one vector (et_hip_linear_step_supported says 1). x: 16-byte
+ * aligned floats that no y_i overlaps. residuals may be NULL, as may each of them. No counterpart in the reference, whose
+ * executor runs one operator at a time. */
+typedef struct et_step_input {
+    const float* x;             /* [columns] */
+    int32_t normed;             /* 0: x as it is */
+    int32_t norm_weight_dtype;  /* ET_DTYPE_F32 or ET_DTYPE_F16 */
+    const void* norm_weight;
+    double eps;
+} et_step_input;
+int et_hip_linear_step_supported(const et_linear_plan* const* plans, uint32_t count, int32_t silu_mul);
+int et_hip_linear_enqueue_step(const et_linear_plan* const* plans, uint32_t count, const et_step_input* input,
+                               const uint8_t* const* weights, const float* const* residuals, float* const* ys,
+                               int32_t silu_mul, void* stream, const volatile int32_t* cancel);
+
 /* ---- quantized_embedding (= bit-exact dequantisation of selected rows) ---- */
 
 /* Plan step = embedding_requirements (crates/runtime-cpu/src/quantized.rs:340-365).
