@@ -183,4 +183,149 @@ __device__ __forceinline__ void decode4<kQ6_K>(const uint8_t* block, uint32_t e,
     }
 }
 
+// Span<CODEC>: the values that share the bytes a lane reads once - kGroups runs of four values, run g at columns
+// first(lane) + g * kStride of the block; kLanes lanes take a block. The same operations as decode4, on a header read in one
+// or two loads: a Q4_K lane reads 20 bytes in two loads for eight values (decode4: six loads for four).
+typedef uint32_t __attribute__((ext_vector_type(2), aligned(1))) Unaligned64;
+typedef uint32_t __attribute__((ext_vector_type(4), aligned(1))) Unaligned128;
+__device__ __forceinline__ uint2 load64(const uint8_t* at) {
+    const Unaligned64 v = *reinterpret_cast<const Unaligned64*>(at);
+    return make_uint2(v.x, v.y);
+}
+__device__ __forceinline__ uint4 load128(const uint8_t* at) {
+    const Unaligned128 v = *reinterpret_cast<const Unaligned128*>(at);
+    return make_uint4(v.x, v.y, v.z, v.w);
+}
+
+template <int CODEC>
+struct Span {  // one run of decode4 (Q8_0)
+    static constexpr int kGroups = 1;
+    static constexpr uint32_t kLanes = block_values(CODEC) / 4, kStride = 0;
+    static __device__ __forceinline__ uint32_t first(uint32_t lane) { return 4 * lane; }
+    static __device__ __forceinline__ void decode(const uint8_t* block, uint32_t lane, float (&out)[1][4]) {
+        decode4<CODEC>(block, 4 * lane, out[0]);
+    }
+};
+
+template <>
+struct Span<kQ4_0> {
+    static constexpr int kGroups = 2;
+    static constexpr uint32_t kLanes = 4, kStride = 16;
+    static __device__ __forceinline__ uint32_t first(uint32_t lane) { return 4 * lane; }
+    static __device__ __forceinline__ void decode(const uint8_t* block, uint32_t lane, float (&out)[2][4]) {
+        const float d = f16_at(block, 0);
+        const uint32_t q = load32(block + 2 + 4 * lane);
+#pragma unroll
+        for (int g = 0; g < 2; g++)
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                out[g][i] = d * static_cast<float>(static_cast<int>((byte_of(q, i) >> (4 * g)) & 0x0fu) - 8);
+    }
+};
+
+// Q4_K and Q5_K: groups 2 p and 2 p + 1 of the block, the nibbles of one dword.
+template <bool FIFTH>
+struct SpanK45 {
+    static constexpr int kGroups = 2;
+    static constexpr uint32_t kLanes = 32, kStride = 32;
+    static __device__ __forceinline__ uint32_t first(uint32_t lane) { return (lane >> 3) * 64 + 4 * (lane & 7u); }
+    static __device__ __forceinline__ void decode(const uint8_t* block, uint32_t lane, float (&out)[2][4]) {
+        const uint32_t pair = lane >> 3, i0 = 4 * (lane & 7u);
+        const uint4 header = load128(block);  // d, dmin, the twelve packed scales
+        const uint32_t high = FIFTH ? load32(block + 16 + i0) : 0u;
+        const uint32_t q = load32(block + (FIFTH ? 48 : 16) + pair * 32 + i0);
+        const float d = f16_bits_to_f32(header.x & 0xffffu), dmin = f16_bits_to_f32(header.x >> 16);
+#pragma unroll
+        for (int g = 0; g < 2; g++) {
+            // scale_min_k4 of group 2 * pair + g
+            const uint32_t shift = 8u * ((2 * pair + g) & 3u);
+            const uint32_t s0 = (header.y >> shift) & 0xffu, s1 = (header.z >> shift) & 0xffu, s2 = (header.w >> shift) & 0xffu;
+            const uint32_t scale = pair < 2 ? s0 & 63u : (s2 & 0x0fu) | ((s0 >> 6) << 4);
+            const uint32_t min = pair < 2 ? s1 & 63u : (s2 >> 4) | ((s1 >> 6) << 4);
+            const float dl = d * static_cast<float>(scale), ml = dmin * static_cast<float>(min);
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                uint32_t quant = (byte_of(q, i) >> (4 * g)) & 0x0fu;
+                if (FIFTH) quant |= ((byte_of(high, i) >> (2 * pair + g)) & 1u) << 4;
+                const float prod = dl * static_cast<float>(quant);
+                out[g][i] = prod - ml;
+            }
+        }
+    }
+};
+template <>
+struct Span<kQ4_K> : SpanK45<false> {};
+template <>
+struct Span<kQ5_K> : SpanK45<true> {};
+
+// Q2_K, Q3_K and Q6_K: the four runs of a half block whose two-bit parts share a dword.
+struct SpanFour {
+    static constexpr int kGroups = 4;
+    static constexpr uint32_t kLanes = 16, kStride = 32;
+    static __device__ __forceinline__ uint32_t first(uint32_t lane) { return (lane >> 3) * 128 + 4 * (lane & 7u); }
+};
+template <>
+struct Span<kQ2_K> : SpanFour {
+    static __device__ __forceinline__ void decode(const uint8_t* block, uint32_t lane, float (&out)[4][4]) {
+        const uint32_t half = lane >> 3, i0 = 4 * (lane & 7u);
+        const uint2 scales = load64(block + 8 * half);
+        const uint32_t q = load32(block + 16 + half * 32 + i0), dd = load32(block + 80);
+        const float d = f16_bits_to_f32(dd & 0xffffu), dmin = f16_bits_to_f32(dd >> 16);
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            const uint32_t scale = ((g < 2 ? scales.x : scales.y) >> (8 * (2 * (g & 1) + (i0 >> 4)))) & 0xffu;
+            const float dl = d * static_cast<float>(scale & 0x0fu), ml = dmin * static_cast<float>(scale >> 4);
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const float prod = dl * static_cast<float>((byte_of(q, i) >> (2 * g)) & 3u);
+                out[g][i] = prod - ml;
+            }
+        }
+    }
+};
+template <>
+struct Span<kQ3_K> : SpanFour {
+    static __device__ __forceinline__ void decode(const uint8_t* block, uint32_t lane, float (&out)[4][4]) {
+        const uint32_t half = lane >> 3, i0 = 4 * (lane & 7u);
+        const uint32_t hm = load32(block + i0), q = load32(block + 32 + half * 32 + i0);
+        const uint2 low = load64(block + 96);
+        const uint32_t high = load32(block + 104);
+        const float d = f16_at(block, 108);
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            const uint32_t at = 2 * (g & 1) + (i0 >> 4);  // of the group's byte in its word
+            const uint32_t bits = (((g < 2 ? low.x : low.y) >> (8 * at + 4 * half)) & 0x0fu) |
+                                  (((high >> (8 * at + 2 * (2 * half + (g >> 1)))) & 3u) << 4);
+            const float dl = d * static_cast<float>(static_cast<int>(bits) - 32);
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int two = static_cast<int>((byte_of(q, i) >> (2 * g)) & 3u);
+                const int four = ((byte_of(hm, i) >> (half * 4 + g)) & 1u) == 0 ? 4 : 0;
+                out[g][i] = dl * static_cast<float>(two - four);
+            }
+        }
+    }
+};
+template <>
+struct Span<kQ6_K> : SpanFour {
+    static __device__ __forceinline__ void decode(const uint8_t* block, uint32_t lane, float (&out)[4][4]) {
+        const uint32_t half = lane >> 3, i0 = 4 * (lane & 7u);
+        const uint32_t even = load32(block + half * 64 + i0), odd = load32(block + half * 64 + 32 + i0);
+        const uint32_t qh = load32(block + 128 + half * 32 + i0);
+        const uint2 scales = load64(block + 192 + 8 * half);
+        const float d = f16_at(block, 208);
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            const uint32_t byte = ((g < 2 ? scales.x : scales.y) >> (8 * (2 * (g & 1) + (i0 >> 4)))) & 0xffu;
+            const float ds = d * static_cast<float>(static_cast<int>(static_cast<int8_t>(byte)));
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const uint32_t nib = (byte_of(g & 1 ? odd : even, i) >> (g < 2 ? 0 : 4)) & 0x0fu;
+                const uint32_t two = (byte_of(qh, i) >> (2 * g)) & 3u;
+                out[g][i] = ds * static_cast<float>(static_cast<int>(nib | (two << 4)) - 32);
+            }
+        }
+    }
+};
+
 }  // namespace et

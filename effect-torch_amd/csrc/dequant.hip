@@ -41,7 +41,8 @@ __device__ __forceinline__ uint64_t source_index(const IndexLayout& layout, uint
 }
 
 constexpr uint64_t kNoBadIndex = ~0ull;
-constexpr uint32_t kChunksPerPass = 4;  // 1024-column chunks a workgroup decodes per pass
+template <int CODEC>
+constexpr uint32_t kSpansPerThread = 4 / Span<CODEC>::kGroups;  // sixteen values
 
 // The value of an index as 64 bits, and whether the table has such a row.
 __device__ __forceinline__ uint64_t index_value(const void* indexes, int index_is_i64, uint64_t source, uint64_t table_rows, bool& bad) {
@@ -63,27 +64,30 @@ __device__ __forceinline__ uint64_t index_value(const void* indexes, int index_i
 // Many, or strided: the block is cleared first, the workgroups that decode check their own index, and a third launch
 // adds the value.
 constexpr uint32_t kChecksInFlight = 16;                        // loads in flight per thread of the checking workgroup
-constexpr uint64_t kMostSelfChecked = 256u * kChecksInFlight;  // indexes it takes in one round
+constexpr uint64_t kMostSelfChecked = 2 * 256u * kChecksInFlight;  // indexes it takes in two rounds
 
 // Two launches less (contiguous ids in a captured graph, three launches / one in us: one id of 4096 Q4_K columns 6.9 / 4.8,
-// 1000 ids 10.6 / 7.7, 4096 ids 22.1 / 20.1; 4096 ids of 32 Q8_0 columns 8.2 / 5.7). One workgroup takes more than 4096 ids
-// in rounds, each a memory latency that narrow rows do not hide (100 000 ids of 256 columns 73 / 97), and strided
-// ids cost each of its threads sixteen times a division per dimension (1000 ids 7.1 / 11.4).
+// 1000 ids 10.6 / 7.7, 4096 ids 22.1 / 20.1; 4096 ids of 32 Q8_0 columns 8.2 / 5.7, 8192 ids 10.0 / 7.0). One workgroup takes
+// more than 4096 ids in rounds, each a memory latency: the second is hidden also by the narrowest rows, further ones are not
+// (100 000 ids of 256 columns took 73 in three launches and 97 in one), and strided ids cost each of its threads sixteen
+// times a division per dimension (1000 ids 7.1 / 11.4).
 bool lookup_checks_itself(const IndexLayout& layout, uint64_t count) { return layout.contiguous && count <= kMostSelfChecked; }
 
 __device__ void report_bad_index(const void* indexes, int index_is_i64, uint64_t offset, uint32_t count, uint64_t table_rows,
                                  unsigned long long* status) {
     __shared__ unsigned long long lowest[256];
     unsigned long long position = kNoBadIndex;
-    bool bad[kChecksInFlight];
+    for (uint32_t first = threadIdx.x; first < count && position == kNoBadIndex; first += 256u * kChecksInFlight) {
+        bool bad[kChecksInFlight];
 #pragma unroll
-    for (uint32_t i = 0; i < kChecksInFlight; i++) {
-        const uint32_t p = threadIdx.x + 256u * i;
-        index_value(indexes, index_is_i64, offset + (p < count ? p : 0u), table_rows, bad[i]);
+        for (uint32_t i = 0; i < kChecksInFlight; i++) {
+            const uint32_t p = first + 256u * i;
+            index_value(indexes, index_is_i64, offset + (p < count ? p : 0u), table_rows, bad[i]);
+        }
+#pragma unroll
+        for (int i = kChecksInFlight - 1; i >= 0; i--)
+            if (bad[i] && first + 256u * i < count) position = first + 256u * i;
     }
-#pragma unroll
-    for (int i = kChecksInFlight - 1; i >= 0; i--)
-        if (bad[i] && threadIdx.x + 256u * i < count) position = threadIdx.x + 256u * i;
     lowest[threadIdx.x] = position;
     __syncthreads();
     for (uint32_t step = 128; step > 0; step >>= 1) {
@@ -111,51 +115,61 @@ __global__ void status_finalize_kernel(const void* indexes, int index_is_i64, In
     status[1] = index_value(indexes, index_is_i64, source_index(layout, status[0]), table_rows, ignored);
 }
 
-// One workgroup per (output row, four 1024-column chunks): the row's index is read once per workgroup
-// and everything per lane is 32-bit arithmetic (a 64-bit division per item, as a flat grid-stride
-// loop over all outputs needs, costs more than the decode itself). CHECKER: workgroup (0, 0) checks all the indexes.
+// A workgroup decodes one output row, or sixteen values per thread of a wider one, or as many rows as its threads hold: the
+// row's index is read once per thread and everything else is 32-bit arithmetic. A thread takes spans (decode_device.h) of
+// sixteen values in all and decodes them before its first store, so that their loads are in flight together; the stores of a
+// wave are whole 128-byte lines. CHECKER: workgroup (0, 0) checks all the indexes.
+//
+// Bound: stores (4 bytes out per 0.3 to 1.1 in) now that the loads are few. With a load per header field and dword of
+// quants (24 a thread for Q4_K) the address path of a compute unit alone took half the time. In a graph, before / after (us):
+// 5000 ids of 4096 columns Q4_K 24.5 / 17.4 (5.4 TB/s), Q5_K 25.2 / 17.5, Q3_K 23.9 / 16.6, Q6_K 21.2 / 17.7, Q8_0 21.4 / 18.4;
+// 20 000 Q4_K 126 / 87; rows that left threads idle: 100 000 ids of 256 columns 73 / 25.
 template <int CODEC, bool CHECKER>
 __global__ __launch_bounds__(256) void dequant_rows_kernel(
     const uint8_t* __restrict__ weight, const void* __restrict__ indexes, int index_is_i64,
-    IndexLayout layout, uint64_t out_rows, uint64_t table_rows, uint32_t columns,
+    IndexLayout layout, uint64_t out_rows, uint64_t table_rows, uint32_t columns, uint32_t rows_per_wg,
     uint64_t row_bytes, float* __restrict__ out, unsigned long long* status) {
-    constexpr uint32_t kValues = block_values(CODEC);
+    using S = Span<CODEC>;
     constexpr uint32_t kBytes = block_bytes(CODEC);
+    constexpr uint32_t kSpans = kSpansPerThread<CODEC>;
     constexpr uint32_t kCheckers = CHECKER ? 1u : 0u;
-    const uint32_t chunks = (columns + 1023u) >> 10;
     if (blockIdx.x < kCheckers) {
         if (blockIdx.y == 0) report_bad_index(indexes, index_is_i64, layout.offset, static_cast<uint32_t>(out_rows), table_rows, status);
         return;
     }
-    for (uint64_t p = blockIdx.x - kCheckers; p < out_rows; p += gridDim.x - kCheckers) {
+    const uint32_t spans = columns / (4 * S::kGroups);  // of a row
+    const uint32_t sub_row = rows_per_wg == 1 ? 0u : threadIdx.x / spans;
+    const uint32_t thread = threadIdx.x - sub_row * spans;  // among those of its row
+    if (sub_row >= rows_per_wg) return;
+    const uint64_t stride = static_cast<uint64_t>(gridDim.x - kCheckers) * rows_per_wg;
+    for (uint64_t p = static_cast<uint64_t>(blockIdx.x - kCheckers) * rows_per_wg + sub_row; p < out_rows; p += stride) {
         uint64_t row = p;
         if (indexes != nullptr) {
             bool bad;
             row = index_value(indexes, index_is_i64, source_index(layout, p), table_rows, bad);
             if (bad) {  // skipped, like the reference's Metal kernel
-                if (!CHECKER && blockIdx.y == 0 && threadIdx.x == 0) atomicMin(status, static_cast<unsigned long long>(p));
+                if (!CHECKER && blockIdx.y == 0 && thread == 0) atomicMin(status, static_cast<unsigned long long>(p));
                 continue;
             }
         }
         const uint8_t* packed_row = weight + row * row_bytes;
         float* out_row = out + p * columns;
-        // Four chunks per pass, all decoded before the first store: their loads are in flight together.
-        for (uint32_t first = blockIdx.y * kChunksPerPass; first < chunks; first += gridDim.y * kChunksPerPass) {
-            float values[kChunksPerPass][4];
+        for (uint32_t at = blockIdx.y * (256u * kSpans); at < spans; at += gridDim.y * (256u * kSpans)) {
+            float values[kSpans][S::kGroups][4];
 #pragma unroll
-            for (uint32_t u = 0; u < kChunksPerPass; u++) {
-                const uint32_t column = ((first + u) << 10) + (threadIdx.x << 2);
-                if (column >= columns) continue;  // columns is a multiple of the block width, so of four
-                const uint32_t block_index = column / kValues;
-                decode4<CODEC>(packed_row + static_cast<uint64_t>(block_index) * kBytes, column - block_index * kValues,
-                               values[u]);
+            for (uint32_t u = 0; u < kSpans; u++) {
+                const uint32_t span = at + 256u * u + thread;
+                if (span < spans) S::decode(packed_row + static_cast<uint64_t>(span / S::kLanes) * kBytes, span % S::kLanes, values[u]);
             }
 #pragma unroll
-            for (uint32_t u = 0; u < kChunksPerPass; u++) {
-                const uint32_t column = ((first + u) << 10) + (threadIdx.x << 2);
-                if (column >= columns) continue;
-                *reinterpret_cast<float4*>(out_row + column) =
-                    make_float4(values[u][0], values[u][1], values[u][2], values[u][3]);
+            for (uint32_t u = 0; u < kSpans; u++) {
+                const uint32_t span = at + 256u * u + thread;
+                if (span >= spans) continue;
+                float* to = out_row + span / S::kLanes * block_values(CODEC) + S::first(span % S::kLanes);
+#pragma unroll
+                for (int g = 0; g < S::kGroups; g++)
+                    *reinterpret_cast<float4*>(to + g * S::kStride) =
+                        make_float4(values[u][g][0], values[u][g][1], values[u][g][2], values[u][g][3]);
             }
         }
     }
@@ -168,14 +182,17 @@ hipError_t launch_dequant(const uint8_t* weight, const void* indexes, int index_
     const uint64_t row_bytes = columns / block_values(CODEC) * block_bytes(CODEC);
     if (out_rows == 0 || columns == 0) return hipSuccess;
     // The loops in the kernel take what the grid limits leave over.
-    const uint64_t chunks = (((columns + 1023) >> 10) + kChunksPerPass - 1) / kChunksPerPass;
-    const uint32_t grid_x = static_cast<uint32_t>(out_rows < (1u << 24) ? out_rows : (1u << 24));
-    const uint32_t grid_y = static_cast<uint32_t>(chunks < 1024 ? chunks : 1024);
+    const uint64_t spans = columns / (4 * Span<CODEC>::kGroups);
+    const uint32_t rows_per_wg = spans >= 256 ? 1u : static_cast<uint32_t>(256 / spans);
+    const uint64_t parts = (spans + 256 * kSpansPerThread<CODEC> - 1) / (256 * kSpansPerThread<CODEC>);
+    const uint64_t groups = (out_rows + rows_per_wg - 1) / rows_per_wg;
+    const uint32_t grid_x = static_cast<uint32_t>(groups < (1u << 24) ? groups : (1u << 24));
+    const uint32_t grid_y = static_cast<uint32_t>(parts < 1024 ? parts : 1024);
     auto* status_words = static_cast<unsigned long long*>(status);
     if (indexes != nullptr && lookup_checks_itself(layout, out_rows)) {
         hipLaunchKernelGGL((dequant_rows_kernel<CODEC, true>), dim3(grid_x + 1, grid_y), dim3(256), 0,
                            stream, weight, indexes, index_is_i64, layout, out_rows, table_rows,
-                           static_cast<uint32_t>(columns), row_bytes, out, status_words);
+                           static_cast<uint32_t>(columns), rows_per_wg, row_bytes, out, status_words);
         return hipGetLastError();
     }
     if (indexes != nullptr) {
@@ -183,7 +200,7 @@ hipError_t launch_dequant(const uint8_t* weight, const void* indexes, int index_
     }
     hipLaunchKernelGGL((dequant_rows_kernel<CODEC, false>), dim3(grid_x, grid_y), dim3(256), 0,
                        stream, weight, indexes, index_is_i64, layout, out_rows, table_rows,
-                       static_cast<uint32_t>(columns), row_bytes, out, status_words);
+                       static_cast<uint32_t>(columns), rows_per_wg, row_bytes, out, status_words);
     if (indexes != nullptr) {
         hipLaunchKernelGGL(status_finalize_kernel, dim3(1), dim3(64), 0, stream, indexes,
                            index_is_i64, layout, table_rows, status_words);
