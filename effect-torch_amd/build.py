@@ -46,6 +46,7 @@ SOURCES = {
     "gemm_h16_wide.hip": [],
     "kv_attention.hip": [],
     "kv_chunk.hip": [],
+    "kv_bytes.hip": [],
     "decode_ops.hip": ["-ffp-contract=off"],
     "quantized.cpp": [],
     "static_workspace.cpp": [],

@@ -295,6 +295,7 @@ struct KvLaunchShape {
     uint32_t splits;
     uint64_t workgroups;
     uint64_t workspace_bytes;
+    bool bytes;  // kv_bytes.hip stands in for the streaming kernel
 };
 KvLaunchShape kv_attention_shape(const KvAttention& p);
 // Attends, appends the new rows, merges; `workspace` holds kv_attention_shape(p).workspace_bytes.

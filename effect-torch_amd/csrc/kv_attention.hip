@@ -292,66 +292,12 @@ __device__ __forceinline__ void attend_step_scatter(const float (&q)[G][Piece<T>
     }
 }
 
-// out[query, column] = sum_i w_i acc_i / sum_i w_i l_i with w_i = exp2(m_i - max m) over the
-// partial records of the context splits.
-__device__ __forceinline__ void merge_splits(const KvArgs& a, uint64_t query, uint32_t column) {
-    const uint32_t stride = a.width + 2;
-    const float* records = a.partial + query * a.splits * stride;
-    float top = kLowest, total = 0.f, value = 0.f;
-#pragma unroll 4
-    for (uint32_t i = 0; i < a.splits; i++) {
-        const float m = records[i * stride], l = records[i * stride + 1], part = records[i * stride + 2 + column];
-        const float next = fmaxf(top, m);
-        const float keep = __builtin_amdgcn_exp2f(top - next), weight = __builtin_amdgcn_exp2f(m - next);
-        total = fmaf(total, keep, weight * l);
-        value = fmaf(value, keep, weight * part);
-        top = next;
-    }
-    a.out[query * a.width + column] = value / total;
-}
-
 // Streaming kernel. LPT lanes share one position (each holds Piece<T>::kDims of the width,
 // width == LPT * kDims), so a wave covers 64 / LPT positions per load and the workgroup
 // WAVES * 64 / LPT; U such loads are in flight per step. G query heads of one kv head are
 // served from the same K / V registers. WAVES = 8 when the launch has enough rows of queries to give
 // every compute unit a workgroup without splitting the context (no partial records, no merge
 // launch), else 4.
-// q of the workgroup's G heads, then k and v of its kv head, for one slot, from the K shares of the
-// projection: the sums in share order, the bias, the rotary pairs of q and k - what
-// reduce_group_rotary_kernel (gemm_h16.hip) stores. out: [(G + 2)][width] floats in LDS.
-template <int G>
-__device__ void project_rows(const KvArgs& a, uint32_t slot, uint32_t head0, uint32_t kv_head, float* out,
-                             uint32_t threads) {
-    const KvProjected& s = a.projected;
-    const uint32_t width = a.width, half = width / 2;
-    const uint64_t share_stride = s.launch_rows * s.vectors;
-    const auto summed = [&](uint32_t first_row, const float* bias, uint32_t row) {
-        const float* first = s.shares + static_cast<uint64_t>(slot) * s.launch_rows + first_row + row;
-        float total = first[0];
-        for (uint32_t k = 1; k < s.count; k++) total += first[k * share_stride];
-        return bias != nullptr ? total + bias[row] : total;
-    };
-    const uint32_t offset = s.offsets_len == 1 ? s.offsets[0] : s.offsets[slot];
-    const uint32_t rotated = (G + 1) * half;  // the pairs of the G query heads, then of the key head
-    for (uint32_t item = threadIdx.x; item < rotated + width; item += threads) {
-        if (item < rotated) {
-            const uint32_t h = item / half, index = item - h * half;
-            const uint32_t head = h < G ? head0 + h : kv_head;
-            const uint32_t first_row = h < G ? s.q_row : s.k_row;
-            const float* bias = h < G ? s.q_bias : s.k_bias;
-            const uint32_t lo = s.interleaved ? 2u * index : index, hi = s.interleaved ? lo + 1u : lo + half;
-            float value_lo = summed(first_row, bias, head * width + lo);
-            float value_hi = summed(first_row, bias, head * width + hi);
-            rotate_pair(value_lo, value_hi, offset, 0u, index, width, s.theta, s.sign, value_lo, value_hi);
-            out[h * width + lo] = value_lo;
-            out[h * width + hi] = value_hi;
-        } else {
-            const uint32_t d = item - rotated;
-            out[(G + 1) * width + d] = summed(s.v_row, s.v_bias, kv_head * width + d);
-        }
-    }
-}
-
 // PROJECTED: q, k, v arrive as the K shares of their projections (KvArgs::projected, one token per slot).
 template <typename T, int LPT, int G, int U, int WAVES, bool PROJECTED>
 __global__ __launch_bounds__(64 * WAVES) void kv_attend_kernel(const KvArgs a) {
@@ -407,7 +353,7 @@ __global__ __launch_bounds__(64 * WAVES) void kv_attend_kernel(const KvArgs a) {
         }
     }
     constexpr bool from_shares = PROJECTED;
-    if constexpr (from_shares) project_rows<G>(a, slot, head0, kv_head, projected, kThreads);
+    if constexpr (from_shares) project_rows(a, slot, G, head0, kv_head, projected, kThreads);
     __syncthreads();
 
     float q[G][DPL];
@@ -713,12 +659,46 @@ __global__ __launch_bounds__(64) void kv_attend_any_kernel(const KvArgs a) {
     }
 }
 
-// Combines the partial records of the context splits: a workgroup per query row, a thread per column.
+// out[query, column] = sum_i w_i acc_i / sum_i w_i l_i with w_i = exp2(m_i - max m) over the partial records of the context
+// splits: a workgroup per query row, a thread per column. A wave's lanes take a split each for the maximum and the weights,
+// while the first records' values are on their way: two round trips to L2 where a chain over the records took one for
+// every four (32 heads of 64 splits: 7.5 -> 4.4 us).
 __global__ void kv_merge_kernel(const KvArgs a) {
     const uint64_t query = blockIdx.x;
     const uint32_t slot = static_cast<uint32_t>(query / (static_cast<uint64_t>(a.query_heads) * a.tokens));
     if (!slot_span(a, slot).ok) return;
-    for (uint32_t column = threadIdx.x; column < a.width; column += blockDim.x) merge_splits(a, query, column);
+    constexpr uint32_t kAhead = 8;
+    const uint32_t stride = a.width + 2, lane = threadIdx.x & 63u;
+    const float* records = a.partial + query * a.splits * stride;
+    for (uint32_t first = 0; first < a.width; first += blockDim.x) {
+        const uint32_t column = min(first + threadIdx.x, a.width - 1);  // whole waves: the lanes past the end help with the weights
+        float top = kLowest, total = 0.f, value = 0.f;
+        for (uint32_t base = 0; base < a.splits; base += 64) {
+            const uint32_t count = min(a.splits - base, 64u);
+            const float* record = records + static_cast<uint64_t>(base) * stride;
+            const bool mine = lane < count;
+            const float m = mine ? record[lane * stride] : kLowest, l = mine ? record[lane * stride + 1] : 0.f;
+            float part[kAhead];
+            const auto load = [&](uint32_t from) {
+#pragma unroll
+                for (uint32_t j = 0; j < kAhead; j++) part[j] = record[min(from + j, count - 1) * stride + 2 + column];
+            };
+            load(0);
+            const float next = fmaxf(top, group_max<64>(m));
+            const float keep = __builtin_amdgcn_exp2f(top - next), weight = mine ? __builtin_amdgcn_exp2f(m - next) : 0.f;
+            top = next;
+            total = fmaf(total, keep, group_sum<64>(mine ? weight * l : 0.f));
+            value *= keep;
+            for (uint32_t from = 0; from < count; from += kAhead) {
+#pragma unroll
+                for (uint32_t j = 0; j < kAhead; j++)
+                    if (from + j < count)
+                        value = fmaf(__uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(weight), from + j)), part[j], value);
+                if (from + kAhead < count) load(from + kAhead);
+            }
+        }
+        if (first + threadIdx.x < a.width) a.out[query * a.width + column] = value / total;
+    }
 }
 
 template <typename T, int LPT, int G>
@@ -842,6 +822,34 @@ bool streaming_is_faster(const KvAttention& p, const KvLaunchShape& streaming, u
     return chunk > 0.95 * streamed;
 }
 
+// Whether kv_bytes.hip attends in the streaming kernel's place, and its launch: one token per slot over u8 slabs. Measured
+// (us, streaming / bytes kernel with their merge launches; slots at context, 32/8 heads x 128): 32 at 2048 53.4 / 29.8, 64 at
+// 1000 59.0 / 34.5, 12 at 1000 19.6 / 15.6, 4 at 2000 15.7 / 13.9, 3 at 10000 to 30000 61.3 / 37.3, 1 at 60000 52.0 / 34.0;
+// 24/8 heads x 128, 40 at 500 to 1500 67.7 / 32.8; 16/8 heads x 64, 32 at 1000 19.7 / 11.8. It starts more slowly (limbs of q, a
+// longer fill): 1 at 1000 (8 Ki rows of kv heads) 12.0 / 13.4, 4 at 700 (22 Ki) 11.7 / 13.4, 4 at 1000 (32 Ki) 12.6 / 13.9 but 12
+// at 400 (38 Ki) 13.6 / 11.6 and 1 at 6000 16.3 / 14.5; 64 at 64 17.6 / 18.3 but 64 at 200 23.3 / 21.3. One query head per kv head
+// leaves it a quarter of its matrix rows: 32 at 2000 128 / 138. Workgroups of eight waves, one per compute unit, need the
+// fewest partial records (30 at 1000, 16/8 heads x 64: 11.3, four waves 14.0); where a split has many positions, two
+// workgroups of four share a compute unit more evenly (12 at 2000 20.5 / 19.7, 3 at 10000 to 30000 39.7 / 37.3).
+constexpr uint64_t kBytesMinRows = 32 * 1024, kBytesFourWavesRows = 192 * 1024;
+constexpr uint32_t kBytesMinContext = 128;
+void streaming_bytes(const KvAttention& p, KvLaunchShape& shape) {
+    const uint32_t group = p.query_heads / p.kv_heads;
+    const uint64_t units = static_cast<uint64_t>(p.active_batch) * p.kv_heads, context = p.max_context;
+    if (!shape.streaming || p.slab_dtype != ET_DTYPE_U8 || p.tokens != 1 || group < 2 || group > 4 ||
+        (p.width != 64 && p.width != 128) || context < kBytesMinContext || units * context < kBytesMinRows)
+        return;
+    const uint64_t reach = static_cast<uint64_t>(kKvTableEntries - 2) * p.block_size - 63;  // positions a split's table lists
+    shape.bytes = true;
+    shape.waves = units < 256 && units * context >= kBytesFourWavesRows ? 4 : 8;
+    uint64_t splits = units >= 256 ? 1 : (shape.waves == 4 ? 512 : 256) / units;
+    splits = std::min<uint64_t>(splits, (context + 64 * shape.waves - 1) / (64 * shape.waves));  // a tile for every wave
+    splits = std::max<uint64_t>({splits, (context + reach - 1) / reach, 1});
+    shape.splits = static_cast<uint32_t>(splits);
+    shape.workgroups = units * splits;
+    shape.workspace_bytes = splits > 1 ? units * group * splits * (p.width + 2) * sizeof(float) : 0;
+}
+
 }  // namespace
 
 KvLaunchShape kv_attention_shape(const KvAttention& p) {
@@ -870,6 +878,7 @@ KvLaunchShape kv_attention_shape(const KvAttention& p) {
             shape.workspace_bytes = splits > 1 ? queries * splits * (p.width + 2) * sizeof(float) : 0;
         }
     }
+    streaming_bytes(p, shape);
     return shape;
 }
 
@@ -907,9 +916,9 @@ hipError_t kv_attention(const KvAttention& p, void* workspace, hipStream_t strea
     a.partial = static_cast<float*>(workspace);
     // The streaming kernel quantises the rows itself when it writes them in one piece (no context
     // splits), every slot is active and its heads are whole stages; else a quantiser launch follows.
+    const uint64_t served = shape.bytes ? p.query_heads / p.kv_heads : streaming_group(p);  // heads of a workgroup
     const bool fused_tiles = p.prepared != nullptr && p.tokens == 1 && shape.streaming && shape.splits == 1 &&
-                             p.active_batch == p.batch &&
-                             (static_cast<uint64_t>(streaming_group(p)) * p.width) % 256 == 0;
+                             p.active_batch == p.batch && (served * p.width) % 256 == 0;
     a.prepared = fused_tiles ? p.prepared : nullptr;
     a.vector_tiles = (p.batch + 31u) / 32u;
     a.projected = p.projected;
@@ -933,6 +942,8 @@ hipError_t kv_attention(const KvAttention& p, void* workspace, hipStream_t strea
     hipError_t error;
     if (shape.chunk) {
         error = kv_chunk(p.slab_dtype, a, kv_chunk_grid(p).row_waves, static_cast<uint32_t>(shape.workgroups), stream);
+    } else if (shape.bytes) {
+        error = kv_bytes(a, shape.waves, static_cast<uint32_t>(shape.workgroups), stream);
     } else if (shape.streaming) {
         const int g = streaming_group(p);
         const uint32_t workgroups = static_cast<uint32_t>(shape.workgroups);

@@ -7,6 +7,7 @@
 
 #include <cstdint>
 
+#include "decode_math.h"
 #include "kernels.h"
 #include "quantize_halves.h"  // dpp_f32
 
@@ -157,6 +158,41 @@ __device__ __forceinline__ void query_range(const KvArgs& a, const Span& s, uint
     begin = min(begin, end);
 }
 
+// q of the workgroup's G heads, then k and v of its kv head, for one slot, from the K shares of the
+// projection: the sums in share order, the bias, the rotary pairs of q and k - what
+// reduce_group_rotary_kernel (gemm_h16.hip) stores. out: [(G + 2)][width] floats in LDS.
+__device__ __forceinline__ void project_rows(const KvArgs& a, uint32_t slot, uint32_t G, uint32_t head0, uint32_t kv_head,
+                                             float* out, uint32_t threads) {
+    const KvProjected& s = a.projected;
+    const uint32_t width = a.width, half = width / 2;
+    const uint64_t share_stride = s.launch_rows * s.vectors;
+    const auto summed = [&](uint32_t first_row, const float* bias, uint32_t row) {
+        const float* first = s.shares + static_cast<uint64_t>(slot) * s.launch_rows + first_row + row;
+        float total = first[0];
+        for (uint32_t k = 1; k < s.count; k++) total += first[k * share_stride];
+        return bias != nullptr ? total + bias[row] : total;
+    };
+    const uint32_t offset = s.offsets_len == 1 ? s.offsets[0] : s.offsets[slot];
+    const uint32_t rotated = (G + 1) * half;  // the pairs of the G query heads, then of the key head
+    for (uint32_t item = threadIdx.x; item < rotated + width; item += threads) {
+        if (item < rotated) {
+            const uint32_t h = item / half, index = item - h * half;
+            const uint32_t head = h < G ? head0 + h : kv_head;
+            const uint32_t first_row = h < G ? s.q_row : s.k_row;
+            const float* bias = h < G ? s.q_bias : s.k_bias;
+            const uint32_t lo = s.interleaved ? 2u * index : index, hi = s.interleaved ? lo + 1u : lo + half;
+            float value_lo = summed(first_row, bias, head * width + lo);
+            float value_hi = summed(first_row, bias, head * width + hi);
+            rotate_pair(value_lo, value_hi, offset, 0u, index, width, s.theta, s.sign, value_lo, value_hi);
+            out[h * width + lo] = value_lo;
+            out[h * width + hi] = value_hi;
+        } else {
+            const uint32_t d = item - rotated;
+            out[(G + 1) * width + d] = summed(s.v_row, s.v_bias, kv_head * width + d);
+        }
+    }
+}
+
 // Sum over the LANES lanes of an aligned group; every lane gets the total.
 template <int LANES>
 __device__ __forceinline__ float group_sum(float v) {
@@ -180,6 +216,8 @@ __device__ __forceinline__ float group_max(float v) {
     return v;
 }
 
+// kv_bytes.hip: decode steps over u8 slabs on the int8 matrix cores; a.splits context splits per (slot, kv head).
+hipError_t kv_bytes(const KvArgs& a, int waves, uint32_t workgroups, hipStream_t stream);
 // kv_chunk.hip: calls of several tokens per slot on the matrix cores. `workgroups` = grid.units * splits.
 hipError_t kv_chunk(int32_t slab_dtype, const KvArgs& a, int row_waves, uint32_t workgroups, hipStream_t stream);
 
