@@ -22,7 +22,8 @@
 // Bound: reads of 128 bytes a position and head, with the ends of a launch. Per 64 positions of 128 columns a wave issues
 // about 700 vector and 16 matrix instructions (of 16 cycles) where the streaming kernel - a conversion, a scale and four
 // multiply-adds per byte - issues 2000. 32 slots at 2048 (138 MB): 53.4 -> 29.8 us, 4.7 TB/s; with the loads left out 17.
-// Ordinary loads: a row's two halves come in two instructions, and non-temporal ones fetched its line twice (37.5).
+// K comes by ordinary loads: the two halves of a row are two instructions', and non-temporal ones fetched its line twice
+// (37.5). Inputs from memory and not from the Infinity Cache: 49.0 -> 34.6.
 #include <hip/hip_runtime.h>
 
 #include <atomic>
@@ -52,9 +53,10 @@ struct BytesLds {
     static_assert(kBytes <= 160 * 1024, "LDS of a compute unit");
 };
 
-// A copy of sixteen bytes per lane to LDS (lane i to `to` + 16 i) that the compiler does not see (see kv_chunk.hip).
-__device__ __forceinline__ void copy_unseen(const void* from, uint32_t to) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(from), "s"(to) : "memory", "m0");
+// A non-temporal copy of sixteen bytes per lane to LDS (lane i to `to` + 16 i) that the compiler does not see (see
+// kv_chunk.hip). Its eight lanes a row take whole lines.
+__device__ __forceinline__ void copy_streamed(const void* from, uint32_t to) {
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt" : : "v"(from), "s"(to) : "memory", "m0");
 }
 
 // Eight rows of sixteen bytes to sixteen lanes of eight: lane i names row (i & 15) / 2, columns 8 (i & 1) .. + 7, and
@@ -108,18 +110,19 @@ __global__ __launch_bounds__(64 * WAVES, 2) void kv_bytes_kernel(const KvArgs a)
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     uint32_t* rows_of_block = reinterpret_cast<uint32_t*>(lds + L::kTableAt);
 
-    // The heads of a (slot, split) run side by side on one XCD (workgroups go to the eight in turn): a position's row holds
-    // all of them, 128 bytes each, and their scales share a line.
-    const uint32_t pairs = a.active_batch * a.splits, whole = pairs / 8 * 8;
-    uint32_t pair, kv_head;
-    if (blockIdx.x < whole * a.kv_heads) {
-        pair = blockIdx.x / (8 * a.kv_heads) * 8 + blockIdx.x % 8;
+    // Whole slots: the heads of one run side by side on one XCD (workgroups go to the eight in turn), as a position's row holds
+    // all of them and their scales share a line (32 slots at 2048, inputs from memory: 35.3 -> 34.6 us). Splits of a slot run
+    // side by side instead (one slot at 60000: 39.4 -> 37.6).
+    uint32_t split = 0, kv_head, slot;
+    if (a.splits == 1 && blockIdx.x < a.active_batch / 8 * 8 * a.kv_heads) {
+        slot = blockIdx.x / (8 * a.kv_heads) * 8 + blockIdx.x % 8;
         kv_head = blockIdx.x / 8 % a.kv_heads;
     } else {
-        pair = blockIdx.x / a.kv_heads;
-        kv_head = blockIdx.x % a.kv_heads;
+        const uint32_t pair = blockIdx.x / a.splits;
+        split = blockIdx.x % a.splits;
+        kv_head = pair % a.kv_heads;
+        slot = pair / a.kv_heads;
     }
-    const uint32_t split = pair % a.splits, slot = pair / a.splits;
     const uint32_t heads = a.query_heads / a.kv_heads, head0 = kv_head * heads;
     const int lane = threadIdx.x & 63, column = lane & 15, group = lane >> 4;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -186,7 +189,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void kv_bytes_kernel(const KvArgs a)
 #pragma unroll
         for (int c = 0; c < kCopies; c++) {
             const uint32_t r = c * kRowsPerCopy + lane / kPieces;
-            copy_unseen(v_base + slab_row(tile + r, shifts) * row_bytes + ((lane % kPieces) ^ swizzle(r)) * 16u,
+            copy_streamed(v_base + slab_row(tile + r, shifts) * row_bytes + ((lane % kPieces) ^ swizzle(r)) * 16u,
                           __builtin_amdgcn_readfirstlane(wave_lds + buffer * L::kValueTile + c * 1024u));
         }
 #pragma unroll
