@@ -10,7 +10,7 @@
 // vectors cost on v_dot4 (gemv_limb.hip: 48 dots per vector, row and lane) is here one matrix
 // instruction per 32-column block and sixteen rows: v_mfma_i32_16x16x32_i8 with the weights' quants
 // as its B operand (sixteen rows of W) and, as its A operand, the three signed-byte limbs of four
-// activation vectors in rows 4v + limb (row 4v + 3 is zero). A lane of the result then holds, for its
+// activation vectors in rows 4v + limb (row 4v + 3 is zero, or a limb of a fifth vector). A lane of the result then holds, for its
 // weight row and its vector, the three limb dots of the block side by side.
 //
 // Work split. A workgroup owns a contiguous range of rows (one per compute unit when the matrix
@@ -105,6 +105,22 @@ __device__ __forceinline__ void scaled_limbs(int (&acc)[3], float unit, float& s
     acc[0] = acc[1] = acc[2] = 0;
 }
 
+// A fifth vector (FIFTH): its three limbs are the rows 4v + 3 that four vectors leave empty, limb i in the fourth result of
+// lane group i (row 15 stays zero). Once per unit the groups' parts are put together, in every lane: limb i's `pos` is worth
+// 256^i, `neg` is the group's share of the minima. (Kept apart until the end of the row, positive and negative sums cost
+// two instructions less and a sixth more error where activations do not cancel.)
+__device__ __forceinline__ void join_groups(uint32_t q, float& pos, float& neg) {
+    pos = q == 3u ? 0.f : pos * __uint_as_float((127u + 8u * q) << 23);
+    // the two small limbs first: one rounding of the whole sum's size, as in scaled_limbs
+    const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(pos), __float_as_uint(neg), false, false);
+    const uint32_t two = __float_as_uint(__uint_as_float(rows[0]) + __uint_as_float(rows[1]));  // pos in even groups, neg in odd
+    const auto halves = __builtin_amdgcn_permlane32_swap(two, two, false, false);
+    const uint32_t four = __float_as_uint(__uint_as_float(halves[0]) + __uint_as_float(halves[1]));
+    const auto both = __builtin_amdgcn_permlane16_swap(four, four, false, false);
+    pos = __uint_as_float(both[0]);
+    neg = __uint_as_float(both[1]);
+}
+
 // ---------------------------------------------------------------------------
 // Codec traits: one 256-column unit (kUnitBytes) of sixteen rows against the A operands.
 //   rp     the unit in the lane's row of the LDS image
@@ -113,13 +129,15 @@ __device__ __forceinline__ void scaled_limbs(int (&acc)[3], float unit, float& s
 //   sums   f32 sums of the lane's vector over the unit's eight blocks, then the value of one unit of limb 0:
 //          SCALES = 1 for all of the unit's columns, SCALES = 4 for every 64 of them
 //          (next vector group: + sums_step floats)
+//   fifth_sums  the same of a fifth vector, whose part is added to total[VG]
 // ---------------------------------------------------------------------------
 struct Q4KMma {
     static constexpr uint32_t kUnitBytes = 144u;  // one super-block
+    static constexpr bool kTakesFifth = true;
     static __device__ __forceinline__ uint32_t chunk(uint32_t q) { return q; }
-    template <int VG, int UNIT, int SCALES, int BLOCKS>
-    static __device__ __forceinline__ void contract(const uint8_t* rp, uint32_t q, const long (&a)[VG][BLOCKS],
-                                                    const float* sums, uint32_t sums_step, float (&total)[VG]) {
+    template <int VG, int UNIT, int SCALES, bool FIFTH, int BLOCKS>
+    static __device__ __forceinline__ void contract(const uint8_t* rp, uint32_t q, const long (&a)[VG][BLOCKS], const float* sums,
+                                                    uint32_t sums_step, const float* fifth_sums, float (&total)[VG + FIFTH]) {
         const uint4 h = *reinterpret_cast<const uint4*>(rp);
         const float d = half_bits_to_float(h.x & 0xffffu), dmin = half_bits_to_float(h.x >> 16);
         // (scale, min) of the eight sub-blocks, a byte each: crates/runtime-cpu/src/quantized.rs:77-86
@@ -127,8 +145,8 @@ struct Q4KMma {
         uint32_t mn[2] = {h.z & 0x3f3f3f3fu, ((h.w >> 4) & 0x0f0f0f0fu) | ((h.z >> 2) & 0x30303030u)};
         // keeps the minima packed, a byte-to-float conversion each, instead of a mask per byte
         asm volatile("" : "+v"(mn[0]), "+v"(mn[1]));
-        int acc[VG][3];
-        float pos[VG];
+        int acc[VG][3], fifth_acc = 0;
+        float pos[VG], fifth_pos = 0.f;
 #pragma unroll
         for (int g = 0; g < VG; g++) acc[g][0] = acc[g][1] = acc[g][2] = 0, pos[g] = 0.f;
         const v4i zero = {0, 0, 0, 0};
@@ -148,6 +166,10 @@ struct Q4KMma {
 #pragma unroll
                 for (int k = 0; k < 3; k++) acc[g][k] += __mul24(c0[k], s_lo) + __mul24(c1[k], s_hi);
                 if constexpr (SCALES == 4) scaled_limbs(acc[g], sums[sums_step * g + 8 + p], pos[g]);
+                if constexpr (FIFTH) {
+                    fifth_acc += __mul24(c0[3], s_lo) + __mul24(c1[3], s_hi);
+                    if constexpr (SCALES == 4) fifth_pos = fmaf(fifth_sums[8 + p], static_cast<float>(fifth_acc), fifth_pos), fifth_acc = 0;
+                }
             }
         }
         // (the compiler turns these into v_cvt_f32_ubyte0..3)
@@ -170,6 +192,15 @@ struct Q4KMma {
             if constexpr (SCALES == 1) scaled_limbs(acc[g], sums[sums_step * g + 8], pos[g]);
             total[g] += d * pos[g] - dmin * neg;
         }
+        if constexpr (FIFTH) {  // the minima of sub-blocks 2q and 2q + 1 are this lane's part
+            const uint32_t mine = (q & 2u ? mn[1] : mn[0]) >> (16 * (q & 1u));
+            const float2 s = *reinterpret_cast<const float2*>(fifth_sums + 2 * q);
+            float neg = fmaf(static_cast<float>((mine >> 8) & 0xffu), s.y, static_cast<float>(mine & 0xffu) * s.x);
+            if constexpr (SCALES == 1) fifth_pos = static_cast<float>(fifth_acc);
+            join_groups(q, fifth_pos, neg);
+            if constexpr (SCALES == 1) fifth_pos *= fifth_sums[8];
+            total[VG] += d * fifth_pos - dmin * neg;
+        }
     }
 };
 
@@ -180,11 +211,13 @@ struct Q4KMma {
 // activations once per block.
 struct Q40Mma {
     static constexpr uint32_t kUnitBytes = 144u;  // eight blocks of 18 bytes
+    static constexpr bool kTakesFifth = false;
     static __device__ __forceinline__ uint32_t chunk(uint32_t q) { return ((q & 1u) << 1) | (q >> 1); }
-    template <int VG, int UNIT, int SCALES, int BLOCKS>
-    static __device__ __forceinline__ void contract(const uint8_t* rp, uint32_t q, const long (&a)[VG][BLOCKS],
-                                                    const float* sums, uint32_t sums_step, float (&total)[VG]) {
+    template <int VG, int UNIT, int SCALES, bool FIFTH, int BLOCKS>
+    static __device__ __forceinline__ void contract(const uint8_t* rp, uint32_t q, const long (&a)[VG][BLOCKS], const float* sums,
+                                                    uint32_t sums_step, const float* fifth_sums, float (&total)[VG + FIFTH]) {
         const uint32_t half = q >> 1, shift = (q & 1u) * 4u;
+        static_assert(!FIFTH, "scales by the block: see launch_vectors");
         float pos[VG], corr[VG], s[VG][8];
 #pragma unroll
         for (int g = 0; g < VG; g++) {
@@ -229,18 +262,19 @@ struct Q40Mma {
 // value in qh[32] between the scales and the nibbles - bit g of qh[i] belongs to column i of sub-block g.
 struct Q5KMma {
     static constexpr uint32_t kUnitBytes = 176u;
+    static constexpr bool kTakesFifth = true;
     static __device__ __forceinline__ uint32_t chunk(uint32_t q) { return q; }
-    template <int VG, int UNIT, int SCALES, int BLOCKS>
-    static __device__ __forceinline__ void contract(const uint8_t* rp, uint32_t q, const long (&a)[VG][BLOCKS],
-                                                    const float* sums, uint32_t sums_step, float (&total)[VG]) {
+    template <int VG, int UNIT, int SCALES, bool FIFTH, int BLOCKS>
+    static __device__ __forceinline__ void contract(const uint8_t* rp, uint32_t q, const long (&a)[VG][BLOCKS], const float* sums,
+                                                    uint32_t sums_step, const float* fifth_sums, float (&total)[VG + FIFTH]) {
         const uint4 h = *reinterpret_cast<const uint4*>(rp);
         const float d = half_bits_to_float(h.x & 0xffffu), dmin = half_bits_to_float(h.x >> 16);
         const uint32_t sc[2] = {h.y & 0x3f3f3f3fu, (h.w & 0x0f0f0f0fu) | ((h.y >> 2) & 0x30303030u)};
         uint32_t mn[2] = {h.z & 0x3f3f3f3fu, ((h.w >> 4) & 0x0f0f0f0fu) | ((h.z >> 2) & 0x30303030u)};
         asm volatile("" : "+v"(mn[0]), "+v"(mn[1]));
         const uint2 fifth = *reinterpret_cast<const uint2*>(rp + 16 + 8 * q);  // columns 8q..8q+7, all sub-blocks
-        int acc[VG][3];
-        float pos[VG];
+        int acc[VG][3], fifth_acc = 0;
+        float pos[VG], fifth_pos = 0.f;
 #pragma unroll
         for (int g = 0; g < VG; g++) acc[g][0] = acc[g][1] = acc[g][2] = 0, pos[g] = 0.f;
         const v4i zero = {0, 0, 0, 0};
@@ -261,6 +295,10 @@ struct Q5KMma {
 #pragma unroll
                 for (int k = 0; k < 3; k++) acc[g][k] += __mul24(c0[k], s_lo) + __mul24(c1[k], s_hi);
                 if constexpr (SCALES == 4) scaled_limbs(acc[g], sums[sums_step * g + 8 + p], pos[g]);
+                if constexpr (FIFTH) {
+                    fifth_acc += __mul24(c0[3], s_lo) + __mul24(c1[3], s_hi);
+                    if constexpr (SCALES == 4) fifth_pos = fmaf(fifth_sums[8 + p], static_cast<float>(fifth_acc), fifth_pos), fifth_acc = 0;
+                }
             }
         }
         const float m0 = static_cast<float>(mn[0] & 0xffu), m1 = static_cast<float>((mn[0] >> 8) & 0xffu);
@@ -282,6 +320,15 @@ struct Q5KMma {
             if constexpr (SCALES == 1) scaled_limbs(acc[g], sums[sums_step * g + 8], pos[g]);
             total[g] += d * pos[g] - dmin * neg;
         }
+        if constexpr (FIFTH) {  // the minima of sub-blocks 2q and 2q + 1 are this lane's part
+            const uint32_t mine = (q & 2u ? mn[1] : mn[0]) >> (16 * (q & 1u));
+            const float2 s = *reinterpret_cast<const float2*>(fifth_sums + 2 * q);
+            float neg = fmaf(static_cast<float>((mine >> 8) & 0xffu), s.y, static_cast<float>(mine & 0xffu) * s.x);
+            if constexpr (SCALES == 1) fifth_pos = static_cast<float>(fifth_acc);
+            join_groups(q, fifth_pos, neg);
+            if constexpr (SCALES == 1) fifth_pos *= fifth_sums[8];
+            total[VG] += d * fifth_pos - dmin * neg;
+        }
     }
 };
 
@@ -289,10 +336,12 @@ struct Q5KMma {
 // 32 signed bytes. The lanes with K index q take columns 8q..8q+7.
 struct Q80Mma {
     static constexpr uint32_t kUnitBytes = 272u;
+    static constexpr bool kTakesFifth = false;
     static __device__ __forceinline__ uint32_t chunk(uint32_t q) { return q; }
-    template <int VG, int UNIT, int SCALES, int BLOCKS>
-    static __device__ __forceinline__ void contract(const uint8_t* rp, uint32_t q, const long (&a)[VG][BLOCKS],
-                                                    const float* sums, uint32_t sums_step, float (&total)[VG]) {
+    template <int VG, int UNIT, int SCALES, bool FIFTH, int BLOCKS>
+    static __device__ __forceinline__ void contract(const uint8_t* rp, uint32_t q, const long (&a)[VG][BLOCKS], const float* sums,
+                                                    uint32_t sums_step, const float* fifth_sums, float (&total)[VG + FIFTH]) {
+        static_assert(!FIFTH, "scales by the block: see launch_vectors");
         float pos[VG];
 #pragma unroll
         for (int g = 0; g < VG; g++) pos[g] = 0.f;
@@ -325,14 +374,15 @@ struct Q80Mma {
     }
 };
 
-template <class T, int VG, int LOADERS, int DEPTH>
+template <class T, int VG, bool FIFTH, int LOADERS, int DEPTH>
 __global__ __launch_bounds__(64 * (kConsumers + LOADERS)) void gemv_mma_kernel(
     const uint8_t* __restrict__ weight, const float* __restrict__ x, uint64_t x_row_stride,
     const float* __restrict__ bias, float* __restrict__ y, uint32_t rows, uint32_t columns, uint32_t rows_per_wg,
     uint32_t vectors, uint32_t spin_limit, uint32_t* timeouts) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     static_assert(DEPTH >= 1 && DEPTH <= 8 && LOADERS >= 1 && LOADERS <= 8, "wait_copies_in_flight counts to seven");
-    constexpr int VEC = 4 * VG;
+    static_assert(!FIFTH || VG == 1, "a fifth vector takes the rows of four");
+    constexpr int VEC = 4 * VG + FIFTH, kSlots = VG + FIFTH;
     Control* control = reinterpret_cast<Control*>(lds + kControlAt);
 
     const uint32_t lane_id = threadIdx.x & 63u;
@@ -461,12 +511,16 @@ __global__ __launch_bounds__(64 * (kConsumers + LOADERS)) void gemv_mma_kernel(
         if ((lane_id & 3u) == 0u) of_unit[(lane_id & 31u) >> 2] = total;
         if ((lane_id & 31u) == 0u) of_unit[8] = unit;
         asm volatile("" ::: "memory");  // LDS serves a wave in order: written above, read below
-        if (((lane_id & 15u) >> 2) == static_cast<uint32_t>(v & 3) && (lane_id & 3u) != 3u) {
-            const uint8_t* plane = scratch + (lane_id & 3u) * kLimbPitch + T::chunk(lane_id >> 4) * 8u;
+        // row 4 * vector + limb; of a fifth vector row 4 * limb + 3
+        const uint32_t upper = (lane_id & 15u) >> 2, lower = lane_id & 3u;
+        const bool is_fifth = FIFTH && v == 4;
+        const uint32_t limb = is_fifth ? upper : lower;
+        if (is_fifth ? lower == 3u && upper < 3u : upper == static_cast<uint32_t>(v & 3) && lower != 3u) {
+            const uint8_t* plane = scratch + limb * kLimbPitch + T::chunk(lane_id >> 4) * 8u;
 #pragma unroll
             for (int s = 0; s < 16; s++) {
                 const uint2 w = *reinterpret_cast<const uint2*>(plane + s * 32);
-                a[v >> 2][s] = pack(w.x, w.y);
+                a[is_fifth ? 0 : v >> 2][s] = pack(w.x, w.y);
             }
         }
     }
@@ -478,28 +532,30 @@ __global__ __launch_bounds__(64 * (kConsumers + LOADERS)) void gemv_mma_kernel(
     for (uint32_t group = 0; group < groups; group++) {
         const uint32_t last_row = min(group * kGroupRows + kGroupRows, wg_rows) - 1u;
         const bool landed = await_copies_in_turn<LOADERS>(control->landed, lane_id, (last_row * pitch + row_bytes + 1023u) >> 10, patience);
-        float total[VG];
+        float total[kSlots];
 #pragma unroll
-        for (int g = 0; g < VG; g++) total[g] = 0.f;
+        for (int g = 0; g < kSlots; g++) total[g] = 0.f;
         if (landed && my_units != 0u) {
             // rows past the end of the range read its last row again and are not stored
             const uint8_t* rp = lds + min(group * kGroupRows + n, wg_rows - 1u) * pitch + first_unit * T::kUnitBytes;
             const float* of_vector = sums + 2u * q * kSumsFloats;
             constexpr uint32_t kStep = 4u * 2u * kSumsFloats;  // to the next vector group
-            T::template contract<VG, 0, 1>(rp, q, a, of_vector, kStep, total);
+            const float* of_fifth = sums + 8u * kSumsFloats;
+            T::template contract<VG, 0, 1, FIFTH>(rp, q, a, of_vector, kStep, of_fifth, total);
             // in one block with the first: the second unit's LDS reads overtake the first's arithmetic
-            if (my_units > 1u) T::template contract<VG, 1, 1>(rp + T::kUnitBytes, q, a, of_vector + kSumsFloats, kStep, total);
+            if (my_units > 1u)
+                T::template contract<VG, 1, 1, FIFTH>(rp + T::kUnitBytes, q, a, of_vector + kSumsFloats, kStep, of_fifth + kSumsFloats, total);
         }
 #pragma unroll
-        for (int g = 0; g < VG; g++) partial[(group * VG + g) * 64u + lane_id] = total[g];
+        for (int g = 0; g < kSlots; g++) partial[(group * kSlots + g) * 64u + lane_id] = total[g];
     }
     // The eight partial sums of every (group, vector group) meet here: each consumer adds those of one
     // pair in wave order (the same bits on every run) and stores sixteen rows of four vectors.
     const uint32_t summed_address = lds_address(&control->summed);
     lds_arrive(summed_address, lane_id == 0);
     if (!lds_await(summed_address, kConsumers, patience)) return;
-    for (uint32_t pair = wave; pair < groups * VG; pair += kConsumers) {
-        const uint32_t group = pair / VG, g = pair - group * VG;
+    for (uint32_t pair = wave; pair < groups * kSlots; pair += kConsumers) {
+        const uint32_t group = pair / kSlots, g = pair - group * kSlots;
         float value = 0.f;
 #pragma unroll
         for (int w = 0; w < kConsumers; w++)
@@ -588,13 +644,15 @@ __global__ __launch_bounds__(64) void gemv_mma_prepare_kernel(const float* __res
     }
 }
 
-template <class T, int VG, int LOADERS, int DEPTH, int AHEAD>
+template <class T, int VG, bool FIFTH, int LOADERS, int DEPTH, int AHEAD>
 __global__ __launch_bounds__(64 * (kConsumers + LOADERS)) void gemv_mma_wide_kernel(
     const uint8_t* __restrict__ weight, const uint8_t* __restrict__ prepared, const float* __restrict__ bias,
     float* __restrict__ y, uint32_t rows, uint32_t columns, uint32_t rows_per_wg, uint32_t vectors, uint32_t spin_limit,
     uint32_t* timeouts) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     static_assert(DEPTH >= 1 && DEPTH <= 8 && LOADERS >= 1 && LOADERS <= 8, "wait_copies_in_flight counts to seven");
+    static_assert(!FIFTH || VG == 1, "a fifth vector takes the rows of four");
+    constexpr int kSlots = VG + FIFTH;
     Control* control = reinterpret_cast<Control*>(lds + kControlAt);
 
     const uint32_t lane_id = threadIdx.x & 63u;
@@ -680,15 +738,18 @@ __global__ __launch_bounds__(64 * (kConsumers + LOADERS)) void gemv_mma_wide_ker
         uint4 raw[VG][4];
         long a[VG][8];
     };
-    const auto load = [&](Operands& operands, uint32_t slice) {  // as A operand: row n = 4 * vector + limb
+    // as A operand: row n = 4 * vector + limb; of a fifth vector 4 * limb + 3
+    const bool in_fifth = FIFTH && (n & 3u) == 3u;
+    const uint32_t limb = in_fifth ? n >> 2 : n & 3u;
+    const auto load = [&](Operands& operands, uint32_t slice) {
 #pragma unroll
         for (int g = 0; g < VG; g++) {
-            const uint32_t vector = 4u * g + (n >> 2);
-            const uint8_t* from = my_units + slice * slice_stride + vector * kWideRecord + ((n & 3u) * 4u + q) * 16u;
+            const uint32_t vector = in_fifth ? 4u : 4u * g + (n >> 2);
+            const uint8_t* from = my_units + slice * slice_stride + vector * kWideRecord + (limb * 4u + q) * 16u;
 #pragma unroll
             for (int p = 0; p < 4; p++) {
                 operands.raw[g][p] = make_uint4(0u, 0u, 0u, 0u);
-                if (vector < vectors && (n & 3u) != 3u) operands.raw[g][p] = *reinterpret_cast<const uint4*>(from + p * 192);
+                if (vector < vectors && limb != 3u) operands.raw[g][p] = *reinterpret_cast<const uint4*>(from + p * 192);
             }
         }
     };
@@ -709,11 +770,11 @@ __global__ __launch_bounds__(64 * (kConsumers + LOADERS)) void gemv_mma_wide_ker
     const uint32_t groups = (wg_rows + kGroupRows - 1u) / kGroupRows;
     const float* of_result = sums + min(q, vectors - 1u) * kSumsFloats;  // result rows past `vectors` are not stored
     const uint32_t sums_step = (min(q + 4u, vectors - 1u) - min(q, vectors - 1u)) * kSumsFloats;
-    float total[kWideGroups][VG];
+    float total[kWideGroups][kSlots];
 #pragma unroll
     for (int i = 0; i < kWideGroups; i++)
 #pragma unroll
-        for (int g = 0; g < VG; g++) total[i][g] = 0.f;
+        for (int g = 0; g < kSlots; g++) total[i][g] = 0.f;
     for (uint32_t first = 0; first < my_slices; first += AHEAD + 1) {
 #pragma unroll
         for (int i = 0; i <= AHEAD; i++) {  // unrolled: operand sets change their roles, not their registers
@@ -731,7 +792,8 @@ __global__ __launch_bounds__(64 * (kConsumers + LOADERS)) void gemv_mma_wide_ker
                     continue;
                 // rows past the end of the range read its last row again and are not stored
                 const uint8_t* rp = lds + slice_at + min(group * kGroupRows + n, wg_rows - 1u) * pitch + wave * T::kUnitBytes;
-                T::template contract<VG, 0, 4>(rp, q, operands[i].a, of_result + slice * vectors * kSumsFloats, sums_step, total[group]);
+                T::template contract<VG, 0, 4, FIFTH>(rp, q, operands[i].a, of_result + slice * vectors * kSumsFloats, sums_step,
+                                                      sums + (slice * vectors + 4u) * kSumsFloats, total[group]);
             }
         }
     }
@@ -740,13 +802,13 @@ __global__ __launch_bounds__(64 * (kConsumers + LOADERS)) void gemv_mma_wide_ker
 #pragma unroll
     for (int group = 0; group < kWideGroups; group++)
 #pragma unroll
-        for (int g = 0; g < VG; g++) partial[(group * VG + g) * 64u + lane_id] = total[group][g];
+        for (int g = 0; g < kSlots; g++) partial[(group * kSlots + g) * 64u + lane_id] = total[group][g];
     // as in gemv_mma_kernel: the eight partial sums of a pair are added in wave order
     const uint32_t summed_address = lds_address(&control->summed);
     lds_arrive(summed_address, lane_id == 0);
     if (!lds_await(summed_address, kConsumers, patience)) return;
-    for (uint32_t pair = wave; pair < groups * VG; pair += kConsumers) {
-        const uint32_t group = pair / VG, g = pair - group * VG;
+    for (uint32_t pair = wave; pair < groups * kSlots; pair += kConsumers) {
+        const uint32_t group = pair / kSlots, g = pair - group * kSlots;
         float value = 0.f;
 #pragma unroll
         for (int w = 0; w < kConsumers; w++)
@@ -795,11 +857,11 @@ hipError_t allow_lds(Kernel kernel, std::atomic<bool> (&allowed)[64]) {
     return hipSuccess;
 }
 
-template <class T, int VG, int LOADERS, int DEPTH>
+template <class T, int VG, bool FIFTH, int LOADERS, int DEPTH>
 hipError_t launch(const uint8_t* weight, const float* x, uint64_t x_row_stride, const float* bias, float* y,
                   uint32_t rows, uint32_t columns, uint32_t vectors, hipStream_t stream) {
     static std::atomic<bool> allowed[64];
-    const auto kernel = gemv_mma_kernel<T, VG, LOADERS, DEPTH>;
+    const auto kernel = gemv_mma_kernel<T, VG, FIFTH, LOADERS, DEPTH>;
     if (hipError_t status = allow_lds(kernel, allowed)) return status;
     HandoverState handover;
     if (hipError_t status = handover_state(&handover)) return status;
@@ -810,11 +872,11 @@ hipError_t launch(const uint8_t* weight, const float* x, uint64_t x_row_stride, 
     return hipGetLastError();
 }
 
-template <class T, int VG, int LOADERS, int DEPTH, int AHEAD>
+template <class T, int VG, bool FIFTH, int LOADERS, int DEPTH, int AHEAD>
 hipError_t launch_wide(const uint8_t* weight, const float* x, uint64_t x_row_stride, const float* bias, float* y,
                        uint32_t rows, uint32_t columns, uint32_t vectors, uint8_t* prepared, hipStream_t stream) {
     static std::atomic<bool> allowed[64];
-    const auto kernel = gemv_mma_wide_kernel<T, VG, LOADERS, DEPTH, AHEAD>;
+    const auto kernel = gemv_mma_wide_kernel<T, VG, FIFTH, LOADERS, DEPTH, AHEAD>;
     if (hipError_t status = allow_lds(kernel, allowed)) return status;
     HandoverState handover;
     if (hipError_t status = handover_state(&handover)) return status;
@@ -830,14 +892,22 @@ hipError_t launch_wide(const uint8_t* weight, const float* x, uint64_t x_row_str
 template <class T>
 hipError_t launch_vectors(const uint8_t* weight, const float* x, uint64_t x_row_stride, const float* bias, float* y,
                           uint32_t rows, uint32_t columns, uint32_t vectors, uint8_t* prepared, hipStream_t stream) {
-    // two vector groups keep 64 registers of A operands: twelve waves leave each 168
+    // Two vector groups keep 64 registers of A operands: twelve waves leave each 168. Five vectors are fifteen limbs and fit one
+    // operand: half the matrix instructions of two groups, a multiply-add per block and eight instructions per unit more than
+    // four vectors (us, two groups / one; inputs from memory): Q4_K 4096 x 14336 18.9 / 17.1, 14336 x 4096 12.6 / 11.9, 4096 x 4096
+    // 7.2 / 6.8; Q5_K 31.7 / 27.4, 17.9 / 17.1, 7.6 / 7.1. The fifth vector's error against 64 bits is what it was. Not Q4_0 and Q8_0: a scale per block would have to meet the limbs'
+    // sums one by one, where an infinite one makes NaN of two signs, or the groups be put together for every block.
     if (columns > kNarrowColumns) {
         if (prepared == nullptr) return hipErrorInvalidValue;
-        if (vectors <= 4) return launch_wide<T, 1, 8, 4, 2>(weight, x, x_row_stride, bias, y, rows, columns, vectors, prepared, stream);
-        return launch_wide<T, 2, 4, 8, 1>(weight, x, x_row_stride, bias, y, rows, columns, vectors, prepared, stream);
+        if (vectors <= 4) return launch_wide<T, 1, false, 8, 4, 2>(weight, x, x_row_stride, bias, y, rows, columns, vectors, prepared, stream);
+        if constexpr (T::kTakesFifth)
+            if (vectors == 5) return launch_wide<T, 1, true, 8, 4, 2>(weight, x, x_row_stride, bias, y, rows, columns, vectors, prepared, stream);
+        return launch_wide<T, 2, false, 4, 8, 1>(weight, x, x_row_stride, bias, y, rows, columns, vectors, prepared, stream);
     }
-    if (vectors <= 4) return launch<T, 1, 8, 4>(weight, x, x_row_stride, bias, y, rows, columns, vectors, stream);
-    return launch<T, 2, 4, 8>(weight, x, x_row_stride, bias, y, rows, columns, vectors, stream);
+    if (vectors <= 4) return launch<T, 1, false, 8, 4>(weight, x, x_row_stride, bias, y, rows, columns, vectors, stream);
+    if constexpr (T::kTakesFifth)
+        if (vectors == 5) return launch<T, 1, true, 8, 4>(weight, x, x_row_stride, bias, y, rows, columns, vectors, stream);
+    return launch<T, 2, false, 4, 8>(weight, x, x_row_stride, bias, y, rows, columns, vectors, stream);
 }
 
 }  // namespace

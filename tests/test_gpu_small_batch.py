@@ -116,6 +116,35 @@ def test_wide_rows_beside_a_large_activation(et, device, codec, vectors):
     assert (np.abs(got - x.astype(np.float64) @ w.T) <= bound).all()
 
 
+@pytest.mark.parametrize("codec", [oracle.Q4_K, oracle.Q5_K])
+@pytest.mark.parametrize("rows,columns", [
+    (2048, 256),    # one unit: seven consumer waves hold no columns
+    (5000, 3840),   # a last group of four rows; the last wave holds one unit
+    (2100, 4096),
+    (2064, 4352),   # wider rows: a last slice of one unit
+    (4096, 14336),  # seven whole slices
+])
+def test_a_fifth_vector_in_the_rows_of_four(et, device, codec, rows, columns):
+    # Its limbs lie in the rows that the four others leave empty: it gets its own value whatever they hold. Fixed point is off
+    # by at most 1.5 units (127 * 2^16 to the largest of 64 columns, 4161000 to that of 256 in rows of up to 4096), the rest
+    # is f32 sums of at most 64 terms per chain, the minima's apart from the quants'.
+    rng = np.random.default_rng(500 + codec + rows + columns)
+    weight = synth.random_weight(codec, rows, columns, rng)
+    x = synth.random_activations(5, columns, rng)
+    x[4] += 0.5  # the minima weigh as much as the quants
+    x[1] = 0.0
+    x[2, ::7] = np.nan
+    got = run_linear(et, device, codec, rows, columns, x, weight)
+    w = oracle.decode_rows(codec, weight, columns).astype(np.float64)
+    size, most = (256, 4161000) if columns <= 4096 else (64, 127 * 65536)
+    unit = np.abs(x[4].astype(np.float64)).reshape(-1, size).max(-1) / most
+    parts = np.abs(w) + 2 * np.abs(w).max(1, keepdims=True)
+    bound = 1.5 * np.abs(w).reshape(rows, -1, size).sum(-1) @ unit + 64 * 2.0 ** -24 * parts @ np.abs(x[4].astype(np.float64))
+    assert (np.abs(got[4] - w @ x[4].astype(np.float64)) <= bound).all()
+    assert not got[1].any() and np.isnan(got[2]).all() and np.isfinite(got[[0, 3, 4]]).all()
+    close(got[[0, 3]], x[[0, 3]].astype(np.float64) @ w.T)
+
+
 def test_wide_rows_without_a_workspace(et, device):
     # aligned activations need no workspace in the vector kernels: the call then runs the launches that quantise themselves
     rows, columns, vectors = 2048, 8192, 5
