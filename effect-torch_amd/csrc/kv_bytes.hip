@@ -2,9 +2,9 @@
 // semantics of kv_attention_into (crates/runtime-cpu/src/napi/mod.rs:3320-3544) as in kv_attention.hip, whose streaming
 // kernel this one stands in for (streaming_bytes there says where).
 //
-// The bytes never become floats. q enters as 31-bit fixed point in four balanced signed-byte limbs per head; a row of K less 128 is signed bytes as it lies in the slab, and v_mfma_i32_16x16x64_i8
-// contracts sixteen positions with the limbs of up to four query heads (rows 4 * limb + head of one operand) in exact
-// integers. A score is the sum of its four integers times q's unit, the softmax scale and the row's K scale. The weights
+// The bytes never become floats. q enters as 31-bit fixed point in four balanced signed-byte limbs per head; a row of K
+// less 128 is signed bytes as it lies in the slab, and v_mfma_i32_16x16x64_i8 contracts sixteen positions with the limbs of
+// up to four query heads (rows 4 * limb + head of one operand) in exact integers. A score is the sum of its four integers times q's unit, the softmax scale and the row's K scale. The weights
 // times the rows' V scales, 64 positions at a time, are fixed point in four limbs as well and contract with V's bytes,
 // which ds_read_b64_tr_b8 transposes out of LDS; the sums of a step are added up in f32.
 //
