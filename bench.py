@@ -570,9 +570,9 @@ def kv_decode(args, et):
         "roofline": {"bound": "hbm", "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(gbs / HBM_PEAK_GBS, 4),
                      "traffic": measured_traffic(("kv_attention_decode", context),
-                                                 et.kv_attention_kernel(states[0], query_heads, 1))
+                                                 et.kv_attention_variant(states[0], query_heads, 1))
                      if args.kv_dtype == "f16" else None,
-                     "kernel": et.kv_attention_kernel(states[0], query_heads, 1),
+                     "kernel": et.kv_attention_variant(states[0], query_heads, 1),
                      "algorithmic_bytes_per_launch": algorithmic, "avg_launch_us": round(ms * 1e3, 3)},
     }
     if not args.no_cpu:

@@ -208,6 +208,7 @@ SIGNATURES = {
                                                           _u64, _vp, _vp, _vp, _u64, _vp, _vp]),
     "et_hip_kv_attention_status_check": (ctypes.c_int, [_KV, _u64, _vp]),
     "et_hip_kv_attention_kernel": (ctypes.c_char_p, [_KV, _u64, _u64]),
+    "et_hip_kv_attention_variant": (ctypes.c_char_p, [_KV, _u64, _u64]),
     "et_hip_kv_commit": (ctypes.c_int, [_KV, _vp]),
     "et_hip_rms_norm_into": (ctypes.c_int, [_T, _T, ctypes.c_double, _T, _vp]),
     "et_hip_rotary_into": (ctypes.c_int, [_T, _vp, _u64, ctypes.c_double, ctypes.c_double, _i32, _T, _vp]),

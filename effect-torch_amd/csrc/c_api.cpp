@@ -446,7 +446,11 @@ uint64_t et_hip_kv_attention_workspace_bytes(const et_kv_layer* layer, uint64_t 
 }
 
 const char* et_hip_kv_attention_kernel(const et_kv_layer* layer, uint64_t query_heads, uint64_t tokens) {
-    return layer ? et::kv::kernel_name(*layer, query_heads, tokens) : "";
+    return layer ? et::kv::kernel_name(*layer, query_heads, tokens, false) : "";
+}
+
+const char* et_hip_kv_attention_variant(const et_kv_layer* layer, uint64_t query_heads, uint64_t tokens) {
+    return layer ? et::kv::kernel_name(*layer, query_heads, tokens, true) : "";
 }
 
 int et_hip_kv_attention_into(const et_kv_layer* layer, const et_tensor* q, const et_tensor* k,

@@ -79,13 +79,14 @@ int workspace_bytes(const et_kv_layer& layer, uint64_t query_heads, uint64_t tok
     return ET_OK;
 }
 
-const char* kernel_name(const et_kv_layer& layer, uint64_t query_heads, uint64_t tokens) {
+const char* kernel_name(const et_kv_layer& layer, uint64_t query_heads, uint64_t tokens, bool variant) {
     KvAttention p{};
     std::string error;
     if (layer_geometry(layer, &p, &error) != ET_OK || query_geometry(query_heads, tokens, &p, &error) != ET_OK)
         return "";
     const KvLaunchShape shape = kv_attention_shape(p);
     if (shape.chunk) return shape.splits > 1 ? "kv_append+kv_chunk+kv_merge" : "kv_append+kv_chunk";
+    if (variant && shape.bytes) return shape.splits > 1 ? "kv_bytes+kv_merge" : "kv_bytes";
     if (shape.streaming) return shape.splits > 1 ? "kv_attend+kv_merge" : "kv_attend";
     return shape.splits > 1 ? "kv_attend_any+kv_merge" : "kv_attend_any";
 }

@@ -28,7 +28,8 @@ int attention_projected_into(const et_kv_layer& layer, const et_kv_projected& pr
                              void* status, void* stream, const volatile int32_t* cancel, std::string* error,
                              const et_linear_plan* consumer, void* prepared, uint64_t prepared_bytes);
 int status_check(const et_kv_layer& layer, uint64_t tokens, const void* status_host, std::string* error);
-const char* kernel_name(const et_kv_layer& layer, uint64_t query_heads, uint64_t tokens);
+// `variant`: the streaming family's kernels told apart.
+const char* kernel_name(const et_kv_layer& layer, uint64_t query_heads, uint64_t tokens, bool variant);
 
 }  // namespace kv
 }  // namespace et

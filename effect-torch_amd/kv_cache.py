@@ -81,6 +81,11 @@ def kv_attention_kernel(layer: KvLayer, query_heads: int, tokens: int) -> str:
     return N.lib().et_hip_kv_attention_kernel(ctypes.byref(layer.struct()), query_heads, tokens).decode()
 
 
+def kv_attention_variant(layer: KvLayer, query_heads: int, tokens: int) -> str:
+    """The kernels that run: ``kv_attention_kernel`` with the two of the ``kv_attend`` family told apart."""
+    return N.lib().et_hip_kv_attention_variant(ctypes.byref(layer.struct()), query_heads, tokens).decode()
+
+
 def kv_commit(layer: "KvLayer", *, stream=None) -> None:
     """``cursor += advance`` for the layer's active slots, on the device (``et_hip_kv_commit``): the commit
     of a decode step (crates/runtime-cpu/src/napi/mod.rs:4511-4517). Layers sharing one cursor tensor are

@@ -446,9 +446,12 @@ int et_hip_kv_attention_status_check(const et_kv_layer* layer, uint64_t tokens,
  * one call. */
 int et_hip_kv_commit(const et_kv_layer* layer, void* stream);
 
-/* Name of the kernel variant these sizes select, for profiles and diagnostics. */
+/* Name of the kernel family these sizes select, for profiles and diagnostics. */
 const char* et_hip_kv_attention_kernel(const et_kv_layer* layer, uint64_t query_heads,
                                        uint64_t tokens);
+/* The kernels that run, the two of the "kv_attend" family told apart: "kv_bytes" where u8 slabs are attended to on the
+ * int8 matrix cores, "kv_attend" where the streaming kernel runs. Other names are those of et_hip_kv_attention_kernel. */
+const char* et_hip_kv_attention_variant(const et_kv_layer* layer, uint64_t query_heads, uint64_t tokens);
 
 /* ---- the small operators of a decode step ---------------------------------
  *

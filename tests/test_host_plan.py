@@ -299,6 +299,23 @@ def test_few_tokens_per_slot_attend_on_the_kernel_that_is_faster(et, query_heads
     assert et.kv_attention_kernel(layer, query_heads, tokens) == kernel
 
 
+@pytest.mark.parametrize("query_heads,dtype,slots,tokens,context,kernel,variant", [
+    (32, "uint8", 32, 1, 2048, "kv_attend", "kv_bytes"),
+    (32, "uint8", 3, 1, 30000, "kv_attend+kv_merge", "kv_bytes+kv_merge"),
+    (32, "uint8", 1, 1, 1000, "kv_attend+kv_merge", "kv_attend+kv_merge"),   # too few rows
+    (8, "uint8", 32, 1, 2048, "kv_attend", "kv_attend"),                     # a query head per kv head
+    (32, "float16", 32, 1, 2048, "kv_attend", "kv_attend"),
+    (32, "uint8", 2, 500, 2000, "kv_append+kv_chunk", "kv_append+kv_chunk"),
+])
+def test_the_kernel_that_runs_is_named(et, query_heads, dtype, slots, tokens, context, kernel, variant):
+    import torch
+    scales = {name: torch.ones(4096, 8) for name in ("k_scales", "v_scales")} if dtype == "uint8" else {}
+    layer = _kv_layer(et, torch, slots=slots, kv_heads=8, width=128, max_tokens=4096, block_size=16,
+                      dtype=getattr(torch, dtype), max_context=context, **scales)
+    assert et.kv_attention_kernel(layer, query_heads, tokens) == kernel
+    assert et.kv_attention_variant(layer, query_heads, tokens) == variant
+
+
 def test_kv_attention_launch_shapes_and_status_wording(et):
     import ctypes
     import struct
