@@ -85,17 +85,19 @@ __device__ __forceinline__ float reduce_scatter(const float (&v)[4]) {
     return __uint_as_float(s[0]) + __uint_as_float(s[1]);
 }
 
-// Fixed point in units of a power of two, `bits` being those of the largest magnitude: below 2^30 units, so that a float
-// loses nothing unless it is smaller than the largest by 2^6 or more, and then what lies under 2^-30 of that. A NaN or
-// infinity makes the unit NaN, and with it every result that the values take part in. Units stay normal numbers.
-__device__ __forceinline__ void fixed_point(uint32_t bits, float& unit, float& inverse) {
-    const uint32_t exponent = min(max(bits >> 23, 40u), 254u);  // the largest is below 2^(exponent - 126)
-    inverse = __uint_as_float((283u - exponent) << 23);         // 2^(156 - exponent)
-    unit = bits < 0x7f800000u ? __uint_as_float((exponent - 29u) << 23) : NAN;
+// Fixed point in units of 2^-up, `bits` being those of the largest magnitude: below 2^30 units, so that a float loses
+// nothing unless it is smaller than the largest by 2^6 or more, and then what lies under 2^-30 of that. `top` is the worth
+// of the top limb, 2^24 units: a normal number down to values of 2^-121, where the unit itself is not, and below that
+// all floats are whole units. A NaN or infinity makes it NaN, and with it every result that the values take part in.
+__device__ __forceinline__ void fixed_point(uint32_t bits, float& top, int& up) {
+    const int exponent = max(static_cast<int>(bits >> 23), 7);  // the largest is below 2^(exponent - 126)
+    up = 156 - exponent;
+    top = bits < 0x7f800000u ? __uint_as_float(static_cast<uint32_t>(exponent - 5) << 23) : NAN;
 }
-// Balanced digits: X + 0x808080 with the top bits of its three low bytes flipped is sum_i 256^i x_i in signed bytes.
-__device__ __forceinline__ uint32_t digits(float value, float inverse) {
-    return static_cast<uint32_t>(static_cast<int>(rintf(value * inverse))) + 0x00808080u;
+// Balanced digits: X + 0x808080 with the top bits of its three low bytes flipped is sum_i 256^i x_i in signed bytes. (2^up is
+// no float where the values are small.)
+__device__ __forceinline__ uint32_t digits(float value, int up) {
+    return static_cast<uint32_t>(static_cast<int>(rintf(__builtin_amdgcn_ldexpf(value, up)))) + 0x00808080u;
 }
 
 // PROJECTED: q, k and v arrive as the K shares of their projections (KvArgs::projected).
@@ -167,7 +169,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void kv_bytes_kernel(const KvArgs a)
                 q_in[h][i] = *reinterpret_cast<const v4f*>(q_rows + min(head, heads - 1) * W + 64 * h + 16 * group + 4 * i);
     };
     if constexpr (!PROJECTED) load_q();  // on their way in front of the first tile
-    const float limb_weight = __uint_as_float((127u + 8u * group) << 23);  // 256^group
+    const float limb_weight = __uint_as_float((103u + 8u * group) << 23);  // of limb `group`, 256^(group - 3) of the top one
 
     const uint32_t row_bytes = a.kv_heads * W;
     const uint8_t* k_base = static_cast<const uint8_t*>(a.k_slab) + kv_head * W;
@@ -228,7 +230,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void kv_bytes_kernel(const KvArgs a)
     if (tile < cached_end) fetch(tile, 0);
 
     v4i q[kHalves];
-    float q_unit;
+    float q_unit;  // the worth of q's top limb
     {
         if constexpr (PROJECTED) load_q();
         uint32_t most = 0;
@@ -238,8 +240,9 @@ __global__ __launch_bounds__(64 * WAVES, 2) void kv_bytes_kernel(const KvArgs a)
             for (int i = 0; i < 16; i++) most = max(most, __float_as_uint(q_in[h][i / 4][i % 4]) & 0x7fffffffu);
         most = max(most, static_cast<uint32_t>(__shfl_xor(static_cast<int>(most), 16)));
         most = max(most, static_cast<uint32_t>(__shfl_xor(static_cast<int>(most), 32)));
-        float unit, inverse;
-        fixed_point(most, unit, inverse);
+        float worth;
+        int up;
+        fixed_point(most, worth, up);
         const bool used = head < heads;
 #pragma unroll
         for (int h = 0; h < kHalves; h++)
@@ -247,10 +250,10 @@ __global__ __launch_bounds__(64 * WAVES, 2) void kv_bytes_kernel(const KvArgs a)
             for (int i = 0; i < 4; i++) {
                 uint32_t word = 0;
 #pragma unroll
-                for (int e = 0; e < 4; e++) word |= ((digits(q_in[h][i][e], inverse) >> (8 * limb)) & 0xffu) << (8 * e);
+                for (int e = 0; e < 4; e++) word |= ((digits(q_in[h][i][e], up) >> (8 * limb)) & 0xffu) << (8 * e);
                 q[h][i] = used ? static_cast<int>(limb < 3 ? word ^ 0x80808080u : word) : 0;
             }
-        q_unit = __shfl(unit, group) * a.scale_log2;  // of head `group`, whose scores this lane will hold
+        q_unit = __shfl(worth, group) * a.scale_log2;  // of head `group`, whose scores this lane will hold
     }
 
     for (; tile < cached_end; tile += WAVES * kTile) {
@@ -301,9 +304,10 @@ __global__ __launch_bounds__(64 * WAVES, 2) void kv_bytes_kernel(const KvArgs a)
             most = max(most, __float_as_uint(w[t]) & 0x7fffffffu);  // NaN and infinities are the largest
         }
         l = fmaf(l, keep, total);
-        float unit, inverse;
-        fixed_point(row_max(most), unit, inverse);
-        const uint32_t x0 = digits(w[0], inverse), x1 = digits(w[1], inverse), x2 = digits(w[2], inverse), x3 = digits(w[3], inverse);
+        float worth;
+        int up;
+        fixed_point(row_max(most), worth, up);
+        const uint32_t x0 = digits(w[0], up), x1 = digits(w[1], up), x2 = digits(w[2], up), x3 = digits(w[3], up);
         // 4x4 byte transpose: limb k of the four weights into one dword
         const uint32_t ab = __builtin_amdgcn_perm(x1, x0, 0x05010400u), cd = __builtin_amdgcn_perm(x3, x2, 0x05010400u);
         const uint32_t ah = __builtin_amdgcn_perm(x1, x0, 0x07030602u), ch = __builtin_amdgcn_perm(x3, x2, 0x07030602u);
@@ -319,7 +323,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void kv_bytes_kernel(const KvArgs a)
 #pragma unroll
         for (int i = 0; i < 4; i++) {  // head i's are those of lane group i
             kept[i] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(keep), 16 * i));
-            units[i] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(unit), 16 * i)) * limb_weight;
+            units[i] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(worth), 16 * i)) * limb_weight;
         }
         if (__builtin_amdgcn_ballot_w64(keep != 1.0f) != 0) {  // some maximum moved
 #pragma unroll

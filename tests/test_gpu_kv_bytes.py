@@ -67,3 +67,26 @@ def test_what_is_not_finite_stays_with_the_heads_that_see_it(et, device):
     finite = np.isfinite(got[0])
     assert np.isfinite(want[0][finite]).all()
     assert np.abs(got[0][finite] - want[0][finite]).max() <= 1e-5
+
+
+@pytest.mark.parametrize("exponent", [-60, -95, -117])
+@pytest.mark.parametrize("width", [64, 128])
+def test_small_scales_and_queries_keep_their_bits(et, device, width, exponent):
+    # A slab may hold rows of any scale, and the limbs of q and of the weights are fixed point. Bar: f32 sums of 300 terms,
+    # 300 * 2^-24 / sqrt(300) = 1e-6 of the result; the streaming kernel shows 2.6e-7.
+    relative = lambda got, want: (np.linalg.norm((got.astype(np.float64) - want) / np.abs(want).max()) /  # noqa: E731
+                                  np.linalg.norm(want / np.abs(want).max()))
+    factor = np.float32(2.0 ** exponent)
+    make = lambda: make_case(np.random.default_rng(width), slots=2, query_heads=8, kv_heads=2, width=width, block_size=16,  # noqa: E731
+                             contexts=[300, 200], tokens=1, advances=[1, 1], dtype="u8")
+    small_values = make()
+    small_values["v_scales"] *= factor
+    small_values["v"] *= factor * np.float32(0)
+    small_queries = make()  # the scores are those of ordinary q and K
+    small_queries["q"] *= factor
+    small_queries["k_scales"] /= factor
+    small_queries["k"] *= 0
+    for case in (small_values, small_queries):
+        got, want = run_gpu(et, device, case, 0.1, max_context=BOUND), run_oracle(case, 0.1)
+        assert et.kv_attention_variant(got[3], 8, 1).startswith("kv_bytes")
+        assert relative(got[0], want[0].astype(np.float64)) <= 1e-6
