@@ -822,29 +822,50 @@ bool streaming_is_faster(const KvAttention& p, const KvLaunchShape& streaming, u
     return chunk > 0.95 * streamed;
 }
 
-// Whether kv_bytes.hip attends in the streaming kernel's place, and its launch: one token per slot over u8 slabs. Measured
-// (us, streaming / bytes kernel with their merge launches; slots at context, 32/8 heads x 128): 32 at 2048 53.4 / 29.8, 64 at
-// 1000 59.0 / 34.5, 12 at 1000 19.6 / 15.6, 4 at 2000 15.7 / 13.9, 3 at 10000 to 30000 61.3 / 37.3, 1 at 60000 52.0 / 34.0;
-// 24/8 heads x 128, 40 at 500 to 1500 67.7 / 32.8; 16/8 heads x 64, 32 at 1000 19.7 / 11.8. It starts more slowly (limbs of q, a
-// longer fill): 1 at 1000 (8 Ki rows of kv heads) 12.0 / 13.4, 4 at 700 (22 Ki) 11.7 / 13.4, 4 at 1000 (32 Ki) 12.6 / 13.9 but 12
-// at 400 (38 Ki) 13.6 / 11.6 and 1 at 6000 16.3 / 14.5; 64 at 64 17.6 / 18.3 but 64 at 200 23.3 / 21.3. One query head per kv head
-// leaves it a quarter of its matrix rows: 32 at 2000 128 / 138. Workgroups of eight waves, one per compute unit, need the
-// fewest partial records (30 at 1000, 16/8 heads x 64: 11.3, four waves 14.0); where a split has many positions, two
-// workgroups of four share a compute unit more evenly (12 at 2000 20.5 / 19.7, 3 at 10000 to 30000 39.7 / 37.3).
+// Whether kv_bytes.hip attends in the streaming kernel's place, and its launch: one token per slot over u8 slabs. Measured over
+// 1100 launches (slots at context, kv heads; us, streaming / bytes kernel with their merge launches, inputs from memory): 32/8
+// heads x 128: 32 at 1000 29.9 / 21.4, 12 at 1536 23.0 / 21.4, 1 at 12288 21.9 / 18.0; 24/8 heads x 128: 32 at 384 25.9 / 13.5;
+// 16/8 heads x 64: 32 at 384 13.8 / 9.6. The bytes kernel starts more slowly (limbs of q, a longer fill) and its time does not
+// depend on the query heads of a kv head; the streaming kernel's does, three heads being three passes of one each. One head
+// leaves the bytes kernel a quarter of its matrix rows (32 at 2000, 32/32 heads: 128 / 138).
+//   Least context, of two / four heads x 128 (one or two steps of the streaming kernel do it): 64 at 192 20.0 / 20.6, 64 at 300
+// 24.4 / 22.6; 64 at 128 19.2 / 21.6, 64 at 160 23.8 / 22.3.
+//   Least rows where the context is split, as a merge launch follows: two heads x 64 8 at 768 (48 Ki) 12.5 / 12.6 but 8 at 1536
+// 15.0 / 13.9; two x 128 8 at 1408 (88 Ki) 14.2 / 16.0 but 4 at 3104 (97 Ki) 16.2 / 16.0; four x 128 4 at 1312 (41 Ki) 14.6 /
+// 15.5 but 4 at 2080 19.1 / 15.8. A long context leaves the streaming kernel so many records that it loses earlier: one slot at
+// 4224, four x 128 16.4 / 16.1; at 7168, two x 128 16.0 / 15.6.
+//   Eight waves, one workgroup per compute unit, need the fewest records (30 at 1000, 16/8 heads x 64: 11.3, four waves 14.0);
+// with many positions in a split two workgroups of four share a compute unit more evenly (3 at 10000 to 30000 39.7 / 37.3), but
+// not with two splits a unit (31 at 1238, 32/8 heads x 64: one piece of eight waves 18.3, two of four 25.0).
+//   All by the declared bound: contexts far below it can lose what the slower start costs (32 at 100 under a bound of 2048:
+// 10.4 / 11.6; 3 at 500 under 30000: 13.6 / 15.2).
+struct BytesLimits {
+    uint32_t context;       // least context
+    uint64_t split_rows;    // least rows of kv heads (slots * kv heads * context) where the context is split
+    uint32_t long_context;  // and shorter than this; kBytesMinRows everywhere
+};
+constexpr BytesLimits kBytesLimits[3][2] = {  // of two, three, four query heads per kv head; widths 64, 128
+    {{128, 64 * 1024, 6144}, {288, 96 * 1024, 6144}},
+    {{128, 0, 0}, {128, 0, 0}},
+    {{128, 48 * 1024, 4096}, {160, 48 * 1024, 4096}}};
 constexpr uint64_t kBytesMinRows = 32 * 1024, kBytesFourWavesRows = 192 * 1024;
-constexpr uint32_t kBytesMinContext = 128;
+constexpr uint64_t kBytesFourWavesUnits = 170;  // at least three splits
 void streaming_bytes(const KvAttention& p, KvLaunchShape& shape) {
     const uint32_t group = p.query_heads / p.kv_heads;
     const uint64_t units = static_cast<uint64_t>(p.active_batch) * p.kv_heads, context = p.max_context;
     if (!shape.streaming || p.slab_dtype != ET_DTYPE_U8 || p.tokens != 1 || group < 2 || group > 4 ||
-        (p.width != 64 && p.width != 128) || context < kBytesMinContext || units * context < kBytesMinRows)
+        (p.width != 64 && p.width != 128))
         return;
+    const BytesLimits& limits = kBytesLimits[group - 2][p.width == 128];
     const uint64_t reach = static_cast<uint64_t>(kKvTableEntries - 2) * p.block_size - 63;  // positions a split's table lists
-    shape.bytes = true;
-    shape.waves = units < 256 && units * context >= kBytesFourWavesRows ? 4 : 8;
-    uint64_t splits = units >= 256 ? 1 : (shape.waves == 4 ? 512 : 256) / units;
-    splits = std::min<uint64_t>(splits, (context + 64 * shape.waves - 1) / (64 * shape.waves));  // a tile for every wave
+    const int waves = units <= kBytesFourWavesUnits && units * context >= kBytesFourWavesRows ? 4 : 8;
+    uint64_t splits = units >= 256 || units == 0 ? 1 : (waves == 4 ? 512 : 256) / units;
+    splits = std::min<uint64_t>(splits, (context + 64 * waves - 1) / (64 * waves));  // a tile for every wave
     splits = std::max<uint64_t>({splits, (context + reach - 1) / reach, 1});
+    const bool many_records = splits > 1 && context < limits.long_context;
+    if (context < limits.context || units * context < std::max(kBytesMinRows, many_records ? limits.split_rows : 0)) return;
+    shape.bytes = true;
+    shape.waves = waves;
     shape.splits = static_cast<uint32_t>(splits);
     shape.workgroups = units * splits;
     shape.workspace_bytes = splits > 1 ? units * group * splits * (p.width + 2) * sizeof(float) : 0;

@@ -15,7 +15,7 @@ BOUND = 40000  # units * bound picks the kernel; 1 slot x 2 kv heads x 40000 pos
 
 def check(et, device, case, scale, heads, **options):
     got = run_gpu(et, device, case, scale, max_context=options.pop("max_context", BOUND), **options)
-    assert et.kv_attention_kernel(got[3], heads, 1) in ("kv_attend", "kv_attend+kv_merge")
+    assert et.kv_attention_variant(got[3], heads, 1).startswith("kv_bytes")
     want = run_oracle(case, scale, **options)
     compare(got, want)
     assert np.abs(got[0] - want[0]).max() <= 1e-5
@@ -41,7 +41,7 @@ def test_blocks_of_any_size_and_windows(et, device, block_size, window, context_
     check(et, device, case, -0.09, 8, window=window, context_window=context_window)
 
 
-@pytest.mark.parametrize("bound", [1100, 140000])  # eight waves, and two workgroups of four to a compute unit
+@pytest.mark.parametrize("bound", [1700, 140000])  # eight waves, and two workgroups of four to a compute unit
 def test_long_contexts_in_splits(et, device, bound):
     rng = np.random.default_rng(bound)
     case = make_case(rng, slots=2, query_heads=64, kv_heads=16, width=64, block_size=16, contexts=[1099, 700], tokens=1,

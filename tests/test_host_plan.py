@@ -316,6 +316,43 @@ def test_the_kernel_that_runs_is_named(et, query_heads, dtype, slots, tokens, co
     assert et.kv_attention_variant(layer, query_heads, tokens) == variant
 
 
+@pytest.mark.parametrize("query_heads,kv_heads,width,slots,context,variant", [
+    # us measured, streaming / bytes kernel, inputs from memory
+    (32, 8, 128, 64, 128, "kv_attend"),               # 19.2 / 21.6
+    (32, 8, 128, 64, 160, "kv_bytes"),                # 23.8 / 22.3
+    (32, 8, 128, 4, 1312, "kv_attend+kv_merge"),      # 14.6 / 15.5
+    (32, 8, 128, 4, 2080, "kv_bytes+kv_merge"),       # 19.1 / 15.8
+    (32, 8, 128, 1, 4224, "kv_bytes+kv_merge"),       # 16.4 / 16.1: a long context
+    (16, 8, 128, 64, 256, "kv_attend"),               # 21.1 / 22.0
+    (16, 8, 128, 64, 300, "kv_bytes"),                # 24.4 / 22.6
+    (16, 8, 128, 8, 1536, "kv_bytes+kv_merge"),       # 96 Ki rows: 15.7 / 16.1, even
+    (16, 8, 128, 8, 1408, "kv_attend+kv_merge"),      # 14.2 / 16.0
+    (16, 8, 64, 64, 128, "kv_bytes"),                 # 16.5 / 9.8
+    (16, 8, 64, 8, 768, "kv_attend+kv_merge"),        # 12.5 / 12.6
+    (16, 8, 64, 10, 422, "kv_bytes"),                 # in one piece: no merge launch
+    (16, 8, 64, 1, 7168, "kv_bytes+kv_merge"),
+    (24, 8, 128, 2, 2112, "kv_bytes+kv_merge"),       # 14.9 / 14.8
+    (24, 8, 64, 64, 128, "kv_bytes"),
+    (24, 8, 64, 64, 127, "kv_attend"),
+    (24, 8, 128, 1, 4000, "kv_attend+kv_merge"),      # fewer than 32 Ki rows
+])
+def test_u8_decode_steps_attend_on_the_kernel_that_is_faster(et, query_heads, kv_heads, width, slots, context, variant):
+    import torch
+    layer = _kv_layer(et, torch, slots=slots, kv_heads=kv_heads, width=width, max_tokens=4096, block_size=16, dtype=torch.uint8,
+                      max_context=context, k_scales=torch.ones(4096, kv_heads), v_scales=torch.ones(4096, kv_heads))
+    assert et.kv_attention_variant(layer, query_heads, 1) == variant
+
+
+@pytest.mark.parametrize("slots,records", [(20, 3), (24, 1), (31, 1)])
+def test_two_workgroups_of_four_waves_only_in_three_pieces_or_more(et, slots, records):
+    # 31 at 1238: one piece of eight waves 18.3 us, two of four 25.0
+    import torch
+    layer = _kv_layer(et, torch, slots=slots, kv_heads=8, width=64, max_tokens=4096, block_size=16, dtype=torch.uint8,
+                      max_context=1400, k_scales=torch.ones(4096, 8), v_scales=torch.ones(4096, 8))
+    assert et.kv_attention_variant(layer, 32, 1) == ("kv_bytes+kv_merge" if records > 1 else "kv_bytes")
+    assert et.kv_attention_workspace_bytes(layer, 32, 1) == (slots * 32 * records * 66 * 4 if records > 1 else 0)
+
+
 def test_kv_attention_launch_shapes_and_status_wording(et):
     import ctypes
     import struct
