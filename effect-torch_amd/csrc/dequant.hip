@@ -115,16 +115,19 @@ __global__ void status_finalize_kernel(const void* indexes, int index_is_i64, In
     status[1] = index_value(indexes, index_is_i64, source_index(layout, status[0]), table_rows, ignored);
 }
 
-// A workgroup decodes one output row, or sixteen values per thread of a wider one, or as many rows as its threads hold: the
-// row's index is read once per thread and everything else is 32-bit arithmetic. A thread takes spans (decode_device.h) of
-// sixteen values in all and decodes them before its first store, so that their loads are in flight together; the stores of a
-// wave are whole 128-byte lines. CHECKER: workgroup (0, 0) checks all the indexes.
+// A workgroup decodes one output row, or sixteen values per thread of a wider one, or (SHORT_ROWS) as many rows as its
+// threads hold. The row's index is read once, and its address held, by the workgroup or by each thread of a short row (per thread
+// for all rows: 20 000 ids of 4096 columns, inputs from memory, Q8_0 101.5 us for 98.2, Q4_K 86.5 for 80.1); everything else is
+// 32-bit arithmetic. A thread takes spans (decode_device.h) of sixteen values in all and decodes them before its first
+// store, so that their loads are in flight together; the stores of a wave are whole 128-byte lines (of Q4_0:
+// halves). CHECKER: workgroup (0, 0) checks all the indexes.
 //
 // Bound: stores (4 bytes out per 0.3 to 1.1 in) now that the loads are few. With a load per header field and dword of
 // quants (24 a thread for Q4_K) the address path of a compute unit alone took half the time. In a graph, before / after (us):
-// 5000 ids of 4096 columns Q4_K 24.5 / 17.4 (5.4 TB/s), Q5_K 25.2 / 17.5, Q3_K 23.9 / 16.6, Q6_K 21.2 / 17.7, Q8_0 21.4 / 18.4;
-// 20 000 Q4_K 126 / 87; rows that left threads idle: 100 000 ids of 256 columns 73 / 25.
-template <int CODEC, bool CHECKER>
+// 5000 ids of 4096 columns Q4_K 24.3 / 17.3 (5.4 TB/s), Q5_K 24.9 / 17.9, Q3_K 23.8 / 17.1, Q2_K 19.7 / 17.2, Q6_K 21.3 / 18.8, Q8_0
+// 21.2 / 18.5; inputs and outputs from memory Q4_K 33.6 / 21.3, Q6_K 29.7 / 23.0, Q8_0 28.2 / 25.8; 20 000 Q4_K
+// 124 / 80; rows that left threads idle: 100 000 ids of 256 columns 73 / 25.
+template <int CODEC, bool CHECKER, bool SHORT_ROWS>
 __global__ __launch_bounds__(256) void dequant_rows_kernel(
     const uint8_t* __restrict__ weight, const void* __restrict__ indexes, int index_is_i64,
     IndexLayout layout, uint64_t out_rows, uint64_t table_rows, uint32_t columns, uint32_t rows_per_wg,
@@ -138,11 +141,12 @@ __global__ __launch_bounds__(256) void dequant_rows_kernel(
         return;
     }
     const uint32_t spans = columns / (4 * S::kGroups);  // of a row
-    const uint32_t sub_row = rows_per_wg == 1 ? 0u : threadIdx.x / spans;
+    const uint32_t my_rows = SHORT_ROWS ? rows_per_wg : 1u;
+    const uint32_t sub_row = SHORT_ROWS ? threadIdx.x / spans : 0u;
     const uint32_t thread = threadIdx.x - sub_row * spans;  // among those of its row
-    if (sub_row >= rows_per_wg) return;
-    const uint64_t stride = static_cast<uint64_t>(gridDim.x - kCheckers) * rows_per_wg;
-    for (uint64_t p = static_cast<uint64_t>(blockIdx.x - kCheckers) * rows_per_wg + sub_row; p < out_rows; p += stride) {
+    if (sub_row >= my_rows) return;
+    const uint64_t stride = static_cast<uint64_t>(gridDim.x - kCheckers) * my_rows;
+    for (uint64_t p = static_cast<uint64_t>(blockIdx.x - kCheckers) * my_rows + sub_row; p < out_rows; p += stride) {
         uint64_t row = p;
         if (indexes != nullptr) {
             bool bad;
@@ -175,22 +179,21 @@ __global__ __launch_bounds__(256) void dequant_rows_kernel(
     }
 }
 
-template <int CODEC>
-hipError_t launch_dequant(const uint8_t* weight, const void* indexes, int index_is_i64,
-                          const IndexLayout& layout, uint64_t out_rows, uint64_t table_rows,
-                          uint64_t columns, float* out, void* status, hipStream_t stream) {
+template <int CODEC, bool SHORT_ROWS>
+hipError_t launch_rows(const uint8_t* weight, const void* indexes, int index_is_i64,
+                       const IndexLayout& layout, uint64_t out_rows, uint64_t table_rows,
+                       uint64_t columns, float* out, void* status, hipStream_t stream) {
     const uint64_t row_bytes = columns / block_values(CODEC) * block_bytes(CODEC);
-    if (out_rows == 0 || columns == 0) return hipSuccess;
     // The loops in the kernel take what the grid limits leave over.
     const uint64_t spans = columns / (4 * Span<CODEC>::kGroups);
-    const uint32_t rows_per_wg = spans >= 256 ? 1u : static_cast<uint32_t>(256 / spans);
+    const uint32_t rows_per_wg = SHORT_ROWS ? static_cast<uint32_t>(256 / spans) : 1u;
     const uint64_t parts = (spans + 256 * kSpansPerThread<CODEC> - 1) / (256 * kSpansPerThread<CODEC>);
     const uint64_t groups = (out_rows + rows_per_wg - 1) / rows_per_wg;
     const uint32_t grid_x = static_cast<uint32_t>(groups < (1u << 24) ? groups : (1u << 24));
     const uint32_t grid_y = static_cast<uint32_t>(parts < 1024 ? parts : 1024);
     auto* status_words = static_cast<unsigned long long*>(status);
     if (indexes != nullptr && lookup_checks_itself(layout, out_rows)) {
-        hipLaunchKernelGGL((dequant_rows_kernel<CODEC, true>), dim3(grid_x + 1, grid_y), dim3(256), 0,
+        hipLaunchKernelGGL((dequant_rows_kernel<CODEC, true, SHORT_ROWS>), dim3(grid_x + 1, grid_y), dim3(256), 0,
                            stream, weight, indexes, index_is_i64, layout, out_rows, table_rows,
                            static_cast<uint32_t>(columns), rows_per_wg, row_bytes, out, status_words);
         return hipGetLastError();
@@ -198,7 +201,7 @@ hipError_t launch_dequant(const uint8_t* weight, const void* indexes, int index_
     if (indexes != nullptr) {
         hipLaunchKernelGGL(status_init_kernel, dim3(1), dim3(64), 0, stream, status_words);
     }
-    hipLaunchKernelGGL((dequant_rows_kernel<CODEC, false>), dim3(grid_x, grid_y), dim3(256), 0,
+    hipLaunchKernelGGL((dequant_rows_kernel<CODEC, false, SHORT_ROWS>), dim3(grid_x, grid_y), dim3(256), 0,
                        stream, weight, indexes, index_is_i64, layout, out_rows, table_rows,
                        static_cast<uint32_t>(columns), rows_per_wg, row_bytes, out, status_words);
     if (indexes != nullptr) {
@@ -206,6 +209,16 @@ hipError_t launch_dequant(const uint8_t* weight, const void* indexes, int index_
                            index_is_i64, layout, table_rows, status_words);
     }
     return hipGetLastError();
+}
+
+template <int CODEC>
+hipError_t launch_dequant(const uint8_t* weight, const void* indexes, int index_is_i64,
+                          const IndexLayout& layout, uint64_t out_rows, uint64_t table_rows,
+                          uint64_t columns, float* out, void* status, hipStream_t stream) {
+    if (out_rows == 0 || columns == 0) return hipSuccess;
+    const bool short_rows = columns / (4 * Span<CODEC>::kGroups) <= 128;  // a workgroup holds two or more
+    return (short_rows ? launch_rows<CODEC, true> : launch_rows<CODEC, false>)(
+        weight, indexes, index_is_i64, layout, out_rows, table_rows, columns, out, status, stream);
 }
 
 }  // namespace

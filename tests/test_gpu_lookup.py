@@ -10,7 +10,9 @@ from effect_torch_amd import synth
 
 pytestmark = pytest.mark.gpu
 
-WIDTHS = {"Q4_0": [32, 96, 2080], "Q8_0": [32, 160, 4128], **{c: [256, 768, 4352] for c in ("Q2_K", "Q3_K", "Q4_K", "Q5_K", "Q6_K")}}
+# 1024 of Q4_0, 512 of Q8_0, 1024 and 2048 of the others are the widest rows that share a workgroup
+WIDTHS = {"Q4_0": [32, 96, 1024, 1056, 2080, 2112], "Q8_0": [32, 160, 512, 544, 4128],
+          **{c: [256, 768, 1024, 2048, 2304, 4352] for c in ("Q2_K", "Q3_K", "Q4_K", "Q5_K", "Q6_K")}}
 
 
 @pytest.mark.parametrize("codec,columns", [(codec, columns) for codec, widths in WIDTHS.items() for columns in widths])
