@@ -115,17 +115,36 @@ __global__ void status_finalize_kernel(const void* indexes, int index_is_i64, In
     status[1] = index_value(indexes, index_is_i64, source_index(layout, status[0]), table_rows, ignored);
 }
 
+// Q4_0: the two runs of a lane lie in the two halves of a block's 128-byte line. The lanes of two blocks swap runs, lane i
+// with lane i ^ 4, so that a store of eight lanes fills a line, in order. In a graph, inputs from memory, half / whole lines (us):
+// 5000 ids of 4096 columns 22.3 / 21.0, 20 000 94.4 / 82.4, 9000 of 11008 columns 119.5 / 103.1.
+__device__ __forceinline__ void store_two_blocks(float* blocks, uint32_t lane, const float (&values)[2][4]) {
+    const bool second = lane >= 4;
+    float first_block[4], second_block[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int given = __float_as_int(second ? values[0][i] : values[1][i]);
+        int got = __builtin_amdgcn_update_dpp(given, given, 0x104, 0xF, 0x5, false);  // row_shl:4 in lanes 0..3 of eight,
+        got = __builtin_amdgcn_update_dpp(got, given, 0x114, 0xF, 0xA, false);        // row_shr:4 in the others
+        first_block[i] = second ? __int_as_float(got) : values[0][i];
+        second_block[i] = second ? values[1][i] : __int_as_float(got);
+    }
+    float* to = blocks + 4u * lane;
+    *reinterpret_cast<float4*>(to) = make_float4(first_block[0], first_block[1], first_block[2], first_block[3]);
+    *reinterpret_cast<float4*>(to + 32) = make_float4(second_block[0], second_block[1], second_block[2], second_block[3]);
+}
+
 // A workgroup decodes one output row, or sixteen values per thread of a wider one, or (SHORT_ROWS) as many rows as its
 // threads hold. The row's index is read once, and its address held, by the workgroup or by each thread of a short row (per thread
 // for all rows: 20 000 ids of 4096 columns, inputs from memory, Q8_0 101.5 us for 98.2, Q4_K 86.5 for 80.1); everything else is
 // 32-bit arithmetic. A thread takes spans (decode_device.h) of sixteen values in all and decodes them before its first
-// store, so that their loads are in flight together; the stores of a wave are whole 128-byte lines (of Q4_0:
+// store, so that their loads are in flight together; the stores of a wave are whole 128-byte lines (of short Q4_0 rows:
 // halves). CHECKER: workgroup (0, 0) checks all the indexes.
 //
 // Bound: stores (4 bytes out per 0.3 to 1.1 in) now that the loads are few. With a load per header field and dword of
 // quants (24 a thread for Q4_K) the address path of a compute unit alone took half the time. In a graph, before / after (us):
 // 5000 ids of 4096 columns Q4_K 24.3 / 17.3 (5.4 TB/s), Q5_K 24.9 / 17.9, Q3_K 23.8 / 17.1, Q2_K 19.7 / 17.2, Q6_K 21.3 / 18.8, Q8_0
-// 21.2 / 18.5; inputs and outputs from memory Q4_K 33.6 / 21.3, Q6_K 29.7 / 23.0, Q8_0 28.2 / 25.8; 20 000 Q4_K
+// 21.2 / 18.5, Q4_0 20.3 / 17.4; inputs and outputs from memory Q4_K 33.6 / 21.3, Q6_K 29.7 / 23.0, Q8_0 28.2 / 25.8; 20 000 Q4_K
 // 124 / 80; rows that left threads idle: 100 000 ids of 256 columns 73 / 25.
 template <int CODEC, bool CHECKER, bool SHORT_ROWS>
 __global__ __launch_bounds__(256) void dequant_rows_kernel(
@@ -170,6 +189,12 @@ __global__ __launch_bounds__(256) void dequant_rows_kernel(
                 const uint32_t span = at + 256u * u + thread;
                 if (span >= spans) continue;
                 float* to = out_row + span / S::kLanes * block_values(CODEC) + S::first(span % S::kLanes);
+                if constexpr (CODEC == kQ4_0 && !SHORT_ROWS) {
+                    if ((span | 7u) < spans) {  // both blocks of these eight lanes are there
+                        store_two_blocks(out_row + (span >> 3) * 64u, span & 7u, values[u]);
+                        continue;
+                    }
+                }
 #pragma unroll
                 for (int g = 0; g < S::kGroups; g++)
                     *reinterpret_cast<float4*>(to + g * S::kStride) =
