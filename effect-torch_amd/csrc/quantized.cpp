@@ -726,7 +726,10 @@ int linear_enqueue_step(const et_linear_plan* const* plans, uint32_t count, cons
     step.row_bytes = plans[0]->encoded_row_bytes;
     step.silu_mul = silu_mul;
     step.count = count;
-    const uintptr_t x_begin = reinterpret_cast<uintptr_t>(input.x), x_end = x_begin + 4 * step.columns;
+    const auto overlap = [](const void* a, uint64_t a_bytes, const void* b, uint64_t b_bytes) {
+        const uintptr_t first = reinterpret_cast<uintptr_t>(a), second = reinterpret_cast<uintptr_t>(b);
+        return a != nullptr && b != nullptr && first < second + b_bytes && second < first + a_bytes;
+    };
     for (uint32_t i = 0; i < count; i++) {
         step.rows[i] = plans[i]->rows;
         step.weight[i] = weights[i];
@@ -734,10 +737,21 @@ int linear_enqueue_step(const et_linear_plan* const* plans, uint32_t count, cons
         step.y[i] = ys[i];
         if (weights[i] == nullptr || (ys[i] == nullptr && !(silu_mul && i == 1)))
             return fail(error, ET_ERR_INVALID, "quantized_linear: NULL device pointer");
-        // every workgroup reads all of x while others already write
-        const uintptr_t y_begin = reinterpret_cast<uintptr_t>(ys[i]);
-        if (ys[i] != nullptr && y_begin < x_end && x_begin < y_begin + 4 * plans[i]->rows)
+    }
+    // The rows of all members run side by side: what one workgroup writes another must neither read nor write. A row's own
+    // residual is read by the thread that then writes it.
+    const uint64_t norm_bytes = step.norm_weight_is_half ? 2 * step.columns : 4 * step.columns;
+    for (uint32_t i = 0; i < (silu_mul ? 1 : count); i++) {
+        const uint64_t bytes = 4 * step.rows[i];
+        if (overlap(step.y[i], bytes, step.x, 4 * step.columns) || overlap(step.y[i], bytes, step.norm_weight, norm_bytes))
             return fail(error, ET_ERR_INVALID, "quantized_linear: a result overlaps the activations of its launch");
+        for (uint32_t j = 0; j < count; j++) {
+            const float* residual = step.residual[j];
+            if (overlap(step.y[i], bytes, step.weight[j], step.rows[j] * step.row_bytes) ||
+                (!silu_mul && j != i && overlap(step.y[i], bytes, step.y[j], 4 * step.rows[j])) ||
+                (!(j == i && residual == step.y[i]) && overlap(step.y[i], bytes, residual, 4 * step.rows[j])))
+                return fail(error, ET_ERR_INVALID, "quantized_linear: a result overlaps another operand of its launch");
+        }
     }
     if (cancelled(cancel)) return fail(error, ET_ERR_CANCELLED, "operation aborted");
     if (hipError_t status = gemv_step(plans[0]->codec, step, as_stream(stream)))

@@ -516,3 +516,29 @@ def test_host_calls_leave_other_arguments_to_the_ctypes_path(et):
     flag.cancel()
     with pytest.raises(et.Cancelled, match="operation aborted"):
         et.linear_into(x, w, None, et.GgmlQuant.Q4_K, y, plan, flag, stream=0)
+
+
+@pytest.mark.parametrize("what", ["x", "norm weight", "weight", "result", "residual of another", "own residual, shifted"])
+def test_a_step_refuses_results_that_its_other_rows_read_or_write(et, what):
+    # the rows of all members run side by side; host tensors: the refusal comes in front of any launch
+    import torch
+    step = et.LinearStep([et.RawLinear(et.GgmlQuant.Q4_K, rows, 1024, 1) for rows in (512, 256)])
+    buffer = torch.zeros(8192)
+    x, norm, ys = buffer[:1024].view(1, 1024), buffer[1024:2048], [buffer[2048:2560], buffer[2560:2816]]
+    weights = [torch.zeros(512, 576, dtype=torch.uint8), torch.zeros(256, 576, dtype=torch.uint8)]
+    residuals = [ys[0], None]
+    if what == "x":
+        ys[1] = buffer[1000:1256]
+    elif what == "norm weight":
+        ys[1] = buffer[1792:2048]
+    elif what == "weight":
+        floats = torch.zeros(512 * 144)
+        weights[0], ys[1] = floats.view(torch.uint8).view(512, 576), floats[-256:]
+    elif what == "result":
+        ys[1] = buffer[2559:2815]
+    elif what == "residual of another":
+        residuals[1] = buffer[2304:2560]
+    else:
+        residuals[0] = buffer[2049:2561]
+    with pytest.raises(et.QuantizedError, match="a result overlaps (the activations|another operand) of its launch"):
+        step.enqueue(x, weights, ys, norm=(norm, 1e-5), residuals=residuals, stream=0)
