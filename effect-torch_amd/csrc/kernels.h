@@ -49,7 +49,7 @@ hipError_t gemv_limb(int32_t codec, const uint8_t* weight, const float* x, uint6
 
 // ---- gemv_step.hip: one vector against up to four matrices of one codec and width in one launch ----
 // y_i = W_i f(x) (+ residual_i, which may be y_i), f(x) = x, or rms_norm(x) * norm_weight (null: ones; floats or halves)
-// when `normed`; silu_mul (two matrices of the same rows): y_0 = silu(W_0 f(x)) * (W_1 f(x)), residuals and y_1 unused.
+// when `normed`; silu_mul (two matrices of the same rows): y_0 = silu(W_0 f(x)) * (W_1 f(x)), y_1 unused, no residuals.
 // x is 16-byte aligned.
 constexpr uint32_t kGemvStepMost = 4;
 struct GemvStep {

@@ -733,7 +733,9 @@ int linear_enqueue_step(const et_linear_plan* const* plans, uint32_t count, cons
     for (uint32_t i = 0; i < count; i++) {
         step.rows[i] = plans[i]->rows;
         step.weight[i] = weights[i];
-        step.residual[i] = residuals != nullptr && !silu_mul ? residuals[i] : nullptr;
+        step.residual[i] = residuals != nullptr ? residuals[i] : nullptr;
+        if (silu_mul && step.residual[i] != nullptr)
+            return fail(error, ET_ERR_INVALID, "quantized_linear: silu(gate) * up takes no residuals");
         step.y[i] = ys[i];
         if (weights[i] == nullptr || (ys[i] == nullptr && !(silu_mul && i == 1)))
             return fail(error, ET_ERR_INVALID, "quantized_linear: NULL device pointer");

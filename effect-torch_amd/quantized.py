@@ -574,11 +574,12 @@ class LinearStep:
                 norm: Optional[tuple] = None, residuals: Optional[Sequence[Optional[torch.Tensor]]] = None, stream=None,
                 cancelled: Optional[CancellationFlag] = None) -> None:
         """``ys[i] = W_i f(x) (+ residuals[i])``, ``f(x) = rms_norm(x) * weight`` for ``norm = (weight, eps)``; ``silu_mul``:
-        ``ys[0] = silu(W_0 f(x)) * (W_1 f(x))``."""
+        ``ys[0] = silu(W_0 f(x)) * (W_1 f(x))``, without residuals."""
         count = len(self.plans)
-        if len(weights) != count or len(ys) != (1 if self.silu_mul else count):
-            raise QuantizedError(N.ERR_INVALID, f"quantized_linear: a launch of {count} plans got {len(weights)} weights and "
-                                                f"{len(ys)} results")
+        if (len(weights) != count or len(ys) != (1 if self.silu_mul else count) or
+                (residuals is not None and len(residuals) != len(ys))):
+            raise QuantizedError(N.ERR_INVALID, f"quantized_linear: a launch of {count} plans got {len(weights)} weights, "
+                                                f"{len(ys)} results and {len(residuals or ())} residuals")
         for index, plan in enumerate(self.plans):
             plan._check_input(x)
             plan._check_weight(weights[index])

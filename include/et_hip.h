@@ -285,7 +285,7 @@ int et_hip_linear_enqueue_prepared_then_norm(const et_linear_plan* plan, const v
 /* Up to ET_HIP_LINEAR_GROUP_MOST contractions of ONE vector in one launch together with the operators around them, for a
  * decode step of a single sequence: y_i = W_i f(x) (+ residual_i, which may be y_i), f(x) = x or, `normed`,
  * rms_norm(x) * norm_weight (rms_norm_forward_into_impl; [columns] f32 or f16, or NULL); with `silu_mul`, two plans of
- * the same rows: y_0 = silu(W_0 f(x)) * (W_1 f(x)), residuals and ys[1] unused. Plans of one vector, one codec and one
+ * the same rows: y_0 = silu(W_0 f(x)) * (W_1 f(x)), ys[1] unused, no residuals (ET_ERR_INVALID). Plans of one vector, one codec and one
  * width, without bias, whose kernel is the dequant-GEMV of one vector (et_hip_linear_step_supported says 1). x: 16-byte
  * aligned floats. No y_i overlaps x, the norm weight, a weight, another y_j or a residual, but for residual_i = y_i: refused
  * (ET_ERR_INVALID). residuals may be NULL, as may each of them. No counterpart in the reference, whose

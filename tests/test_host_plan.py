@@ -542,3 +542,14 @@ def test_a_step_refuses_results_that_its_other_rows_read_or_write(et, what):
         residuals[0] = buffer[2049:2561]
     with pytest.raises(et.QuantizedError, match="a result overlaps (the activations|another operand) of its launch"):
         step.enqueue(x, weights, ys, norm=(norm, 1e-5), residuals=residuals, stream=0)
+
+
+def test_a_step_drops_no_residual(et):
+    import torch
+    plan = et.RawLinear(et.GgmlQuant.Q4_K, 512, 1024, 1)
+    x, y, residual = torch.zeros(1, 1024), torch.zeros(1, 512), torch.zeros(1, 512)
+    weight = torch.zeros(512, 576, dtype=torch.uint8)
+    with pytest.raises(et.QuantizedError, match="takes no residuals"):
+        et.LinearStep([plan, plan], silu_mul=True).enqueue(x, [weight, weight], [y], residuals=[residual], stream=0)
+    with pytest.raises(et.QuantizedError, match="2 weights, 2 results and 1 residuals"):
+        et.LinearStep([plan, plan]).enqueue(x, [weight, weight], [y, residual], residuals=[None], stream=0)
