@@ -849,7 +849,7 @@ def llama_decode(args, et, emit=True):
         kv.append(et.KvLayer(k_slab, v_slab, block, table, cursors, advances, max_context, k_scales=k_scales,
                              v_scales=v_scales))
     decoder = et.LlamaDecoder(shape, et.GgmlQuant.Q4_K, slots, weights, base["head"], norms, final_norm, embedding, kv,
-                              tokens, mode=mode, fused=not args.unfused)
+                              tokens, mode=mode, fused=not args.unfused, chain=not args.unfused)
     start_cursors, start_tokens = cursors.clone(), tokens.clone()
 
     def restart():

@@ -63,13 +63,15 @@ class LlamaDecoder:
     norms / SiLU * up / rotary computed inside the launches next to them where the plans can
     (``on_the_fly``); otherwise one launch sequence per operator, as the reference's executor runs
     them, except that a single sequence whose plans can (``chained``) has norms, residual sums and
-    SiLU * up computed inside the contractions' launches. The results agree within the f32 bars either way.
+    SiLU * up computed inside the contractions' launches, unless ``chain`` is false. The results agree within the
+    f32 bars either way; what an operator of its own would leave in ``h``, ``q``, ``k``, ``up``, ``projected`` and ``down``
+    is there only where it has one.
     """
 
     def __init__(self, shape: LlamaShape, codec: GgmlQuant, slots: int, weights: Sequence[Dict[str, torch.Tensor]],
                  head: torch.Tensor, norms: Sequence[torch.Tensor], final_norm: torch.Tensor,
                  embedding: torch.Tensor, kv: Sequence[KvLayer], tokens: torch.Tensor, *,
-                 mode: ActivationMode = ActivationMode.F32, fused: bool = True):
+                 mode: ActivationMode = ActivationMode.F32, fused: bool = True, chain: bool = True):
         self.shape, self.slots, self.weights, self.head = shape, slots, weights, head
         self.norms, self.final_norm, self.embedding, self.kv, self.tokens = norms, final_norm, embedding, kv, tokens
         self.layers = len(weights)
@@ -95,7 +97,7 @@ class LlamaDecoder:
         self.chain = {"qkv": LinearStep([plans["wq"], plans["wk"], plans["wv"]]), "wo": LinearStep([plans["wo"]]),
                       "ffn": LinearStep([plans["gate"], plans["up"]], silu_mul=True), "down": LinearStep([plans["down"]]),
                       "head": LinearStep([plans["head"]])}
-        self.chained = not fused and all(step.supported for step in self.chain.values())
+        self.chained = chain and not fused and all(step.supported for step in self.chain.values())
         self.kv_ws = kv_attention_workspace(kv[0], shape.heads, 1)
         # q / k / v can stay the K shares of their group launch when the attention kernel is the one that sums them
         streaming = lambda layer: kv_attention_kernel(layer, shape.heads, 1).split("+")[0] == "kv_attend"  # noqa: E731

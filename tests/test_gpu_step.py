@@ -90,3 +90,91 @@ def test_what_has_no_such_launch_is_refused(et, device):
 @pytest.mark.parametrize("contexts", [(40, 41), (2030, 2060)], ids=["one_attention_launch_or_more", "context_2048"])
 def test_decode_steps_of_one_sequence_follow_the_oracle_chain(et, device, contexts):
     _follow_the_oracle_chain(et, device, False, 1, contexts)
+
+
+def small_decoder(et, device, codec, slab, head_dim, bound, chain):
+    """Two layers, one sequence, eight query heads over two kv heads; every call makes the same one."""
+    rng = np.random.default_rng(0x5DEC + head_dim)
+    code = getattr(synth, codec)
+    shape = et.LlamaShape(hidden=8 * head_dim, heads=8, kv_heads=2, head_dim=head_dim, ffn=1280, vocab=1000, layers=2)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(device)  # noqa: E731
+    shapes = shape.linear_shapes()
+    weights = [{name: dev(synth.random_weight(code, *size, rng)) for name, size in shapes.items() if name != "head"} for _ in range(2)]
+    head = dev(synth.random_weight(code, *shapes["head"], rng))
+    norm = lambda *size: dev((1 + 0.1 * rng.standard_normal((*size, shape.hidden))).astype(np.float32))  # noqa: E731
+    norms, final_norm = [norm(2) for _ in range(2)], norm()
+    embedding = dev(rng.standard_normal((shape.vocab, shape.hidden)).astype(np.float16))
+    cursors, advances = (torch.full((1,), n, dtype=torch.int32, device=device) for n in (77, 1))
+    table = dev(rng.permutation(8).reshape(1, 8).astype(np.int32))
+
+    def layer():
+        size = (128, 2, head_dim)
+        if slab == torch.uint8:
+            values = [dev(rng.integers(1, 256, size).astype(np.uint8)) for _ in range(2)]
+            scales = {name: dev(rng.uniform(0.01, 0.03, size[:2]).astype(np.float32)) for name in ("k_scales", "v_scales")}
+        else:
+            values, scales = [dev(rng.standard_normal(size).astype(np.float32)).to(slab) for _ in range(2)], {}
+        return et.KvLayer(*values, 16, table, cursors, advances, bound, **scales)
+
+    tokens = torch.full((1,), 5, dtype=torch.int32, device=device)
+    return et.LlamaDecoder(shape, et.GgmlQuant[codec], 1, weights, head, norms, final_norm, embedding, [layer(), layer()], tokens,
+                           fused=False, chain=chain)
+
+
+@pytest.mark.parametrize("codec,slab,head_dim,bound,attention,bar", [
+    ("Q4_K", torch.float32, 64, 100, "kv_attend", 2e-6),
+    ("Q6_K", torch.float16, 128, 5000, "kv_attend+kv_merge", 2e-3),
+    ("Q8_0", torch.bfloat16, 64, 100, "kv_attend", 1e-2),
+    ("Q5_K", torch.uint8, 128, 40000, "kv_bytes+kv_merge", 1e-2),
+    ("Q4_0", torch.uint8, 64, 40000, "kv_bytes+kv_merge", 1e-2),
+    ("Q3_K", torch.float32, 96, 100, "kv_attend_any", 2e-6),          # q and k are rotated by a launch of their own
+])
+def test_a_chained_step_is_that_of_its_operators_one_by_one(et, device, codec, slab, head_dim, bound, attention, bar):
+    # Bar: f32 sums; where a row of the step rounds to the slab's next value the two part by that step (2^-11, 2^-9, 1/254 of the
+    # row's largest) in one of 78 positions.
+    one = small_decoder(et, device, codec, slab, head_dim, bound, chain=False)
+    chained = small_decoder(et, device, codec, slab, head_dim, bound, chain=True)
+    assert chained.chained and not one.chained
+    assert et.kv_attention_variant(chained.kv[0], 8, 1).startswith(attention)
+    assert chained.project_in_attention == (not attention.startswith("kv_attend_any"))
+    relative = lambda got, want: ((got - want).norm() / want.norm()).item()  # noqa: E731
+    for decoder in (one, chained):
+        for name in ("h", "q", "k", "v", "up", "projected", "down"):
+            getattr(decoder, name).fill_(float("nan"))
+        decoder.step()
+    torch.cuda.synchronize()
+    for decoder in (one, chained):
+        et.gather_rows_status_check(1000, decoder.status[0])
+        for index in range(2):
+            et.kv_attention_status_check(decoder.kv[index], 1, decoder.status[1 + index])
+    assert relative(chained.logits, one.logits) <= bar
+    assert torch.isfinite(one.logits).all() and one.cursors.item() == chained.cursors.item() == 78
+    # one operator per launch: each has left its result behind
+    assert all(torch.isfinite(getattr(one, name)).all() for name in ("h", "q", "k", "v", "up", "projected", "down"))
+    for name, source, result in (("wo", one.attended, one.projected), ("down", one.gate, one.down)):
+        want = torch.empty_like(result)
+        one.plans[name].enqueue(source, one.weights[1][name], None, want, one.linear_ws)
+        assert torch.equal(result, want)
+
+
+def test_a_chained_step_as_a_replayed_graph(et, device):
+    eager, graphed = (small_decoder(et, device, "Q4_K", torch.uint8, 128, 40000, chain=True) for _ in range(2))
+    start = [t.clone() for layer in graphed.kv for t in (layer.k_slab, layer.v_slab, layer.k_scales, layer.v_scales)]
+    graphed.step()  # warm up, then back to the start
+    for tensor, value in zip([t for layer in graphed.kv for t in (layer.k_slab, layer.v_slab, layer.k_scales, layer.v_scales)], start):
+        tensor.copy_(value)
+    graphed.tokens.fill_(5)
+    graphed.cursors.fill_(77)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        graphed.step()
+    for _ in range(4):
+        eager.step()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        for a, b in ((eager.logits, graphed.logits), (eager.tokens, graphed.tokens), (eager.cursors, graphed.cursors)):
+            assert torch.equal(a, b)
+    for a, b in zip(eager.kv, graphed.kv):
+        assert torch.equal(a.k_slab, b.k_slab) and torch.equal(a.v_slab, b.v_slab) and torch.equal(a.k_scales, b.k_scales)
