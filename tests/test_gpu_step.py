@@ -2,13 +2,15 @@
 one after the other, and the decode step of a single sequence that is made of them.
 
 Sizes: one, two and four slices of columns (4096 each, the last one ragged), one to eight rows per wave and the loop above
-that, matrices whose rows end inside a wave's rows or a workgroup's range. Bars: ``close`` of test_gpu_parity (f32 bars)."""
+that, matrices whose rows end inside a wave's rows or a workgroup's range. Bars: ``close`` of test_gpu_parity (f32 bars); the
+sums alone: the bits of the launch per matrix. Chained steps against the same step with one operator per launch."""
 import numpy as np
 import pytest
 import torch
 
 import oracle
 from effect_torch_amd import synth
+import test_gpu_decode_step
 from test_gpu_decode_step import test_decode_steps_follow_the_oracle_chain as _follow_the_oracle_chain
 from test_gpu_parity import close
 
@@ -71,6 +73,49 @@ def test_gate_and_up_with_silu(et, device, codec, rows, columns):
     close(y.cpu().numpy(), oracle.silu_mul(linear(code, gate, rows, columns, h), linear(code, up, rows, columns, h)))
 
 
+@pytest.mark.parametrize("codec", CODECS)
+@pytest.mark.parametrize("rows,columns", [((1000, 77), 1792), ((14336,), 4096), ((2500, 40), 4352), ((4099,), 14336)])
+def test_the_sums_are_those_of_a_launch_per_matrix(et, device, codec, rows, columns):
+    # the same limbs, folds and order: the same bits, also where an activation is not finite
+    code, weights, x, norm, _ = case(codec, rows, columns, 0xB175 + columns)
+    plans = [et.RawLinear(et.GgmlQuant[codec], r, columns, 1) for r in rows]
+    step, wd = et.LinearStep(plans), tensors(device, *weights)
+    for spoilt in (None, np.nan, np.inf, -np.inf):
+        if spoilt is not None:
+            x[0, columns - 3] = spoilt
+        xd, = tensors(device, x)
+        ys, want = ([torch.full((1, r), 7.0, device=device) for r in rows] for _ in range(2))
+        step.enqueue(xd, wd, ys)
+        for plan, weight, y in zip(plans, wd, want):
+            plan.enqueue(xd, weight, None, y, torch.empty(max(plan.requirements.workspace_bytes, 16), dtype=torch.uint8, device=device))
+        for y, w in zip(ys, want):
+            assert torch.equal(y.isnan(), w.isnan()) and torch.equal(y.nan_to_num(), w.nan_to_num())
+
+
+@pytest.mark.parametrize("columns", [256, 1792, 4096, 4352, 14336])
+@pytest.mark.parametrize("weight", ["f32", "none"])
+def test_norms_with_float_weights_or_none(et, device, columns, weight):
+    rows = 300
+    code, (packed,), x, norm, (residual,) = case("Q4_K", (rows,), columns, 0xF32 + columns)
+    step = et.LinearStep([et.RawLinear(et.GgmlQuant.Q4_K, rows, columns, 1)])
+    norm = (norm.astype(np.float32) + np.float32(1e-5)) if weight == "f32" else None  # no half floats
+    for spoilt in (False, True):
+        if spoilt:
+            x[:] = np.inf
+        xd, wd, rd = tensors(device, x, packed, residual)
+        nd = None
+        if norm is not None:
+            nd, = tensors(device, np.concatenate([norm[:1], norm]))
+            nd = nd[1:]  # 4-byte aligned only
+        y = torch.empty(1, rows, device=device)
+        step.enqueue(xd, [wd], [y], norm=(nd, 1e-5), residuals=[rd])
+        got = y.cpu().numpy()
+        if spoilt:
+            assert np.isnan(got).all()
+        else:
+            close(got, linear(code, packed, rows, columns, oracle.rms_norm(x, norm, 1e-5)) + residual)
+
+
 def test_what_has_no_such_launch_is_refused(et, device):
     plan = lambda *a, **k: et.RawLinear(et.GgmlQuant.Q4_K, *a, **k)  # noqa: E731
     one = plan(512, 1024, 1)
@@ -88,8 +133,12 @@ def test_what_has_no_such_launch_is_refused(et, device):
 
 
 @pytest.mark.parametrize("contexts", [(40, 41), (2030, 2060)], ids=["one_attention_launch_or_more", "context_2048"])
-def test_decode_steps_of_one_sequence_follow_the_oracle_chain(et, device, contexts):
+def test_decode_steps_of_one_sequence_follow_the_oracle_chain(et, device, contexts, monkeypatch):
+    made = []
+    model = test_gpu_decode_step.Model
+    monkeypatch.setattr(test_gpu_decode_step, "Model", lambda *args: made.append(model(*args)) or made[-1])
     _follow_the_oracle_chain(et, device, False, 1, contexts)
+    assert made[0].decoder.chained and made[0].decoder.project_in_attention
 
 
 def small_decoder(et, device, codec, slab, head_dim, bound, chain):
