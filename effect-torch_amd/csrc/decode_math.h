@@ -1,6 +1,8 @@
-// Arithmetic shared by the stand-alone decode operators (decode_ops.hip) and the activation
-// quantisers that apply them on the fly (quantize_act.hip), so that the fused and the separate
-// forms produce the same bits. Both translation units are compiled with -ffp-contract=off.
+// Arithmetic shared by the stand-alone decode operators (decode_ops.hip), the activation quantisers that apply them on
+// the fly (quantize_act.hip) and the launches that take them in (gemm_h16.hip, gemv_step.hip, kv_attention.hip,
+// kv_bytes.hip). The first two are compiled with -ffp-contract=off, the others are not: what is to give the same bits in
+// all of them (rotate_pair, silu_mul_one) switches contraction off itself, and rms_one is products alone. The sums of
+// squares of an RMS norm may differ in their last f64 bit, and the norm by a rounding to f32 once in many elements.
 #pragma once
 
 #include <hip/hip_runtime.h>

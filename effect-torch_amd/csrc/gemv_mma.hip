@@ -10,8 +10,8 @@
 // vectors cost on v_dot4 (gemv_limb.hip: 48 dots per vector, row and lane) is here one matrix
 // instruction per 32-column block and sixteen rows: v_mfma_i32_16x16x32_i8 with the weights' quants
 // as its B operand (sixteen rows of W) and, as its A operand, the three signed-byte limbs of four
-// activation vectors in rows 4v + limb (row 4v + 3 is zero, or a limb of a fifth vector). A lane of the result then holds, for its
-// weight row and its vector, the three limb dots of the block side by side.
+// activation vectors in rows 4v + limb (row 4v + 3 is zero, or a limb of a fifth vector). A lane of the result then holds,
+// for its weight row and its vector, the three limb dots of the block side by side.
 //
 // Work split. A workgroup owns a contiguous range of rows (one per compute unit when the matrix
 // fits). LOADER waves copy that range into LDS as it lies in memory, with 1 KiB global-to-LDS copies
@@ -192,7 +192,9 @@ struct Q4KMma {
             if constexpr (SCALES == 1) scaled_limbs(acc[g], sums[sums_step * g + 8], pos[g]);
             total[g] += d * pos[g] - dmin * neg;
         }
-        if constexpr (FIFTH) {  // the minima of sub-blocks 2q and 2q + 1 are this lane's part
+        // The minima of sub-blocks 2q and 2q + 1 are this lane's part. (Written out here and in Q5KMma: as a function of both, Q4_K
+        // 4096 x 14336 takes 16.5 us for 15.4.)
+        if constexpr (FIFTH) {
             const uint32_t mine = (q & 2u ? mn[1] : mn[0]) >> (16 * (q & 1u));
             const float2 s = *reinterpret_cast<const float2*>(fifth_sums + 2 * q);
             float neg = fmaf(static_cast<float>((mine >> 8) & 0xffu), s.y, static_cast<float>(mine & 0xffu) * s.x);
@@ -892,11 +894,13 @@ hipError_t launch_wide(const uint8_t* weight, const float* x, uint64_t x_row_str
 template <class T>
 hipError_t launch_vectors(const uint8_t* weight, const float* x, uint64_t x_row_stride, const float* bias, float* y,
                           uint32_t rows, uint32_t columns, uint32_t vectors, uint8_t* prepared, hipStream_t stream) {
-    // Two vector groups keep 64 registers of A operands: twelve waves leave each 168. Five vectors are fifteen limbs and fit one
-    // operand: half the matrix instructions of two groups, a multiply-add per block and eight instructions per unit more than
-    // four vectors (us, two groups / one; inputs from memory): Q4_K 4096 x 14336 18.9 / 17.1, 14336 x 4096 12.6 / 11.9, 4096 x 4096
-    // 7.2 / 6.8; Q5_K 31.7 / 27.4, 17.9 / 17.1, 7.6 / 7.1. The fifth vector's error against 64 bits is what it was. Not Q4_0 and Q8_0: a scale per block would have to meet the limbs'
-    // sums one by one, where an infinite one makes NaN of two signs, or the groups be put together for every block.
+    // Two vector groups keep 64 registers of A operands: twelve waves leave each 168. Five vectors are fifteen limbs and fit
+    // one operand: half the matrix instructions of two groups, a multiply-add per block and eight instructions per unit more
+    // than four vectors. In a graph, two groups / one (us; the same inputs again | inputs from memory): Q4_K 4096 x 14336 17.9 /
+    // 15.7 | 18.0 / 16.6, 14336 x 4096 12.0 / 11.2 | 12.9 / 12.0, 4096 x 4096 7.4 / 7.0 | 7.3 / 6.9; Q5_K 31.6 / 27.2 | 31.1 / 27.3, 17.2 /
+    // 16.3 | 17.3 / 16.4, 7.4 / 6.9 | 7.5 / 7.2. The fifth vector's error against 64 bits is what it was. Not Q4_0 and Q8_0: a
+    // scale per block would have to meet the limbs' sums one by one, where an infinite one makes NaN of two signs, or the
+    // groups be put together for every block.
     if (columns > kNarrowColumns) {
         if (prepared == nullptr) return hipErrorInvalidValue;
         if (vectors <= 4) return launch_wide<T, 1, false, 8, 4, 2>(weight, x, x_row_stride, bias, y, rows, columns, vectors, prepared, stream);

@@ -834,9 +834,9 @@ bool streaming_is_faster(const KvAttention& p, const KvLaunchShape& streaming, u
 // 15.0 / 13.9; two x 128 8 at 1408 (88 Ki) 14.2 / 16.0 but 4 at 3104 (97 Ki) 16.2 / 16.0; four x 128 4 at 1312 (41 Ki) 14.6 /
 // 15.5 but 4 at 2080 19.1 / 15.8. A long context leaves the streaming kernel so many records that it loses earlier: one slot at
 // 4224, four x 128 16.4 / 16.1; at 7168, two x 128 16.0 / 15.6.
-//   Eight waves, one workgroup per compute unit, need the fewest records (30 at 1000, 16/8 heads x 64: 11.3, four waves 14.0);
-// with many positions in a split two workgroups of four share a compute unit more evenly (3 at 10000 to 30000 39.7 / 37.3), but
-// not with two splits a unit (31 at 1238, 32/8 heads x 64: one piece of eight waves 18.3, two of four 25.0).
+//   Workgroups of eight waves, one per compute unit, leave the fewest records; with many positions in a split two workgroups
+// of four share a compute unit more evenly (3 at 10000 to 30000 39.7 / 37.3), but not with two splits a unit (31 at 1238, 32/8
+// heads x 64: one piece of eight waves 18.3, two of four 25.0).
 //   All by the declared bound: contexts far below it can lose what the slower start costs (32 at 100 under a bound of 2048:
 // 10.4 / 11.6; 3 at 500 under 30000: 13.6 / 15.2).
 struct BytesLimits {

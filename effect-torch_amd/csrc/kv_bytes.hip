@@ -4,9 +4,10 @@
 //
 // The bytes never become floats. q enters as 31-bit fixed point in four balanced signed-byte limbs per head; a row of K
 // less 128 is signed bytes as it lies in the slab, and v_mfma_i32_16x16x64_i8 contracts sixteen positions with the limbs of
-// up to four query heads (rows 4 * limb + head of one operand) in exact integers. A score is the sum of its four integers times q's unit, the softmax scale and the row's K scale. The weights
-// times the rows' V scales, 64 positions at a time, are fixed point in four limbs as well and contract with V's bytes,
-// which ds_read_b64_tr_b8 transposes out of LDS; the sums of a step are added up in f32.
+// up to four query heads (rows 4 * limb + head of one operand) in exact integers. A score is the sum of its four integers
+// times q's unit, the softmax scale and the row's K scale. The weights times the rows' V scales, 64 positions at a time,
+// are fixed point in four limbs as well and contract with V's bytes, which ds_read_b64_tr_b8 transposes out of LDS; the sums
+// of a step are added up in f32.
 //
 // Layout. A wave takes 64 positions a step on its own: K straight into the registers of the lanes that hold it as an
 // operand (lane = position l % 16, sixteen columns per lane group l / 16), V by copies into an LDS tile of its own, both
@@ -17,13 +18,18 @@
 // Precision: limbs hold 31 bits, a float's 24 and more, the integer sums are exact, and an exponent is rounded once, next to
 // the row's maximum. Relative error against 64 bits (2-norm, 1e-7; streaming kernel / this), 32/8 heads x 128: 32 slots at
 // 2048 3.3 / 1.3, three at 10000 to 30000 3.3 / 1.7, one at 60000 3.7 / 2.0. Three limbs (24 bits) and exponents of a rounded
-// score had 4.5.
+// score had 4.5. The fixed point is that of the largest of a row of q, and of the largest of 64 weights: what is smaller than
+// it by 2^-6 and more loses bits, which shows only where the largest meets a byte of 128, a value of zero. V scales and
+// queries keep their bits down to 2^-121.
+// What is not finite: a NaN or infinity in q, a K scale or a V scale makes all columns of the heads that see it NaN, as in
+// the streaming kernel (whose values are byte * scale - 128 * scale).
 //
 // Bound: reads of 128 bytes a position and head, with the ends of a launch. Per 64 positions of 128 columns a wave issues
 // about 700 vector and 16 matrix instructions (of 16 cycles) where the streaming kernel - a conversion, a scale and four
-// multiply-adds per byte - issues 2000. 32 slots at 2048 (138 MB): 53.4 -> 29.8 us, 4.7 TB/s; with the loads left out 17.
-// K comes by ordinary loads: the two halves of a row are two instructions', and non-temporal ones fetched its line twice
-// (37.5). Inputs from memory and not from the Infinity Cache: 49.0 -> 34.6.
+// multiply-adds per byte - issues 2000. 32 slots at 2048 (138 MB, which the Infinity Cache holds), streaming kernel / this, in a
+// graph: the same inputs again 50.4 / 31.8 us (4.3 TB/s), inputs from memory 51.1 / 35.7; with the loads left out 17. K comes by
+// ordinary loads: the two halves of a row are two instructions', and non-temporal ones fetched its line twice (a quarter
+// more time).
 #include <hip/hip_runtime.h>
 
 #include <atomic>
@@ -174,7 +180,8 @@ __global__ __launch_bounds__(64 * WAVES, 2) void kv_bytes_kernel(const KvArgs a)
     const uint32_t row_bytes = a.kv_heads * W;
     const uint8_t* k_base = static_cast<const uint8_t*>(a.k_slab) + kv_head * W;
     const uint8_t* v_base = static_cast<const uint8_t*>(a.v_slab) + kv_head * W;
-    const auto slab_row = [&](uint32_t position, auto shifts) __attribute__((always_inline)) -> uint64_t {  // positions past the end read the last cached row
+    // positions past the end read the last cached row
+    const auto slab_row = [&](uint32_t position, auto shifts) __attribute__((always_inline)) -> uint64_t {
         position = min(position, cached_end - 1);
         const uint32_t block = shifts ? position >> a.block_shift : position / a.block_size;
         const uint32_t within = shifts ? position & (a.block_size - 1) : position - block * a.block_size;
@@ -203,7 +210,8 @@ __global__ __launch_bounds__(64 * WAVES, 2) void kv_bytes_kernel(const KvArgs a)
             v_scale[t] = a.v_scales[row * a.kv_heads + kv_head];
         }
     };
-    const auto fetch = [&](uint32_t tile, uint32_t buffer) __attribute__((always_inline)) {  // one branch on the block size, not one per row
+    // one branch on the block size, not one per row
+    const auto fetch = [&](uint32_t tile, uint32_t buffer) __attribute__((always_inline)) {
         if (a.block_shift >= 0)
             fetch_rows(tile, buffer, std::true_type{});
         else
