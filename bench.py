@@ -37,47 +37,48 @@ ROTATE_BYTES = 640 << 20       # > 2x the 256 MB Infinity Cache
 # HBM bytes per launch measured with rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE, scaled by the same
 # counters' reading for a plain copy of known size. The counters cannot be collected from inside
 # this script, so each figure is tied to the kernel it was taken from: the kernel's name as the
-# planner reports it and the SHA-256 of the source file that defines it at the time of the profile.
+# planner reports it and the SHA-256 of the source files that define it, one after the other, at the time of the profile.
 # When either differs from what runs now, `roofline.traffic` is null until the profile is re-taken.
 MEASURED_TRAFFIC = {
     ("q4_k_gemv_14336x4096", 1, "f32"): {
-        "bytes": 33283900, "kernel": "gemv_limb_dma", "source": "gemv_limb.hip",
-        "sha256": "4fa7d816114655dcc55c2445c3543c2c2a4ee75ef28d65d3e37a1ac4883848cb",
+        "bytes": 33284000, "kernel": "gemv_limb_dma", "sources": ("gemv_limb.hip", "gemv_limb_device.h"),
+        "sha256": "4816172f76e164fc94ed8f30e01bc2b88e1e96ad473a314b8e5a361afa7e1098",
         "profile": "profiles/gemv_limb_q4k_14336x4096_m1_hbm_traffic.md"},
     ("q4_0_gemv_11008x4096", 1, "f32"): {
-        "bytes": 25614000, "kernel": "gemv_limb_dma", "source": "gemv_limb.hip",
-        "sha256": "4fa7d816114655dcc55c2445c3543c2c2a4ee75ef28d65d3e37a1ac4883848cb",
+        "bytes": 25614000, "kernel": "gemv_limb_dma", "sources": ("gemv_limb.hip", "gemv_limb_device.h"),
+        "sha256": "4816172f76e164fc94ed8f30e01bc2b88e1e96ad473a314b8e5a361afa7e1098",
         "profile": "profiles/gemv_limb_q4k_14336x4096_m1_hbm_traffic.md"},
     ("q4_k_gemv_14336x4096", 4, "f32"): {
-        "bytes": 33895200, "kernel": "gemv_mma", "source": "gemv_mma.hip",
-        "sha256": "f3bf93df89988bc17bec99050bd1b47eecb979a5c848917aad42700dfb58aba2",
+        "bytes": 33901400, "kernel": "gemv_mma", "sources": ("gemv_mma.hip",),
+        "sha256": "0b585507674e24af341b701c61cbc8563864749030dc18312122180f27abb1c0",
         "profile": "profiles/gemv_mma_small_batch_2_to_8_vectors.md"},
     ("q4_k_gemv_14336x4096", 8, "f32"): {
-        "bytes": 34754600, "kernel": "gemv_mma", "source": "gemv_mma.hip",
-        "sha256": "f3bf93df89988bc17bec99050bd1b47eecb979a5c848917aad42700dfb58aba2",
+        "bytes": 34769400, "kernel": "gemv_mma", "sources": ("gemv_mma.hip",),
+        "sha256": "0b585507674e24af341b701c61cbc8563864749030dc18312122180f27abb1c0",
         "profile": "profiles/gemv_mma_small_batch_2_to_8_vectors.md"},
     ("kv_attention_decode", 2048): {
-        "bytes": 270024900, "kernel": "kv_attend", "source": "kv_attention.hip",
-        "sha256": "590105a686a613206e4bfe632266890d8f03aa1f6a00829b1aa81122a1f041fd",
+        "bytes": 270026900, "kernel": "kv_attend", "sources": ("kv_attention.hip",),
+        "sha256": "99fb132fdc8aadf54121f3367e7a5e484a25388563590e2de301d40caf019f60",
         "profile": "profiles/kv_attend_decode_32slots_ctx2048_f16.md"},
 }
 
 
 def measured_traffic(key, kernel_name):
     """The profiled HBM bytes per launch of `key`, or None when the kernel that runs now is not the
-    one that was profiled (another kernel name, or its source file has changed since)."""
+    one that was profiled (another kernel name, or one of its source files has changed since)."""
     import hashlib
 
     entry = MEASURED_TRAFFIC.get(key)
     if entry is None or not str(kernel_name).startswith(entry["kernel"]):
         return None
-    path = os.path.join(ROOT, "effect-torch_amd", "csrc", entry["source"])
+    digest = hashlib.sha256()
     try:
-        with open(path, "rb") as source:
-            digest = hashlib.sha256(source.read()).hexdigest()
+        for name in entry["sources"]:
+            with open(os.path.join(ROOT, "effect-torch_amd", "csrc", name), "rb") as source:
+                digest.update(source.read())
     except OSError:
         return None
-    return entry["bytes"] if digest == entry["sha256"] else None
+    return entry["bytes"] if digest.hexdigest() == entry["sha256"] else None
 
 
 def cpu_model():
