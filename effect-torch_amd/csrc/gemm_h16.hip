@@ -2,7 +2,7 @@
 // matrix cores: weights times their sub-block scales are exact small integers in half floats, activations two half floats each.
 //
 //   y[m, n] = sum_s  unit[m, s] * d[n, s] * sum_g sum_i (sc_g[n] * nib[n, g, i]) * X[m, g, i]
-//           - sum_s  dmin[n, s] * sum_g m_g[n] * xsum[m, g]
+//           - sum_s  unit[m, s] * dmin[n, s] * sum_g m_g[n] * xsum[m, g]
 // s = 256-column stage (one Q4_K super-block), g = its eight 32-column sub-blocks.
 //
 // Activations are scaled per vector and stage, X = x * (2^23 - 1) / max|x|, and split into X = 4096 * hi + lo with
@@ -351,14 +351,15 @@ __global__ __launch_bounds__(kThreads) void gemm_h16_kernel(
         uint4 fifth = make_uint4(0u, 0u, 0u, 0u);  // Q5_K: qh of this lane half's sixteen columns
         if constexpr (CODEC == kQ5_K) fifth = *reinterpret_cast<const uint4*>(row_in_slot + 16u + 16u * half);
 
-        // min term: acc_min[m, n] += sum_g (dmin * m_g)[n] * xsum[m, g]; K = 2 per MFMA, lane half h
+        // min term: acc_min[m, n] += sum_g (dmin * m_g)[n] * (unit * xsum[g])[m]; K = 2 per MFMA, lane half h
         // supplies sub-block 2j + h.
+        const float vector_unit = *reinterpret_cast<const float*>(slot + kUnitAt + in_half * 4u);
 #pragma unroll
         for (int jj = 0; jj < NB / 2; jj++) {
             const uint32_t g = b_base + 2u * jj + half;
             uint32_t sc, mn;
             q4k_scale_min(header, g, sc, mn);
-            const float a_operand = *reinterpret_cast<const float*>(slot + kSumsAt + g * 128u + in_half * 4u);
+            const float a_operand = vector_unit * *reinterpret_cast<const float*>(slot + kSumsAt + g * 128u + in_half * 4u);
             acc_min = __builtin_amdgcn_mfma_f32_32x32x2f32(a_operand, dmin_block * static_cast<float>(mn), acc_min,
                                                            0, 0, 0);
         }

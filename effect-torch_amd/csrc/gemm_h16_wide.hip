@@ -2,26 +2,31 @@
 // vectors with 256 weight rows (Q2_K, Q6_K: 128), so that weights are unpacked once for 128 (64) vectors instead of for
 // every 32, and an activation tile is copied for 256 rows instead of 64 or 128.
 //
-// Bound: instruction issue. Eight waves, two per SIMD, each 128 vectors x 32 rows (Q2_K, Q6_K, which contract two operands
-// per weight: 64 x 32). Matrix and vector instructions of a SIMD take their time one after the other on this device, also
-// from two waves: a Q4_K wave's stage of 256 columns is 128 half-float matrix instructions (32 cycles each), 16 f32 ones for
-// the minima (64) and about 510 vector instructions (4): 7160 cycles by that sum, 7860 measured at the 2.1 GHz the
-// device holds. What helped was therefore fewer vector instructions (waves of 64 x 64 unpack every weight twice: 282 ->
-// 296 us) and not the latencies: operands fetched only behind each barrier measured the same. Counted at
-// 14336 x 4096 with 1000 vectors: matrix 60 %, vector 22 % of the cycles of busy compute units, which are busy 81 % of the
-// launch (448 workgroups on 256 compute units), no LDS bank conflicts.
+// Bound: the matrix pipe, at the clock that its power leaves. Eight waves, two per SIMD, each 128 vectors x 32 rows (Q2_K,
+// Q6_K, which contract two operands per weight: 64 x 32). A Q4_K wave's stage of 256 columns is 128 half-float matrix
+// instructions, eight bfloat16 ones for the minima (32 cycles each) and about 520 vector instructions. With two waves on a SIMD
+// up to seven vector instructions (of four cycles) run in the shadow of each matrix instruction (measured in loops of both; with
+// one wave four do), so what counts is how evenly they lie between them: the next sub-block's operands are made between
+// this one's matrix instructions, and a stage's sums are folded into the accumulators tile by tile between the next tile's.
+// The minima were f32 matrix instructions (16 of 64 cycles per stage, a fifth of the pipe's time); now the sums of a
+// sub-block, whole numbers, are cut into three bfloat16 pieces once per workgroup, and the products are exact.
+// Both steps, 14336 x 4096 with 1000 vectors: 289 -> 253 us, clocks of busy compute units 122.5 -> 99.6 million, of which matrix
+// instructions 60 -> 63 %. The clock falls from 2.02 to 1.93 GHz on the way: a loop of these instructions alone holds 1.75 GHz on
+// random operands (2.1 on zeros). Without any copies 7 % less; 448 workgroups on 256 compute units leave an eighth of them idle.
 // Every wave unpacks its own weight rows from the packed bytes in LDS. There are no loader waves (a third wave per SIMD
 // would leave 168 registers each): the waves ask for the next sub-blocks' activations and the next stage's weights
 // themselves, through inline assembly, because any LDS read next to a copy that the compiler can see waits for it.
 //
-// Whole calls (us, gemm_h16_kernel / this): 14336 x 4096 with 1000 vectors Q4_K 420 / 288 (407 TFLOP/s), Q5_K 453 / 285,
-// Q6_K 724 / 460, Q3_K 415 / 255, Q2_K 512 / 405; Q4_K 4096 x 14336 with 1000 396 / 278, 14336 x 4096 with 256 115 / 85.
+// Whole calls (us, gemm_h16_kernel / this before / this): 14336 x 4096 with 1000 vectors Q4_K 420 / 284 / 262 (448 TFLOP/s), Q5_K
+// 453 / 292 / 270, Q6_K 724 / 461 / 429, Q3_K 415 / 259 / 246, Q2_K 512 / 418 / 397; Q4_K 4096 x 14336 with 1000 396 / 280 / 261,
+// 14336 x 4096 with 256 115 / 93 / 90.
 // Relative error against 64 bits there (2-norm, 1e-7): Q4_K 1.75 / 1.71, Q6_K 1.66 / 1.63, Q2_K 1.84 / 1.76: one chain of
 // sums over the stage's eight sub-blocks instead of two or four, from activations that are rounded less (quantize_halves.h).
 #include <hip/hip_runtime.h>
 
 #include <atomic>
 #include <cstdint>
+#include <type_traits>
 
 #include "gemm_h16_device.h"
 
@@ -32,6 +37,9 @@ constexpr int kWaves = 8;
 constexpr int kTiles = kGemmWideVectors / 32;        // activation tiles per workgroup
 constexpr int kSlots = 4;                            // sub-blocks of activations in LDS: two landed, two on their way
 constexpr uint32_t kSlotBytes = kTiles * 2 * 2048u;  // per tile and plane four 8-column parts of 512 bytes
+constexpr int kCutAt = 3;                            // the sub-block in which the stage's sums are cut: they have landed by then
+typedef short v8s __attribute__((ext_vector_type(8)));
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 constexpr int kActivationCopies = 2;                 // per wave and sub-block: one plane of one tile
 static_assert(kTiles * 2 == kWaves && kStageBlocks % kSlots == 0, "a wave copies one plane of one tile; slots start anew per stage");
 
@@ -50,8 +58,9 @@ struct Wide {
     static constexpr int kRounds = (kWeightJobs + kWaves - 1) / kWaves;  // weight copies per wave and stage, one per sub-block
     static_assert(kRounds <= kStageBlocks - 2, "landed before the last sub-block");
     // the activation slots; one stage of unit[m] (512 bytes, copied twice) and of xsum; two stages of weights
+    // (and, in their place, the sums cut into three bfloat16 pieces, [tile][piece][vector][sub-block])
     static constexpr uint32_t kUnitsAt = kSlots * kSlotBytes, kSumsAt = kUnitsAt + 1024u,
-                              kWeightsAt = kSumsAt + (kMinima ? 4096u : 0u), kLdsBytes = kWeightsAt + 2 * kWeightBytes;
+                              kWeightsAt = kSumsAt + (kMinima ? kTiles * 1536u : 0u), kLdsBytes = kWeightsAt + 2 * kWeightBytes;
     static_assert(kLdsBytes <= 160 * 1024, "LDS of a gfx950 CU: 160 KiB, all of it dynamic here");
     // copies that a wave asks for in front of the activations during sub-block b: the stage's tables, next weights
     static constexpr int ahead(int b, bool last) { return (b == 0 ? 1 : 0) + (!last && b < kRounds ? 1 : 0); }
@@ -61,7 +70,7 @@ struct Wide {
 __device__ __forceinline__ void copy_to_lds(const uint8_t* base, uint32_t lane_offset, uint32_t to) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                  :
-                 : "s"(to), "v"(lane_offset), "s"(base)
+                 : "s"(__builtin_amdgcn_readfirstlane(to)), "v"(lane_offset), "s"(base)
                  : "memory");  // m0 is a reserved register: nothing else in this file sets it
 }
 
@@ -152,6 +161,32 @@ __device__ __forceinline__ void operands(const Raw& raw, const Shared& shared, i
     }
 }
 
+// f32 bits as three bfloat16 numbers that add up to it, eight significant bits each: the top halves of `x`, of
+// what is left of it, and of what is left then (nothing is lost above 2^-110, and S is a whole number).
+struct Pieces {
+    uint32_t high, mid, low;  // in the upper sixteen bits
+};
+__device__ __forceinline__ Pieces cut(float x) {
+    Pieces p;
+    p.high = __float_as_uint(x) & 0xffff0000u;
+    const float rest = x - __uint_as_float(p.high);
+    p.mid = __float_as_uint(rest) & 0xffff0000u;
+    p.low = __float_as_uint(rest - __uint_as_float(p.mid));
+    return p;
+}
+__device__ __forceinline__ v8bf as_bf16(const v8s& bits) { return __builtin_bit_cast(v8bf, bits); }
+// The eight minima of this lane's row, against the high (lane half 0) and middle pieces, and against the low ones
+// (half 0 alone: the operand's other eight columns are zero).
+__device__ __forceinline__ void minimum_operands(const uint4& header, uint32_t half, v8s out[2]) {
+#pragma unroll
+    for (uint32_t g = 0; g < kStageBlocks; g++) {
+        uint32_t sc, mn;
+        q4k_scale_min(header, g, sc, mn);
+        out[0][g] = static_cast<short>(__float_as_uint(static_cast<float>(mn)) >> 16);  // at most 63: exact
+    }
+    out[1] = half == 0 ? out[0] : v8s{0, 0, 0, 0, 0, 0, 0, 0};
+}
+
 template <int CODEC>
 __global__ __launch_bounds__(64 * kWaves, 2) void gemm_h16_wide_kernel(const Group group, const uint8_t* __restrict__ tiles,
                                                                        uint32_t vector_tiles, uint32_t columns,
@@ -222,6 +257,23 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_h16_wide_kernel(const Gro
             copy_to_lds(base + kUnitAt, min((lane >> 3) & 3u, tiles_left) * kBlob + (lane & 7u) * 16u, lds0 + W::kUnitsAt);
     };
 
+    // Between the barriers of sub-blocks kCutAt and kCutAt + 1 every thread reads and cuts the sums of two sub-blocks of one
+    // vector, behind the second one the pieces take the sums' place; they are read in the last sub-block.
+    uint32_t piece[3];
+    const uint32_t cut_vector = threadIdx.x & 31u, cut_group = ((threadIdx.x >> 5) & 3u) * 2u;
+    const auto cut_sums = [&] {
+        const float* sums = reinterpret_cast<const float*>(lds + W::kSumsAt + (wave >> 1) * 1024u) + cut_group * 32u + cut_vector;
+        const Pieces a = cut(sums[0]), b = cut(sums[32]);
+        piece[0] = __builtin_amdgcn_perm(b.high, a.high, 0x07060302u);
+        piece[1] = __builtin_amdgcn_perm(b.mid, a.mid, 0x07060302u);
+        piece[2] = __builtin_amdgcn_perm(b.low, a.low, 0x07060302u);
+    };
+    const auto put_pieces = [&] {
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+            *reinterpret_cast<uint32_t*>(lds + W::kSumsAt + (wave >> 1) * 1536u + i * 512u + cut_vector * 16u + cut_group * 2u) = piece[i];
+    };
+
     v16f acc[MT], zero;
 #pragma unroll
     for (int r = 0; r < 16; r++) zero[r] = 0.f;
@@ -232,24 +284,26 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_h16_wide_kernel(const Gro
         return lds + W::kWeightsAt + (stage & 1u) * W::kWeightBytes + (wave_n * 32u + in_half) * kRowBytes;
     };
     const uint8_t* const activations = lds + wave_m * MT * 4096u + half * 1024u + in_half * 16u;
-    const auto load = [&](int b, int plane, int chunk, v8h x[MT]) {
-#pragma unroll
-        for (int m = 0; m < MT; m++)
-            x[m] = *reinterpret_cast<const v8h*>(activations + (b % kSlots) * kSlotBytes + m * 4096u + plane * 2048u + chunk * 512u);
+    const auto operand = [&](int b, int m, int turn) {  // turn: low and high plane of one sixteen-column chunk, then of the other
+        return *reinterpret_cast<const v8h*>(activations + (b % kSlots) * kSlotBytes + m * 4096u + (turn & 1) * 2048u + (turn >> 1) * 512u);
     };
 
     // Sub-block b of a stage begins. Landed behind its barrier: the activations of sub-block b + 1, and whatever was
     // asked for before them two sub-blocks ago. Free: the slot of sub-block b - 1, in a stage's first sub-block also the
     // other stage's weights and the tables of the stage before.
-    const auto begin = [&](uint32_t stage, bool last, int b) {
+    const auto begin = [&](uint32_t stage, auto is_last, int b) {
+        constexpr bool last = decltype(is_last)::value;
         if (!last) wait_copies_in_flight(kActivationCopies + (b > 0 ? W::ahead(b - 1, false) : 0));
         else wait_copies_in_flight(b < 6 ? kActivationCopies + (b > 0 ? W::ahead(b - 1, true) : 0) : 0);
+        if (W::kMinima && b == kCutAt + 1) asm volatile("" : "+v"(piece[0]), "+v"(piece[1]), "+v"(piece[2]));  // read before others write
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         if (b == 0) copy_tables(stage);
         if (!last && b < W::kRounds) copy_weights(stage + 1u, b);
         if (b + kSlots - 1 < kStageBlocks) copy_activations(stage, b + kSlots - 1);
         else if (!last) copy_activations(stage + 1u, b + kSlots - 1 - kStageBlocks);
+        if (W::kMinima && b == kCutAt) cut_sums();
+        if (W::kMinima && b == kCutAt + 1) put_pieces();
     };
 #pragma unroll
     for (int i = 0; i < W::kRounds; i++) copy_weights(0, i);
@@ -259,127 +313,178 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_h16_wide_kernel(const Gro
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     if (!working) {
-        for (uint32_t stage = 0; stage < stages; stage++) {
+        const auto pass = [&](uint32_t stage, auto is_last) {
 #pragma unroll
-            for (int b = 0; b < kStageBlocks; b++) begin(stage, stage + 1u == stages, b);
-        }
+            for (int b = 0; b < kStageBlocks; b++) begin(stage, is_last, b);
+        };
+        for (uint32_t stage = 0; stage + 1u < stages; stage++) pass(stage, std::false_type{});
+        pass(stages - 1u, std::true_type{});
         return;
     }
     Shared shared = fetch_shared<CODEC>(row_of(0), half);
-    v8h w[2][P], x[2][MT];
+    v8h w[2][P], x[2][4];  // x: the operands of MT tiles in one turn, in the last sub-block of one tile in four turns
     operands<CODEC>(fetch<CODEC>(row_of(0), 0, half), shared, 0, w);
-    load(0, 0, 0, x[0]);
+    const auto load_turn = [&](int b, int turn, v8h to[4]) {
+#pragma unroll
+        for (int m = 0; m < MT; m++) to[m] = operand(b, m, turn);
+    };
+    const auto load_tile = [&](int b, int m, v8h to[4]) {
+#pragma unroll
+        for (int turn = 0; turn < 4; turn++) to[turn] = operand(b, m, turn);
+    };
+    load_turn(0, 0, x[0]);
 
-    for (uint32_t stage = 0; stage < stages; stage++) {
-        const bool last = stage + 1u == stages;
+    // One stage. A wave issues in order and a matrix instruction keeps its pipe busy for eight issue cycles, so what keeps the
+    // pipe fed is that no run of vector instructions stands alone: the sums of one tile of vectors are finished before the
+    // next tile's begin, the packed bytes of the next sub-block become operands between the matrix instructions of
+    // this one, and a tile's sums of the stage are folded into acc between the last matrix instructions of the next tile.
+    // The last stage is compiled apart: a branch between sub-blocks would let the compiler move that arithmetic behind it.
+    const auto contract = [&](uint32_t stage, auto is_last) {
+        constexpr bool last = decltype(is_last)::value;
         v16f p[P][MT];
         Shared shared_next;
+        // what the fold needs of this lane's row
+        float d = 0.f, dmin = 0.f;
+        v8s minima[2];
 #pragma unroll
         for (int b = 0; b < kStageBlocks; b++) {
-            begin(stage, last, b);
-            // Four turns of matrix instructions, low and high plane of both sixteen-column chunks. Behind each the next
-            // turn's activations are read; behind the first also the next sub-block's packed bytes, which become weight
-            // operands behind the third.
+            begin(stage, is_last, b);
+            const bool more = !last || b + 1 < kStageBlocks;
             const int bn = (b + 1) % kStageBlocks;
             const uint8_t* const row_n = row_of(b + 1 < kStageBlocks ? stage : stage + 1u);
             Raw raw;
             v8h next[2][P];
-#pragma unroll
-            for (int turn = 0; turn < 4; turn++) {
-                const int chunk = turn >> 1, plane = turn & 1;
-                if (turn < 3) load(b, (turn + 1) & 1, (turn + 1) >> 1, x[(turn + 1) & 1]);
-                else load(bn, 0, 0, x[0]);
-                if (turn == 0) {
-                    if (bn == 0) shared_next = fetch_shared<CODEC>(row_n, half);
-                    raw = fetch<CODEC>(row_n, bn, half);
-                }
-                if (turn == 2) operands<CODEC>(raw, bn == 0 ? shared_next : shared, bn, next);
-#pragma unroll
-                for (int m = 0; m < MT; m++)
-#pragma unroll
-                    for (int k = 0; k < P; k++)
-                        p[k][m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[plane][m], w[chunk][k], b + turn == 0 ? zero : p[k][m], 0, 0, 0);
-                // reads first, then the matrix instructions with the operands' arithmetic between them
-                __builtin_amdgcn_sched_group_barrier(0x100, MT + 1, 0);
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x002, 10, 0);
-                }
-                __builtin_amdgcn_sched_barrier(0);
+            if (b + 1 == kStageBlocks) {
+                const uint8_t* row = row_of(stage);
+                uint32_t dd = 0;
+                if constexpr (W::kMinima) dd = shared.header.x;
+                else if constexpr (CODEC == kQ3_K) dd = *reinterpret_cast<const uint16_t*>(row + HalfStage<CODEC>::in_tail(108u));
+                else if constexpr (CODEC == kQ6_K) dd = *reinterpret_cast<const uint16_t*>(row + HalfStage<CODEC>::in_tail(208u));
+                else dd = *reinterpret_cast<const uint32_t*>(row + HalfStage<CODEC>::in_tail(80u));
+                d = kPlaneRatio * half_bits_to_float(dd & 0xffffu), dmin = half_bits_to_float(dd >> 16);
+                if constexpr (W::kMinima) minimum_operands(shared.header, half, minima);
             }
-#pragma unroll
-            for (int chunk = 0; chunk < 2; chunk++)
-#pragma unroll
-                for (int k = 0; k < P; k++) w[chunk][k] = next[chunk][k];
-        }
-        // acc += p * unit[m] * d[n] - sum_g (dmin * m_g)[n] * xsum[m, g]; vectors of a lane: 8 (r / 4) + 4 half + r % 4
-        const uint8_t* row = row_of(stage);
-        uint32_t dd = 0;
-        if constexpr (W::kMinima) dd = shared.header.x;
-        else if constexpr (CODEC == kQ3_K) dd = *reinterpret_cast<const uint16_t*>(row + HalfStage<CODEC>::in_tail(108u));
-        else if constexpr (CODEC == kQ6_K) dd = *reinterpret_cast<const uint16_t*>(row + HalfStage<CODEC>::in_tail(208u));
-        else dd = *reinterpret_cast<const uint32_t*>(row + HalfStage<CODEC>::in_tail(80u));
-        const float d = kPlaneRatio * half_bits_to_float(dd & 0xffffu), dmin = half_bits_to_float(dd >> 16);
-        float minimum[kStageBlocks / 2];  // of sub-blocks 2 j + half
-        if constexpr (W::kMinima) {
-#pragma unroll
-            for (int j = 0; j < kStageBlocks / 2; j++) {
-                uint32_t sc, mn;
-                q4k_scale_min(shared.header, 2u * j + half, sc, mn);
-                minimum[j] = dmin * static_cast<float>(mn);
-            }
-        }
-#pragma unroll
-        for (int m = 0; m < MT; m++) {
-            v16f below = zero;  // K = 2 per instruction, lane half h supplies sub-block 2 j + h
-            if constexpr (W::kMinima) {
-#pragma unroll
-                for (int j = 0; j < kStageBlocks / 2; j++)
-                    below = __builtin_amdgcn_mfma_f32_32x32x2f32(
-                        *reinterpret_cast<const float*>(lds + W::kSumsAt + (wave_m * MT + m) * 1024u + (2u * j + half) * 128u + in_half * 4u),
-                        minimum[j], below, 0, 0, 0);
-            }
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const float4 units = *reinterpret_cast<const float4*>(lds + W::kUnitsAt + (wave_m * MT + m) * 128u + (8u * j + 4u * half) * 4u);
+            // acc += unit[m] * (p * d[n] - (sum_g S[m, g] * m_g[n]) * dmin[n]); vectors of a lane: 8 (r / 4) + 4 half + r % 4
+            v16f below;
+            const auto units_of = [&](int m, int j) {
+                return *reinterpret_cast<const float4*>(lds + W::kUnitsAt + (wave_m * MT + m) * 128u + (8u * j + 4u * half) * 4u);
+            };
+            const auto fold = [&](int m, int j, const float4& units) {
                 const float unit[4] = {units.x, units.y, units.z, units.w};
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
                     const int r = 4 * j + i;
-                    if constexpr (W::kMinima) acc[m][r] += fmaf(p[0][m][r], unit[i] * d, -below[r]);
+                    if constexpr (W::kMinima) acc[m][r] = fmaf(fmaf(p[0][m][r], d, -dmin * below[r]), unit[i], acc[m][r]);
                     else if constexpr (CODEC == kQ6_K) acc[m][r] = fmaf(fmaf(16.0f, p[P - 1][m][r], p[0][m][r]), unit[i] * d, acc[m][r]);
                     else if constexpr (CODEC == kQ2_K)
                         acc[m][r] = fmaf(fmaf(p[0][m][r], d, -p[P - 1][m][r] * (kPlaneRatio * dmin)), unit[i], acc[m][r]);
                     else acc[m][r] = fmaf(p[0][m][r], unit[i] * d, acc[m][r]);
                 }
+            };
+            float4 units = {};
+            if (b + 1 < kStageBlocks) {
+                // four turns; x[0] holds the first one's operands
+#pragma unroll
+                for (int turn = 0; turn < 4; turn++) {
+                    if (turn < 3) load_turn(b, turn + 1, x[(turn + 1) & 1]);
+                    else if (b + 2 < kStageBlocks) load_turn(bn, 0, x[0]);
+                    else load_tile(bn, 0, x[0]);
+                    if (turn == 0) raw = fetch<CODEC>(row_n, bn, half);
+                    if (turn == 1) operands<CODEC>(raw, shared, bn, next);
+#pragma unroll
+                    for (int m = 0; m < MT; m++)
+#pragma unroll
+                        for (int k = 0; k < P; k++)
+                            p[k][m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[turn & 1][m], w[turn >> 1][k], b + turn == 0 ? zero : p[k][m], 0, 0, 0);
+                    // reads first, then the matrix instructions, from the second turn on with the next operands' arithmetic between them
+                    __builtin_amdgcn_sched_group_barrier(0x100, MT, 0);
+                    if (turn == 0) {
+                        __builtin_amdgcn_sched_group_barrier(0x008, 4 * P * MT / 4, 0);
+                        __builtin_amdgcn_sched_barrier(0);
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < P * MT; i++) {
+                            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                            __builtin_amdgcn_sched_group_barrier(0x002, P == 1 ? 3 : 5, 0);
+                        }
+                    }
+                }
+            } else {
+                // tile after tile; x[0] holds the first one's operands
+#pragma unroll
+                for (int m = 0; m < MT; m++) {
+                    if (m + 1 < MT) load_tile(b, m + 1, x[(m + 1) & 1]);
+                    else if (more) load_turn(bn, 0, x[(m + 1) & 1]);
+                    if (m == 0 && more) {
+                        shared_next = fetch_shared<CODEC>(row_n, half);
+                        raw = fetch<CODEC>(row_n, bn, half);
+                    }
+                    if (m == MT / 2 && more) operands<CODEC>(raw, shared_next, bn, next);
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        float4 units_next = units;
+                        if (m + (i + 1) / 4 > 0) units_next = units_of(m - 1 + (i + 1) / 4, (i + 1) % 4);
+#pragma unroll
+                        for (int k = 0; k < P; k++)
+                            p[k][m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[m & 1][i], w[i >> 1][k], p[k][m], 0, 0, 0);
+                        if (m > 0) fold(m - 1, i, units);
+                        units = units_next;
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                    if (W::kMinima) {
+                        const uint8_t* pieces = lds + W::kSumsAt + (wave_m * MT + m) * 1536u + in_half * 16u;
+                        below = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16(*reinterpret_cast<const v8s*>(pieces + half * 512u)),
+                                                                        as_bf16(minima[0]), zero, 0, 0, 0);
+                        below = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16(*reinterpret_cast<const v8s*>(pieces + 1024u)),
+                                                                        as_bf16(minima[1]), below, 0, 0, 0);
+                    }
+                }
+            }
+            if (b + 1 == kStageBlocks) {
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const float4 now = units;
+                    if (j < 3) units = units_of(MT - 1, j + 1);
+                    fold(MT - 1, j, now);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (more) {
+#pragma unroll
+                for (int chunk = 0; chunk < 2; chunk++)
+#pragma unroll
+                    for (int k = 0; k < P; k++) w[chunk][k] = next[chunk][k];
             }
         }
-        shared = shared_next;
-    }
+        if (!last) shared = shared_next;
+    };
+    for (uint32_t stage = 0; stage + 1u < stages; stage++) contract(stage, std::false_type{});
+    contract(stages - 1u, std::true_type{});
 
-    // ---- add bias, store ----
+    // ---- add bias, store: y, or this K share's sums ----
     const uint64_t launch_rows = static_cast<uint64_t>(group.row_tiles) * W::kRows;
     const uint32_t in_tile = wave_n * 32u + in_half, n_out = row0 + in_tile;
     if (n_out >= rows) return;
-    const float bias = member.bias != nullptr ? member.bias[n_out] : 0.f;
-    const uint32_t launch_row = row_tile * W::kRows + in_tile;  // among the rows of all members
+    const bool direct = k_splits == 1;
+    const float bias = direct && member.bias != nullptr ? member.bias[n_out] : 0.f;
+    const uint64_t stride = direct ? rows : launch_rows;  // of a vector; row_tile * kRows + in_tile is among the rows of all members
+    float* const out = direct ? member.y + n_out : partials + k_share * (vectors * launch_rows) + row_tile * W::kRows + in_tile;
+    const float* const residual = direct && member.residual != nullptr ? member.residual + n_out : nullptr;
+    const auto store = [&](auto all_vectors) {
 #pragma unroll
-    for (int m = 0; m < MT; m++) {
+        for (int m = 0; m < MT; m++) {
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const uint32_t v = (first_vector_tile + m) * 32u + 8u * (r >> 2) + 4u * half + (r & 3u);
-            if (v >= vectors) continue;
-            if (k_splits == 1) {
+            for (int r = 0; r < 16; r++) {
+                const uint32_t v = (first_vector_tile + m) * 32u + 8u * (r >> 2) + 4u * half + (r & 3u);
+                if (!decltype(all_vectors)::value && v >= vectors) continue;
                 // residual may be y itself: every output is read, then written, by this lane only
-                const uint64_t at = static_cast<uint64_t>(v) * rows + n_out;
                 const float value = acc[m][r] + bias;
-                member.y[at] = member.residual != nullptr ? value + member.residual[at] : value;
-            } else {
-                partials[(static_cast<uint64_t>(k_share) * vectors + v) * launch_rows + launch_row] = acc[m][r];
+                out[v * stride] = residual != nullptr ? value + residual[v * stride] : value;
             }
         }
-    }
+    };
+    if ((first_vector_tile + MT) * 32u <= vectors && residual == nullptr) store(std::true_type{});
+    else store(std::false_type{});
 }
 
 template <int CODEC>
