@@ -34,11 +34,14 @@
 // is copied (global_load_lds; the u8 tier passes through registers, where it becomes half floats and bfloat16) while
 // this one is contracted.
 //
-// Bound: instruction issue. Matrix and vector instructions of a SIMD take their time one after the other on this device;
-// two slots of 500 tokens at context 2000, 32/8 heads x 128: matrix 38 %, vector (softmax, the weights' pieces, the adds of
-// the short chains) 45 % of the cycles of busy compute units (u8: 33 and 51 %), no LDS bank conflicts, compute units busy 76 %
-// of the launch (their workgroups have 1500 to 2000 positions). 93 us with the append launch, where the streaming kernel
-// took 1036; bf16 115 / 1097, u8 126 / 1322.
+// Bound: instruction issue. A wave's scores, weights and products follow one another, and the matrix and vector instructions
+// of the two waves of a SIMD hardly run side by side in such long runs (with the waves half a step apart the same time); two
+// slots of 500 tokens at context 2000, 32/8 heads x 128: matrix 38 %, vector (softmax, the weights' pieces, the adds of
+// the short chains) about 40 % of the cycles of busy compute units, no LDS bank conflicts, compute units busy 76 %
+// of the launch (their workgroups have 1500 to 2000 positions). What a tile costs besides: its addresses, found by a lane per
+// position one tile ahead and handed out with ds_bpermute; two LDS offsets per lane, from which every operand's address is
+// one exclusive or; a row's maximum that is followed to within kSlack. Before these three, and now (us): two slots of 500 at
+// 2000 96.7 / 93.4, bf16 115.3 / 106.2, u8 127.1 / 121.2, at 8000 289 / 280 (the streaming kernel took 1036, 1097 and 1322).
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 
@@ -167,6 +170,10 @@ struct Slab<U8> {
     }
 };
 
+// Weights are at most exp2(kSlack), 4 * 4096 in a half float's pieces, and the rounding of a positive exponent is that of the
+// exponents between -2 and 0. With a maximum that is followed exactly nearly every step of 64 positions has one row of 32 that
+// moves, and all 32 pay 70 vector instructions for it.
+constexpr float kSlack = 2.0f;
 constexpr int kChunkWaves = 8, kChunkThreads = 64 * kChunkWaves;
 
 // RW row waves share a tile (32 * RW query rows per workgroup), 8 / RW groups of them take tiles in turn.
@@ -183,6 +190,8 @@ struct ChunkShape {
     static constexpr uint32_t kTableAt = 2u * kGroups * kBufferBytes;
     static constexpr uint32_t kLdsBytes = kTableAt + kKvTableEntries * 4u;
     static_assert(kLdsBytes <= 160 * 1024, "LDS of a compute unit");
+    static_assert(kTile <= 64 || (kTile == 128 && kCopies % 2 == 0 && 64 % (RW * kRowsPerCopy) == 0), "half of the copies to each 64 positions");
+    static_assert(kBufferBytes % 256 == 0 && kTileBytes % 256 == 0, "rows start where the bits of their pieces are zero");
     static_assert(kChunkWaves * (W / 32) * 1024 * 4 <= kTableAt && kChunkWaves * 128 * 4 <= kKvTableEntries * 4,
                   "the waves' sums meet where the tiles and the table were");
     // Piece p of position r of a tile lies in slot p ^ swizzle(r): the 32 positions of a K operand read and the
@@ -394,7 +403,7 @@ __global__ __launch_bounds__(kChunkThreads, 2) void kv_chunk_kernel(const KvArgs
     constexpr int kGroups = Shape::kGroups, kRows = Shape::kRows, kTile = Shape::kTile, kCopies = Shape::kCopies;
     constexpr int kKeyChunks = W / 16, kDimTiles = W / 32, kQueryPieces = S::kQueryPieces, kWeightPieces = S::kWeightPieces;
     constexpr int U = S::kBlocksPerStep < kTile / 32 ? S::kBlocksPerStep : kTile / 32;
-    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    extern __shared__ __attribute__((aligned(256))) uint8_t lds[];
     uint32_t* rows_of_block = reinterpret_cast<uint32_t*>(lds + Shape::kTableAt);
 
     // Workgroups of one (slot, kv head) share their K and V in an XCD's L2: the pair runs fastest over the
@@ -456,15 +465,36 @@ __global__ __launch_bounds__(kChunkThreads, 2) void kv_chunk_kernel(const KvArgs
     Raw k_raw[S::kScaled ? kCopies : 1], v_raw[S::kScaled ? kCopies : 1];
     float k_scale[S::kScaled ? kCopies : 1], v_scale[S::kScaled ? kCopies : 1];
     const auto tile_row = [&](int i) { return static_cast<uint32_t>((i * RW + row_wave) * Shape::kRowsPerCopy + lane / Shape::kPieces); };
-    const auto fetch = [&](uint32_t tile_begin, uint32_t buffer) {
+    // Slab rows of a tile's positions, found a tile ahead, a lane to a position.
+    constexpr int kPlaces = (kTile + 63) / 64;
+    uint32_t place[kPlaces];
+    const auto locate = [&](uint32_t tile_begin) {
+        uint32_t block[kPlaces], within[kPlaces];
+        // positions past the end read the last row again; their weights are zero
+        const auto position = [&](int i) { return min(tile_begin + 64 * i + lane, my_end - 1); };
+#pragma unroll
+        for (int i = 0; i < kPlaces; i++) {
+            if (a.block_shift >= 0) {
+                block[i] = position(i) >> a.block_shift;
+                within[i] = position(i) & (a.block_size - 1);
+            } else {
+                block[i] = position(i) / a.block_size;
+                within[i] = position(i) - block[i] * a.block_size;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < kPlaces; i++) {
+            const uint32_t base = rows_of_block[min(block[i] - first_block, kKvTableEntries - 1u)];
+            const uint32_t at = min(base + within[i], a.max_tokens - 1);
+            place[i] = base == kNoBlock ? 0u : at;
+        }
+    };
+    const auto fetch = [&](uint32_t buffer) {
 #pragma unroll
         for (int i = 0; i < kCopies; i++) {
-            // positions past the end read the last row again; their weights are zero
-            const uint32_t r = tile_row(i), position = min(tile_begin + r, my_end - 1);
-            const uint32_t piece = (lane % Shape::kPieces) ^ Shape::swizzle(r);
-            const uint32_t base = rows_of_block[min(block_of(a, position) - first_block, kKvTableEntries - 1u)];
-            const uint32_t at = base == kNoBlock ? 0u : min(base + within_block(a, position), a.max_tokens - 1);
-            const uint64_t from = at * slab_row + piece * (8 * S::kBytes);
+            const uint32_t r = tile_row(i), piece = (lane % Shape::kPieces) ^ Shape::swizzle(r);
+            const uint32_t at = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute((r & 63u) << 2, place[i * kPlaces / kCopies]));
+            const uint64_t from = static_cast<uint64_t>(at) * slab_row + piece * (8 * S::kBytes);
             if constexpr (S::kScaled) {
                 k_raw[i] = *reinterpret_cast<const Raw*>(k_base + from);
                 v_raw[i] = *reinterpret_cast<const Raw*>(v_base + from);
@@ -504,7 +534,11 @@ __global__ __launch_bounds__(kChunkThreads, 2) void kv_chunk_kernel(const KvArgs
     __syncthreads();  // the table is in LDS
     const uint32_t rounds = (my_end - my_begin + kRound - 1) / kRound;
     uint32_t tile_begin = my_begin + group * kTile;
-    if (rounds != 0) fetch(tile_begin, 0);
+    if (rounds != 0) {
+        locate(tile_begin);
+        fetch(0);
+        locate(tile_begin + kRound);
+    }
 
     // q in pieces, scaled so that the row's largest component lies in [2^9, 2^10); the score's unit undoes it.
     typename KE::v8 q[kQueryPieces][kKeyChunks];
@@ -552,12 +586,16 @@ __global__ __launch_bounds__(kChunkThreads, 2) void kv_chunk_kernel(const KvArgs
     for (int t = 0; t < kDimTiles; t++) o[t] = zero;
 
     // K operand of a 32-position block: position in_half, pieces 2c + half. V operand: positions
-    // 16c + 8a + 4 half + (0..3), of which this lane's address names row (lane & 15) / 4 and four of sixteen columns.
-    const uint32_t key_row = in_half * Shape::kRowBytes, key_swizzle = Shape::swizzle(in_half);
+    // 16c + 8h + 4 half + (0..3), of which this lane's address names row (lane & 15) / 4 and four of sixteen columns.
+    // A row's pieces fill the bits of the address that the swizzle changes, so c, h and the column tile come in with one
+    // exclusive or each, and no lane keeps more than these two offsets.
+    const uint32_t key_at = in_half * Shape::kRowBytes + ((half ^ Shape::swizzle(in_half)) << 4);
     const uint32_t value_row = 4 * half + ((lane & 15) >> 2), value_piece = ((lane >> 4) & 1) * 2 + ((lane & 3) >> 1);
-    const auto contract = [&](const uint8_t* buffer, uint32_t tile) {
-        const uint8_t* values = buffer + Shape::kTileBytes;
-        const float* scales = reinterpret_cast<const float*>(buffer + 2 * Shape::kTileBytes);
+    const uint32_t value_at = Shape::kTileBytes + value_row * Shape::kRowBytes +
+                              ((value_piece ^ Shape::swizzle(value_row)) << 4) + (lane & 1) * 8;
+    const auto contract = [&](uint32_t buffer, uint32_t tile) {
+        const uint32_t keys = buffer + key_at, values = buffer + value_at;
+        const float* scales = reinterpret_cast<const float*>(lds + buffer + 2 * Shape::kTileBytes);
 #pragma unroll
         for (int b = 0; b < kTile / 32; b += U) {
             const uint32_t step = tile + 32 * b;
@@ -570,8 +608,7 @@ __global__ __launch_bounds__(kChunkThreads, 2) void kv_chunk_kernel(const KvArgs
                     typename KE::v8 key[4];
 #pragma unroll
                     for (int c = 0; c < 4; c++)
-                        key[c] = *reinterpret_cast<const typename KE::v8*>(buffer + 32 * (b + u) * Shape::kRowBytes + key_row +
-                                                                           (((2 * (first + c) + half) ^ key_swizzle) << 4));
+                        key[c] = *reinterpret_cast<const typename KE::v8*>(lds + (keys ^ ((first + c) << 5)) + 32 * (b + u) * Shape::kRowBytes);
                     v16f sum = zero;
 #pragma unroll
                     for (int p = kQueryPieces - 1; p >= 0; p--)
@@ -606,8 +643,9 @@ __global__ __launch_bounds__(kChunkThreads, 2) void kv_chunk_kernel(const KvArgs
 #pragma unroll
                 for (int r = 0; r < 16; r++) top = fmaxf(top, score[u][r]);
             top = fmaxf(top, other_half(top, lane));
+            // The reference point of a row's exponents may lie up to kSlack below its maximum.
             const float next = fmaxf(m, top * unit);
-            if (__builtin_amdgcn_ballot_w64(next != m) != 0) {
+            if (__builtin_amdgcn_ballot_w64(next > m + kSlack) != 0) {
                 const float keep = __builtin_amdgcn_exp2f(m - next);
                 m = next;
                 l *= keep;
@@ -654,11 +692,8 @@ __global__ __launch_bounds__(kChunkThreads, 2) void kv_chunk_kernel(const KvArgs
 #pragma unroll
                 for (int c = 0; c < 2 * U; c++)
 #pragma unroll
-                    for (int h = 0; h < 2; h++) {
-                        const uint32_t r = 32 * b + 16 * c + 8 * h + value_row;
-                        value[c].raw[h] = read_transposed(values + r * Shape::kRowBytes +
-                                                          (((4 * t + value_piece) ^ Shape::swizzle(r)) << 4) + (lane & 1) * 8);
-                    }
+                    for (int h = 0; h < 2; h++)
+                        value[c].raw[h] = read_transposed(lds + (values ^ (t * 64 + h * 32)) + (32 * b + 16 * c + 8 * h) * Shape::kRowBytes);
                 v16f sum = zero;
 #pragma unroll
                 for (int p = kWeightPieces - 1; p >= 0; p--)
@@ -675,8 +710,11 @@ __global__ __launch_bounds__(kChunkThreads, 2) void kv_chunk_kernel(const KvArgs
         __syncthreads();
         for (uint32_t round = 0; round < rounds; round++, tile_begin += kRound) {
             const bool more = round + 1 < rounds;
-            if (more) fetch(tile_begin + kRound, (round + 1) & 1);
-            if (has_rows && tile_begin < my_end) contract(buffers + (round & 1) * Shape::kBufferBytes, tile_begin);
+            if (more) {
+                fetch((round + 1) & 1);
+                locate(tile_begin + 2 * kRound);
+            }
+            if (has_rows && tile_begin < my_end) contract((2u * group + (round & 1)) * Shape::kBufferBytes, tile_begin);
             if (more) deposit((round + 1) & 1);
             __syncthreads();
         }
