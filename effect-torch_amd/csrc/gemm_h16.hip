@@ -2,7 +2,7 @@
 // matrix cores: weights times their sub-block scales are exact small integers in half floats, activations two half floats each.
 //
 //   y[m, n] = sum_s  unit[m, s] * d[n, s] * sum_g sum_i (sc_g[n] * nib[n, g, i]) * X[m, g, i]
-//           - sum_s  unit[m, s] * dmin[n, s] * sum_g m_g[n] * xsum[m, g]
+//           - sum_s  dmin[n, s] * sum_g m_g[n] * xsum[m, g]
 // s = 256-column stage (one Q4_K super-block), g = its eight 32-column sub-blocks.
 //
 // Activations are scaled per vector and stage, X = x * (2^23 - 1) / max|x|, and split into X = 4096 * hi + lo with
@@ -345,56 +345,70 @@ __global__ __launch_bounds__(kThreads) void gemm_h16_kernel(
             continue;
         }
 
+        // Everything the stage needs of LDS is asked for first: a wave that reads each operand where it uses it waits for
+        // LDS half a dozen times per stage, and the two consumers of a SIMD wait at the same time. With the nibbles' eight
+        // instructions less per sub-block (packed_nibbles_times), Q4_K, whole calls in us: 128256 x 4096 with 32 vectors 134.5 ->
+        // 129, 14336 x 4096 with 16 and 64 26.3 -> 25.5 and 38.8 -> 37.0, with 32 the same (29.1; its copies take that long).
+        // (The other three codecs read where they use: reading first 1 to 3 % slower there.)
         const uint4 header = *reinterpret_cast<const uint4*>(row_in_slot);
-        const float d_scaled = kPlaneRatio * half_bits_to_float(header.x & 0xffffu);
-        const float dmin_block = half_bits_to_float(header.x >> 16);
+        uint4 raw[NB / 2];  // the 32 bytes of a pair of sub-blocks: low and high nibbles; this lane half's sixteen columns
+#pragma unroll
+        for (int j = 0; j < NB / 2; j++) raw[j] = *reinterpret_cast<const uint4*>(row_in_slot + kQuantsAt + 16u * b_base + 32u * j + 16u * half);
         uint4 fifth = make_uint4(0u, 0u, 0u, 0u);  // Q5_K: qh of this lane half's sixteen columns
         if constexpr (CODEC == kQ5_K) fifth = *reinterpret_cast<const uint4*>(row_in_slot + 16u + 16u * half);
-
-        // min term: acc_min[m, n] += sum_g (dmin * m_g)[n] * (unit * xsum[g])[m]; K = 2 per MFMA, lane half h
-        // supplies sub-block 2j + h.
-        const float vector_unit = *reinterpret_cast<const float*>(slot + kUnitAt + in_half * 4u);
+        constexpr int kAhead = NB < 2 ? NB : 2;  // sub-blocks whose activations are read ahead
+        Operands<NARROW> x[kAhead];
 #pragma unroll
-        for (int jj = 0; jj < NB / 2; jj++) {
-            const uint32_t g = b_base + 2u * jj + half;
-            uint32_t sc, mn;
-            q4k_scale_min(header, g, sc, mn);
-            const float a_operand = vector_unit * *reinterpret_cast<const float*>(slot + kSumsAt + g * 128u + in_half * 4u);
-            acc_min = __builtin_amdgcn_mfma_f32_32x32x2f32(a_operand, dmin_block * static_cast<float>(mn), acc_min,
-                                                           0, 0, 0);
-        }
+        for (int bb = 0; bb < kAhead; bb++) x[bb].load(slot, b_base + bb, half, in_half);
+        float sums[NB / 2];
+#pragma unroll
+        for (int j = 0; j < NB / 2; j++)
+            sums[j] = *reinterpret_cast<const float*>(slot + kSumsAt + (b_base + 2u * j + half) * 128u + in_half * 4u);
+        float4 units[R / 4];
+#pragma unroll
+        for (int j = 0; j < R / 4; j++) units[j] = *reinterpret_cast<const float4*>(slot + kUnitAt + (8u * j + 4u * half) * 4u);
+        __builtin_amdgcn_sched_barrier(0);
+
+        // Scales and minima of the wave's sub-blocks, a byte each from b_base on (q4k_scale_min for four at once; b_base is
+        // uniform, and a select of bits instead of a branch on it).
+        const uint32_t upper = b_base >= 4u ? 0xffffffffu : 0u, down = (b_base & 3u) * 8u;
+        const uint32_t scales = ((((header.w & 0x0f0f0f0fu) | ((header.y >> 2) & 0x30303030u)) & upper) |
+                                 ((header.y & 0x3f3f3f3fu) & ~upper)) >> down;
+        const uint32_t minima = ((((header.w >> 4) & 0x0f0f0f0fu) | ((header.z >> 2) & 0x30303030u)) & upper |
+                                 ((header.z & 0x3f3f3f3fu) & ~upper)) >> (down + 8u * half);
+        const float d_scaled = kPlaneRatio * half_bits_to_float(header.x & 0xffffu);
+        const float dmin_block = half_bits_to_float(header.x >> 16);
 
         // The stage's products: both halves of X against sc_g * nib, summed over this wave's sub-blocks.
         // The weight operands of sub-block bb + 1 are prepared (VALU) between the MFMAs of sub-block bb.
         const auto prepare = [&](int bb, v8h& b0, v8h& b1) {
-            const uint32_t b = b_base + bb;
-            // sub-block 2p + side: low (side 0) or high (side 1) nibbles of the 32 bytes of pair p; this
-            // lane half takes bytes 16 * half .. + 16 = columns 16 * half .. + 16 of the sub-block
-            const uint4 raw = *reinterpret_cast<const uint4*>(row_in_slot + kQuantsAt + 32u * (b >> 1) + 16u * half);
-            const uint32_t shift = (b & 1u) * 4u;
-            uint32_t w0 = (raw.x >> shift) & 0x0f0f0f0fu, w1 = (raw.y >> shift) & 0x0f0f0f0fu,
-                     w2 = (raw.z >> shift) & 0x0f0f0f0fu, w3 = (raw.w >> shift) & 0x0f0f0f0fu;
-            if constexpr (CODEC == kQ5_K) {  // the fifth bit of column c of sub-block b: bit b of qh[c]
-                w0 |= ((fifth.x >> b) & 0x01010101u) << 4;
-                w1 |= ((fifth.y >> b) & 0x01010101u) << 4;
-                w2 |= ((fifth.z >> b) & 0x01010101u) << 4;
-                w3 |= ((fifth.w >> b) & 0x01010101u) << 4;
-            }
-            uint32_t sc, mn;
-            q4k_scale_min(header, b, sc, mn);
-            const _Float16 sc_h = static_cast<_Float16>(static_cast<float>(sc));
+            // sub-block 2p + side: low (side 0) or high (side 1) nibbles of the 32 bytes of pair p; b_base is even
+            const uint4& from = raw[bb / 2];
+            const _Float16 sc_h = static_cast<_Float16>(static_cast<float>((scales >> (8 * bb)) & 0xffu));
             const v2h sc2 = {sc_h, sc_h};
-            b0 = nibbles_times(w0, w1, sc2);
-            b1 = nibbles_times(w2, w3, sc2);
+            if constexpr (CODEC == kQ5_K) {  // the fifth bit of column c of sub-block b: bit b of qh[c]
+                const uint32_t b = b_base + bb, shift = (bb & 1) * 4u;
+                const uint32_t w0 = ((from.x >> shift) & 0x0f0f0f0fu) | (((fifth.x >> b) & 0x01010101u) << 4),
+                               w1 = ((from.y >> shift) & 0x0f0f0f0fu) | (((fifth.y >> b) & 0x01010101u) << 4),
+                               w2 = ((from.z >> shift) & 0x0f0f0f0fu) | (((fifth.z >> b) & 0x01010101u) << 4),
+                               w3 = ((from.w >> shift) & 0x0f0f0f0fu) | (((fifth.w >> b) & 0x01010101u) << 4);
+                b0 = nibbles_times(w0, w1, sc2);
+                b1 = nibbles_times(w2, w3, sc2);
+            } else if (bb & 1) {
+                b0 = packed_nibbles_times<true>(from.x, from.y, sc2);
+                b1 = packed_nibbles_times<true>(from.z, from.w, sc2);
+            } else {
+                b0 = packed_nibbles_times<false>(from.x, from.y, sc2);
+                b1 = packed_nibbles_times<false>(from.z, from.w, sc2);
+            }
         };
         v16f p = zero;
         v8h b0, b1;
         prepare(0, b0, b1);
 #pragma unroll
         for (int bb = 0; bb < NB; bb++) {
-            Operands<NARROW> x;
-            x.load(slot, b_base + bb, half, in_half);
-            p = x.contract(b0, b1, p);
+            p = x[bb % kAhead].contract(b0, b1, p);
+            if (bb + kAhead < NB) x[bb % kAhead].load(slot, b_base + bb + kAhead, half, in_half);
             if (bb + 1 < NB) {
                 v8h n0, n1;
                 prepare(bb + 1, n0, n1);
@@ -404,22 +418,24 @@ __global__ __launch_bounds__(kThreads) void gemm_h16_kernel(
 #pragma unroll
                 for (int i = 0; i < kMatrix; i++) {
                     __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);             // one MFMA
-                    __builtin_amdgcn_sched_group_barrier(0x002, 48 / kMatrix, 0);  // its share of the VALU work
+                    __builtin_amdgcn_sched_group_barrier(0x002, 32 / kMatrix, 0);  // its share of the VALU work
                 }
             }
         }
-        // unit[m] * d[n] for the sixteen vectors this lane accumulates, m = 8 * (r / 4) + 4 * half + r % 4:
-        // four 16-byte LDS reads that every lane of a half shares, sixteen multiplications. (The same
-        // products as a rank-1 v_mfma_f32_32x32x2f32 in the result layout cost 64 cycles of the matrix
-        // pipe, and matrix and VALU instructions do not run side by side on this device.)
+        // min term: acc_min[m, n] += sum_g (dmin * m_g)[n] * xsum[m, g]; K = 2 per MFMA, lane half h
+        // supplies sub-block 2j + h. Behind the products: these take twice the time and cover the wait for the last of them.
+#pragma unroll
+        for (int j = 0; j < NB / 2; j++)
+            acc_min = __builtin_amdgcn_mfma_f32_32x32x2f32(sums[j], dmin_block * static_cast<float>((minima >> (16 * j)) & 0xffu), acc_min, 0, 0, 0);
+        // unit[m] * d[n] for the sixteen vectors this lane accumulates, m = 8 * (r / 4) + 4 * half + r % 4
+        // (as a rank-1 v_mfma_f32_32x32x2f32 in the result layout: 64 cycles of the matrix pipe instead of 16 multiplications)
         float sd[R];
 #pragma unroll
         for (int j = 0; j < R / 4; j++) {
-            const float4 units = *reinterpret_cast<const float4*>(slot + kUnitAt + (8u * j + 4u * half) * 4u);
-            sd[4 * j + 0] = units.x * d_scaled;
-            sd[4 * j + 1] = units.y * d_scaled;
-            sd[4 * j + 2] = units.z * d_scaled;
-            sd[4 * j + 3] = units.w * d_scaled;
+            sd[4 * j + 0] = units[j].x * d_scaled;
+            sd[4 * j + 1] = units[j].y * d_scaled;
+            sd[4 * j + 2] = units[j].z * d_scaled;
+            sd[4 * j + 3] = units[j].w * d_scaled;
         }
 #pragma unroll
         for (int r = 0; r < R; r++) acc[r] = fmaf(stage_sum<NARROW>(p, r), sd[r], acc[r]);

@@ -9,18 +9,18 @@
 // one wave four do), so what counts is how evenly they lie between them: the next sub-block's operands are made between
 // this one's matrix instructions, and a stage's sums are folded into the accumulators tile by tile between the next tile's.
 // The minima were f32 matrix instructions (16 of 64 cycles per stage, a fifth of the pipe's time); now the sums of a
-// sub-block, whole numbers, are cut into three bfloat16 pieces once per workgroup, and the products are exact.
+// sub-block, in units of the vector whole numbers of up to 28 bits, are cut into three bfloat16 pieces once per workgroup, and the products are exact.
 // Both steps, 14336 x 4096 with 1000 vectors: 289 -> 253 us, clocks of busy compute units 122.5 -> 99.6 million, of which matrix
-// instructions 60 -> 63 %. The clock falls from 2.02 to 1.93 GHz on the way: a loop of these instructions alone holds 1.75 GHz on
+// instructions 60 -> 63 %; the nibbles' eight instructions less per sub-block (packed_nibbles_times) 5 % more. The clock falls from 2.02 to 1.93 GHz on the way: a loop of these instructions alone holds 1.75 GHz on
 // random operands (2.1 on zeros). Without any copies 7 % less; 448 workgroups on 256 compute units leave an eighth of them idle.
 // Every wave unpacks its own weight rows from the packed bytes in LDS. There are no loader waves (a third wave per SIMD
 // would leave 168 registers each): the waves ask for the next sub-blocks' activations and the next stage's weights
 // themselves, through inline assembly, because any LDS read next to a copy that the compiler can see waits for it.
 //
-// Whole calls (us, gemm_h16_kernel / this before / this): 14336 x 4096 with 1000 vectors Q4_K 420 / 284 / 262 (448 TFLOP/s), Q5_K
-// 453 / 292 / 270, Q6_K 724 / 461 / 429, Q3_K 415 / 259 / 246, Q2_K 512 / 418 / 397; Q4_K 4096 x 14336 with 1000 396 / 280 / 261,
+// Whole calls (us, gemm_h16_kernel / this before / this): 14336 x 4096 with 1000 vectors Q4_K 420 / 289 / 259 (454 TFLOP/s), Q5_K
+// 453 / 296 / 265, Q6_K 724 / 481 / 438, Q3_K 415 / 259 / 246, Q2_K 512 / 429 / 398; Q4_K 4096 x 14336 with 1000 396 / 274 / 256,
 // 14336 x 4096 with 256 115 / 93 / 90.
-// Relative error against 64 bits there (2-norm, 1e-7): Q4_K 1.75 / 1.71, Q6_K 1.66 / 1.63, Q2_K 1.84 / 1.76: one chain of
+// Relative error against 64 bits there (2-norm, 1e-7): Q4_K 1.75 / 1.69 / 1.66, Q6_K 1.66 / 1.63 / 1.63, Q2_K 1.84 / 1.76 / 1.76: one chain of
 // sums over the stage's eight sub-blocks instead of two or four, from activations that are rounded less (quantize_halves.h).
 #include <hip/hip_runtime.h>
 
@@ -38,16 +38,13 @@ constexpr int kTiles = kGemmWideVectors / 32;        // activation tiles per wor
 constexpr int kSlots = 4;                            // sub-blocks of activations in LDS: two landed, two on their way
 constexpr uint32_t kSlotBytes = kTiles * 2 * 2048u;  // per tile and plane four 8-column parts of 512 bytes
 constexpr int kCutAt = 3;                            // the sub-block in which the stage's sums are cut: they have landed by then
-typedef short v8s __attribute__((ext_vector_type(8)));
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 constexpr int kActivationCopies = 2;                 // per wave and sub-block: one plane of one tile
 static_assert(kTiles * 2 == kWaves && kStageBlocks % kSlots == 0, "a wave copies one plane of one tile; slots start anew per stage");
 
 template <int CODEC>
 struct Wide {
     static constexpr bool kMinima = CODEC == kQ4_K || CODEC == kQ5_K;  // a minimum per sub-block, against xsum
-    // weight operands per sixteen columns: Q6_K splits its scale, Q2_K contracts its minima
-    static constexpr int kParts = CODEC == kQ6_K || CODEC == kQ2_K ? 2 : 1;
+    static constexpr int kParts = weight_parts(CODEC);
     static constexpr int kMT = kParts == 2 ? 2 : 4;  // 32-vector tiles per wave, against 32 rows
     static constexpr int kWavesM = kTiles / kMT, kWavesN = kWaves / kWavesM;
     static constexpr uint32_t kRows = 32u * kWavesN;
@@ -65,127 +62,6 @@ struct Wide {
     // copies that a wave asks for in front of the activations during sub-block b: the stage's tables, next weights
     static constexpr int ahead(int b, bool last) { return (b == 0 ? 1 : 0) + (!last && b < kRounds ? 1 : 0); }
 };
-
-// 1 KiB from `base` + a byte offset per lane to LDS address `to` + 16 bytes per lane.
-__device__ __forceinline__ void copy_to_lds(const uint8_t* base, uint32_t lane_offset, uint32_t to) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                 :
-                 : "s"(__builtin_amdgcn_readfirstlane(to)), "v"(lane_offset), "s"(base)
-                 : "memory");  // m0 is a reserved register: nothing else in this file sets it
-}
-
-// The packed bytes of one lane's columns 32 b + 16 half .. + 16 of a row, as they come out of LDS.
-struct Raw {
-    uint4 low, high;
-    uint32_t scale, scale_top;
-};
-// What all of a row's sub-blocks share: d, dmin and the scales (Q4_K, Q5_K); the fifth (Q5_K) or top (Q3_K) bits.
-struct Shared {
-    uint4 header, bits;
-};
-template <int CODEC>
-__device__ __forceinline__ Shared fetch_shared(const uint8_t* row, uint32_t half) {
-    Shared s = {};
-    if constexpr (CODEC == kQ4_K || CODEC == kQ5_K) s.header = *reinterpret_cast<const uint4*>(row);
-    if constexpr (CODEC == kQ5_K) s.bits = *reinterpret_cast<const uint4*>(row + 16u + 16u * half);
-    if constexpr (CODEC == kQ3_K) s.bits = *reinterpret_cast<const uint4*>(row + 16u * half);
-    return s;
-}
-template <int CODEC>
-__device__ __forceinline__ Raw fetch(const uint8_t* row, int b, uint32_t half) {
-    const uint32_t n = b >> 2, t = b & 3;
-    Raw r = {};
-    if constexpr (CODEC == kQ4_K || CODEC == kQ5_K) {
-        r.low = *reinterpret_cast<const uint4*>(row + HalfStage<CODEC>::kQuantsAt + 32u * (b >> 1) + 16u * half);
-    } else if constexpr (CODEC == kQ6_K) {
-        r.low = *reinterpret_cast<const uint4*>(row + 64u * n + 32u * (t & 1u) + 16u * half);
-        r.high = *reinterpret_cast<const uint4*>(row + 128u + 32u * n + 16u * half);
-        r.scale = row[192u + 8u * n + 2u * t + half];
-    } else if constexpr (CODEC == kQ3_K) {
-        r.low = *reinterpret_cast<const uint4*>(row + 32u + 32u * n + 16u * half);
-        r.scale = row[HalfStage<CODEC>::in_tail(96u) + 2u * t + half];
-        r.scale_top = row[HalfStage<CODEC>::in_tail(104u) + 2u * (t & 1u) + half];
-    } else {
-        r.low = *reinterpret_cast<const uint4*>(row + 16u + 32u * n + 16u * half);
-        r.scale = row[2u * b + half];
-    }
-    return r;
-}
-__device__ __forceinline__ v2h twice(int value) {
-    const _Float16 h = static_cast<_Float16>(static_cast<float>(value));
-    return v2h{h, h};
-}
-// The weight operands of those columns, eight by eight: gemm_h16_kernel's values.
-template <int CODEC>
-__device__ __forceinline__ void operands(const Raw& raw, const Shared& shared, int b, v8h out[2][Wide<CODEC>::kParts]) {
-    const uint32_t n = b >> 2, t = b & 3;
-    const uint32_t low[4] = {raw.low.x, raw.low.y, raw.low.z, raw.low.w}, high[4] = {raw.high.x, raw.high.y, raw.high.z, raw.high.w};
-    const uint32_t bits[4] = {shared.bits.x, shared.bits.y, shared.bits.z, shared.bits.w};
-    uint32_t w[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        if constexpr (CODEC == kQ4_K || CODEC == kQ5_K) {
-            w[i] = (low[i] >> ((b & 1) * 4)) & 0x0f0f0f0fu;
-            if constexpr (CODEC == kQ5_K) w[i] |= ((bits[i] >> b) & 0x01010101u) << 4;
-        } else if constexpr (CODEC == kQ6_K) {
-            w[i] = ((low[i] >> ((t >> 1) * 4u)) & 0x0f0f0f0fu) | (((high[i] >> (2u * t)) & 0x03030303u) << 4);
-        } else {
-            w[i] = (low[i] >> (2u * t)) & 0x03030303u;
-            if constexpr (CODEC == kQ3_K) w[i] |= ((bits[i] >> (4u * n + t)) & 0x01010101u) << 2;
-        }
-    }
-    if constexpr (CODEC == kQ4_K || CODEC == kQ5_K) {
-        uint32_t sc, mn;
-        q4k_scale_min(shared.header, b, sc, mn);
-        const v2h scale = twice(sc);
-        out[0][0] = nibbles_times(w[0], w[1], scale);
-        out[1][0] = nibbles_times(w[2], w[3], scale);
-    } else if constexpr (CODEC == kQ6_K) {
-        const int sc = static_cast<int8_t>(raw.scale);
-        const v2h scale_low = twice(sc & 15), scale_high = twice(sc >> 4);
-        out[0][0] = nibbles_times<32>(w[0], w[1], scale_low);
-        out[1][0] = nibbles_times<32>(w[2], w[3], scale_low);
-        out[0][1] = nibbles_times<32>(w[0], w[1], scale_high);
-        out[1][1] = nibbles_times<32>(w[2], w[3], scale_high);
-    } else if constexpr (CODEC == kQ3_K) {
-        const int sc = static_cast<int>(((raw.scale >> (4u * n)) & 15u) |
-                                        (((raw.scale_top >> (2u * (2u * n + (t >> 1)))) & 3u) << 4)) - 32;
-        const v2h scale = twice(sc);
-        out[0][0] = bytes_minus_times<4>(w[0], w[1], scale);
-        out[1][0] = bytes_minus_times<4>(w[2], w[3], scale);
-    } else {
-        const v2h scale = twice(raw.scale & 15u), m = twice(raw.scale >> 4);
-        out[0][0] = nibbles_times(w[0], w[1], scale);
-        out[1][0] = nibbles_times(w[2], w[3], scale);
-        out[0][1] = out[1][1] = v8h{m.x, m.x, m.x, m.x, m.x, m.x, m.x, m.x};
-    }
-}
-
-// f32 bits as three bfloat16 numbers that add up to it, eight significant bits each: the top halves of `x`, of
-// what is left of it, and of what is left then (nothing is lost above 2^-110, and S is a whole number).
-struct Pieces {
-    uint32_t high, mid, low;  // in the upper sixteen bits
-};
-__device__ __forceinline__ Pieces cut(float x) {
-    Pieces p;
-    p.high = __float_as_uint(x) & 0xffff0000u;
-    const float rest = x - __uint_as_float(p.high);
-    p.mid = __float_as_uint(rest) & 0xffff0000u;
-    p.low = __float_as_uint(rest - __uint_as_float(p.mid));
-    return p;
-}
-__device__ __forceinline__ v8bf as_bf16(const v8s& bits) { return __builtin_bit_cast(v8bf, bits); }
-// The eight minima of this lane's row, against the high (lane half 0) and middle pieces, and against the low ones
-// (half 0 alone: the operand's other eight columns are zero).
-__device__ __forceinline__ void minimum_operands(const uint4& header, uint32_t half, v8s out[2]) {
-#pragma unroll
-    for (uint32_t g = 0; g < kStageBlocks; g++) {
-        uint32_t sc, mn;
-        q4k_scale_min(header, g, sc, mn);
-        out[0][g] = static_cast<short>(__float_as_uint(static_cast<float>(mn)) >> 16);  // at most 63: exact
-    }
-    out[1] = half == 0 ? out[0] : v8s{0, 0, 0, 0, 0, 0, 0, 0};
-}
 
 template <int CODEC>
 __global__ __launch_bounds__(64 * kWaves, 2) void gemm_h16_wide_kernel(const Group group, const uint8_t* __restrict__ tiles,
@@ -258,12 +134,14 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_h16_wide_kernel(const Gro
     };
 
     // Between the barriers of sub-blocks kCutAt and kCutAt + 1 every thread reads and cuts the sums of two sub-blocks of one
-    // vector, behind the second one the pieces take the sums' place; they are read in the last sub-block.
+    // vector, in units of the vector (pieces of numbers around 10^-35 would not be normal), behind the second one the pieces take the sums' place; they are read in the last sub-block.
     uint32_t piece[3];
     const uint32_t cut_vector = threadIdx.x & 31u, cut_group = ((threadIdx.x >> 5) & 3u) * 2u;
     const auto cut_sums = [&] {
         const float* sums = reinterpret_cast<const float*>(lds + W::kSumsAt + (wave >> 1) * 1024u) + cut_group * 32u + cut_vector;
-        const Pieces a = cut(sums[0]), b = cut(sums[32]);
+        const float unit = *reinterpret_cast<const float*>(lds + W::kUnitsAt + (wave >> 1) * 128u + cut_vector * 4u);
+        const auto whole = [&](float sum) { return unit != 0.f ? sum / unit : 0.f; };
+        const Pieces a = cut(whole(sums[0])), b = cut(whole(sums[32]));
         piece[0] = __builtin_amdgcn_perm(b.high, a.high, 0x07060302u);
         piece[1] = __builtin_amdgcn_perm(b.mid, a.mid, 0x07060302u);
         piece[2] = __builtin_amdgcn_perm(b.low, a.low, 0x07060302u);
@@ -364,7 +242,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_h16_wide_kernel(const Gro
                 d = kPlaneRatio * half_bits_to_float(dd & 0xffffu), dmin = half_bits_to_float(dd >> 16);
                 if constexpr (W::kMinima) minimum_operands(shared.header, half, minima);
             }
-            // acc += unit[m] * (p * d[n] - (sum_g S[m, g] * m_g[n]) * dmin[n]); vectors of a lane: 8 (r / 4) + 4 half + r % 4
+            // acc += unit[m] * (p * d[n] - (sum_g xsum[m, g] / unit[m] * m_g[n]) * dmin[n]); vectors of a lane: 8 (r / 4) + 4 half + r % 4
             v16f below;
             const auto units_of = [&](int m, int j) {
                 return *reinterpret_cast<const float4*>(lds + W::kUnitsAt + (wave_m * MT + m) * 128u + (8u * j + 4u * half) * 4u);

@@ -106,9 +106,10 @@ hipError_t quantize_activations(const float* x, uint64_t x_row_stride, uint64_t 
 // limbs = 3: 24-bit fixed point in three balanced signed bytes, scale = max|x| / (127 * 65536).
 // limbs = 2 is the layout of gemm_h16: x in units of max|x| / (2^23 - 1) per vector and 256-column stage, as a whole
 // multiple of 4096 and a rest, each a half float (quantize_halves.h):
-//   half l (0: low / 4096, 1: high), 8-column part c (0..31), vector m: 8 half floats at  l*16384 + c*512 + m*16
+//   half l (0: low / 4096, 1: high), 8-column part c (0..31), vector m: 8 half floats at  l*16384 + c*512 + m*16, the
+//   columns of each four in the order 0, 2, 1, 3
 //   unit[m] f32 (max|x| / (2^23 - 1)) at  32768 + m*4
-//   xsum[sub-block g (0..7)][m] f32, in units of unit[m], at  32768 + 128 + g*128 + m*4
+//   xsum[sub-block g (0..7)][m] f32 at  32768 + 128 + g*128 + m*4
 // and padding up to 34 KiB.
 constexpr uint32_t tile_blob_bytes(int limbs) { return limbs == 1 ? 12288u : limbs == 2 ? 34816u : 28672u; }
 constexpr uint64_t tile_workspace_bytes(int limbs, uint64_t vectors, uint64_t columns) {

@@ -26,7 +26,7 @@ __device__ __forceinline__ int dpp_i32(int v) {
 // of the stage's largest value) and by less wherever lo is small. X is x / unit to within one rounding: the quotient by a multiplication with 1 / unit, corrected
 // by its remainder. (A whole number lo from the product alone: relative error of a contraction with 20 vectors x 4096
 // columns, 1e-7, before / now Q5_K 1.46 / 1.20, Q6_K 1.58 / 1.37, Q2_K 1.64 / 1.43; no slower.) The two products of a weight with these operands add
-// up to X * w / 4096 in one accumulator. xsum[g] = sum of X over sub-block g, rounded to an f32.
+// up to X * w / 4096 in one accumulator. xsum[g] = unit * (sum of X over sub-block g).
 // One wave per (vector, stage): lane `quad` holds columns 4 quad .. 4 quad + 3 of the stage. Blob
 // layout: see tile_blob_bytes() in kernels.h.
 __device__ __forceinline__ void quantize_halves_store(const float4& in, uint32_t v, uint32_t stage, uint32_t quad,
@@ -62,8 +62,9 @@ __device__ __forceinline__ void quantize_halves_store(const float4& in, uint32_t
         const float hi = rintf(r * (1.0f / 4096.0f)), lo = fmaf(-4096.0f, hi, r);  // lo is exact
         sum_hi += hi;  // exact: whole numbers up to 2^16
         sum_lo += lo;
-        low.h[i] = static_cast<_Float16>(lo * (1.0f / 4096.0f));
-        high.h[i] = static_cast<_Float16>(hi);
+        constexpr int kPlace[4] = {0, 2, 1, 3};  // where the weight operands have column i of four (gemm_h16_device.h)
+        low.h[kPlace[i]] = static_cast<_Float16>(lo * (1.0f / 4096.0f));
+        high.h[kPlace[i]] = static_cast<_Float16>(hi);
     }
     sum_hi += dpp_f32<0xB1>(sum_hi);  // the eight lanes of a 32-column sub-block
     sum_lo += dpp_f32<0xB1>(sum_lo);
@@ -78,7 +79,7 @@ __device__ __forceinline__ void quantize_halves_store(const float4& in, uint32_t
     *reinterpret_cast<uint2*>(blob + 16384u + at) = high.words;
     float* tables = reinterpret_cast<float*>(blob + 32768u);
     if (quad == 0) tables[v & 31u] = unit;
-    if ((quad & 7u) == 0) tables[32u + (quad >> 3) * 32u + (v & 31u)] = fmaf(4096.0f, sum_hi, sum_lo);
+    if ((quad & 7u) == 0) tables[32u + (quad >> 3) * 32u + (v & 31u)] = unit * fmaf(4096.0f, sum_hi, sum_lo);
 }
 
 }  // namespace et
