@@ -29,6 +29,7 @@
 #include <cstdint>
 #include <type_traits>
 
+#include "et_hip.h"
 #include "gemm_h16_device.h"
 
 namespace et {
@@ -565,8 +566,9 @@ __global__ __launch_bounds__(256) void reduce_group_rotary_kernel(const Group gr
 
 }  // namespace
 
-// Up to here two of the wide kernel's four activation tiles would be padding.
-constexpr uint64_t kGemmWideFrom = 64;
+// Up to here two of the wide kernel's four activation tiles would be padding. With two operands per weight the waves of the
+// second two tiles have nothing to do then, and the others no more than with them.
+constexpr uint64_t kGemmWideFrom = 64, kGemmWideFromTwoParts = 48;
 // Its weight copies add 32-bit byte offsets to a tile's first row: 256 rows of less than 2^23 bytes each.
 constexpr uint64_t kGemmWideColumns = 1u << 23;
 
@@ -602,22 +604,24 @@ GemmGroupGeometry gemm_h16_group_geometry(int32_t codec, const uint64_t* rows, u
     const GemmGroupGeometry narrow = codec != kQ6_K && large * vector_tiles >= 192
                                          ? GemmGroupGeometry{128, large, 1}
                                          : GemmGroupGeometry{64, small, shares(small * vector_tiles)};
-    if (vectors <= kGemmWideFrom || columns >= kGemmWideColumns || vectors > 0xffffffffull) return narrow;
+    const uint64_t wide_from = weight_parts(codec) == 2 ? kGemmWideFromTwoParts : kGemmWideFrom;
+    if (vectors <= wide_from || columns >= kGemmWideColumns || vectors > 0xffffffffull) return narrow;
     // Prompts: the wide kernel where it takes less time. A compute unit runs one workgroup at a time, so a launch takes
     // as many turns of a share's stages as its busiest XCD has workgroups per compute unit; a stage of 256 columns takes,
-    // from launches of 1000 vectors on 14336 x 4096, the microseconds of StageTimes. K shares cost what their sums move,
-    // written and read at 4 TB/s, and a launch; the wide kernel also its first copies and its stores, which no other
-    // workgroup covers. (Whole calls, narrow / wide in us: Q4_K 14336 x 4096 with 1000, 256 and 70 vectors 419 / 288,
-    // 115 / 85, 55 / 47; 4096 x 4096 with 1000, 512 and 200 vectors 129 / 95, 65 / 59 and 33 / 38, the last one stays
-    // narrow; 11008 x 2048 with 300 vectors 66 / 71, narrow as well; Q6_K 14336 x 4096 with 1000 and 70 724 / 460, 71 / 63.)
+    // from 90 shapes of all codecs (512 to 16384 rows, 1024 to 14336 columns, 40 to 1000 vectors, both kernels, the wide one with up to
+    // sixteen shares), the microseconds of StageTimes. K shares cost what their sums move, written and read at 4 TB/s, and a
+    // launch. With leads of 2 and 4 us what the rule takes needs 1.014 of the better kernel's time in the geometric
+    // mean (with the times of the wide kernel before its even schedule and a lead of 6 us: 1.031). (Whole calls, narrow / wide in us: Q4_K 10438 x 6400 with 816
+    // vectors 385 / 305, 2816 x 4096 with 233 40.5 / 36.8, 4854 x 11008 with 58 41.7 / 47.2; Q6_K 1422 x 3328 with 998 87 / 67,
+    // 10385 x 2816 with 56 39.5 / 30.6; Q3_K 2392 x 1536 with 915 51.5 / 40.7.)
     struct StageTimes {
         double rows64, rows128, wide;
     };
-    const StageTimes us = codec == kQ2_K   ? StageTimes{1.3, 2.2, 6.1}
-                          : codec == kQ3_K ? StageTimes{1.1, 1.8, 7.6}
-                          : codec == kQ5_K ? StageTimes{1.15, 1.95, 8.5}
-                          : codec == kQ6_K ? StageTimes{1.6, 0.0, 6.9}
-                                           : StageTimes{1.05, 1.8, 8.4};
+    const StageTimes us = codec == kQ2_K   ? StageTimes{1.3, 2.2, 5.25}
+                          : codec == kQ3_K ? StageTimes{1.1, 1.8, 6.55}
+                          : codec == kQ5_K ? StageTimes{1.15, 1.95, 7.3}
+                          : codec == kQ6_K ? StageTimes{1.6, 0.0, 5.95}
+                                           : StageTimes{1.05, 1.8, 7.2};
     uint64_t launch_rows = 0;
     for (uint32_t i = 0; i < count; i++) launch_rows += rows[i];
     const auto cost = [&](uint64_t on_an_xcd, uint64_t splits, double stage_us) {
@@ -628,16 +632,25 @@ GemmGroupGeometry gemm_h16_group_geometry(int32_t codec, const uint64_t* rows, u
     const double narrow_us = cost((narrow.row_tiles + 7) / 8 * vector_tiles * narrow.k_splits, narrow.k_splits,
                                   narrow.tile_rows == 128 ? us.rows128 : us.rows64);
     GemmGroupGeometry best = narrow;
-    double best_us = narrow_us - 6.0;
+    double best_us = narrow_us - (weight_parts(codec) == 2 ? 4.0 : 2.0);
+    const auto scratch = [&](const GemmGroupGeometry& g) {
+        return tile_workspace_bytes(2, vectors, columns) + (g.k_splits > 1 ? g.k_splits * vectors * g.row_tiles * g.tile_rows * 4u : 0);
+    };
+    const bool static_scratch = scratch(narrow) <= ET_HIP_STATIC_WORKSPACE_BYTES;
     const uint64_t wide_groups = (vectors + kGemmWideVectors - 1) / kGemmWideVectors;
     for (uint64_t splits = 1; splits <= stages && splits <= 16; splits++) {
         const uint64_t share = (stages + splits - 1) / splits;
         if ((stages + share - 1) / share != splits) continue;  // an empty share
-        const double wide_us = cost((wide * splits + 7) / 8 * wide_groups, splits, us.wide);
-        if (wide_us < best_us) {
-            best_us = wide_us;
-            best = GemmGroupGeometry{wide_rows, wide, static_cast<uint32_t>(splits), true};
-        }
+        const GemmGroupGeometry candidate{wide_rows, wide, static_cast<uint32_t>(splits), true};
+        const uint64_t on_an_xcd = (wide * splits + 7) / 8 * wide_groups;
+        const double wide_us = cost(on_an_xcd, splits, us.wide);
+        if (wide_us >= best_us) continue;
+        // Shares that outgrow the library's own scratch, where the narrow kernel would not, leave callers of that entry point
+        // without a path: only for a clear gain.
+        const bool clear = vectors > kGemmWideFrom && cost(on_an_xcd, splits, us.wide / 0.86) < narrow_us - 6.0;
+        if (!clear && static_scratch && scratch(candidate) > ET_HIP_STATIC_WORKSPACE_BYTES) continue;
+        best_us = wide_us;
+        best = candidate;
     }
     return best;
 }

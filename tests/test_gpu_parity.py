@@ -316,6 +316,8 @@ def test_linear_many_vectors_f32_matrix_core_tiles(et, device, codec, vectors, r
     (oracle.Q6_K, 225, 4097, 2304),
     (oracle.Q2_K, 161, 14336, 4096),
     (oracle.Q2_K, 480, 4096, 4352),
+    (oracle.Q6_K, 49, 10385, 2816),   # the fewest vectors of the codecs with two operands per weight
+    (oracle.Q4_K, 300, 14336, 512),   # two stages: the first is followed by the last
 ])
 def test_prompts_on_the_wide_kernel(et, device, codec, vectors, rows, columns):
     rng = np.random.default_rng(rows + columns + vectors)
