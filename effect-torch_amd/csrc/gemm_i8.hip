@@ -360,10 +360,9 @@ __global__ __launch_bounds__(kThreads) void gemm_i8_kernel(
                 const uint4 first_four = *reinterpret_cast<const LdsQuad*>(window);
                 const uint32_t d0 = first_four.x, d1 = first_four.y, d2 = first_four.z, d3 = first_four.w, d4 = window[4];
                 const bool odd = (b & 1u) != 0;  // (row * pitch + b * 34 or 18) & 2, pitch % 4 == 0
-                // The scale sits at the block start: for the second half of Q8_0 in another dword.
-                const uint32_t scale_word =
-                    CODEC == kQ8_0 ? *reinterpret_cast<const uint32_t*>(row_in_slot + ((b * W::kBlockBytes) & ~3u)) : d0;
-                w_scale[bb] = half_bits_to_float(odd ? scale_word >> 16 : scale_word & 0xffffu);
+                // The scale sits at the block start: the window of the second half of Q8_0 lacks it, but the operand of the
+                // scale products takes it from the first lane half alone.
+                w_scale[bb] = half_bits_to_float(odd ? d0 >> 16 : d0 & 0xffffu);
                 uint32_t words[4];
                 words[0] = odd ? d1 : __builtin_amdgcn_alignbit(d1, d0, 16);
                 words[1] = odd ? d2 : __builtin_amdgcn_alignbit(d2, d1, 16);
