@@ -245,6 +245,29 @@ def test_chunks_are_as_close_to_64_bits_as_the_streaming_kernel(et, device, dtyp
 
 
 @pytest.mark.parametrize("dtype", [np.float16, "bf16"])
+@pytest.mark.parametrize("rise", [0.4, 0.9, 1.9, 5.0])
+def test_chunks_whose_maximum_rises_slowly(et, device, dtype, rise):
+    # Scores (log2 units) that rise by `rise` every 32 positions: the chunk kernel's reference point of the exponents trails a
+    # row's maximum by up to two, so it moves every few steps, every step, or by more than that in one. This file's bar: a
+    # score near 170 (rise 5) carries 2^-24 of itself, 1e-5 of a weight.
+    rng = np.random.default_rng(int(10 * rise))
+    slots, tokens, scale = 20, 40, 128 ** -0.5
+    case = make_case(rng, slots=slots, query_heads=8, kv_heads=2, width=128, block_size=16, contexts=[700, 500] * 10, tokens=tokens,
+                     advances=[tokens] * slots, dtype=dtype)
+    case["q"] *= np.float32(0.2)
+    case["q"][..., 0] = 1.0
+    level = (np.arange(740) // 32 * rise / np.log2(np.e) / scale).astype(np.float32)
+    stored = torch.from_numpy(level).to(torch.bfloat16).view(torch.int16).numpy().view(np.uint16) if dtype == "bf16" else level.astype(dtype)
+    for slot in range(slots):
+        at = np.arange(int(case["cursors"][slot]))
+        case["k_slab"][case["table"][slot, at // 16] * 16 + at % 16, :, 0] = stored[at][:, None]
+        case["k"][slot, :, :, 0] = level[len(at):len(at) + tokens]
+    got = run_gpu(et, device, case, scale)
+    assert et.kv_attention_kernel(got[3], 8, tokens).startswith("kv_append+kv_chunk")
+    compare(got, run_oracle(case, scale))
+
+
+@pytest.mark.parametrize("dtype", [np.float16, "bf16"])
 @pytest.mark.parametrize("width,bound", [(128, 300), (128, 9000), (64, 300)])  # one split, several, the narrow kernel
 def test_values_that_are_not_finite_stay_with_the_rows_that_see_them(et, device, dtype, width, bound):
     rng = np.random.default_rng(width + bound)
