@@ -27,9 +27,9 @@
 
 #include <atomic>
 #include <cstdint>
+#include <limits>
 #include <type_traits>
 
-#include "et_hip.h"
 #include "gemm_h16_device.h"
 
 namespace et {
@@ -578,7 +578,7 @@ bool gemm_h16_supported(int32_t codec, uint64_t columns) {
 }
 
 GemmGroupGeometry gemm_h16_group_geometry(int32_t codec, const uint64_t* rows, uint32_t count, uint64_t columns,
-                                          uint64_t vectors) {
+                                          uint64_t vectors, uint64_t most_partial_bytes) {
     const uint64_t stages = columns / 256, vector_tiles = (vectors + 31) / 32;
     // The rule of gemm_i8_k_splits: a launch with far fewer workgroups than compute units shares the
     // stages of K out over several workgroups per tile, no share empty.
@@ -631,24 +631,16 @@ GemmGroupGeometry gemm_h16_group_geometry(int32_t codec, const uint64_t* rows, u
     };
     const double narrow_us = cost((narrow.row_tiles + 7) / 8 * vector_tiles * narrow.k_splits, narrow.k_splits,
                                   narrow.tile_rows == 128 ? us.rows128 : us.rows64);
+    const auto fits = [&](const GemmGroupGeometry& g) { return gemm_h16_partial_bytes(g, vectors) <= most_partial_bytes; };
     GemmGroupGeometry best = narrow;
-    double best_us = narrow_us - (weight_parts(codec) == 2 ? 4.0 : 2.0);
-    const auto scratch = [&](const GemmGroupGeometry& g) {
-        return tile_workspace_bytes(2, vectors, columns) + (g.k_splits > 1 ? g.k_splits * vectors * g.row_tiles * g.tile_rows * 4u : 0);
-    };
-    const bool static_scratch = scratch(narrow) <= ET_HIP_STATIC_WORKSPACE_BYTES;
+    double best_us = fits(narrow) ? narrow_us - (weight_parts(codec) == 2 ? 4.0 : 2.0) : std::numeric_limits<double>::infinity();
     const uint64_t wide_groups = (vectors + kGemmWideVectors - 1) / kGemmWideVectors;
     for (uint64_t splits = 1; splits <= stages && splits <= 16; splits++) {
         const uint64_t share = (stages + splits - 1) / splits;
         if ((stages + share - 1) / share != splits) continue;  // an empty share
         const GemmGroupGeometry candidate{wide_rows, wide, static_cast<uint32_t>(splits), true};
-        const uint64_t on_an_xcd = (wide * splits + 7) / 8 * wide_groups;
-        const double wide_us = cost(on_an_xcd, splits, us.wide);
-        if (wide_us >= best_us) continue;
-        // Shares that outgrow the library's own scratch, where the narrow kernel would not, leave callers of that entry point
-        // without a path: only for a clear gain.
-        const bool clear = vectors > kGemmWideFrom && cost(on_an_xcd, splits, us.wide / 0.86) < narrow_us - 6.0;
-        if (!clear && static_scratch && scratch(candidate) > ET_HIP_STATIC_WORKSPACE_BYTES) continue;
+        const double wide_us = cost((wide * splits + 7) / 8 * wide_groups, splits, us.wide);
+        if (wide_us >= best_us || !fits(candidate)) continue;
         best_us = wide_us;
         best = candidate;
     }
@@ -657,8 +649,7 @@ GemmGroupGeometry gemm_h16_group_geometry(int32_t codec, const uint64_t* rows, u
 
 uint64_t gemm_h16_group_partial_bytes(int32_t codec, const uint64_t* rows, uint32_t count, uint64_t columns,
                                       uint64_t vectors) {
-    const GemmGroupGeometry g = gemm_h16_group_geometry(codec, rows, count, columns, vectors);
-    return g.k_splits > 1 ? g.k_splits * vectors * g.row_tiles * g.tile_rows * 4u : 0;
+    return gemm_h16_partial_bytes(gemm_h16_group_geometry(codec, rows, count, columns, vectors), vectors);
 }
 
 namespace {
@@ -740,7 +731,7 @@ GemmShares gemm_h16_shares_layout(int32_t codec, uint64_t rows, uint64_t columns
 
 hipError_t gemm_h16_group(int32_t codec, const GemmMember* members, uint32_t count, const uint8_t* tiles,
                           float* partials, uint64_t columns64, uint64_t vectors64, hipStream_t stream,
-                          bool leave_shares, const GemmRotary* rotary) {
+                          bool leave_shares, const GemmRotary* rotary, uint64_t most_partial_bytes) {
     if (!gemm_h16_supported(codec, columns64)) return hipErrorInvalidValue;
     if (count == 0 || count > kGemmGroupMost || columns64 % 256 != 0 || columns64 == 0) return hipErrorInvalidValue;
     const uint32_t columns = static_cast<uint32_t>(columns64), vectors = static_cast<uint32_t>(vectors64);
@@ -749,7 +740,7 @@ hipError_t gemm_h16_group(int32_t codec, const GemmMember* members, uint32_t cou
         if (members[i].rows == 0 || members[i].rows > 0xffffffffull) return hipErrorInvalidValue;
         rows[i] = members[i].rows;
     }
-    GemmGroupGeometry g = gemm_h16_group_geometry(codec, rows, count, columns, vectors);
+    GemmGroupGeometry g = gemm_h16_group_geometry(codec, rows, count, columns, vectors, most_partial_bytes);
     // the rotary rides on the launch that sums K shares: without shares the caller rotates itself
     if (rotary != nullptr && (g.k_splits == 1 || partials == nullptr)) return hipErrorInvalidValue;
     if (partials == nullptr && g.k_splits > 1) {  // nowhere to keep shares: 64-row workgroups, whole K each
@@ -824,7 +815,8 @@ hipError_t gemm_h16_probe(int probe, const uint8_t* weight, const uint8_t* tiles
 hipError_t gemm_h16(int32_t codec, const uint8_t* weight, const uint8_t* tiles, const GemmOutput& out,
                     uint64_t rows, uint64_t columns, uint64_t vectors, hipStream_t stream) {
     const GemmMember one = {weight, out.bias, out.residual, out.y, rows};
-    return gemm_h16_group(codec, &one, 1, tiles, out.partials, columns, vectors, stream, out.leave_shares);
+    return gemm_h16_group(codec, &one, 1, tiles, out.partials, columns, vectors, stream, out.leave_shares, nullptr,
+                          out.most_partial_bytes);
 }
 
 }  // namespace et

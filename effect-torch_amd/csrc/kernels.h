@@ -141,6 +141,7 @@ constexpr uint32_t kGemmMinVectors = 7;
 // Launches with few output tiles share K out over this many workgroups per tile (1 = no sharing);
 // `partials` then holds k_splits * vectors * rows floats. partials == nullptr: never share.
 uint32_t gemm_i8_k_splits(int32_t codec, int limbs, uint64_t rows, uint64_t columns, uint64_t vectors);
+constexpr uint64_t kAnyPartials = ~0ull;
 struct GemmOutput {
     const float* bias;      // [rows] or null
     const float* residual;  // [vectors, rows] added to the result, or null; may be y itself
@@ -149,6 +150,7 @@ struct GemmOutput {
     // gemm_h16 only: leave the K shares in `partials` unsummed ([share][vector][launch row], see
     // gemm_h16_shares_layout) for a consumer that sums them itself; bias, residual and y are then unused.
     bool leave_shares = false;
+    uint64_t most_partial_bytes = kAnyPartials;  // gemm_h16 only: what `partials` holds, where that is less than it could take
 };
 hipError_t gemm_i8(int32_t codec, int limbs, const uint8_t* weight, const uint8_t* tiles,
                    const GemmOutput& out, uint64_t rows, uint64_t columns, uint64_t vectors,
@@ -184,8 +186,12 @@ struct GemmGroupGeometry {
 };
 constexpr uint32_t kGemmWideVectors = 128;
 constexpr uint32_t gemm_h16_wide_rows(int32_t codec) { return codec == kQ2_K || codec == kQ6_K ? 128u : 256u; }
+constexpr uint64_t gemm_h16_partial_bytes(const GemmGroupGeometry& g, uint64_t vectors) {
+    return g.k_splits > 1 ? g.k_splits * vectors * g.row_tiles * g.tile_rows * 4u : 0;
+}
+// The fastest tiles and K shares whose partial results take at most that many bytes (gemm_h16_kernel's own where none do).
 GemmGroupGeometry gemm_h16_group_geometry(int32_t codec, const uint64_t* rows, uint32_t count, uint64_t columns,
-                                          uint64_t vectors);
+                                          uint64_t vectors, uint64_t most_partial_bytes = kAnyPartials);
 uint64_t gemm_h16_group_partial_bytes(int32_t codec, const uint64_t* rows, uint32_t count, uint64_t columns,
                                       uint64_t vectors);
 // A rotary embedding applied to some members of a group launch in the launch that sums their K
@@ -201,7 +207,8 @@ struct GemmRotary {
 };
 hipError_t gemm_h16_group(int32_t codec, const GemmMember* members, uint32_t count, const uint8_t* tiles,
                           float* partials, uint64_t columns, uint64_t vectors, hipStream_t stream,
-                          bool leave_shares = false, const GemmRotary* rotary = nullptr);
+                          bool leave_shares = false, const GemmRotary* rotary = nullptr,
+                          uint64_t most_partial_bytes = kAnyPartials);
 // Measurement only (et_hip_calibration_contraction): the Q4_K kernel of 64-row tiles without K shares
 // as it is (probe 0), without its consumers' arithmetic (1), without its copies (2), without the weight
 // (3) or the activation copies (4), with the weight (5) or the activation copies (6) and nothing else; at

@@ -135,7 +135,8 @@ int select_kernel(et_linear_plan* plan, std::string* error) {
         if (limbs == 2) {  // gemm_h16 chooses its own tile height and keeps partial results by whole tiles
             const GemmGroupGeometry g = gemm_h16_group_geometry(plan->codec, &plan->rows, 1, plan->columns, plan->vectors);
             plan->k_splits = g.k_splits;
-            if (plan->k_splits > 1) plan->partial_offset = take({g.k_splits, plan->vectors, g.row_tiles, g.tile_rows, 4});
+            plan->partial_offset = cursor;
+            if (plan->k_splits > 1) take({g.k_splits, plan->vectors, g.row_tiles, g.tile_rows, 4});
             return;
         }
         plan->k_splits = gemm_i8_k_splits(plan->codec, limbs, plan->rows, plan->columns, plan->vectors);
@@ -761,10 +762,25 @@ int linear_enqueue_step(const et_linear_plan* const* plans, uint32_t count, cons
     return ET_OK;
 }
 
+uint64_t workspace_bytes_within(const et_linear_plan& plan, uint64_t limit) {
+    if (plan.workspace_bytes <= limit || plan.kernel != LinearKernel::kGemmHalf || plan.partial_offset > limit) return plan.workspace_bytes;
+    return plan.partial_offset + gemm_h16_partial_bytes(gemm_h16_group_geometry(plan.codec, &plan.rows, 1, plan.columns, plan.vectors,
+                                                                                limit - plan.partial_offset),
+                                                        plan.vectors);
+}
+
 int linear_enqueue(const et_linear_plan& plan, const float* x, uint64_t x_row_stride,
                    const uint8_t* weight, const float* bias, float* y, void* workspace,
                    uint64_t workspace_bytes, void* stream, const volatile int32_t* cancel,
                    std::string* error) {
+    return linear_enqueue_within(plan, x, x_row_stride, weight, bias, y, workspace, workspace_bytes, plan.workspace_bytes, stream,
+                                 cancel, error);
+}
+
+int linear_enqueue_within(const et_linear_plan& plan, const float* x, uint64_t x_row_stride,
+                          const uint8_t* weight, const float* bias, float* y, void* workspace,
+                          uint64_t workspace_bytes, uint64_t limit, void* stream, const volatile int32_t* cancel,
+                          std::string* error) {
     if ((bias != nullptr) != plan.has_bias)
         return fail(error, ET_ERR_EXECUTION, "quantized_linear: bias does not match the immutable plan");
     if (cancelled(cancel)) return fail(error, ET_ERR_CANCELLED, "operation aborted");
@@ -800,19 +816,20 @@ int linear_enqueue(const et_linear_plan& plan, const float* x, uint64_t x_row_st
     }
 
     if (on_matrix_cores(plan)) {
-        if (scratch == nullptr || workspace_bytes < plan.workspace_bytes)
+        const uint64_t needed = workspace_bytes_within(plan, limit);
+        if (scratch == nullptr || workspace_bytes < needed)
             return fail(error, ET_ERR_EXECUTION,
                         "quantized_linear: workspace of " + std::to_string(workspace_bytes) +
-                            " bytes is smaller than the planned " +
-                            std::to_string(plan.workspace_bytes));
+                            " bytes is smaller than the planned " + std::to_string(needed));
         auto* tiles = scratch + plan.q_offset;
         if (hipError_t status =
                 quantize_tiles(x, x_row_stride, plan.vectors, plan.columns, limbs_of(plan), tiles, s))
             return hip_failure(error, "quantized_linear", status);
         // between the launches of one call, as the reference polls between rows (quantized.rs:451,459)
         if (cancelled(cancel)) return fail(error, ET_ERR_CANCELLED, "operation aborted");
-        float* partials = plan.k_splits > 1 ? reinterpret_cast<float*>(scratch + plan.partial_offset) : nullptr;
-        if (hipError_t status = contract_tiles(plan, weight, tiles, GemmOutput{bias, nullptr, y, partials}, s))
+        GemmOutput out = {bias, nullptr, y, plan.k_splits > 1 ? reinterpret_cast<float*>(scratch + plan.partial_offset) : nullptr};
+        if (limit < plan.workspace_bytes) out.most_partial_bytes = limit - plan.partial_offset;
+        if (hipError_t status = contract_tiles(plan, weight, tiles, out, s))
             return hip_failure(error, "quantized_linear", status);
         return ET_OK;
     }

@@ -57,7 +57,7 @@ struct et_linear_plan {
     uint64_t gather_offset, gather_bytes;  // densified f32 input
     uint64_t bias_offset;                  // densified f32 bias
     uint64_t q_offset;                     // quantised activation tiles (matrix-core kernels)
-    uint64_t partial_offset;               // partial results of the K shares (0 splits: unused)
+    uint64_t partial_offset;               // partial results of the K shares
     uint32_t k_splits;
     uint64_t workspace_bytes;
 };
@@ -95,6 +95,14 @@ int linear_enqueue(const et_linear_plan& plan, const float* x, uint64_t x_row_st
                    uint64_t workspace_bytes, void* stream, const volatile int32_t* cancel,
                    std::string* error);
 
+// What the plan's call takes of a workspace of `limit` bytes, and that call: the plan's own tiles and K shares where
+// they fit, else (gemm_h16) the fastest that do; more than `limit` where none do.
+uint64_t workspace_bytes_within(const et_linear_plan& plan, uint64_t limit);
+int linear_enqueue_within(const et_linear_plan& plan, const float* x, uint64_t x_row_stride,
+                          const uint8_t* weight, const float* bias, float* y, void* workspace,
+                          uint64_t workspace_bytes, uint64_t limit, void* stream, const volatile int32_t* cancel,
+                          std::string* error);
+
 // The quantised form of the activations a matrix-core plan consumes, made once and shared by every
 // plan of the same columns, vectors and activation mode; 0 bytes when the plan's kernel reads x itself.
 uint64_t prepared_input_bytes(const et_linear_plan& plan);
@@ -108,7 +116,7 @@ int linear_prepare_input_from(const et_linear_plan& plan, const et_prepare_sourc
 // Several plans of the same columns and vectors against one prepared input in one launch (see
 // et_hip_linear_enqueue_prepared_group in et_hip.h).
 // linear_enqueue with the workspace in a device array of the library's own (static_workspace.cpp): for
-// callers that cannot allocate. Plans that need more than ET_HIP_STATIC_WORKSPACE_BYTES are refused.
+// callers that cannot allocate. Plans that do not fit ET_HIP_STATIC_WORKSPACE_BYTES with any tiles and K shares are refused.
 int linear_enqueue_static_workspace(const et_linear_plan& plan, const float* x, uint64_t x_row_stride,
                                     const uint8_t* weight, const float* bias, float* y, void* stream,
                                     const volatile int32_t* cancel, std::string* error);

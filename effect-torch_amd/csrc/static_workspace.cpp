@@ -6,9 +6,9 @@
 // `scratch` is ONE array per GPU, held from the first use of the library on that GPU until the
 // process ends, and every call on a GPU uses it: calls that overlap in time on one GPU (two
 // streams, two threads) race on it and must be serialised by the caller. A call needs the bytes
-// et_hip_linear_plan_workspace_bytes reports for its plan; plans that need more than
-// ET_HIP_STATIC_WORKSPACE_BYTES are refused. What a call finds in the array is what the last call
-// left there: the kernels write every byte they later read (activation tiles, K-share partials,
+// et_hip_linear_plan_workspace_bytes reports for its plan; where those are more than
+// ET_HIP_STATIC_WORKSPACE_BYTES it runs on the fastest tiles and K shares that fit, and is refused
+// where none do. What a call finds in the array is what the last call left there: the kernels write every byte they later read (activation tiles, K-share partials,
 // the dense copy of strided input rows), nothing has to start at zero.
 #include <hip/hip_runtime.h>
 
@@ -81,17 +81,16 @@ void warm_device_symbols() {
 int linear_enqueue_static_workspace(const et_linear_plan& plan, const float* x, uint64_t x_row_stride,
                                     const uint8_t* weight, const float* bias, float* y, void* stream,
                                     const volatile int32_t* cancel, std::string* error) {
-    const uint64_t needed = plan.workspace_bytes;
-    if (needed > ET_HIP_STATIC_WORKSPACE_BYTES) {
-        *error = "quantized_linear: this plan needs a workspace of " + std::to_string(needed) +
+    if (workspace_bytes_within(plan, ET_HIP_STATIC_WORKSPACE_BYTES) > ET_HIP_STATIC_WORKSPACE_BYTES) {
+        *error = "quantized_linear: this plan needs a workspace of " + std::to_string(plan.workspace_bytes) +
                  " bytes, the static workspace holds " + std::to_string(ET_HIP_STATIC_WORKSPACE_BYTES) +
                  "; use et_hip_linear_enqueue with a workspace of the caller's";
         return ET_ERR_UNSUPPORTED;
     }
     uint8_t* pointer = nullptr;
     if (int status = scratch_pointer(&pointer, error)) return status;
-    return linear_enqueue(plan, x, x_row_stride, weight, bias, y, pointer, ET_HIP_STATIC_WORKSPACE_BYTES, stream, cancel,
-                          error);
+    return linear_enqueue_within(plan, x, x_row_stride, weight, bias, y, pointer, ET_HIP_STATIC_WORKSPACE_BYTES,
+                                 ET_HIP_STATIC_WORKSPACE_BYTES, stream, cancel, error);
 }
 
 }  // namespace quantized

@@ -384,8 +384,8 @@ class RawLinear:
     def enqueue_static_workspace(self, x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor],
                                  y: torch.Tensor, stream=None, cancelled: Optional[CancellationFlag] = None) -> None:
         """:meth:`enqueue` with the library's own static device workspace (``et_hip_linear_enqueue_static_workspace``):
-        no allocation anywhere; plans that need more than ``STATIC_WORKSPACE_BYTES`` are refused; calls that
-        overlap in time on one GPU race on the array."""
+        no allocation anywhere; plans that need more than ``STATIC_WORKSPACE_BYTES`` run on tiles and K shares that
+        take less, or are refused where none do; calls that overlap in time on one GPU race on the array."""
         self._check_input(x)
         self._check_weight(weight, bias)
         self._check_output(y)

@@ -175,11 +175,13 @@ int et_hip_linear_enqueue(const et_linear_plan* plan, const float* x, uint64_t x
  * library, ET_HIP_STATIC_WORKSPACE_BYTES per GPU, held from its first use on that GPU until the
  * process ends. It has no counterpart in the reference; it exists for callers that cannot allocate
  * device memory: code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc.
- * The call allocates nothing and frees nothing. A plan whose et_hip_linear_plan_workspace_bytes
- * exceeds the array is refused (ET_ERR_UNSUPPORTED, "... the static workspace holds ..."): such
- * callers bring their own workspace to et_hip_linear_enqueue. Every call on a GPU uses the same
+ * The call allocates nothing and frees nothing. Every call on a GPU uses the same
  * array: calls that overlap in time on one GPU race on it - serialise them (one stream, or events).
- * Results are those of et_hip_linear_enqueue, bit for bit. The array's device address is looked up
+ * Results are those of et_hip_linear_enqueue, bit for bit, where et_hip_linear_plan_workspace_bytes
+ * does not exceed the array. A plan that would take more only for its K-share partials runs on the
+ * fastest tiles and K shares that fit (the same products, summed in another order); a plan for which
+ * none fit is refused (ET_ERR_UNSUPPORTED, "... the static workspace holds ..."): such callers bring
+ * their own workspace to et_hip_linear_enqueue. The array's device address is looked up
  * when a plan is made on that GPU (et_hip_linear_plan_create / et_hip_linear_requirements), not by
  * this call, so that the call may be recorded into a stream capture: make the plan, with the GPU
  * current, before the capture begins. */

@@ -171,6 +171,59 @@ def test_workspace_sizes_are_checked_products(et):
     assert plan.requirements.workspace_bytes >= 512 * 4096 * 4
 
 
+def _takes(et, codec, rows, columns, vectors):
+    """Whether the entry point with the library's own workspace takes the plan: past the size check it stops at the
+    set cancellation flag, or before that for want of a device; nothing is launched."""
+    import ctypes
+    plan = et.RawLinear(codec, rows, columns, vectors)
+    x, stop = torch.zeros(16), et.CancellationFlag()
+    stop.cancel()
+    from effect_torch_amd import _native
+    lib = _native.lib()
+    status = lib.et_hip_linear_enqueue_static_workspace(plan.requirements._handle, x.data_ptr(), columns, x.data_ptr(), None,
+                                                        x.data_ptr(), None, stop.ptr)
+    assert status != 0
+    return "the static workspace holds" not in ctypes.string_at(lib.et_hip_last_error()).decode()
+
+
+def test_the_static_workspace_takes_every_plan_whose_narrow_tiles_fit(et):
+    import math
+    import random
+    codecs = {"Q2_K": 128, "Q3_K": 256, "Q4_K": 256, "Q5_K": 256, "Q6_K": 128}
+
+    def up(value, to):
+        return -(-value // to) * to
+
+    def narrow_bytes(codec, rows, columns, vectors):
+        """The whole workspace of a call on gemm_h16_kernel: dense x and bias, activation tiles, K shares of 64-row tiles."""
+        stages, vector_tiles, small, shares = columns // 256, -(-vectors // 32), -(-rows // 64), 1
+        if not (codec != "Q6_K" and -(-rows // 128) * vector_tiles >= 192) and stages >= 2 and small * vector_tiles < 192:
+            splits = min(256 // (small * vector_tiles), stages)
+            if splits >= 2:
+                shares = -(-stages // -(-stages // splits))
+        sums = 4 * shares * vectors * small * 64 if shares > 1 else 0
+        return up(4 * vectors * columns, 256) + up(4 * rows, 256) + stages * vector_tiles * 34816 + up(sums, 256)
+
+    # at the limit; and where the faster tiles' shares need several times the array
+    shapes = [("Q4_K", 4096, 4096, m) for m in (128, 129, 133, 142, 143)] + [
+        ("Q2_K", 4096, 4096, 170), ("Q6_K", 4096, 5120, 108), ("Q6_K", 4096, 5120, 118), ("Q2_K", 768, 3072, 281),
+        ("Q4_K", 4096, 13824, 123), ("Q2_K", 5044, 13056, 76), ("Q3_K", 4623, 3072, 126), ("Q5_K", 10009, 10496, 96),
+        ("Q6_K", 2975, 3072, 317), ("Q4_K", 1334, 2560, 768)]
+    rng = random.Random(16)
+    for _ in range(1500):
+        shapes.append((rng.choice(list(codecs)), int(math.exp(rng.uniform(math.log(256), math.log(16384)))),
+                       256 * int(math.exp(rng.uniform(0, math.log(57)))), int(math.exp(rng.uniform(math.log(33), math.log(1200))))))
+    fitted = beyond = 0
+    for codec, rows, columns, vectors in shapes:
+        if narrow_bytes(codec, rows, columns, vectors) > et.STATIC_WORKSPACE_BYTES:
+            continue
+        fitted += 1
+        beyond += et.RawLinear(et.GgmlQuant[codec], rows, columns, vectors).requirements.workspace_bytes > et.STATIC_WORKSPACE_BYTES
+        assert _takes(et, et.GgmlQuant[codec], rows, columns, vectors), (codec, rows, columns, vectors)
+    assert fitted > 800 and beyond > 50
+    assert not _takes(et, et.GgmlQuant.Q4_K, 256, 14336, 2048)  # 112 MiB of dense rows alone
+
+
 def test_embedding_plan(et):
     Q5 = et.GgmlQuant.Q5_K
     plan = et.embedding_requirements(torch.zeros((2, 3), dtype=torch.int64), _w(3, 176), Q5, (3, 256))

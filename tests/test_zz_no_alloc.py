@@ -109,3 +109,33 @@ def test_static_workspace_entry_point_refuses_what_does_not_fit(et, device):
     out = torch.empty((1, 300), device=device)
     small.enqueue_static_workspace(torch.from_numpy(xs).to(device), torch.from_numpy(w).to(device), None, out)
     close(out.cpu().numpy(), oracle.linear_into(oracle.Q4_K, 300, 512, xs, w))
+
+
+@pytest.mark.parametrize("codec,rows,columns,vectors", [
+    (oracle.Q4_K, 4096, 4096, 142),
+    (oracle.Q6_K, 2975, 3072, 317),
+    (oracle.Q2_K, 5044, 13056, 76),
+    (oracle.Q5_K, 4096, 5376, 150),
+])
+def test_static_workspace_entry_point_runs_plans_whose_shares_outgrow_it(et, device, codec, rows, columns, vectors):
+    # the plan's own K shares need more than the array: other tiles or fewer shares, the same products
+    rng = np.random.default_rng(rows + columns + vectors)
+    weight = torch.from_numpy(synth.random_weight(codec, rows, columns, rng)).to(device)
+    x = torch.from_numpy(synth.random_activations(vectors, columns, rng)).to(device)
+    bias = torch.from_numpy(rng.standard_normal(rows).astype(np.float32)).to(device)
+    plan = et.RawLinear(et.GgmlQuant(codec), rows, columns, vectors, True)
+    assert plan.requirements.workspace_bytes > et.STATIC_WORKSPACE_BYTES
+    y, again = (torch.full((vectors, rows), float("nan"), device=device) for _ in range(2))
+    plan.enqueue_static_workspace(x, weight, bias, y)
+    plan.enqueue_static_workspace(x, weight, bias, again)
+    decoded = et.dequantize_rows(weight, et.GgmlQuant(codec), (rows, columns)).double()
+    exact = x.double() @ decoded.T + bias.double()
+    torch.cuda.synchronize()
+    assert torch.equal(y, again)
+    # As in the prompts' test: 32 matrix instructions per stage chain, 51 stages at most, a handful of roundings per element of
+    # rms 2^-24 / sqrt(3): sqrt(32/2 + 51/2 + 4) of them are 2.3e-7, the activations' own rounding 1e-7
+    assert ((y - exact).norm() / exact.norm()).item() <= 2.5e-7
+    # with a workspace of its own the plan runs its own shares
+    own = torch.full((vectors, rows), float("nan"), device=device)
+    plan.enqueue(x, weight, bias, own, torch.empty(plan.requirements.workspace_bytes, dtype=torch.uint8, device=device))
+    assert ((own - exact).norm() / exact.norm()).item() <= 2.5e-7
