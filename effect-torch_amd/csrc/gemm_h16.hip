@@ -607,33 +607,39 @@ GemmGroupGeometry gemm_h16_group_geometry(int32_t codec, const uint64_t* rows, u
     const uint64_t wide_from = weight_parts(codec) == 2 ? kGemmWideFromTwoParts : kGemmWideFrom;
     if (vectors <= wide_from || columns >= kGemmWideColumns || vectors > 0xffffffffull) return narrow;
     // Prompts: the wide kernel where it takes less time. A compute unit runs one workgroup at a time, so a launch takes
-    // as many turns of a share's stages as its busiest XCD has workgroups per compute unit; a stage of 256 columns takes,
-    // from 90 shapes of all codecs (512 to 16384 rows, 1024 to 14336 columns, 40 to 1000 vectors, both kernels, the wide one with up to
-    // sixteen shares), the microseconds of StageTimes. K shares cost what their sums move, written and read at 4 TB/s, and a
-    // launch. With leads of 2 and 4 us what the rule takes needs 1.014 of the better kernel's time in the geometric
-    // mean (with the times of the wide kernel before its even schedule and a lead of 6 us: 1.031). (Whole calls, narrow / wide in us: Q4_K 10438 x 6400 with 816
-    // vectors 385 / 305, 2816 x 4096 with 233 40.5 / 36.8, 4854 x 11008 with 58 41.7 / 47.2; Q6_K 1422 x 3328 with 998 87 / 67,
-    // 10385 x 2816 with 56 39.5 / 30.6; Q3_K 2392 x 1536 with 915 51.5 / 40.7.)
-    struct StageTimes {
-        double rows64, rows128, wide;
+    // as many turns as its busiest XCD has workgroups per compute unit; a turn costs the microseconds of Turn for every 256
+    // columns of a share and once (first copies, last stores), K shares a launch and what their sums move (0.42 us per MiB,
+    // written and read). From 1120 random shapes of all codecs (256 to 16384 rows, 256 to 14336 columns, 49 to 1500 vectors) and 300
+    // with more than 16 MiB of sums, both kernels, the wide one with up to sixteen shares; estimates are off by 6 to 8 %
+    // (rms), hence a lead of 3 us. What the rule takes needs 1.006 of the better kernel's time in the geometric mean over
+    // the random shapes (5 of them more than 3 % above the rule before), 1.009 over the others; stage times without Turn::once and
+    // no shares beyond 16 MiB needed 1.027 and 1.08. (Whole calls, gemm_h16_kernel / wide in us: Q4_K 8540 x 9216
+    // with 612 vectors 352 / 238, 2104 x 3584 with 198 38.0 / 30.6, 8167 x 2304 with 125 24.9 / 34.9; Q6_K 16372 x 3584 with 469
+    // 345 / 205, 8678 x 11264 with 51 119 / 63, 711 x 3584 with 62 15.8 / 20.7; Q3_K 995 x 1280 with 112 13.4 / 23.5.)
+    struct Turn {
+        double stage, once;
     };
-    const StageTimes us = codec == kQ2_K   ? StageTimes{1.3, 2.2, 5.25}
-                          : codec == kQ3_K ? StageTimes{1.1, 1.8, 6.55}
-                          : codec == kQ5_K ? StageTimes{1.15, 1.95, 7.3}
-                          : codec == kQ6_K ? StageTimes{1.6, 0.0, 5.95}
-                                           : StageTimes{1.05, 1.8, 7.2};
+    struct Times {
+        Turn rows64, rows128, wide;
+    };
+    Times us = codec == kQ2_K   ? Times{{1.13, 2.8}, {1.84, 4.0}, {4.6, 2.8}}
+               : codec == kQ3_K ? Times{{0.90, 1.8}, {1.50, 2.8}, {5.5, 3.8}}
+               : codec == kQ5_K ? Times{{0.90, 2.6}, {1.56, 3.5}, {5.9, 4.9}}
+               : codec == kQ6_K ? Times{{1.32, 3.7}, {}, {5.1, 3.8}}
+                                : Times{{0.82, 2.8}, {1.37, 3.9}, {5.8, 3.8}};
+    if (weight_parts(codec) == 2 && vectors <= 64) us.wide.stage = codec == kQ2_K ? 3.1 : 3.3;  // half of the waves have no vectors
     uint64_t launch_rows = 0;
     for (uint32_t i = 0; i < count; i++) launch_rows += rows[i];
-    const auto cost = [&](uint64_t on_an_xcd, uint64_t splits, double stage_us) {
+    const auto cost = [&](uint64_t on_an_xcd, uint64_t splits, const Turn& turn) {
         const double turns = static_cast<double>((on_an_xcd + 31) / 32);
-        const double sums = splits > 1 ? 3.0 + 8.0e-6 / 4 * static_cast<double>(splits) * static_cast<double>(vectors) * static_cast<double>(launch_rows) : 0.0;
-        return turns * static_cast<double>((stages + splits - 1) / splits) * stage_us + sums;
+        const double sums = splits > 1 ? 3.0 + 0.42 / 262144 * static_cast<double>(splits) * static_cast<double>(vectors) * static_cast<double>(launch_rows) : 0.0;
+        return turns * (static_cast<double>((stages + splits - 1) / splits) * turn.stage + turn.once) + sums;
     };
     const double narrow_us = cost((narrow.row_tiles + 7) / 8 * vector_tiles * narrow.k_splits, narrow.k_splits,
                                   narrow.tile_rows == 128 ? us.rows128 : us.rows64);
     const auto fits = [&](const GemmGroupGeometry& g) { return gemm_h16_partial_bytes(g, vectors) <= most_partial_bytes; };
     GemmGroupGeometry best = narrow;
-    double best_us = fits(narrow) ? narrow_us - (weight_parts(codec) == 2 ? 4.0 : 2.0) : std::numeric_limits<double>::infinity();
+    double best_us = fits(narrow) ? narrow_us - 3.0 : std::numeric_limits<double>::infinity();
     const uint64_t wide_groups = (vectors + kGemmWideVectors - 1) / kGemmWideVectors;
     for (uint64_t splits = 1; splits <= stages && splits <= 16; splits++) {
         const uint64_t share = (stages + splits - 1) / splits;
