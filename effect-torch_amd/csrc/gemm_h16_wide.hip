@@ -193,7 +193,12 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_h16_wide_kernel(const Gro
     if (!working) {
         const auto pass = [&](uint32_t stage, auto is_last) {
 #pragma unroll
-            for (int b = 0; b < kStageBlocks; b++) begin(stage, is_last, b);
+            for (int b = 0; b < kStageBlocks; b++) {
+                begin(stage, is_last, b);
+                // The pieces are in LDS before this wave's next barrier. (Waves with vectors wait for operands that they read
+                // behind these writes, and LDS answers in order.)
+                if (W::kMinima && b == kCutAt + 1) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            }
         };
         for (uint32_t stage = 0; stage + 1u < stages; stage++) pass(stage, std::false_type{});
         pass(stages - 1u, std::true_type{});
