@@ -240,14 +240,14 @@ __device__ __forceinline__ void operands(const Raw& raw, const Shared& shared, i
 }
 
 // f32 bits as three bfloat16 numbers that add up to it, eight significant bits each: the top halves of `x`, of
-// what is left of it, and of what is left then (nothing is lost above 2^-110).
+// what is left of it, and of what is left then (nothing is lost above 2^-110). Of an infinity nothing is left.
 struct Pieces {
     uint32_t high, mid, low;  // in the upper sixteen bits
 };
 __device__ __forceinline__ Pieces cut(float x) {
     Pieces p;
     p.high = __float_as_uint(x) & 0xffff0000u;
-    const float rest = x - __uint_as_float(p.high);
+    const float rest = __builtin_isinf(x) ? 0.f : x - __uint_as_float(p.high);
     p.mid = __float_as_uint(rest) & 0xffff0000u;
     p.low = __float_as_uint(rest - __uint_as_float(p.mid));
     return p;

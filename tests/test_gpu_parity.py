@@ -339,6 +339,24 @@ def test_prompts_on_the_wide_kernel(et, device, codec, vectors, rows, columns):
     assert np.linalg.norm(got - exact) <= 2.5e-7 * np.linalg.norm(exact)
 
 
+@pytest.mark.parametrize("codec", [oracle.Q4_K, oracle.Q5_K])
+def test_prompts_whose_sums_of_activations_overflow(et, device, codec):
+    # 32 values of 1.2e37 add up to no f32: what the minima take away is an infinity, or a NaN where a sub-block's minimum is 0
+    # (zero times infinity), of that vector alone
+    rng = np.random.default_rng(30 + codec)
+    rows, columns, vectors, block = 14336, 4096, 128, 144 if codec == oracle.Q4_K else 176
+    weight = synth.random_weight(codec, rows, columns, rng)
+    x = synth.random_activations(vectors, columns, rng)
+    x[3, 256:512] = 1.2e37
+    assert "gemm_h16_wide" in et.RawLinear(et.GgmlQuant(codec), rows, columns, vectors).requirements.kernel
+    got = run_linear(et, device, codec, rows, columns, x, weight, None)
+    packed = weight[:, block + 4:block + 16]  # of the second super-block: six bits each of eight scales and eight minima
+    minima = np.concatenate([packed[:, 4:8] & 63, (packed[:, 8:12] >> 4) | ((packed[:, 4:8] >> 6) << 4)], axis=1)
+    assert np.array_equal(np.isnan(got[3]), (minima == 0).any(axis=1))
+    assert np.isneginf(got[3][(minima != 0).all(axis=1)]).all()
+    assert np.isfinite(np.delete(got, 3, axis=0)).all()
+
+
 @pytest.mark.parametrize("mode", ["F32", "INT8"])
 @pytest.mark.parametrize("codec,vectors,rows,columns", [(oracle.Q4_K, 32, 1024, 4096), (oracle.Q4_K, 32, 4096, 4096),
                                                         (oracle.Q4_K, 32, 4096, 14336), (oracle.Q5_K, 32, 4096, 4096),
