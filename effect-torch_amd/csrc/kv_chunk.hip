@@ -173,7 +173,7 @@ struct Slab<U8> {
 // Weights are at most exp2(kSlack), 4 * 4096 in a half float's pieces, and the rounding of a positive exponent is that of the
 // exponents between -2 and 0. With a maximum that is followed exactly nearly every step of 64 positions has one row of 32 that
 // moves, and all 32 pay 70 vector instructions for it.
-constexpr float kSlack = 2.0f;
+constexpr float kSlack = 2.0f, kMostWeight = 4.0f;
 constexpr int kChunkWaves = 8, kChunkThreads = 64 * kChunkWaves;
 
 // RW row waves share a tile (32 * RW query rows per workgroup), 8 / RW groups of them take tiles in turn.
@@ -403,6 +403,8 @@ __global__ __launch_bounds__(kChunkThreads, 2) void kv_chunk_kernel(const KvArgs
     constexpr int kGroups = Shape::kGroups, kRows = Shape::kRows, kTile = Shape::kTile, kCopies = Shape::kCopies;
     constexpr int kKeyChunks = W / 16, kDimTiles = W / 32, kQueryPieces = S::kQueryPieces, kWeightPieces = S::kWeightPieces;
     constexpr int U = S::kBlocksPerStep < kTile / 32 ? S::kBlocksPerStep : kTile / 32;
+    // A weight past that would be infinite, and its row attended to once more: right, and fifteen times slower.
+    static_assert(!std::is_same<VE, Half>::value || kMostWeight * S::kWeightScale <= 65504.0f, "weights are half floats");
     extern __shared__ __attribute__((aligned(256))) uint8_t lds[];
     uint32_t* rows_of_block = reinterpret_cast<uint32_t*>(lds + Shape::kTableAt);
 

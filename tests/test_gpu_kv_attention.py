@@ -244,23 +244,33 @@ def test_chunks_are_as_close_to_64_bits_as_the_streaming_kernel(et, device, dtyp
     assert error <= 2.0e-7
 
 
-@pytest.mark.parametrize("dtype", [np.float16, "bf16"])
+@pytest.mark.parametrize("dtype,width,tokens", [(np.float16, 128, 40), ("bf16", 128, 40), ("u8", 128, 40), (np.float16, 64, 40), ("u8", 64, 40),
+                                                (np.float16, 128, 12), ("u8", 128, 12)])  # 48 query rows: two row waves
 @pytest.mark.parametrize("rise", [0.4, 0.9, 1.9, 5.0])
-def test_chunks_whose_maximum_rises_slowly(et, device, dtype, rise):
+def test_chunks_whose_maximum_rises_slowly(et, device, dtype, width, tokens, rise):
     # Scores (log2 units) that rise by `rise` every 32 positions: the chunk kernel's reference point of the exponents trails a
     # row's maximum by up to two, so it moves every few steps, every step, or by more than that in one. This file's bar: a
-    # score near 170 (rise 5) carries 2^-24 of itself, 1e-5 of a weight.
+    # score near 115 (23 times 5) carries 2^-23 of itself in the pieces of q and as much in its sums: 3e-5, two thirds of that in a
+    # weight, of values up to 4.
     rng = np.random.default_rng(int(10 * rise))
-    slots, tokens, scale = 20, 40, 128 ** -0.5
-    case = make_case(rng, slots=slots, query_heads=8, kv_heads=2, width=128, block_size=16, contexts=[700, 500] * 10, tokens=tokens,
+    slots, scale = 20 if tokens == 40 else 40, width ** -0.5
+    case = make_case(rng, slots=slots, query_heads=8, kv_heads=2, width=width, block_size=16, contexts=[700, 500] * (slots // 2), tokens=tokens,
                      advances=[tokens] * slots, dtype=dtype)
     case["q"] *= np.float32(0.2)
     case["q"][..., 0] = 1.0
     level = (np.arange(740) // 32 * rise / np.log2(np.e) / scale).astype(np.float32)
-    stored = torch.from_numpy(level).to(torch.bfloat16).view(torch.int16).numpy().view(np.uint16) if dtype == "bf16" else level.astype(dtype)
     for slot in range(slots):
         at = np.arange(int(case["cursors"][slot]))
-        case["k_slab"][case["table"][slot, at // 16] * 16 + at % 16, :, 0] = stored[at][:, None]
+        rows = case["table"][slot, at // 16] * 16 + at % 16
+        if dtype == "u8":  # 127 steps of the row's scale in column 0, a step up or down in the others
+            case["k_slab"][rows] = rng.integers(127, 130, (len(at), 2, width))
+            case["k_slab"][rows, :, 0] = 255
+            case["k_scales"][rows] = (level[at] / np.float32(127.0) + np.float32(1e-12))[:, None]
+        elif dtype == "bf16":
+            stored = torch.from_numpy(level[at]).to(torch.bfloat16).view(torch.int16).numpy().view(np.uint16)
+            case["k_slab"][rows, :, 0] = stored[:, None]
+        else:
+            case["k_slab"][rows, :, 0] = level[at].astype(dtype)[:, None]
         case["k"][slot, :, :, 0] = level[len(at):len(at) + tokens]
     got = run_gpu(et, device, case, scale)
     assert et.kv_attention_kernel(got[3], 8, tokens).startswith("kv_append+kv_chunk")
