@@ -340,6 +340,27 @@ def test_prompts_on_the_wide_kernel(et, device, codec, vectors, rows, columns):
 
 
 @pytest.mark.parametrize("codec", [oracle.Q4_K, oracle.Q5_K])
+def test_prompts_of_very_small_and_large_activations(et, device, codec):
+    # the sums of a vector's activations are divided by its unit (its stage's largest magnitude / 2^23) before they are cut: units
+    # of 1e-37, of 7e-39 (no normal number: off by 2^-150 at most, 1e-7 of itself) and of 5e23
+    rng = np.random.default_rng(60 + codec)
+    rows, columns, vectors = 14336, 4096, 128
+    weight = synth.random_weight(codec, rows, columns, rng)
+    x = synth.random_activations(vectors, columns, rng)
+    x /= np.abs(x.reshape(vectors, -1, 256)).max(axis=2).repeat(256, axis=1)  # every stage's largest magnitude is 1
+    sizes = {1: 1e-30, 40: 6e-32, 70: 4e30, 127: 1e-31}
+    for row, size in sizes.items():
+        x[row] *= np.float32(size)
+    assert "gemm_h16_wide" in et.RawLinear(et.GgmlQuant(codec), rows, columns, vectors).requirements.kernel
+    got = run_linear(et, device, codec, rows, columns, x, weight, None).astype(np.float64)
+    decoded = et.dequantize_rows(to_dev(weight, device), et.GgmlQuant(codec), (rows, columns)).double()
+    exact = (to_dev(x, device).double() @ decoded.T).cpu().numpy()
+    error = np.linalg.norm(got - exact, axis=1) / np.linalg.norm(exact, axis=1)
+    # 2.5e-7 as in the test above, row by row, and 1e-7 for the unit of row 40
+    assert error.max() <= 3.5e-7, {row: error[row] for row in sizes}
+
+
+@pytest.mark.parametrize("codec", [oracle.Q4_K, oracle.Q5_K])
 def test_prompts_whose_sums_of_activations_overflow(et, device, codec):
     # 32 values of 1.2e37 add up to no f32: what the minima take away is an infinity, or a NaN where a sub-block's minimum is 0
     # (zero times infinity), of that vector alone
