@@ -17,8 +17,6 @@ namespace et {
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 typedef float v16f __attribute__((ext_vector_type(16)));
-typedef short v8s __attribute__((ext_vector_type(8)));
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 
 constexpr int kStageBlocks = 8;
 constexpr float kPlaneRatio = 4096.0f;          // what the accumulators lack: the tiles hold hi and lo / 4096
@@ -135,135 +133,6 @@ __device__ __forceinline__ v8h bytes_minus_times(uint32_t first, uint32_t second
 
 // Weight operands per sixteen columns: Q6_K splits its scale, Q2_K contracts its minima.
 constexpr int weight_parts(int codec) { return codec == kQ6_K || codec == kQ2_K ? 2 : 1; }
-
-// 1 KiB from `base` + a byte offset per lane to LDS address `to` + 16 bytes per lane.
-__device__ __forceinline__ void copy_to_lds(const uint8_t* base, uint32_t lane_offset, uint32_t to) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                 :
-                 : "s"(__builtin_amdgcn_readfirstlane(to)), "v"(lane_offset), "s"(base)
-                 : "memory");  // m0 is a reserved register: nothing else in this file sets it
-}
-
-// The packed bytes of one lane's columns 32 b + 16 half .. + 16 of a row, as they come out of LDS.
-struct Raw {
-    uint4 low, high;
-    uint32_t scale, scale_top;
-};
-// What all of a row's sub-blocks share: d, dmin and the scales (Q4_K, Q5_K); the fifth (Q5_K) or top (Q3_K) bits.
-struct Shared {
-    uint4 header, bits;
-};
-template <int CODEC>
-__device__ __forceinline__ Shared fetch_shared(const uint8_t* row, uint32_t half) {
-    Shared s = {};
-    if constexpr (CODEC == kQ4_K || CODEC == kQ5_K) s.header = *reinterpret_cast<const uint4*>(row);
-    if constexpr (CODEC == kQ5_K) s.bits = *reinterpret_cast<const uint4*>(row + 16u + 16u * half);
-    if constexpr (CODEC == kQ3_K) s.bits = *reinterpret_cast<const uint4*>(row + 16u * half);
-    return s;
-}
-template <int CODEC>
-__device__ __forceinline__ Raw fetch(const uint8_t* row, int b, uint32_t half) {
-    const uint32_t n = b >> 2, t = b & 3;
-    Raw r = {};
-    if constexpr (CODEC == kQ4_K || CODEC == kQ5_K) {
-        r.low = *reinterpret_cast<const uint4*>(row + HalfStage<CODEC>::kQuantsAt + 32u * (b >> 1) + 16u * half);
-    } else if constexpr (CODEC == kQ6_K) {
-        r.low = *reinterpret_cast<const uint4*>(row + 64u * n + 32u * (t & 1u) + 16u * half);
-        r.high = *reinterpret_cast<const uint4*>(row + 128u + 32u * n + 16u * half);
-        r.scale = row[192u + 8u * n + 2u * t + half];
-    } else if constexpr (CODEC == kQ3_K) {
-        r.low = *reinterpret_cast<const uint4*>(row + 32u + 32u * n + 16u * half);
-        r.scale = row[HalfStage<CODEC>::in_tail(96u) + 2u * t + half];
-        r.scale_top = row[HalfStage<CODEC>::in_tail(104u) + 2u * (t & 1u) + half];
-    } else {
-        r.low = *reinterpret_cast<const uint4*>(row + 16u + 32u * n + 16u * half);
-        r.scale = row[2u * b + half];
-    }
-    return r;
-}
-__device__ __forceinline__ v2h twice(int value) {
-    const _Float16 h = static_cast<_Float16>(static_cast<float>(value));
-    return v2h{h, h};
-}
-// The weight operands of those columns, eight by eight: gemm_h16_kernel's values.
-template <int CODEC>
-__device__ __forceinline__ void operands(const Raw& raw, const Shared& shared, int b, v8h out[2][weight_parts(CODEC)]) {
-    const uint32_t n = b >> 2, t = b & 3;
-    const uint32_t low[4] = {raw.low.x, raw.low.y, raw.low.z, raw.low.w}, high[4] = {raw.high.x, raw.high.y, raw.high.z, raw.high.w};
-    const uint32_t bits[4] = {shared.bits.x, shared.bits.y, shared.bits.z, shared.bits.w};
-    uint32_t w[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        if constexpr (CODEC == kQ4_K || CODEC == kQ5_K) {
-            w[i] = (low[i] >> ((b & 1) * 4)) & 0x0f0f0f0fu;
-            if constexpr (CODEC == kQ5_K) w[i] |= ((bits[i] >> b) & 0x01010101u) << 4;
-        } else if constexpr (CODEC == kQ6_K) {
-            w[i] = ((low[i] >> ((t >> 1) * 4u)) & 0x0f0f0f0fu) | (((high[i] >> (2u * t)) & 0x03030303u) << 4);
-        } else {
-            w[i] = (low[i] >> (2u * t)) & 0x03030303u;
-            if constexpr (CODEC == kQ3_K) w[i] |= ((bits[i] >> (4u * n + t)) & 0x01010101u) << 2;
-        }
-    }
-    if constexpr (CODEC == kQ4_K || CODEC == kQ5_K) {
-        uint32_t sc, mn;
-        q4k_scale_min(shared.header, b, sc, mn);
-        const v2h scale = twice(sc);
-        if (CODEC == kQ4_K && (b & 1)) {
-            out[0][0] = packed_nibbles_times<true>(low[0], low[1], scale);
-            out[1][0] = packed_nibbles_times<true>(low[2], low[3], scale);
-        } else if (CODEC == kQ4_K) {
-            out[0][0] = packed_nibbles_times<false>(low[0], low[1], scale);
-            out[1][0] = packed_nibbles_times<false>(low[2], low[3], scale);
-        } else {
-            out[0][0] = nibbles_times(w[0], w[1], scale);
-            out[1][0] = nibbles_times(w[2], w[3], scale);
-        }
-    } else if constexpr (CODEC == kQ6_K) {
-        const int sc = static_cast<int8_t>(raw.scale);
-        const v2h scale_low = twice(sc & 15), scale_high = twice(sc >> 4);
-        out[0][0] = nibbles_times<32>(w[0], w[1], scale_low);
-        out[1][0] = nibbles_times<32>(w[2], w[3], scale_low);
-        out[0][1] = nibbles_times<32>(w[0], w[1], scale_high);
-        out[1][1] = nibbles_times<32>(w[2], w[3], scale_high);
-    } else if constexpr (CODEC == kQ3_K) {
-        const int sc = static_cast<int>(((raw.scale >> (4u * n)) & 15u) |
-                                        (((raw.scale_top >> (2u * (2u * n + (t >> 1)))) & 3u) << 4)) - 32;
-        const v2h scale = twice(sc);
-        out[0][0] = bytes_minus_times<4>(w[0], w[1], scale);
-        out[1][0] = bytes_minus_times<4>(w[2], w[3], scale);
-    } else {
-        const v2h scale = twice(raw.scale & 15u), m = twice(raw.scale >> 4);
-        out[0][0] = nibbles_times(w[0], w[1], scale);
-        out[1][0] = nibbles_times(w[2], w[3], scale);
-        out[0][1] = out[1][1] = v8h{m.x, m.x, m.x, m.x, m.x, m.x, m.x, m.x};
-    }
-}
-
-// f32 bits as three bfloat16 numbers that add up to it, eight significant bits each: the top halves of `x`, of
-// what is left of it, and of what is left then (nothing is lost above 2^-110). Of an infinity nothing is left.
-struct Pieces {
-    uint32_t high, mid, low;  // in the upper sixteen bits
-};
-__device__ __forceinline__ Pieces cut(float x) {
-    Pieces p;
-    p.high = __float_as_uint(x) & 0xffff0000u;
-    const float rest = __builtin_isinf(x) ? 0.f : x - __uint_as_float(p.high);
-    p.mid = __float_as_uint(rest) & 0xffff0000u;
-    p.low = __float_as_uint(rest - __uint_as_float(p.mid));
-    return p;
-}
-__device__ __forceinline__ v8bf as_bf16(const v8s& bits) { return __builtin_bit_cast(v8bf, bits); }
-// The eight minima of this lane's row, against the high (lane half 0) and middle pieces, and against the low ones
-// (half 0 alone: the operand's other eight columns are zero).
-__device__ __forceinline__ void minimum_operands(const uint4& header, uint32_t half, v8s out[2]) {
-#pragma unroll
-    for (uint32_t g = 0; g < kStageBlocks; g++) {
-        uint32_t sc, mn;
-        q4k_scale_min(header, g, sc, mn);
-        out[0][g] = static_cast<short>(__float_as_uint(static_cast<float>(mn)) >> 16);  // at most 63: exact
-    }
-    out[1] = half == 0 ? out[0] : v8s{0, 0, 0, 0, 0, 0, 0, 0};
-}
 
 // The matrices of one launch: contractions that share their activations (the q / k / v projections
 // of a decode step) run as one grid over the row tiles of all of them.
