@@ -2,26 +2,32 @@
 // vectors with 256 weight rows (Q2_K, Q6_K: 128), so that weights are unpacked once for 128 (64) vectors instead of for
 // every 32, and an activation tile is copied for 256 rows instead of 64 or 128.
 //
-// Bound: the matrix pipe, at the clock that its power leaves. Eight waves, two per SIMD, each 128 vectors x 32 rows (Q2_K,
-// Q6_K, which contract two operands per weight: 64 x 32). A Q4_K wave's stage of 256 columns is 128 half-float matrix
-// instructions, eight bfloat16 ones for the minima (32 cycles each) and about 520 vector instructions. With two waves on a SIMD
-// up to seven vector instructions (of four cycles) run in the shadow of each matrix instruction (measured in loops of both; with
-// one wave four do), so what counts is how evenly they lie between them: the next sub-block's operands are made between
-// this one's matrix instructions, and a stage's sums are folded into the accumulators tile by tile between the next tile's.
-// The minima were f32 matrix instructions (16 of 64 cycles per stage, a fifth of the pipe's time); now the sums of a
-// sub-block, in units of the vector whole numbers of up to 28 bits, are cut into three bfloat16 pieces once per workgroup, and the products are exact.
-// Both steps, 14336 x 4096 with 1000 vectors: 289 -> 253 us, clocks of busy compute units 122.5 -> 99.6 million, of which matrix
-// instructions 60 -> 63 %; the nibbles' eight instructions less per sub-block (packed_nibbles_times) 5 % more. The clock falls from 2.02 to 1.93 GHz on the way: a loop of these instructions alone holds 1.75 GHz on
-// random operands (2.1 on zeros). Without any copies 7 % less; 448 workgroups on 256 compute units leave an eighth of them idle.
+// Bound: matrix instructions together with the LDS reads of their operands. Eight waves, two per SIMD, each 128 vectors x 32 rows
+// (Q2_K, Q6_K, which contract two operands per weight: 64 x 32). A Q4_K wave's stage of 256 columns is 128 half-float matrix
+// instructions, eight bfloat16 ones for the minima (32 cycles each), 165 LDS instructions, as an activation operand (16 bytes a
+// lane, about eight cycles of the compute unit's LDS) serves one matrix instruction, and about 520 vector instructions. 14336 x
+// 4096 with 1000 vectors: 240 us, 27.6 ns per matrix instruction of a SIMD, matrix pipes busy 68 % of the cycles of busy compute units at 1.93
+// GHz. Loops on random operands, two waves per SIMD: matrix instructions alone 21.3 ns (zeros 14.3: their power takes the
+// clock down), with six, ten and twelve LDS reads to ten of them 25.0, 27.5 and 30.8. Left: operands that serve two matrix
+// instructions (64 x 64 per wave, every weight unpacked twice), and 448 workgroups on 256 compute units, an eighth of them idle.
+// Vector instructions, up to seven for a matrix instruction, cost next to nothing where they lie evenly between them (loops of
+// both, two waves per SIMD): the next sub-block's operands are made between this one's matrix instructions, and a stage's sums
+// are folded into the accumulators tile by tile between the next tile's. The minima were f32 matrix instructions (16 of 64
+// cycles per stage, a fifth of the pipe's time); now a sub-block's sum, an f32, is divided by the vector's unit and the
+// quotient, rounded to 24 bits, is cut into three bfloat16 pieces that add up to it exactly, once per workgroup; their products are
+// exact. Clocks of busy compute units before these steps, with them, and with the nibbles' eight instructions less per sub-block
+// (packed_nibbles_times): 122.5, 99.6 and 92.2 million.
 // Every wave unpacks its own weight rows from the packed bytes in LDS. There are no loader waves (a third wave per SIMD
 // would leave 168 registers each): the waves ask for the next sub-blocks' activations and the next stage's weights
 // themselves, through inline assembly, because any LDS read next to a copy that the compiler can see waits for it.
+// Q4_K and Q5_K have all 256 registers and spill 12 and 16, in the last stage and the stores.
 //
-// Whole calls (us, gemm_h16_kernel / this before / this): 14336 x 4096 with 1000 vectors Q4_K 420 / 289 / 259 (454 TFLOP/s), Q5_K
-// 453 / 296 / 265, Q6_K 724 / 481 / 438, Q3_K 415 / 259 / 246, Q2_K 512 / 429 / 398; Q4_K 4096 x 14336 with 1000 396 / 274 / 256,
-// 14336 x 4096 with 256 115 / 93 / 90.
-// Relative error against 64 bits there (2-norm, 1e-7): Q4_K 1.75 / 1.69 / 1.66, Q6_K 1.66 / 1.63 / 1.63, Q2_K 1.84 / 1.76 / 1.76: one chain of
-// sums over the stage's eight sub-blocks instead of two or four, from activations that are rounded less (quantize_halves.h).
+// Whole calls (us, gemm_h16_kernel / this before those steps / this): 14336 x 4096 with 1000 vectors Q4_K 415 / 294 / 259 (453
+// TFLOP/s), Q5_K 445 / 301 / 266, Q6_K 730 / 474 / 437, Q3_K 434 / 268 / 254, Q2_K 534 / 426 / 399; Q4_K 4096 x 14336 with 1000
+// 390 / 293 / 266, 14336 x 4096 with 256 121 / 95 / 88. In launches of one stage per workgroup the separate last stage is no gain: Q6_K
+// 622 x 3584 with 371 vectors 42.0 / 34.3 / 35.2 (one loop for all stages: 35.7, and 1000 vectors 447 instead of 418).
+// Relative error against 64 bits there (2-norm, 1e-7): Q4_K 1.75 / 1.69 / 1.66, Q6_K 1.66 / 1.63 / 1.63, Q2_K 1.84 / 1.76 / 1.76:
+// one chain of sums over the stage's eight sub-blocks instead of two or four, from activations that are rounded less (quantize_halves.h).
 #include <hip/hip_runtime.h>
 
 #include <atomic>
@@ -266,7 +272,8 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_h16_wide_kernel(const Gro
     };
 
     // Between the barriers of sub-blocks kCutAt and kCutAt + 1 every thread reads and cuts the sums of two sub-blocks of one
-    // vector, in units of the vector (pieces of numbers around 10^-35 would not be normal), behind the second one the pieces take the sums' place; they are read in the last sub-block.
+    // vector, in units of the vector (pieces of numbers around 10^-35 would not be normal); behind the second one the
+    // pieces take the sums' place; they are read in the last sub-block.
     uint32_t piece[3];
     const uint32_t cut_vector = threadIdx.x & 31u, cut_group = ((threadIdx.x >> 5) & 3u) * 2u;
     const auto cut_sums = [&] {
