@@ -42,6 +42,9 @@
 // position one tile ahead and handed out with ds_bpermute; two LDS offsets per lane, from which every operand's address is
 // one exclusive or; a row's maximum that is followed to within kSlack. Before these three, and now (us): two slots of 500 at
 // 2000 96.7 / 93.4, bf16 115.3 / 106.2, u8 127.1 / 121.2, at 8000 289 / 280 (the streaming kernel took 1036, 1097 and 1322).
+// The f16 kernel of four row waves and width 128, alone among the twelve, needs nine registers more than the 256: four of them, a query
+// operand, are reloaded at the head of every tile's contraction, and the wait for them is one for the next tile's copies, too,
+// which have just been asked for. (Before the three changes one was, with the same wait, and the u8 and bf16 kernels had such reloads.)
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 
