@@ -279,8 +279,8 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_h16_wide_kernel(const Gro
     const auto cut_sums = [&] {
         const float* sums = reinterpret_cast<const float*>(lds + W::kSumsAt + (wave >> 1) * 1024u) + cut_group * 32u + cut_vector;
         const float unit = *reinterpret_cast<const float*>(lds + W::kUnitsAt + (wave >> 1) * 128u + cut_vector * 4u);
-        const auto whole = [&](float sum) { return unit != 0.f ? sum / unit : 0.f; };
-        const Pieces a = cut(whole(sums[0])), b = cut(whole(sums[32]));
+        const auto in_units = [&](float sum) { return unit != 0.f ? sum / unit : 0.f; };
+        const Pieces a = cut(in_units(sums[0])), b = cut(in_units(sums[32]));
         piece[0] = __builtin_amdgcn_perm(b.high, a.high, 0x07060302u);
         piece[1] = __builtin_amdgcn_perm(b.mid, a.mid, 0x07060302u);
         piece[2] = __builtin_amdgcn_perm(b.low, a.low, 0x07060302u);
